@@ -1,12 +1,26 @@
-// fp32 tile arithmetic: BM x BN x 16 CTA tile (128 x 128 on 2 x 2 waves; 32 x 256 on 1 x 4 waves for small M),
-// v_mfma_f32_32x32x2_f32.
+// fp32 tile arithmetic on v_mfma_f32_16x16x4_f32: B as [K,N] (the reference's layout, streamk_fp32.py:74) or [N,K].
+// Replaces the T.gemm of the reference's fp32 kernel (streamk_fp32.py:109-125).
 //
-// Replaces the T.gemm of the reference's fp32 kernel (streamk_fp32.py:109-125).  B may be [K,N]
-// (the reference's layout, streamk_fp32.py:74) or [N,K].
+// An fp32 MFMA takes 32 cycles for 2048 FLOP, so the LDS reads of even a 32 x 32 wave tile are a third of the LDS
+// bandwidth: what bounds these kernels is the matrix pipe (157 TFLOP/s) for many rows of A and the stream of B from HBM
+// for few.  Both want the same thing, loads far ahead of their use without registers to hold them: a ring of STAGES
+// slots of BK K-values of A and B, filled by direct global -> LDS loads (16 bytes per lane), one wait (vmcnt, in order)
+// and one barrier per iteration, STAGES - 1 iterations in flight.  Tile shapes differ in how many CTAs a problem gives:
+// 128 x 128 where that fills the device, 64 x 64 / 64 x 128 where it does not or M <= 64, 32 x 64 / 32 x 256 for
+// M <= 32 (see the planner's kFamiliesF32).  Measured (B [K,N], weights from HBM) against the register-staged two-slot
+// kernels this replaced, in us: 16 x 16384 x 8192 120 -> 92 (5.8 TB/s), 16 x 4096 x 4096 59.8 -> 20.7, 64 x 4096 x 4096
+// 97 -> 28, 256 x 1024 x 512 23.1 -> 10.0, 512 x 4096 x 4096 163 -> 133, 4096^3 1019 -> 961 (143 TFLOP/s); as [N,K]
+// 149 -> 97, 64.8 -> 20.2, 98 -> 28, 23.4 -> 10.8, 167 -> 131, 1061 -> 933 (147 TFLOP/s).
 //
-// One MFMA multiplies a 32 x 2 slice: lane (r = lane%32, g = lane/32) supplies A[r][k_g].  A lane
-// reads four consecutive K of its row in one 16-byte LDS access and feeds them to four MFMAs, so
-// MFMA e of an 8-wide K step contracts K = {e, 4 + e}; the B operand follows the same rule.
+// LDS layout of a slot: BM rows of A of BK * 4 bytes, then B: [N,K] BN rows like A's, [K,N] BK rows of BN * 4 bytes.
+// 16-byte piece p of a row of 4 / 8 / 16 pieces is kept at position p ^ swizzle(row) ((row >> 2) & 3, (row >> 1) & 7,
+// row & 15: the 16 lanes served together read 16 rows on distinct banks); piece p of K-row k of a [K,N] stage at
+// p ^ 4 ((k >> 2) & 3): the four lane groups of a fragment read, four K-rows apart, fall on the four 64-byte quarters of
+// the 64 banks.
+//
+// Fragments: lane (i = lane % 16, g = lane / 16) takes piece 4 s + g of its row for K-step s of 16, four consecutive
+// K-values, and feeds them to four MFMAs: MFMA e contracts K = 16 s + {e, 4 + e, 8 + e, 12 + e}; from a [K,N] stage it reads the
+// same four K-values of its column one by one.
 #pragma once
 #include "sk_device.h"
 
@@ -20,183 +34,227 @@ struct GemmArgsF32 {
   int64_t lda, ldb, ldc;
 };
 
-template <bool B_KN_, int BM_ = 128, int BN_ = 128, int WM_ = 2, int WN_ = 2>
+template <bool B_KN_, int BM_, int BN_, int BK_, int WM_, int WN_, int STAGES_, int CTAS_>
 struct TileF32 {
   typedef GemmArgsF32 Args;
-  static constexpr bool LEAN_ENTRY = true;  // see run_persistent
+  static constexpr bool LEAN_ENTRY = true;            // see run_persistent
+  static constexpr bool COHERENT_PARTIALS = true;     // partials travel with device-scope accesses
+  static constexpr bool FIXUP_WORD_IN_LDS = true;     // the ring is dead between two calls of mac
   static constexpr bool B_KN = B_KN_;
-  static constexpr int BM = BM_, BN = BN_, BK = 16, WM = WM_, WN = WN_;
-  static constexpr int NT = 256, TM = BM / (WM * 32), TN = BN / (WN * 32), WTM = TM * 32, WTN = TN * 32;
-  static_assert(WM * WN == 4 && BM % (WM * 32) == 0 && BN % (WN * 32) == 0 && BN % 64 == 0, "tile shape");
-  static constexpr int LDA = BK + 4;                 // floats per LDS row of A (and of B when [N,K])
-  static constexpr int LDB = B_KN ? BN + 8 : BK + 4; // floats per LDS row of B
-  static constexpr int A_STAGE = BM * LDA, B_STAGE = B_KN ? BK * LDB : BN * LDB, STAGE = A_STAGE + B_STAGE;
-  static constexpr int LDS_BYTES = 2 * STAGE * 4, LDS_TOTAL = LDS_BYTES;
-  static constexpr int TILE_ELEMS = BM * BN, NV4 = TM * TN * 4;
-  static constexpr int CTAS_PER_CU = 2, WAVES_PER_EU = 2;
-  static constexpr bool COHERENT_PARTIALS = false;
-  // 16-byte loads per thread: a pass of the 256 threads covers 64 rows of 16 K-values (A, and B as
-  // [N,K]) or 1024 / BN K-rows of BN values (B as [K,N])
-  static constexpr int A_LOADS = (BM + 63) / 64, B_LOADS = BN * BK / 4 / NT;
-  static constexpr int B_CPR = BN / 4, B_RPP = NT / B_CPR;  // [K,N]: chunks per K-row, K-rows per pass
+  static constexpr int BM = BM_, BN = BN_, BK = BK_, WM = WM_, WN = WN_, S = STAGES_;
+  static constexpr int NT = 256, FM = BM / (WM * 16), FN = BN / (WN * 16), STEPS = BK / 16;
+  static_assert(WM * WN == 4 && BM % (WM * 16) == 0 && BN % (WN * 16) == 0 && BN % 64 == 0, "tile shape");
+  static_assert(BK == 16 || BK == 32 || BK == 64, "rows of 4, 8 or 16 pieces");
+  static constexpr int ROW = BK * 4, PR = BK / 4;             // bytes / 16-byte pieces of an LDS row along K
+  static constexpr int A_BYTES = BM * ROW, B_BYTES = BN * ROW, SLOT = A_BYTES + B_BYTES;
+  static constexpr int NA = A_BYTES / 1024, NB = B_BYTES / 1024;  // wave-wide loads of a slot
+  // (a slot of A may hold fewer loads than there are waves: the other waves repeat them, which keeps the counts equal)
+  static constexpr int LA = NA >= 4 ? NA / 4 : 1, LB = NB / 4, LOADS = LA + LB;
+  static_assert((NA % 4 == 0 || 4 % NA == 0) && NB % 4 == 0, "the loads are shared out evenly");
+  static constexpr int LDS_BYTES = S * SLOT, LDS_TOTAL = LDS_BYTES;
+  static_assert(LDS_BYTES * CTAS_ <= 160 * 1024, "the rings must fit the LDS of a CU");
+  static constexpr int CTAS_PER_CU = CTAS_, WAVES_PER_EU = CTAS_;
+  static constexpr int TILE_ELEMS = BM * BN, NV4 = FM * FN;
+  static constexpr int OUTSTANDING = (S - 2) * LOADS;
 
+  // c[i][j][e] = C[pm*BM + (wm*FM + i)*16 + lane%16][pn*BN + (wn*FN + j)*16 + 4*(lane/16) + e]
   struct Acc {
-    floatx16 c[TM][TN];
+    floatx4 c[FM][FN];
   };
 
+  static __device__ __forceinline__ int swizzle(int row) {
+    return PR == 4 ? (row >> 2) & 3 : (PR == 8 ? (row >> 1) & 7 : row & 15);
+  }
+
   static __device__ __forceinline__ void mac(const Args &a, Acc &acc, int pm, int pn, int k0, int n, char *smem) {
-    float *lds = reinterpret_cast<float *>(smem);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int wm = wave / WN, wn = wave % WN;
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc.c[i][j][r] = 0.f;
+      for (int j = 0; j < FN; ++j) acc.c[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    // ---- global addressing (buffer descriptors: rows past the matrix read as zero) ----
+    // ---- descriptors: rows past M / N and K-rows past K read as zero ----
     const int rows_a = min(BM, a.M - pm * BM), cols_b = min(BN, a.N - pn * BN);
-    const BufferRsrc rsrc_a = make_rsrc(a.A + (int64_t)pm * BM * a.lda, (uint32_t)(rows_a * a.lda * 4));
-    const int a_row = tid / 4, a_c = tid % 4;  // 4 chunks of 4 floats per K-row of 16
-    const uint32_t voff_a = (BM % 64 == 0 || a_row < BM) ? (uint32_t)(a_row * a.lda + a_c * 4) * 4 : OOB_OFFSET;
-    const uint32_t pass_a = (uint32_t)(64 * a.lda * 4);
-    BufferRsrc rsrc_b;
-    uint32_t voff_b, pass_b, kstep_b;
-    int b_st;  // LDS float offset of this thread's first B chunk
-    if (!B_KN) {
-      rsrc_b = make_rsrc(a.B + (int64_t)pn * BN * a.ldb, (uint32_t)(cols_b * a.ldb * 4));
-      voff_b = (uint32_t)(a_row * a.ldb + a_c * 4) * 4;
-      pass_b = (uint32_t)(64 * a.ldb * 4);
-      kstep_b = BK * 4;
-      b_st = a_row * LDB + a_c * 4;
-    } else {
-      rsrc_b = make_rsrc(a.B + (int64_t)pn * BN, (uint32_t)(((int64_t)(a.K - 1) * a.ldb + cols_b) * 4));
-      const int k_row = tid / B_CPR, c = tid % B_CPR;
-      voff_b = (c * 4 < cols_b) ? (uint32_t)(k_row * a.ldb + c * 4) * 4 : OOB_OFFSET;
-      pass_b = (uint32_t)(B_RPP * a.ldb * 4);
-      kstep_b = (uint32_t)(BK * a.ldb * 4);
-      b_st = k_row * LDB + c * 4;
-    }
-    const int a_st = a_row * LDA + a_c * 4;
-    const int tail_kt = (a.K % BK != 0) ? (a.K / BK) : -1;
+    const uint32_t lda_bytes = (uint32_t)a.lda * 4, ldb_bytes = (uint32_t)a.ldb * 4;
+    const uint4v rsrc_a = uniform_rsrc(make_rsrc_words(a.A + (int64_t)pm * BM * a.lda, (uint32_t)rows_a * lda_bytes));
+    const uint4v rsrc_b = uniform_rsrc(
+        B_KN ? make_rsrc_words(a.B + (int64_t)pn * BN, (uint32_t)(((int64_t)(a.K - 1) * a.ldb + cols_b) * 4))
+             : make_rsrc_words(a.B + (int64_t)pn * BN * a.ldb, (uint32_t)cols_b * ldb_bytes));
 
-    uint4v ra[A_LOADS], rb[B_LOADS];
-    auto load_global = [&](int kt) {
-      uint32_t va = voff_a, vb = voff_b;
-      if (kt == tail_kt && kt * BK + a_c * 4 >= a.K) {
-        va = OOB_OFFSET;
-        if (!B_KN) vb = OOB_OFFSET;
+    // ---- this lane's source of each of its wave's loads: byte offset at K = 0 and its K-values (for the K tail) ----
+    uint32_t off_a[LA], off_b[LB];
+    int ka[LA], kb[LB];
+#pragma unroll
+    for (int j = 0; j < LA; ++j) {
+      const int x = ((wave * LA + j) % NA) * 64 + lane, row = x / PR, piece = (x % PR) ^ swizzle(row);
+      off_a[j] = (uint32_t)row * lda_bytes + (uint32_t)piece * 16;
+      ka[j] = piece * 4;
+    }
+#pragma unroll
+    for (int j = 0; j < LB; ++j) {
+      const int x = (wave * LB + j) * 64 + lane;
+      if constexpr (B_KN) {
+        const int k = x / (BN / 4), piece = (x % (BN / 4)) ^ (4 * ((k >> 2) & 3));
+        off_b[j] = piece * 4 < cols_b ? (uint32_t)k * ldb_bytes + (uint32_t)piece * 16 : OOB_OFFSET;
+        kb[j] = 0;   // (K-rows past K lie past the descriptor's end)
+      } else {
+        const int row = x / PR, piece = (x % PR) ^ swizzle(row);
+        off_b[j] = (uint32_t)row * ldb_bytes + (uint32_t)piece * 16;
+        kb[j] = piece * 4;
       }
+    }
+    // one row of tiles over [N,K] weights: every tile starts K at a different offset (see rotation_of)
+    const int rot = (!B_KN && a.M <= BM) ? rotation_of(pn, n) : 0;
+    const uint32_t base = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_address(smem));
+    auto issue = [&](int t, int slot) {
+      const int kk = (k0 + rotated_iteration(t, rot, n)) * BK;
+      const uint32_t kbytes = (uint32_t)__builtin_amdgcn_readfirstlane(kk * 4);
+      const uint32_t kb_bytes = B_KN ? (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)kk * ldb_bytes)) : kbytes;
+      const uint32_t dst = base + (uint32_t)(slot * SLOT);
+      if (t < n && kk + BK <= a.K) {
 #pragma unroll
-      for (int i = 0; i < A_LOADS; ++i) ra[i] = buffer_load_16(rsrc_a, va, (uint32_t)kt * (BK * 4) + i * pass_a);
+        for (int j = 0; j < LB; ++j) dma_load_16(rsrc_b, dst + A_BYTES + (uint32_t)(wave * LB + j) * 1024, off_b[j], kb_bytes);
 #pragma unroll
-      for (int i = 0; i < B_LOADS; ++i) rb[i] = buffer_load_16(rsrc_b, vb, (uint32_t)kt * kstep_b + i * pass_b);
+        for (int j = 0; j < LA; ++j) dma_load_16(rsrc_a, dst + (uint32_t)((wave * LA + j) % NA) * 1024, off_a[j], kbytes);
+      } else {
+        // the K tail, and iterations past the segment: nothing is fetched for K-values past the end (zeros arrive)
+        const int left = t < n ? a.K - kk : 0;
+#pragma unroll
+        for (int j = 0; j < LB; ++j)
+          dma_load_16(rsrc_b, dst + A_BYTES + (uint32_t)(wave * LB + j) * 1024, kb[j] < left ? off_b[j] : OOB_OFFSET, kb_bytes);
+#pragma unroll
+        for (int j = 0; j < LA; ++j)
+          dma_load_16(rsrc_a, dst + (uint32_t)((wave * LA + j) % NA) * 1024, ka[j] < left ? off_a[j] : OOB_OFFSET, kbytes);
+      }
     };
 
-    const int a_rd = (wm * WTM + (lane & 31)) * LDA + (lane >> 5) * 4;
-    const int b_rd = B_KN ? A_STAGE + (lane >> 5) * 4 * LDB + wn * WTN + (lane & 31)
-                          : A_STAGE + (wn * WTN + (lane & 31)) * LDB + (lane >> 5) * 4;
-
-    load_global(k0);
-    for (int it = 0; it < n; ++it) {
-      float *st = lds + (it & 1) * STAGE;
+    // ---- fragment addresses ----
+    const int fi = lane & 15, fg = lane >> 4;
+    int rd_a[STEPS], rd_b[STEPS], rd_bt[FN];
 #pragma unroll
-      for (int i = 0; i < A_LOADS; ++i)
-        if (BM % 64 == 0 || a_row + i * 64 < BM) *reinterpret_cast<uint4v *>(st + a_st + i * 64 * LDA) = ra[i];
+    for (int s = 0; s < STEPS; ++s) {
+      const int pos = ((4 * s + fg) ^ swizzle(fi)) * 16;
+      rd_a[s] = (wm * FM * 16 + fi) * ROW + pos;
+      rd_b[s] = A_BYTES + (wn * FN * 16 + fi) * ROW + pos;
+    }
+    if constexpr (B_KN) {
 #pragma unroll
-      for (int i = 0; i < B_LOADS; ++i)
-        *reinterpret_cast<uint4v *>(st + A_STAGE + b_st + i * (B_KN ? B_RPP * LDB : 64 * LDB)) = rb[i];
-      __syncthreads();
-      if (it + 1 < n) load_global(k0 + it + 1);
+      for (int j = 0; j < FN; ++j) rd_bt[j] = A_BYTES + (4 * fg * BN + ((16 * (wn * FN + j) + fi) ^ (16 * fg))) * 4;
+    }
+    auto compute = [&](const char *st, auto rows_active) {
+      constexpr int FMA = decltype(rows_active)::value;
 #pragma unroll
-      for (int kk = 0; kk < BK / 8; ++kk) {
-        floatx4 fa[TM], fb[TN];
+      for (int s = 0; s < STEPS; ++s) {
+        floatx4 fa[FMA], fb[FN];
 #pragma unroll
-        for (int i = 0; i < TM; ++i) fa[i] = *reinterpret_cast<const floatx4 *>(st + a_rd + i * 32 * LDA + kk * 8);
+        for (int i = 0; i < FMA; ++i) fa[i] = *reinterpret_cast<const floatx4 *>(st + rd_a[s] + i * 16 * ROW);
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          if (!B_KN) {
-            fb[j] = *reinterpret_cast<const floatx4 *>(st + b_rd + j * 32 * LDB + kk * 8);
+        for (int j = 0; j < FN; ++j) {
+          if constexpr (B_KN) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) fb[j][e] = *reinterpret_cast<const float *>(st + rd_bt[j] + (16 * s + e) * BN * 4);
           } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) fb[j][e] = st[b_rd + (kk * 8 + e) * LDB + j * 32];
+            fb[j] = *reinterpret_cast<const floatx4 *>(st + rd_b[s] + j * 16 * ROW);
           }
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
-          for (int i = 0; i < TM; ++i)
+          for (int i = 0; i < FMA; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
-              acc.c[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][e], fb[j][e], acc.c[i][j], 0, 0, 0);
+            for (int j = 0; j < FN; ++j)
+              acc.c[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[j][e], fa[i][e], acc.c[i][j], 0, 0, 0);
       }
+    };
+
+#pragma unroll
+    for (int j = 0; j < S - 1; ++j) issue(j, j);
+    int slot = 0;
+    // (M <= 16 on a tile of 32 rows: the second block of rows is left out)
+    const bool half = FM == 2 && WM == 1 && a.M <= 16;
+    for (int t = 0; t < n; ++t) {   // (n is the same for every wave of the CTA: the barriers stay matched)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(OUTSTANDING) : "memory");
+      __syncthreads();   // everybody's loads of the iteration have landed; everybody has read the slot refilled next
+      issue(t + S - 1, slot == 0 ? S - 1 : slot - 1);
+      const char *st = smem + slot * SLOT;
+      if (FM == 2 && WM == 1 && half)
+        compute(st, std::integral_constant<int, 1>{});
+      else
+        compute(st, std::integral_constant<int, FM>{});
+      // the fragments are in registers before the next barrier hands the slot back to the loads
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      slot = slot + 1 == S ? 0 : slot + 1;
     }
+    // the loads still in flight (they fetch nothing) write LDS: let them land before the ring is reused
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
   }
 
-  // acc.c[i][j][r] = C[pm*BM + wm*WTM + i*32 + 8*(r/4) + 4*(lane/32) + r%4][pn*BN + wn*WTN + j*32 + lane%32]
   static __device__ __forceinline__ void store_c(const Args &a, const Acc &acc, int pm, int pn, char *,
                                                  const void * /*bias: not offered for fp32*/) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wm = wave / WN, wn = wave % WN;
+    const bool vec_ok = (a.ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(a.C) & 15) == 0);
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < FM; ++i) {
+      const int row = pm * BM + (wm * FM + i) * 16 + (lane & 15);
+      if (row >= a.M) continue;
 #pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int col = pn * BN + wn * WTN + j * 32 + (lane & 31);
+      for (int j = 0; j < FN; ++j) {
+        const int col = pn * BN + (wn * FN + j) * 16 + 4 * (lane >> 4);
+        float *dst = a.C + (int64_t)row * a.ldc + col;
+        if (vec_ok && col + 4 <= a.N) {
+          *reinterpret_cast<floatx4 *>(dst) = acc.c[i][j];
+        } else {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int row = pm * BM + wm * WTM + i * 32 + 8 * (r / 4) + 4 * (lane >> 5) + (r % 4);
-          if (row < a.M && col < a.N) a.C[(int64_t)row * a.ldc + col] = acc.c[i][j][r];
+          for (int e = 0; e < 4; ++e)
+            if (col + e < a.N) dst[e] = acc.c[i][j][e];
         }
       }
+    }
   }
 
-  static __device__ __forceinline__ floatx4 grp(const Acc &acc, int v) {
-    const floatx16 &c = acc.c[(v / 4) / TN][(v / 4) % TN];
-    const int q = (v % 4) * 4;
-    return floatx4{c[q], c[q + 1], c[q + 2], c[q + 3]};
-  }
+  // Partial tiles: block v = i FN + j of thread t at (v NT + t) 4; the accumulating form keeps element e of it at
+  // (v 4 + e) NT + t.  Every access is of device scope (write-through stores, loads that bypass the XCD's L2): no CTA
+  // writes back or invalidates an L2 (128 x 128 tiles split in four used to spend 40 us on that).
   static __device__ __forceinline__ void store_partial(const Acc &acc, float *dst) {
-    dst = pin_here(dst);
+    const BufferRsrc r = make_rsrc(dst, TILE_ELEMS * 4);
 #pragma unroll
     for (int v = 0; v < NV4; ++v)
-      *reinterpret_cast<floatx4 *>(dst + ((size_t)v * NT + threadIdx.x) * 4) = grp(acc, v);
+      st_coherent16(r, threadIdx.x * 16, v * NT * 16, __builtin_bit_cast(uint4v, acc.c[v / FN][v % FN]));
   }
   static __device__ __forceinline__ void add_partial(Acc &acc, const float *src) {
-    src = pin_here(src);
+    const BufferRsrc r = make_rsrc(src, TILE_ELEMS * 4);
+    constexpr int GROUP = NV4 < 16 ? NV4 : 16;   // loads in flight before their sums
 #pragma unroll
-    for (int v = 0; v < NV4; ++v) {
-      floatx4 x = *reinterpret_cast<const floatx4 *>(src + ((size_t)v * NT + threadIdx.x) * 4);
-      floatx16 &c = acc.c[(v / 4) / TN][(v / 4) % TN];
-      const int q = (v % 4) * 4;
+    for (int v0 = 0; v0 < NV4; v0 += GROUP) {
+      floatx4 x[GROUP];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) c[q + e] += x[e];
+      for (int v = 0; v < GROUP; ++v)
+        x[v] = __builtin_bit_cast(floatx4, ld_coherent16(r, threadIdx.x * 16, (v0 + v) * NT * 16));
+#pragma unroll
+      for (int v = 0; v < GROUP; ++v) acc.c[(v0 + v) / FN][(v0 + v) % FN] += x[v];
     }
   }
   static __device__ __forceinline__ void atomic_partial(const Acc &acc, float *dst) {
     dst = pin_here(dst);
 #pragma unroll
-    for (int v = 0; v < NV4; ++v) {
-      floatx4 x = grp(acc, v);
+    for (int v = 0; v < NV4; ++v)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) atomic_add_f32(dst + (size_t)(v * 4 + e) * NT + threadIdx.x, x[e]);
-    }
+      for (int e = 0; e < 4; ++e) atomic_add_f32(dst + (size_t)(v * 4 + e) * NT + threadIdx.x, acc.c[v / FN][v % FN][e]);
   }
   static __device__ __forceinline__ void take_partial(Acc &acc, float *src) {
     src = pin_here(src);
 #pragma unroll
-    for (int v = 0; v < NV4; ++v) {
-      floatx16 &c = acc.c[(v / 4) / TN][(v / 4) % TN];
-      const int q = (v % 4) * 4;
+    for (int v = 0; v < NV4; ++v)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         float *p = src + (size_t)(v * 4 + e) * NT + threadIdx.x;
-        c[q + e] = *p;
-        *p = 0.f;
+        acc.c[v / FN][v % FN][e] = ld_coherent_scalar(p);
+        st_coherent(p, 0.f);
       }
-    }
   }
 };
 

@@ -2382,3 +2382,30 @@ def test_autotune_search_and_cache(sk, oracle, tmp_path):
     with pytest.raises(RuntimeError):
         at.autotune(200, 512, 1024, "float16", "nt", configs=[dict(bm=48, bn=48, bk=64)], cache=False)
     sk.workspace_status()
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt"])
+@pytest.mark.parametrize("bm,bn", [(32, 64), (32, 256), (64, 64), (64, 128), (128, 128)])
+def test_fp32_tile_edges(sk, bm, bn, layout):
+    """Every fp32 tile around the edges of its rows, columns and K-iterations: integer operands keep every partial sum
+    exact, so C must equal the host product.  A's rows are followed by NaN (a K tail must not read past K), C's columns
+    by a marker (an edge tile must not write past N)."""
+    import torch
+    rng = np.random.default_rng(bm * 1000 + bn)
+    for M in (1, 16, 17, bm - 1, bm + 1, 2 * bm):
+        for N, K in ((bn, 16), (bn - 4, 60), (bn + 4, 68), (3 * bn + 8, 260), (2 * bn, 4)):
+            A = rng.integers(-4, 5, (M, K)).astype(np.float32)
+            B = rng.integers(-4, 5, (K, N)).astype(np.float32)
+            Ap = torch.full((M, K + 4), float("nan"), device="cuda")
+            Ap[:, :K] = _t(A)
+            Bt = _t(B if layout == "nn" else np.ascontiguousarray(B.T))
+            Cp = torch.full((M, N + 4), 7.0, device="cuda")
+            for sch in (dict(schedule="dp"), dict(schedule="basic", grid=3), dict(schedule="basic", grid=5, fixup="atomic")):
+                if sch["schedule"] == "basic" and sch["grid"] > -(-M // bm) * -(-N // bn) * -(-K // 64):
+                    continue   # (a CTA keeps at least one iteration)
+                Cp.fill_(7.0)
+                sk.streamk_fp32(Ap[:, :K], Bt, layout=layout, out=Cp[:, :N], bm=bm, bn=bn, **sch)
+                C = Cp.cpu().numpy()
+                assert np.array_equal(C[:, :N], A @ B), (M, N, K, sch)
+                assert (C[:, N:] == 7.0).all(), (M, N, K, sch)
+    sk.workspace_status()
