@@ -109,7 +109,8 @@ struct TileF32 {
     const int rot = (!B_KN && a.M <= BM) ? rotation_of(pn, n) : 0;
     const uint32_t base = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_address(smem));
     auto issue = [&](int t, int slot) {
-      const int kk = (k0 + rotated_iteration(t, rot, n)) * BK;
+      // (past the segment K = 0: the offset of a load that fetches nothing stays at OOB_OFFSET, far past any descriptor)
+      const int kk = t < n ? (k0 + rotated_iteration(t, rot, n)) * BK : 0;
       const uint32_t kbytes = (uint32_t)__builtin_amdgcn_readfirstlane(kk * 4);
       const uint32_t kb_bytes = B_KN ? (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)kk * ldb_bytes)) : kbytes;
       const uint32_t dst = base + (uint32_t)(slot * SLOT);
