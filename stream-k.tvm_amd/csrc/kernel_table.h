@@ -284,6 +284,43 @@ struct KernelInfo {
 // byte of weights -- was measured and is not built: 16 x 16384 x 16384 split in two over K 39.7 us against 39.4 for the
 // 64-row instance and 37.5 for the general kernel, 16 x 8192 x 8192 17.8 against 13.8)
 
+// Up to 16 rows of A, Q4 weights, every wave streaming K on its own (tile_rows_q4.h; dtypes SK_Q4, SK_Q4_ZP and
+// SK_Q4_ZP_TILED, variant 5; taken when asked for by variant or by the planner's rule):
+// X(id, rows of A staged, blocks of 16 weight rows, slots, per-group zero points, scale groups in LDS, tiled weights)
+#define SK_ROWS_Q4_KERNELS(X) \
+  X(310, 4, 1, 4, false, 128, false) \
+  X(311, 4, 2, 2, false, 128, false) \
+  X(312, 4, 3, 4, false, 128, false) \
+  X(313, 4, 4, 3, false, 128, false) \
+  X(314, 8, 1, 4, false, 128, false) \
+  X(315, 8, 2, 3, false, 128, false) \
+  X(316, 8, 3, 3, false, 128, false) \
+  X(317, 8, 4, 2, false, 128, false) \
+  X(318, 4, 1, 4, true, 128, false) \
+  X(319, 4, 2, 2, true, 128, false) \
+  X(320, 4, 3, 4, true, 128, false) \
+  X(321, 4, 4, 3, true, 128, false) \
+  X(322, 8, 1, 4, true, 128, false) \
+  X(323, 8, 2, 3, true, 128, false) \
+  X(324, 8, 3, 3, true, 128, false) \
+  X(325, 8, 4, 2, true, 128, false) \
+  X(326, 16, 1, 3, true, 128, false) \
+  X(327, 16, 2, 2, true, 128, false) \
+  X(328, 16, 3, 2, true, 128, false) \
+  X(329, 16, 4, 2, true, 112, false) \
+  X(330, 4, 1, 4, true, 128, true) \
+  X(331, 4, 2, 2, true, 128, true) \
+  X(332, 4, 3, 4, true, 128, true) \
+  X(333, 4, 4, 3, true, 128, true) \
+  X(334, 8, 1, 4, true, 128, true) \
+  X(335, 8, 2, 3, true, 128, true) \
+  X(336, 8, 3, 3, true, 128, true) \
+  X(337, 8, 4, 2, true, 128, true) \
+  X(338, 16, 1, 3, true, 128, true) \
+  X(339, 16, 2, 2, true, 128, true) \
+  X(340, 16, 3, 2, true, 128, true) \
+  X(341, 16, 4, 2, true, 112, true)
+
 // bfloat16 twins of the fp16 matrix-vector kernels (dtype SK_BF16, variant 2)
 #define SK_GEMV_BF16_KERNELS(X) \
   X(241, 1, 1, 4, 4, 8192)      \

@@ -135,7 +135,7 @@ int launch_gemv_rows(int id, const SkinnyArgs &a, const DevPlan &p, const Worksp
     SK_STREAM_Q4_KERNELS(X)
 #undef X
   }
-  return (int)hipErrorInvalidValue;
+  return launch_rows_q4(id, a, p, ws, s, bias);
 }
 
 int occupancy_gemv_rows(int id) {
@@ -214,7 +214,7 @@ int occupancy_gemv_rows(int id) {
     SK_STREAM_Q4_KERNELS(X)
 #undef X
   }
-  return -1;
+  return occupancy_rows_q4(id);
 }
 
 }  // namespace sk

@@ -24,6 +24,7 @@ int tile_asm8_kernel_infos(KernelInfo *out, int max);
 int tile_q4_kernel_infos(KernelInfo *out, int max);
 int tile_8bit_kernel_infos(KernelInfo *out, int max);
 int skinny_kernel_infos(KernelInfo *out, int max);
+int rows_q4_kernel_infos(KernelInfo *out, int max);
 int f32_kernel_infos(KernelInfo *out, int max);
 
 const KernelInfo *kernel_table(int *count) {
@@ -34,6 +35,7 @@ const KernelInfo *kernel_table(int *count) {
     n += tile_asm8_kernel_infos(g_table + n, 400 - n);
     n += tile_q4_kernel_infos(g_table + n, 400 - n);
     n += skinny_kernel_infos(g_table + n, 400 - n);
+    n += rows_q4_kernel_infos(g_table + n, 400 - n);
     n += f32_kernel_infos(g_table + n, 400 - n);
     g_count = n;
   });
@@ -84,7 +86,8 @@ static const KernelInfo *pick_kernel(int64_t M, int64_t N, int64_t K, int dtype,
     const KernelInfo *found = nullptr;
     for (int i = 0; i < n; ++i)
       if (t[i].dtype == dtype && t[i].layout == layout && t[i].bm == cfg->bm && t[i].bn == cfg->bn &&
-          (cfg->bk <= 0 || t[i].bk == cfg->bk) && (want_variant < 0 || t[i].variant == want_variant) &&
+          (cfg->bk <= 0 || t[i].bk == cfg->bk) &&
+          (want_variant < 0 ? t[i].variant != 5 || t[i].family != FAMILY_SKINNY : t[i].variant == want_variant) &&
           accepts_shape(t[i], M, K) && (found == nullptr || variant_rank(t[i]) > variant_rank(*found)))
         found = &t[i];
     return found;
@@ -158,6 +161,27 @@ static const KernelInfo *pick_kernel(int64_t M, int64_t N, int64_t K, int dtype,
           if (t[i].family == FAMILY_SKINNY && t[i].dtype == dtype && t[i].variant == 2 && t[i].bn == 16 &&
               t[i].bk == bk && accepts_shape(t[i], M, K))
             return &t[i];
+    }
+    // 2 <= M <= 16 with Q4 weights and per-group zero points: the kernels whose waves stream K on their own
+    // (tile_rows_q4.h), as many rows of A staged as M needs, and the tile that gives the busiest CU the least to do -- a
+    // round of tiles costs about 24 weight rows' time beside its own rows (ZP 16 x 28672 x 8192: two rounds of 64 rows
+    // 40.9 us, three of 48 49.9, four of 32 50.0, seven of 16 60.4; 4 x 11008 x 4096: 48 rows 11.1, 64 rows 11.9, two
+    // rounds of 32 13.2).  With one zero point for the matrix up to 8 rows, where 64-row tiles run in one round (beyond,
+    // 4 x 28672 x 8192: 31.9 us on the general kernel against 38); 5 to 8 rows on 32-row tiles stay with the kernel
+    // that streams through shared LDS (8 x 5120 x 5120: 8.1 us against 8.7, 8 x 8192 x 8192: 11.8 / 11.9).
+    if ((dtype == SK_Q4_ZP || dtype == SK_Q4_ZP_TILED || (dtype == SK_Q4 && M <= 8 && cdiv(N, 64) <= num_cus)) && M > 1 && M <= 16 && want_variant < 0) {
+      int64_t least = 0;
+      for (int i = 0; i < n; ++i) {
+        if (t[i].family != FAMILY_SKINNY || t[i].dtype != dtype || t[i].variant != 5 || !accepts_shape(t[i], M, K)) continue;
+        if (best && t[i].max_m > best->max_m) continue;
+        const int64_t busiest = cdiv(cdiv(N, t[i].bn), num_cus) * (t[i].bn + 24);
+        if (!best || t[i].max_m < best->max_m || busiest < least) {
+          best = &t[i];
+          least = busiest;
+        }
+      }
+      if (best && !(dtype == SK_Q4 && M > 4 && best->bn == 32 && K % 256 == 0)) return best;
+      best = nullptr;
     }
     // 2 <= M <= 16 with row-major Q4 weights (scalar zero point), weights from HBM.  Where 64-row tiles give three
     // fifths of the CUs a tile the general kernel with 64 weight rows and K split over two waves, data-parallel
@@ -544,9 +568,14 @@ extern "C" int sk_make_plan(int64_t M, int64_t N, int64_t K, int dtype, int layo
     // fp16 / bfloat16: two fifths -- they run data-parallel rather than pay a fix-up; Q4 16 x 11008 x 4096: 11.5 us
     // against 14.3 us, fp16 16 x 2048 x 8192 on 128 tiles: 11.5 against 14.1, 32 x 11008 x 4096 on 172 tiles of 32 x 64:
     // 19.2 against 22.7; not the 64 x 32 tiles, where the split wins)
-    const bool stream_dp = k->family == FAMILY_SKINNY && (k->variant == 4 || k->dtype == SK_Q4) && k->max_m >= 16 &&
-                           (k->bm == 16 || (k->variant == 4 && k->dtype != SK_Q4 && !(k->bm == 64 && k->bn == 32))) &&
-                           total64 * 5 >= (int64_t)num_cus * (k->variant == 4 && k->dtype != SK_Q4 ? 2 : 3);
+    // (the Q4 kernels whose waves stream K on their own, variant 5: from two fifths on; 8 x 2048 x 8192 on 128 tiles 7.9 us
+    // against 9.9, 16 x 1024 x 16384 on 64 tiles 14.8 / 11.7)
+    const bool stream_dp =
+        k->family == FAMILY_SKINNY &&
+        (k->variant == 5 ? total64 * 5 >= (int64_t)num_cus * 2
+                         : (k->variant == 4 || k->dtype == SK_Q4) && k->max_m >= 16 &&
+                               (k->bm == 16 || (k->variant == 4 && k->dtype != SK_Q4 && !(k->bm == 64 && k->bn == 32))) &&
+                               total64 * 5 >= (int64_t)num_cus * (k->variant == 4 && k->dtype != SK_Q4 ? 2 : 3));
     const bool q4_gemv = k->family == FAMILY_SKINNY && k->variant == 2 && k->max_m == 1 &&
                          (k->dtype == SK_Q4 || k->dtype == SK_Q4_ZP || k->dtype == SK_Q4_TILED || k->dtype == SK_Q4_ZP_TILED);
     if ((total64 >= num_cus || stream_dp) && total64 <= max_grid) {
@@ -588,7 +617,7 @@ extern "C" int sk_make_plan(int64_t M, int64_t N, int64_t K, int dtype, int layo
     // (the kernels that stream the weights through LDS are bound by memory, not by the busiest CU: an uneven last
     // wave costs them less than the fix-up; 16 x 28672 x 8192: 77.8 us data-parallel against 83.6 us.  With 64 rows of
     // A on 64 x 32 tiles it is the other way round, 110 us against 103 us; on 64 x 64 tiles 91.5 against 92.6)
-    if (k->family == FAMILY_SKINNY && k->variant == 4 && (k->bm == 16 || k->bn == 64) && total64 >= grid) sched = SK_SCHED_DP;
+    if (k->family == FAMILY_SKINNY && k->variant >= 4 && (k->bm == 16 || k->bn == 64) && total64 >= grid) sched = SK_SCHED_DP;
     // (the same for the Q4 matrix-vector kernels: 1 x 28672 x 8192 on 1792 tiles 28.0 us data-parallel against 31.2 us,
     // 1 x 14336 x 4096 with K split over four waves 10.8 against 16.1)
     if (k->family == FAMILY_SKINNY && k->variant == 2 && k->max_m == 1 && total64 >= grid &&

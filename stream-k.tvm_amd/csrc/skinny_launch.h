@@ -114,6 +114,26 @@ __global__ __launch_bounds__(P::NT, P::WAVES_PER_EU) void sk_skinny_flat_kernel(
   P::store_c(a, acc, 0, tile, smem, nullptr);
 }
 
+// the same for weights with per-group zero points (ZP_ARGS: row-major, so ldw = K / 2 and groups = K / 128)
+template <class P>
+__global__ __launch_bounds__(P::NT, P::WAVES_PER_EU) void sk_skinny_flat_zp_kernel(const half_t *A, const void *W, const half_t *scales,
+                                                                                 const half_t *zeros, half_t *C, int M, int N, int K) {
+  __shared__ __attribute__((aligned(16))) char smem[P::LDS_BYTES];
+  SkinnyArgs a;
+  a.A = A; a.W = W; a.scales = scales; a.C = C;
+  a.M = M; a.N = N; a.K = K;
+  a.lda = K; a.ldw = K / 2; a.ldc = N;
+  a.zero = 0; a.groups = K / 128; a.zeros = zeros;
+  typename P::Acc acc;
+  const int tile = first_tile_of_block<P>();
+  P::mac(a, acc, 0, tile, 0, (K + P::BKC - 1) / P::BKC, smem);
+  P::store_c(a, acc, 0, tile, smem, nullptr);
+}
+template <class P, class = void>
+struct zp_flat_args { static constexpr bool value = false; };
+template <class P>
+struct zp_flat_args<P, std::void_t<decltype(P::ZP_ARGS)>> { static constexpr bool value = P::ZP_ARGS; };
+
 // NO_FLAT_ARGS: policies whose scalar-argument instance the compiler does not fit into the register budget
 template <class P, class = void>
 struct no_flat_args { static constexpr bool value = false; };
@@ -129,7 +149,13 @@ static inline int launch_policy(const SkinnyArgs &a, const DevPlan &p, const Wor
     else
       hipLaunchKernelGGL((sk_skinny_kernel_bias<P, true>), dim3(p.grid), dim3(P::NT), 0, s, a, p, ws, bias);
   } else if (p.sk_tiles == 0) {
-    if constexpr (!no_flat_args<P>::value) {
+    if constexpr (zp_flat_args<P>::value) {
+      if (p.grid == p.total_tiles && p.ipt == (a.K + P::BKC - 1) / P::BKC && a.lda == a.K && a.ldc == a.N) {
+        hipLaunchKernelGGL((sk_skinny_flat_zp_kernel<P>), dim3(p.grid), dim3(P::NT), 0, s, a.A, a.W, a.scales, a.zeros, a.C, a.M, a.N,
+                           a.K);
+        return (int)hipGetLastError();
+      }
+    } else if constexpr (!no_flat_args<P>::value) {
       if (p.grid == p.total_tiles && p.ipt == (a.K + P::BKC - 1) / P::BKC && a.zeros == nullptr && a.lda == a.K && a.ldc == a.N &&
           a.ldw <= 0x7fffffff) {
         hipLaunchKernelGGL((sk_skinny_flat_kernel<P>), dim3(p.grid), dim3(P::NT), 0, s, a.A, a.W, a.scales, a.C, a.M, a.N, a.K,

@@ -2409,3 +2409,66 @@ def test_fp32_tile_edges(sk, bm, bn, layout):
                 assert np.array_equal(C[:, :N], A @ B), (M, N, K, sch)
                 assert (C[:, N:] == 7.0).all(), (M, N, K, sch)
     sk.workspace_status()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["q4", "q4_zp", "q4_zp_tiled"])
+def test_q4_waves_streaming_k_on_their_own(sk, oracle, dtype):
+    """The Q4 kernels whose waves stream K without a barrier (4, 8 and 16 staged rows of A, tiles of 16 to 64 weight rows):
+    M at the edges of the staged rows, ragged N, K from one scale group to the most groups they hold (waves without a
+    group in the last iteration, fewer groups than a 16-byte piece of scales).  Integer activations and power-of-two
+    scales keep every partial sum exact in fp32, so C must equal the host product to the bit; an infinite activation
+    meets the exact integers q - zero."""
+    import torch
+    rng = np.random.default_rng(310)
+    code = {"q4": 2, "q4_zp": 7, "q4_zp_tiled": 9}[dtype]
+    most = 8 if dtype == "q4" else 16
+    ran = set()
+    for (N, K) in [(16, 128), (200, 1152), (129, 2176), (513, 4096), (40, 14336), (72, 16384)]:
+        Wq = rng.integers(0, 256, (N, K // 2), dtype=np.uint8)
+        sc = (2.0 ** rng.integers(-3, 1, (N, K // 128))).astype(np.float16)
+        zp = rng.integers(0, 16, (N, K // 128)).astype(np.float16) if dtype != "q4" else np.full((N, K // 128), 5, np.float16)
+        Ai = rng.integers(-2, 3, (16, K)).astype(np.float16)
+        exact = oracle.q4_zp_gemm_ref(Ai, Wq, sc, zp)
+        assert np.abs(exact).max() < 2 ** 20 and np.array_equal(exact, np.rint(exact * 8) / 8)   # (exact in fp32)
+        want = exact.astype(np.float16).astype(np.float32)
+        dW, dS, dA = _t(Wq), _t(sc), _t(Ai)
+        if dtype == "q4_zp_tiled":
+            dW = sk.tile_q4(dW)
+        kw = dict(zero=5) if dtype == "q4" else dict(zeros=_t(zp), tiled=dtype == "q4_zp_tiled")
+        for M in (1, 3, 4, 5, 8, 9, 16):
+            if M > most:
+                continue
+            Ap = torch.full((M, K + 8), float("nan"), device="cuda", dtype=torch.float16)   # (rows end in NaN)
+            Ap[:, :K] = dA[:M]
+            for bn in (16, 32, 48, 64):
+                for sch in (dict(schedule="dp"), dict(schedule="dp", grid=3), dict(schedule="basic", fixup="reduce", grid=5),
+                            dict(schedule="basic", fixup="atomic", grid=7)):
+                    try:
+                        plan = sk.make_plan(M, N, K, dtype, "nt", dict(bm=16, bn=bn, bk=1024, variant=6, **sch), cus=256)
+                    except sk.StreamKError:
+                        continue   # (more CTAs than iterations, or more groups than the instance holds)
+                    assert plan.dtype == code and sk.kernel_name(plan.kernel_id).startswith("rows_q4")
+                    C = sk.streamk_q4(Ap[:, :K], dW, dS, plan=plan, **kw)
+                    assert np.array_equal(C.float().cpu().numpy(), want[:M]), (M, N, K, bn, sch)
+                    ran.add(plan.kernel_id)
+            if M > 1:
+                C = sk.streamk_q4(dA[:M].contiguous(), dW, dS, **kw)
+                assert np.array_equal(C.float().cpu().numpy(), want[:M]), (M, N, K)
+        M = min(8, most)
+        Ainf = dA[:M].clone()
+        Ainf[0, 0] = float("inf")
+        plan = sk.make_plan(M, N, K, dtype, "nt", dict(bm=16, bn=16, bk=1024, variant=6, schedule="dp"), cus=256)
+        C = sk.streamk_q4(Ainf, dW, dS, plan=plan, **kw).float().cpu().numpy()
+        first = (Wq[:, 0] & 15).astype(np.float32) - zp[:, 0].astype(np.float32)
+        assert np.array_equal(np.isposinf(C[0]), first > 0) and np.array_equal(np.isneginf(C[0]), first < 0)
+        assert np.array_equal(C[1:], want[1:M])
+    assert len(ran) == (8 if dtype == "q4" else 12), sorted(ran)
+    # refused as before: these tiles without the variant, more rows than staged, more groups than the instance holds
+    for bad in (dict(bm=16, bn=48, bk=1024), dict(bm=16, bn=64, bk=1024)):
+        with pytest.raises(sk.StreamKError):
+            sk.make_plan(4, 1024, 1024, dtype, "nt", bad, cus=256)
+    for m, k in ((most + 1, 1024), (4, 16512)):
+        with pytest.raises(sk.StreamKError):
+            sk.make_plan(m, 1024, k, dtype, "nt", dict(bm=16, bn=16, bk=1024, variant=6), cus=256)
+    sk.workspace_status()
