@@ -111,6 +111,7 @@ typedef struct sk_config {
                              (8 for the 16-bit and fp8 tile kernels, row-major otherwise) */
   int32_t spin_limit;     /* REDUCE fix-up: polls of a peer flag before giving up; 0 = default */
   int32_t reserved[4];    /* reserved[0]: 0 = preferred kernel variant of the tile, v > 0 = variant v - 1
+                             (9 without a tile, fp8 / int8 up to 64 rows: weights streamed through LDS)
                              (implementation alternatives of one tile shape, for the autotuner);
                              reserved[1]: split factor of SK_SCHED_SPLIT_K, 0 = choose;
                              reserved[2]: 1 = interleaved order of the Stream-K tiles (see sk_plan.interleave); with 0 the

@@ -268,6 +268,18 @@ struct KernelInfo {
   X(298, 3, 2, 2, 1, 4, 1, 2, false) \
   X(299, 3, 2, 2, 1, 4, 1, 2, true)
 
+// one-byte twins (dtypes SK_F8E4M3 id, SK_F8E5M2 id + 10, SK_I8 id + 20; bk counts bytes; variant 8, taken when asked
+// for by variant):
+// X(id, MB, WM, WN, RK, DEPTH, NB, AD, padded, KH)
+#define SK_STREAM_BYTES_KERNELS(X)       \
+  X(350, 1, 1, 4, 1, 4, 1, 3, true, 1)   \
+  X(351, 2, 1, 4, 1, 3, 1, 3, true, 1)   \
+  X(352, 1, 1, 2, 2, 3, 1, 3, true, 1)   \
+  X(353, 2, 2, 2, 1, 3, 1, 3, true, 1)   \
+  X(354, 2, 2, 2, 1, 3, 2, 2, false, 2)  \
+  X(355, 1, 1, 1, 4, 3, 1, 2, false, 2)  \
+  X(356, 2, 1, 2, 2, 3, 1, 2, false, 2)
+
 // Up to 16 rows of A, Q4 weights (row-major, scalar zero point) streaming through LDS in contiguous loads
 // (tile_stream_q4.h; dtype SK_Q4, variant 4):  X(id, WN, RK, KH, WD, AD)
 #define SK_STREAM_Q4_KERNELS(X) \

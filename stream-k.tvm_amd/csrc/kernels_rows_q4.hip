@@ -26,7 +26,7 @@ int launch_rows_q4(int id, const SkinnyArgs &a, const DevPlan &p, const Workspac
     SK_ROWS_Q4_KERNELS(X)
 #undef X
   }
-  return (int)hipErrorInvalidValue;
+  return launch_stream_bytes(id, a, p, ws, s, bias);
 }
 
 int occupancy_rows_q4(int id) {
@@ -40,7 +40,7 @@ int occupancy_rows_q4(int id) {
     SK_ROWS_Q4_KERNELS(X)
 #undef X
   }
-  return -1;
+  return occupancy_stream_bytes(id);
 }
 
 }  // namespace sk

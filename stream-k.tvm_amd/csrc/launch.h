@@ -33,6 +33,9 @@ int occupancy_tile_asm8(int id);
 // small-M kernels for Q4 weights without a barrier in their loop (translation unit kernels_rows_q4.hip)
 int launch_rows_q4(int id, const SkinnyArgs &a, const DevPlan &p, const Workspace &ws, hipStream_t s, const void *bias);
 int occupancy_rows_q4(int id);
+// small-M kernels that stream one-byte weights through LDS (translation unit kernels_stream_bytes.hip)
+int launch_stream_bytes(int id, const SkinnyArgs &a, const DevPlan &p, const Workspace &ws, hipStream_t s, const void *bias);
+int occupancy_stream_bytes(int id);
 // tile kernels for Q4 weights (translation unit kernels_tile_q4.hip)
 int tile_q4_kernel_infos(KernelInfo *out, int max);
 int launch_tile_q4(int id, const GemmArgs &a, const DevPlan &p, const Workspace &ws, hipStream_t s, const void *bias);

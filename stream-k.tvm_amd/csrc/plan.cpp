@@ -25,6 +25,7 @@ int tile_q4_kernel_infos(KernelInfo *out, int max);
 int tile_8bit_kernel_infos(KernelInfo *out, int max);
 int skinny_kernel_infos(KernelInfo *out, int max);
 int rows_q4_kernel_infos(KernelInfo *out, int max);
+int stream_bytes_kernel_infos(KernelInfo *out, int max);
 int f32_kernel_infos(KernelInfo *out, int max);
 
 const KernelInfo *kernel_table(int *count) {
@@ -36,6 +37,7 @@ const KernelInfo *kernel_table(int *count) {
     n += tile_q4_kernel_infos(g_table + n, 400 - n);
     n += skinny_kernel_infos(g_table + n, 400 - n);
     n += rows_q4_kernel_infos(g_table + n, 400 - n);
+    n += stream_bytes_kernel_infos(g_table + n, 400 - n);
     n += f32_kernel_infos(g_table + n, 400 - n);
     g_count = n;
   });
@@ -63,6 +65,11 @@ static int variant_rank(const KernelInfo &k) {
     return k.variant == 4 ? -1 : (k.variant == 3 ? 1 : (k.variant == 0 ? 0 : k.variant + 1));
   return k.variant == 7 ? 4 : (k.variant == 4 ? 3 : (k.variant == 1 ? 2 : (k.variant == 2 ? 1 : 0)));
 }
+// kernels that a tile alone does not name: the Q4 ones whose waves stream K on their own, and the ones that stream one-byte
+// weights through LDS
+static bool by_variant_only(const KernelInfo &k) {
+  return k.family == FAMILY_SKINNY && (k.variant == 5 || k.variant == 8);
+}
 static bool accepts_shape(const KernelInfo &k, int64_t M, int64_t K) {
   // (the assembly-loop tile kernels have no K tail: other K go to the next-best variant of the tile)
   return (k.max_m == 0 || M <= k.max_m) && (k.max_ipt == 0 || (K + k.bk - 1) / k.bk <= k.max_ipt) &&
@@ -87,7 +94,7 @@ static const KernelInfo *pick_kernel(int64_t M, int64_t N, int64_t K, int dtype,
     for (int i = 0; i < n; ++i)
       if (t[i].dtype == dtype && t[i].layout == layout && t[i].bm == cfg->bm && t[i].bn == cfg->bn &&
           (cfg->bk <= 0 || t[i].bk == cfg->bk) &&
-          (want_variant < 0 ? t[i].variant != 5 || t[i].family != FAMILY_SKINNY : t[i].variant == want_variant) &&
+          (want_variant < 0 ? !by_variant_only(t[i]) : t[i].variant == want_variant) &&
           accepts_shape(t[i], M, K) && (found == nullptr || variant_rank(t[i]) > variant_rank(*found)))
         found = &t[i];
     return found;
@@ -135,6 +142,26 @@ static const KernelInfo *pick_kernel(int64_t M, int64_t N, int64_t K, int dtype,
       if (t[i].family == FAMILY_SKINNY && t[i].dtype == dtype && t[i].variant == 4 && t[i].bm == bm && t[i].bn == bn &&
           t[i].bk == bk && accepts_shape(t[i], M, K))
         return &t[i];
+  }
+  // up to 64 rows of fp8 / int8: the same kernels on bytes, for a caller who names their variant alone (the operators
+  // do, where no tuned configuration exists).  Up to 32 rows the narrowest tile of which every CU gets at
+  // most one, beyond like the 16-bit ones (weights from HBM, e4m3, in us, tile_skinny.h's kernels / these:
+  // 16 x 4096 x 4096 9.8 / 6.5, 16 x 8192 x 8192 22.5 / 14.3, 16 x 11008 x 4096 16.6 / 11.8 on 64-row tiles and 14.7 on
+  // 32, 32 x 5120 x 5120 14.8 / 10.5 on 32 x 32 tiles and 12.8 on 32 x 64, 64 x 28672 x 8192 67.5 / 56.5,
+  // 64 x 4096 x 4096 14.5 / 9.7 on 64 x 32 tiles and 13.0 on 64 x 64)
+  if (one_byte && want_variant == 8) {
+    if (M > 64) return nullptr;
+    int bm = 64, bn = cdiv(N, 64) * 5 < (int64_t)num_cus * 3 ? 32 : 64, bk = 512;
+    if (M <= 32) {
+      bm = M <= 16 ? 16 : 32;
+      bn = bm == 16 && cdiv(N, 16) <= num_cus ? 16 : (cdiv(N, 32) <= num_cus ? 32 : 64);
+      bk = bn == 16 ? 2048 : (bn == 32 ? 1024 : 512);
+    }
+    for (int i = 0; i < n; ++i)
+      if (t[i].family == FAMILY_SKINNY && t[i].dtype == dtype && t[i].variant == 8 && t[i].bm == bm && t[i].bn == bn &&
+          t[i].bk == bk)
+        return &t[i];
+    return nullptr;
   }
   // 65 to 96 rows of fp16 / bfloat16 where 96 x 32 tiles fill the device in one round (N = 8192 on 256 CUs): the
   // streaming kernel with three blocks of rows per wave -- A is three times the bytes of the weights per CTA, but the
@@ -568,11 +595,16 @@ extern "C" int sk_make_plan(int64_t M, int64_t N, int64_t K, int dtype, int layo
     // fp16 / bfloat16: two fifths -- they run data-parallel rather than pay a fix-up; Q4 16 x 11008 x 4096: 11.5 us
     // against 14.3 us, fp16 16 x 2048 x 8192 on 128 tiles: 11.5 against 14.1, 32 x 11008 x 4096 on 172 tiles of 32 x 64:
     // 19.2 against 22.7; not the 64 x 32 tiles, where the split wins)
+    // (one-byte weights through LDS: always up to 32 rows -- 16 x 1024 x 16384 on 64 tiles 11.0 us against 11.4 -- and on
+    // 64 rows unless a CTA would run many iterations while others idle: 64 x 4096 x 4096 9.7 us against 11.9,
+    // 64 x 5120 x 5120 11.9 / 15.4, 64 x 4096 x 11008 20.2 / 18.9, 64 x 2048 x 8192 15.0 / 12.7)
+    const bool stream_bytes = k->family == FAMILY_SKINNY && k->variant == 8;
     // (the Q4 kernels whose waves stream K on their own, variant 5: from two fifths on; 8 x 2048 x 8192 on 128 tiles 7.9 us
     // against 9.9, 16 x 1024 x 16384 on 64 tiles 14.8 / 11.7)
     const bool stream_dp =
         k->family == FAMILY_SKINNY &&
-        (k->variant == 5 ? total64 * 5 >= (int64_t)num_cus * 2
+        (stream_bytes ? k->bm <= 32 || total64 >= num_cus || out->iters_per_tile * (num_cus - total64) <= 8 * num_cus
+         : k->variant == 5 ? total64 * 5 >= (int64_t)num_cus * 2
                          : (k->variant == 4 || k->dtype == SK_Q4) && k->max_m >= 16 &&
                                (k->bm == 16 || (k->variant == 4 && k->dtype != SK_Q4 && !(k->bm == 64 && k->bn == 32))) &&
                                total64 * 5 >= (int64_t)num_cus * (k->variant == 4 && k->dtype != SK_Q4 ? 2 : 3));

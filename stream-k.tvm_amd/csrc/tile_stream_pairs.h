@@ -1,4 +1,4 @@
-// Up to 64 rows of A against fp16 / bfloat16 weights [N, K] (NT): the weights stream through LDS in loads that
+// Up to 64 rows of A against fp16, bfloat16, fp8 or int8 weights [N, K] (NT): the weights stream through LDS in loads that
 // read CONTIGUOUS bytes.
 //
 // The general small-M kernel (tile_skinny.h) loads the 16x16x32 MFMA's operand layout straight from memory: lane l
@@ -27,6 +27,11 @@
 //    90.8 -> 86.4 us, 16 x 4096 x 4096 9.7 -> 9.2; the other instances gain nothing or lose: 64 x 32 tiles at
 //    64 x 8192 x 8192 28.8 -> 33.8 us).
 //  * Tiles walk K from different offsets (rotation_of, sk_device.h).
+//  * One-byte operands take the same path as pairs (F8_).  Weights from HBM, e4m3, against the general kernels that
+//    load 64 bytes of 16 rows per instruction: 1 x 4096 x 4096 10.2 -> 6.2 us, 16 x 8192 x 8192 22.5 -> 14.3,
+//    24 x 11008 x 4096 17.7 -> 12.9, 64 x 28672 x 8192 67.5 -> 56.5 (4.2 TB/s; A as many bytes per CTA as the weights).
+//    A 32 x 32 tile (K split in two, two waves per K sub-block) is built for them alone: with 16-bit operands it is
+//    behind the 32 x 32 tile of two by two waves (20 x 4096 x 11008 30.7 us against 27.2).
 //
 // Replaces the reference's inner MAC for its own run shape, 16 x 16384 x 8192 (streamk_fp16_nt.py:15, :196-240).
 #pragma once
@@ -35,10 +40,17 @@
 namespace sk {
 
 template <int MB_, int WM_, int WN_, int RK_, int DEPTH_, bool BF16_ = false, int NB_ = 1, int AD_ = 3, bool PADDED_ = true,
-          int KH_ = 1>
+          int KH_ = 1, int F8_ = 0>
 struct TileStreamPairs {
   typedef SkinnyArgs Args;
-  typedef floatx4 AccV;
+  // F8_ (1: OCP e4m3, 2: OCP e5m2, 3: int8): one-byte operands travel as pairs, the launcher halves K, lda and ldw; a
+  // fragment's 16 bytes are 16 K-values, for A and the weights alike.  fp8: a.zero carries the bits of the scalar that
+  // multiplies the fp32 sums, C is fp16; int8: sums, partials and C are int32.
+  static_assert(F8_ == 0 || !BF16_, "one-byte operands exclude bfloat16");
+  static constexpr bool I8 = F8_ == 3;
+  typedef int intx4 __attribute__((ext_vector_type(4)));
+  typedef typename std::conditional<I8, intx4, floatx4>::type AccV;
+  typedef typename std::conditional<I8, int, float>::type AccT;
   static constexpr bool LEAN_ENTRY = false;  // see run_persistent
   static constexpr bool NO_FLAT_ARGS = false;
   static constexpr bool COHERENT_PARTIALS = true;
@@ -187,7 +199,17 @@ struct TileStreamPairs {
         for (int i = 0; i < MB; ++i)
 #pragma unroll
           for (int j = 0; j < NB; ++j) {
-            if constexpr (BF16_) {
+            if constexpr (I8) {
+              acc.c[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(intx4, fw[j][s]), __builtin_bit_cast(intx4, fa[i][s]),
+                                                                  acc.c[i][j], 0, 0, 0);
+            } else if constexpr (F8_ != 0) {
+              typedef long longx2 __attribute__((ext_vector_type(2)));
+              const longx2 w2 = __builtin_bit_cast(longx2, fw[j][s]), a2 = __builtin_bit_cast(longx2, fa[i][s]);
+#pragma unroll
+              for (int h = 0; h < 2; ++h)
+                acc.c[i][j] = F8_ == 1 ? __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(w2[h], a2[h], acc.c[i][j], 0, 0, 0)
+                                       : __builtin_amdgcn_mfma_f32_16x16x32_bf8_bf8(w2[h], a2[h], acc.c[i][j], 0, 0, 0);
+            } else if constexpr (BF16_) {
               typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
               acc.c[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, fw[j][s]), __builtin_bit_cast(bf16x8, fa[i][s]),
                                                                     acc.c[i][j], 0, 0, 0);
@@ -206,7 +228,7 @@ struct TileStreamPairs {
 
     // ---- sum the RK partial accumulators into the rk == 0 waves (through the weights' rings, free by now) ----
     if constexpr (RK * KH > 1) {
-      float *red = reinterpret_cast<float *>(smem);
+      AccT *red = reinterpret_cast<AccT *>(smem);
       if (wave >= WM * WN) {
 #pragma unroll
         for (int v = 0; v < NV4; ++v)
@@ -244,7 +266,7 @@ struct TileStreamPairs {
     if (wave >= WM * WN) return;
     const int wm = wave % WM, wn = wave / WM;
     const int lr = lane & 15, lg = lane >> 4;
-    const bool vec_ok = (a.ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(a.C) & 7) == 0);
+    const bool vec_ok = (a.ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(a.C) & (I8 ? 15 : 7)) == 0);
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
       const int row = pm * BM + (wm * MB + i) * 16 + lr;
@@ -252,10 +274,20 @@ struct TileStreamPairs {
       for (int j = 0; j < NB; ++j) {
         const int col = pn * BN + (wn * NB + j) * 16 + lg * 4;
         if (row < a.M && col < a.N) {
+          if constexpr (I8) {   // int32 C straight from the accumulators (ldc counts int32 elements)
+            int *dst = reinterpret_cast<int *>(a.C) + (int64_t)row * a.ldc + col;
+            if (vec_ok && col + 4 <= a.N) {
+              *reinterpret_cast<intx4 *>(dst) = acc.c[i][j];
+            } else {
+              for (int e = 0; e < 4 && col + e < a.N; ++e) dst[e] = acc.c[i][j][e];
+            }
+            continue;
+          }
           half4v h;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             float x = acc.c[i][j][e];
+            if constexpr (F8_ != 0 && !I8) x *= __builtin_bit_cast(float, a.zero);
             if constexpr (BIAS) x = activate(x + bias_at<BF16_>(bias, col + e, a.N), act);
             if constexpr (BF16_) {
               const __bf16 b = (__bf16)x;
@@ -278,32 +310,41 @@ struct TileStreamPairs {
   // Partial tiles are a few KB: every access is a coherent (write-through / L2-bypassing) one, as in tile_skinny.h.
   // Block v = i NB + j of thread t (one of the NTP threads of the rk == 0 waves) is kept at (v NTP + t) 4; the
   // accumulating form keeps element e of it at (v 4 + e) NTP + t.
-  static __device__ __forceinline__ void store_partial(const Acc &acc, float *dst) {
+  static __device__ __forceinline__ void store_partial(const Acc &acc, float *dst_) {
     if (threadIdx.x >= NTP) return;
+    AccT *dst = reinterpret_cast<AccT *>(dst_);
 #pragma unroll
     for (int v = 0; v < NV4; ++v) st_coherent(dst + ((size_t)v * NTP + threadIdx.x) * 4, acc.c[v / NB][v % NB]);
   }
-  static __device__ __forceinline__ void add_partial(Acc &acc, const float *src) {
+  static __device__ __forceinline__ void add_partial(Acc &acc, const float *src_) {
     if (threadIdx.x >= NTP) return;
+    const AccT *src = reinterpret_cast<const AccT *>(src_);
 #pragma unroll
     for (int v = 0; v < NV4; ++v) acc.c[v / NB][v % NB] += ld_coherent(src + ((size_t)v * NTP + threadIdx.x) * 4);
   }
-  static __device__ __forceinline__ void atomic_partial(const Acc &acc, float *dst) {
+  static __device__ __forceinline__ void atomic_partial(const Acc &acc, float *dst_) {
     if (threadIdx.x >= NTP) return;
-#pragma unroll
-    for (int v = 0; v < NV4; ++v)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) atomic_add_f32(dst + (size_t)(v * 4 + e) * NTP + threadIdx.x, acc.c[v / NB][v % NB][e]);
-  }
-  static __device__ __forceinline__ void take_partial(Acc &acc, float *src) {
-    if (threadIdx.x >= NTP) return;
+    AccT *dst = reinterpret_cast<AccT *>(dst_);
 #pragma unroll
     for (int v = 0; v < NV4; ++v)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        float *p = src + (size_t)(v * 4 + e) * NTP + threadIdx.x;
+        if constexpr (I8)
+          atomic_add_i32(dst + (size_t)(v * 4 + e) * NTP + threadIdx.x, acc.c[v / NB][v % NB][e]);
+        else
+          atomic_add_f32(dst + (size_t)(v * 4 + e) * NTP + threadIdx.x, acc.c[v / NB][v % NB][e]);
+      }
+  }
+  static __device__ __forceinline__ void take_partial(Acc &acc, float *src_) {
+    if (threadIdx.x >= NTP) return;
+    AccT *src = reinterpret_cast<AccT *>(src_);
+#pragma unroll
+    for (int v = 0; v < NV4; ++v)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        AccT *p = src + (size_t)(v * 4 + e) * NTP + threadIdx.x;
         acc.c[v / NB][v % NB][e] = ld_coherent_scalar(p);
-        st_coherent(p, 0.f);
+        st_coherent(p, (AccT)0);
       }
   }
 };

@@ -146,7 +146,8 @@ def _plan_for(config, M, N, K, dtype, layout):
     key = (M, N, K, dtype, layout, config, _plan_mod.tuned_generation(), torch.cuda.current_device() if torch.cuda.is_available() else -1)
     plan = _plan_cache.get(key)
     if plan is None:
-        plan = make_plan(M, N, K, dtype, layout, _parse_config(config) if config else None)
+        plan = make_plan(M, N, K, dtype, layout,
+                         _parse_config(config) if config else _plan_mod.operator_config(M, N, K, dtype, layout))
         if len(_plan_cache) < 4096:
             _plan_cache[key] = plan
     return plan

@@ -2472,3 +2472,54 @@ def test_q4_waves_streaming_k_on_their_own(sk, oracle, dtype):
         with pytest.raises(sk.StreamKError):
             sk.make_plan(m, 1024, k, dtype, "nt", dict(bm=16, bn=16, bk=1024, variant=6), cus=256)
     sk.workspace_status()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["float8_e4m3", "float8_e5m2", "int8"])
+def test_one_byte_weights_streamed_through_lds(sk, dtype):
+    """The kernels that stream one-byte weights through LDS (16, 32 and 64 rows of A, tiles of 16 to 64 weight rows): M
+    and N around the tiles' edges, K from one 16-byte piece over a last iteration hanging over K to several iterations,
+    the schedules and both fix-ups.  Integer operands keep every partial sum exact, so C must equal the host product
+    (fp8: rounded to fp16 once); the rows of A end in a value that would show."""
+    import torch
+    rng = np.random.default_rng(350)
+    kind = {"float8_e4m3": torch.float8_e4m3fn, "float8_e5m2": torch.float8_e5m2, "int8": torch.int8}[dtype]
+    lim = 127 if dtype == "int8" else 4
+    f = sk.streamk_int8 if dtype == "int8" else sk.streamk_fp8
+    as_kind = lambda x: torch.from_numpy(x).to(kind).cuda()   # noqa: E731
+    ran = set()
+    for bm, bn, bk in ((16, 64, 512), (32, 64, 512), (16, 32, 1024), (64, 32, 512), (64, 64, 512), (16, 16, 2048), (32, 32, 1024)):
+        for N, K in ((bn, 16), (bn - 3, bk + 16), (3 * bn + 5, 2 * bk - 16), (2 * bn, 3 * bk)):
+            A = rng.integers(-lim, lim + 1, (bm, K)).astype(np.float32)
+            B = rng.integers(-lim, lim + 1, (N, K)).astype(np.float32)
+            want = A.astype(np.float64) @ B.astype(np.float64).T
+            if dtype != "int8":
+                want = (want * 0.5).astype(np.float32).astype(np.float16)
+            dB = as_kind(B)
+            for M in {1, bm - 1, bm}:
+                Ap = torch.full((M, K + 16), 3.0, device="cuda").to(kind)
+                Ap[:, :K] = as_kind(A[:M])
+                for sch in (dict(schedule="dp"), dict(schedule="dp", grid=2), dict(schedule="basic", fixup="reduce", grid=3),
+                            dict(schedule="basic", fixup="atomic", grid=5)):
+                    if sch["schedule"] == "basic" and sch["grid"] > -(-N // bn) * -(-K // bk):
+                        continue   # (a CTA keeps at least one iteration)
+                    plan = sk.make_plan(M, N, K, dtype, "nt", dict(bm=bm, bn=bn, bk=bk, variant=9, **sch), cus=256)
+                    assert sk.kernel_name(plan.kernel_id).startswith("stream_")
+                    kw = {} if dtype == "int8" else dict(alpha=0.5)
+                    C = f(Ap[:, :K], dB, plan=plan, **kw).cpu().numpy()
+                    assert np.array_equal(C, want[:M]), (M, N, K, bm, bn, sch)
+                    ran.add(plan.kernel_id)
+                if dtype != "int8":   # the epilogue operands
+                    bias = torch.from_numpy(rng.integers(-8, 9, N).astype(np.float16)).cuda()
+                    C = f(Ap[:, :K], dB, plan=plan, alpha=0.5, bias=bias, activation="relu").cpu().numpy()
+                    full = (A[:M].astype(np.float64) @ B.astype(np.float64).T) * 0.5 + bias.cpu().numpy().astype(np.float64)
+                    assert np.array_equal(C, np.maximum(full, 0).astype(np.float32).astype(np.float16)), (M, N, K, bm, bn)
+        # what a caller who gives the tile alone gets is what it was
+        if (bm, bn, bk) in ((64, 32, 512), (16, 16, 2048), (32, 32, 1024)):
+            with pytest.raises(sk.StreamKError):
+                sk.make_plan(1, 256, 4096, dtype, "nt", dict(bm=bm, bn=bn, bk=bk), cus=256)
+    assert len(ran) == 7
+    # what an operator call takes without a tuned configuration
+    for M, N in ((1, 4096), (16, 8192), (16, 8224), (17, 8192), (32, 8224), (33, 4096), (64, 28672)):
+        assert sk.kernel_name(sk.make_plan(M, N, 4096, dtype, "nt", sk.plan.operator_config(M, N, 4096, dtype, "nt"), cus=256).kernel_id).startswith("stream_"), (M, N)
+    sk.workspace_status()
