@@ -7,6 +7,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libstreamk.so")
+TORCH_LIB_PATH = os.path.join(_HERE, "libstreamk_torch.so")
 
 SK_F16, SK_F32, SK_Q4, SK_BF16, SK_Q4_TILED, SK_F8E4M3, SK_I8, SK_Q4_ZP, SK_F8E5M2, SK_Q4_ZP_TILED = 0, 1, 2, 3, 4, 5, 6, 7, 8, 9
 LAYOUT_NT, LAYOUT_NN = 0, 1
@@ -127,6 +128,29 @@ def lib():
         getattr(L, f).restype = ci
     _lib = L
     return L
+
+
+_torch_lib = None
+
+
+def torch_lib():
+    """Loads libstreamk_torch.so, whose static initialisers register the operators' native implementations
+    (csrc/torch_ops.cpp)."""
+    global _torch_lib
+    if _torch_lib is None:
+        lib()
+        if not os.path.exists(TORCH_LIB_PATH):
+            raise ImportError(f"{TORCH_LIB_PATH} is missing: build it with `make -C stream-k.tvm_amd/csrc` "
+                              "(or __graft_entry__.build())")
+        L = ctypes.CDLL(TORCH_LIB_PATH)
+        L.sk_torch_add_plan.argtypes = [ctypes.POINTER(SkPlan), ctypes.c_int]
+        L.sk_torch_add_plan.restype = None
+        L.sk_torch_clear_plans.argtypes = []
+        L.sk_torch_clear_plans.restype = None
+        L.sk_torch_set_workspace.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t]
+        L.sk_torch_set_workspace.restype = None
+        _torch_lib = L
+    return _torch_lib
 
 
 def kernel_name(kernel_id):

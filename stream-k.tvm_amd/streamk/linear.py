@@ -80,7 +80,7 @@ class StreamKLinear(torch.nn.Module):
         if x.dtype != self.dtype or x.shape[-1] != self.in_features:
             raise ValueError(f"input must be {self.dtype} [..., {self.in_features}], got {x.dtype} {tuple(x.shape)}")
         lead = x.shape[:-1]
-        a = x.reshape(-1, self.in_features)
+        a = x if x.dim() == 2 else x.reshape(-1, self.in_features)
         if a.shape[0] == 0:
             return x.new_zeros(*lead, self.out_features)
         # bias and activation are applied in the GEMM's epilogue (fp32, before the rounding to C's type)
@@ -93,7 +93,7 @@ class StreamKLinear(torch.nn.Module):
             zeros = self.zeros if self.weight_format == "q4_zp" else None
             c = torch.ops.streamk.gemm_q4(a, self.qweight, self.scales, zeros, self.zero, self.group, False, "",
                                           self.bias, act)
-        return c.view(*lead, self.out_features)
+        return c if x.dim() == 2 else c.view(*lead, self.out_features)
 
     def extra_repr(self):
         return (f"in_features={self.in_features}, out_features={self.out_features}, bias={self.bias is not None}, "

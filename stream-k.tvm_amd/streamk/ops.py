@@ -10,7 +10,8 @@ Mirrors the reference's operator surface:
 Every GEMM is registered with the PyTorch dispatcher as a custom operator of the `streamk` namespace
 (`torch.ops.streamk.gemm_f16`, `gemm_bf16`, `gemm_f32`, `gemm_q4`, `gemm_f8`, `gemm_i8`, each with an
 `_out` twin that writes a caller's C, plus `dequant_q4`): a HIP implementation that hands data
-pointers and the current stream to the C ABI, and a fake (meta) implementation that gives shape and
+pointers and the current stream to the C ABI (native for ordinary calls, csrc/torch_ops.cpp, which passes every other
+one on to the implementations here, registered as `<name>_general`), and a fake (meta) implementation that gives shape and
 dtype of the result, so that `torch.compile`, FakeTensor tracing and graph capture see an ordinary
 operator.  This is the role of the reference's `@jit(out_idx=[2])` wrapper, which turns the kernel
 into `f(A, B) -> C` (autotune/streamk_fp16_autotune.py:93-94).  The functions below are thin argument
@@ -43,11 +44,13 @@ def _workspace(nbytes, device):
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
         if ws is not None:  # the library must not take a later allocation at this address for this workspace
+            _lib.torch_lib().sk_torch_set_workspace(*key, None, 0)
             _lib.lib().sk_workspace_release(ws.data_ptr())
         ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         _lib.check(_lib.lib().sk_workspace_init(ws.data_ptr(), ws.numel(), _stream_ptr()),
                    "sk_workspace_init")
         _workspaces[key] = ws
+        _lib.torch_lib().sk_torch_set_workspace(*key, ws.data_ptr(), ws.numel())
     return ws
 
 
@@ -61,7 +64,8 @@ def reset_workspaces():
     """Drops cached workspaces.  Needed after workspace_status() (or a launch) has raised StreamKError
     with status SK_ERR_TIMEOUT: the library refuses a workspace on which a fix-up wait gave up until it
     has been initialised again, which the next call on a fresh workspace does."""
-    for ws in _workspaces.values():
+    for key, ws in _workspaces.items():
+        _lib.torch_lib().sk_torch_set_workspace(*key, None, 0)
         _lib.lib().sk_workspace_release(ws.data_ptr())
     _workspaces.clear()
 
@@ -119,6 +123,8 @@ def _plan_handle(plan):
 
 
 def _config_string(plan, config, kw):
+    if plan is None and not config and not kw:
+        return ""
     if plan is not None:
         return _plan_handle(plan)
     d = dict(config or {})
@@ -143,13 +149,18 @@ def _plan_for(config, M, N, K, dtype, layout):
             raise ValueError(f"unknown plan handle {config!r}")
         return plan
     # (a plan depends on the tuned cache it was made from and on the device it was made for)
-    key = (M, N, K, dtype, layout, config, _plan_mod.tuned_generation(), torch.cuda.current_device() if torch.cuda.is_available() else -1)
+    generation, device = _plan_mod.tuned_generation(), torch.cuda.current_device() if torch.cuda.is_available() else -1
+    key = (M, N, K, dtype, layout, config, generation, device)
     plan = _plan_cache.get(key)
     if plan is None:
         plan = make_plan(M, N, K, dtype, layout,
                          _parse_config(config) if config else _plan_mod.operator_config(M, N, K, dtype, layout))
         if len(_plan_cache) < 4096:
             _plan_cache[key] = plan
+            if config == "":   # from now on the native implementation answers calls of this shape
+                with _plan_mod.tuned_lock:
+                    if generation == _plan_mod.tuned_generation():
+                        _lib.torch_lib().sk_torch_add_plan(ctypes.byref(plan), device)
     return plan
 
 
@@ -383,8 +394,11 @@ def _register(name, before_out, after_out, run, out_meta):
     after_out) -> ().  run(*args) with C at position len(before_out arguments) performs the launch;
     out_meta(*functional args) -> (shape, dtype) of C."""
     out_pos = before_out.count("Tensor")
-    _LIBRARY.define(f"{name}({before_out}, {after_out}) -> Tensor")
-    _LIBRARY.define(f"{name}_out({before_out}, Tensor(a!) out, {after_out}) -> ()")
+    native = name.startswith("gemm_")   # csrc/torch_ops.cpp implements these and calls <name>_general for the rest
+    general = "_general" if native else ""
+    for suffix in ("", general) if native else ("",):
+        _LIBRARY.define(f"{name}{suffix}({before_out}, {after_out}) -> Tensor")
+        _LIBRARY.define(f"{name}_out{suffix}({before_out}, Tensor(a!) out, {after_out}) -> ()")
 
     def functional(*args):
         shape, dtype = out_meta(*args)
@@ -401,8 +415,8 @@ def _register(name, before_out, after_out, run, out_meta):
         if args[out_pos].numel() > 0 or args[0].shape[0] > 0:
             run(*args)
 
-    _LIBRARY.impl(name, functional, "CUDA")
-    _LIBRARY.impl(f"{name}_out", out_variant, "CUDA")
+    _LIBRARY.impl(name + general, functional, "CUDA")
+    _LIBRARY.impl(f"{name}_out{general}", out_variant, "CUDA")
     torch.library.register_fake(f"streamk::{name}", functional_fake, lib=_LIBRARY)
     torch.library.register_fake(f"streamk::{name}_out", lambda *args: None, lib=_LIBRARY)
 
@@ -438,6 +452,7 @@ _register("dequant_q4", "Tensor Wq, Tensor scales, Tensor? zeros", "int zero=8, 
           lambda Wq, scales, zeros, W, zero=8, group=128: _run_dequant_q4(Wq, scales, zeros, W, zero, group),
           lambda Wq, scales, *rest: ((Wq.shape[0], Wq.shape[1] * 2), torch.float16))
 
+_lib.torch_lib()
 _ops = torch.ops.streamk
 
 

@@ -1,5 +1,6 @@
 """Host partitioner front-end: the integers of streamk_fp32.py:30-54 for a run-time shape."""
 import ctypes
+import threading
 
 from . import _lib
 from ._lib import SkConfig, SkPlan
@@ -55,14 +56,17 @@ _tuned = None
 
 
 _tuned_generation = 0
+tuned_lock = threading.Lock()   # a plan enters the native operators' table under the generation it was made from
 
 
 def invalidate_tuned_cache():
     """Forget the loaded tuned cache (the autotuner calls this when it has written an entry).  Plans that other
     layers made from the old cache are told apart by tuned_generation()."""
     global _tuned, _tuned_generation
-    _tuned = None
-    _tuned_generation += 1
+    with tuned_lock:
+        _tuned = None
+        _tuned_generation += 1
+        _lib.torch_lib().sk_torch_clear_plans()
 
 
 def tuned_generation():

@@ -157,3 +157,120 @@ def test_operators_pass_opcheck(sk):
     opcheck(ops.gemm_f8.default, (f8a, f8b, 0.5, "e4m3"), test_utils=tests)
     torch.cuda.synchronize()
     sk.workspace_status()
+
+
+def _calls_of(fn):
+    """The streamk operators a call goes through, and its result or the type of its exception."""
+    import torch
+    with torch.autograd.profiler.profile() as prof:
+        try:
+            out = fn()
+        except Exception as e:  # noqa: BLE001
+            out = type(e)
+    return [e.name.split("::")[1] for e in prof.function_events if e.name.startswith("streamk::")], out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["gemm_f16", "gemm_bf16", "gemm_f32", "gemm_f8", "gemm_i8", "gemm_q4"])
+def test_native_operators_answer_like_the_general_ones(name):
+    """Calls of every form, twice each: by the operator -- natively once its plan is known -- and by the Python
+    implementation it stands in for.  Same bits, or the same exception; ordinary forms run natively from the second call
+    on, the others never do."""
+    import torch
+    import streamk
+    ops = torch.ops.streamk
+    op, general = getattr(ops, name), getattr(ops, name + "_general")
+    out_op, out_general = getattr(ops, name + "_out"), getattr(ops, name + "_out_general")
+    torch.manual_seed(5)
+    M, N, K = 5, 264, 384
+    kind = {"gemm_f16": torch.float16, "gemm_bf16": torch.bfloat16, "gemm_f32": torch.float32, "gemm_f8": torch.float8_e4m3fn,
+            "gemm_i8": torch.int8, "gemm_q4": torch.float16}[name]
+    ctype = {"gemm_f8": torch.float16, "gemm_i8": torch.int32}.get(name, kind)
+
+    def mat(rows, cols):
+        if kind == torch.int8:
+            return torch.randint(-9, 10, (rows, cols), device="cuda", dtype=kind)
+        return torch.randint(-3, 4, (rows, cols), device="cuda").float().to(kind)
+
+    A, big = mat(M, K), mat(M + 2, K + 64)
+    q4 = name == "gemm_q4"
+    Wq = torch.randint(0, 256, (N, K // 2), device="cuda", dtype=torch.uint8)
+    sc, zp = torch.rand(N, K // 128, device="cuda").half(), torch.randint(0, 16, (N, K // 128), device="cuda").half()
+    weights = (Wq, sc, None) if q4 else (mat(N, K),)
+    bias = torch.randint(-5, 6, (N,), device="cuda").to(ctype)
+    lead = {"gemm_f8": (0.5, ""), "gemm_q4": (8, 128, False)}.get(name, () if name == "gemm_i8" else ("nt",))
+    epi = (bias, "relu") if name not in ("gemm_f32", "gemm_i8") else ()
+    ordinary = [(A, *weights, *lead), (A[:1], *weights, *lead), (big[1:1 + M, 16:16 + K], *weights, *lead)]
+    other = [(A[:0], *weights, *lead),                                              # no rows
+             (A.cpu(), *weights, *lead), (A.double(), *weights, *lead), (A[:, :-128], *weights, *lead),   # refused
+             (A.t(), *weights, *lead), (A[0], *weights, *lead), (A, *weights, *lead, "schedule=dp")]
+    if epi:
+        ordinary += [(A, *weights, *lead, "", *epi), (A, *weights, *lead, "", None, "silu")]
+        other += [(A, *weights, *lead, "", bias[:-1], "none"), (A, *weights, *lead, "", None, "tanh"),
+                  (A, *weights, *lead, "", bias.double(), "none")]
+    if name in ("gemm_f16", "gemm_bf16", "gemm_f32"):
+        ordinary += [(A, mat(K, N), "nn"), (A, mat(N, K + 8)[:, :K], "nt")]
+        other += [(A, mat(N, K), "tn")]
+    if kind in (torch.float16, torch.bfloat16):
+        other += [(big[:M, 1:1 + K], *weights, *lead)]                              # copied before the launch
+    if name == "gemm_f8":
+        ordinary += [(A, *weights, 0.25, "e4m3")]
+        other += [(A, *weights, 0.25, "e5m2"), (A.view(torch.uint8), weights[0].view(torch.uint8), 1.0, "e4m3"), (A, *weights, float("nan"), "")]
+    if q4:
+        ordinary += [(A, Wq, sc, zp), (A, Wq, sc, None, 3), (torch.randn(80, K, device="cuda").half(), Wq, sc, None)]
+        other += [(A, Wq, sc, zp.to(torch.uint8)), (A, Wq, sc, zp[:, :2]), (A, Wq, sc, None, 16), (A, Wq, sc, None, 8, 64),
+                  (A, Wq.t().contiguous().t(), sc, None), (A, streamk.tile_q4(Wq), sc, None, 8, 128, True),
+                  (torch.randn(80, K, device="cuda").half(), Wq, sc, zp), (torch.randn(1100, K, device="cuda").half(), Wq, sc, None)]
+
+    def same(a, b):
+        return a is b if isinstance(a, type) or isinstance(b, type) else (a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b))
+
+    n_operands = 4 if q4 else 2
+    for native, args in [(True, x) for x in ordinary] + [(False, x) for x in other]:
+        if q4 and len(args) < 4:
+            args = args + (None,)
+        _, want = _calls_of(lambda: general(*args))
+        _, first = _calls_of(lambda: op(*args))
+        names, got = _calls_of(lambda: op(*args))
+        text = [tuple(a.shape) if isinstance(a, torch.Tensor) else a for a in args]
+        assert same(first, want) and same(got, want), (text, want, got)
+        if isinstance(want, torch.Tensor) and native:
+            assert names == [name], (text, names)
+        elif not native:
+            assert names[:1] == [name] and (name + "_general" in names or isinstance(want, type)), (text, names)
+        if isinstance(want, torch.Tensor):   # into a caller's C, rows further apart than they are long
+            C = torch.full((want.shape[0], want.shape[1] + 8), 7, device="cuda", dtype=ctype)
+            out_op(*args[:n_operands], C[:, :-8], *args[n_operands:])
+            assert torch.equal(C[:, :-8], want) and (C[:, -8:] == 7).all(), text
+            bad = torch.empty(want.shape[0] + 1, want.shape[1], device="cuda", dtype=ctype)
+            assert _calls_of(lambda: out_op(*args[:n_operands], bad, *args[n_operands:]))[1] is \
+                _calls_of(lambda: out_general(*args[:n_operands], bad, *args[n_operands:]))[1]
+    # workspaces taken back: the general implementation makes a new one where the plan needs it
+    streamk.reset_workspaces()
+    for args in ordinary:
+        assert torch.equal(op(*args, *((None,) if q4 and len(args) < 4 else ())), general(*args, *((None,) if q4 and len(args) < 4 else ())))
+    # another stream, a graph, and a tuned cache that changed
+    args = ordinary[0]
+    want = general(*args)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        got = op(*args)
+    s.synchronize()
+    assert torch.equal(got, want)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        got = op(*args)
+    for _ in range(3):
+        torch.cuda.synchronize()
+        got.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+    streamk.plan.invalidate_tuned_cache()
+    names, got = _calls_of(lambda: op(*args))
+    assert names == [name, name + "_general"] and torch.equal(got, want)
+    if kind.is_floating_point and kind != torch.float8_e4m3fn:   # an input that requires a gradient: the result as it was
+        x = args[0].clone().requires_grad_()
+        assert op(x, *args[1:]).requires_grad == general(x, *args[1:]).requires_grad
+    streamk.workspace_status()
