@@ -296,6 +296,14 @@ struct KernelInfo {
 // byte of weights -- was measured and is not built: 16 x 16384 x 16384 split in two over K 39.7 us against 39.4 for the
 // 64-row instance and 37.5 for the general kernel, 16 x 8192 x 8192 17.8 against 13.8)
 
+// 65 to 128 rows, fp16 / bfloat16 NT, rings of different depths for weights and A (tile_ring16.h; variant 9, taken when
+// asked for by variant or by the planner's rule):  X(id, BM, BN, BK, WM, WN, KH, slots of weights, slots of A, BF16)
+#define SK_TILE_RING_KERNELS(X)                 \
+  X(380, 128, 64, 64, 2, 2, 2, 9, 5, false)     \
+  X(381, 128, 64, 64, 2, 2, 2, 9, 5, true)      \
+  X(382, 128, 128, 64, 2, 2, 2, 6, 4, false)    \
+  X(383, 128, 128, 64, 2, 2, 2, 6, 4, true)
+
 // Up to 16 rows of A, Q4 weights, every wave streaming K on its own (tile_rows_q4.h; dtypes SK_Q4, SK_Q4_ZP and
 // SK_Q4_ZP_TILED, variant 5; taken when asked for by variant or by the planner's rule):
 // X(id, rows of A staged, blocks of 16 weight rows, slots, per-group zero points, scale groups in LDS, tiled weights)

@@ -47,7 +47,7 @@ int launch_tile_asm8(int id, const GemmArgs &a, const DevPlan &p, const Workspac
     SK_TILE_ASM8_KERNELS(X)
 #undef X
   }
-  return launch_tile_q4(id, a, p, ws, s, bias);
+  return launch_tile_ring(id, a, p, ws, s, bias);
 }
 
 int occupancy_tile_asm8(int id) {
@@ -62,7 +62,7 @@ int occupancy_tile_asm8(int id) {
     SK_TILE_ASM8_KERNELS(X)
 #undef X
   }
-  return occupancy_tile_q4(id);
+  return occupancy_tile_ring(id);
 }
 
 }  // namespace sk

@@ -40,6 +40,9 @@ int occupancy_stream_bytes(int id);
 int tile_q4_kernel_infos(KernelInfo *out, int max);
 int launch_tile_q4(int id, const GemmArgs &a, const DevPlan &p, const Workspace &ws, hipStream_t s, const void *bias);
 int occupancy_tile_q4(int id);
+// tile kernels for 65 to 128 rows of 16-bit operands (translation unit kernels_tile_ring.hip)
+int launch_tile_ring(int id, const GemmArgs &a, const DevPlan &p, const Workspace &ws, hipStream_t s, const void *bias);
+int occupancy_tile_ring(int id);
 // tile kernels for one-byte operands (translation unit kernels_tile_8bit.hip)
 int tile_8bit_kernel_infos(KernelInfo *out, int max);
 int launch_tile_8bit(int id, const GemmArgs &a, const DevPlan &p, const Workspace &ws, hipStream_t s, const void *bias);

@@ -26,6 +26,7 @@ int tile_8bit_kernel_infos(KernelInfo *out, int max);
 int skinny_kernel_infos(KernelInfo *out, int max);
 int rows_q4_kernel_infos(KernelInfo *out, int max);
 int stream_bytes_kernel_infos(KernelInfo *out, int max);
+int tile_ring_kernel_infos(KernelInfo *out, int max);
 int f32_kernel_infos(KernelInfo *out, int max);
 
 const KernelInfo *kernel_table(int *count) {
@@ -38,6 +39,7 @@ const KernelInfo *kernel_table(int *count) {
     n += skinny_kernel_infos(g_table + n, 400 - n);
     n += rows_q4_kernel_infos(g_table + n, 400 - n);
     n += stream_bytes_kernel_infos(g_table + n, 400 - n);
+    n += tile_ring_kernel_infos(g_table + n, 400 - n);
     n += f32_kernel_infos(g_table + n, 400 - n);
     g_count = n;
   });
@@ -66,9 +68,9 @@ static int variant_rank(const KernelInfo &k) {
   return k.variant == 7 ? 4 : (k.variant == 4 ? 3 : (k.variant == 1 ? 2 : (k.variant == 2 ? 1 : 0)));
 }
 // kernels that a tile alone does not name: the Q4 ones whose waves stream K on their own, and the ones that stream one-byte
-// weights through LDS
+// weights through LDS, and the tile kernels for 65 to 128 rows
 static bool by_variant_only(const KernelInfo &k) {
-  return k.family == FAMILY_SKINNY && (k.variant == 5 || k.variant == 8);
+  return k.variant == 9 || (k.family == FAMILY_SKINNY && (k.variant == 5 || k.variant == 8));
 }
 static bool accepts_shape(const KernelInfo &k, int64_t M, int64_t K) {
   // (the assembly-loop tile kernels have no K tail: other K go to the next-best variant of the tile)
@@ -446,6 +448,50 @@ static const KernelInfo *model_pick(int64_t M, int64_t N, int64_t K, int dtype, 
   return best;
 }
 
+// ---- 65 to 128 rows of fp16 / bfloat16, NT: the ring kernels' tile and split of K ----
+// time = o + rounds * iterations * (t + u * busy CUs / CUs) + fix-up(split), fitted to 60 timings, weights from HBM
+// (within 6 % of each).  100 rows, the tile kernels of the table above / these, in us: 4096 x 11008 42.0 / 33.5,
+// 2048 x 8192 29.1 / 21.4, 5120 x 5120 35.2 / 27.2, 8192 x 8192 48.9 / 40.2, 28672 x 8192 130 / 98, 11008 x 4096 37.4 / 34.4.
+// From K = 1536 on: 110 x 22712 x 1688 37.5 / 34.7, 110 x 1024 x 1024 8.8 / 10.3, 110 x 28672 x 1024 20.4 / 21.6.
+struct RingFamily {
+  int bn;
+  double o, t, u, fix, per_log2;
+};
+static const RingFamily kFamiliesRing[] = {{64, 3.9, 0.395, 0.09, 2.6, 2.6}, {128, 2.4, 0.55, 0.22, 3.5, 4.3}};
+static const KernelInfo *model_pick_ring(int64_t N, int64_t K, int dtype, int num_cus, sk_config *out) {
+  const KernelInfo *best = nullptr;
+  double best_time = 0;
+  int count;
+  const KernelInfo *t = kernel_table(&count);
+  for (const RingFamily &f : kFamiliesRing) {
+    const KernelInfo *k = nullptr;
+    for (int i = 0; i < count && !k; ++i)
+      if (t[i].family == FAMILY_TILE && t[i].variant == 9 && t[i].dtype == dtype && t[i].bn == f.bn) k = &t[i];
+    if (!k) continue;
+    const int64_t tiles = cdiv(N, f.bn), ipt = cdiv(K, k->bk);
+    for (int s = 1; s <= 8; s *= 2) {
+      if (s > 1 && (tiles * s > num_cus || ipt / s < 8)) continue;
+      const double busy = tiles * s < num_cus ? (double)(tiles * s) / num_cus : 1.0;
+      const double time = f.o + (double)cdiv(tiles * s, num_cus) * ((double)ipt / s) * (f.t + f.u * busy) +
+                          (s == 1 ? 0.0 : f.fix + f.per_log2 * (s == 2 ? 1 : (s == 4 ? 2 : 3)));
+      if (best && time >= best_time) continue;
+      best = k;
+      best_time = time;
+      const bool even = ipt % s == 0;
+      out->schedule = s == 1 ? SK_SCHED_DP : (even ? SK_SCHED_SPLIT_K : SK_SCHED_SK_BASIC);
+      out->grid = s > 1 && !even ? (int)(tiles * s) : 0;
+      out->reserved[1] = s > 1 && even ? s : 0;
+    }
+  }
+  if (best) {
+    out->bm = best->bm;
+    out->bn = best->bn;
+    out->bk = best->bk;
+    out->reserved[0] = best->variant + 1;
+  }
+  return best;
+}
+
 // ---- fp32: tile, schedule and grid, when the caller leaves all three open ----
 // The matrix pipe is slow enough (64 FLOP per cycle and SIMD) that tiles of 64 x 64 keep it busy; what decides is how
 // many CTAs there are and whether two of them share a CU (one computes while the other waits at its barrier).  Model,
@@ -545,10 +591,18 @@ extern "C" int sk_make_plan(int64_t M, int64_t N, int64_t K, int dtype, int layo
   // tile, variant, schedule and grid all left open for a 16-bit or one-byte problem with more rows than the
   // weight-streaming kernels take: the cost model chooses kernel and split
   sk_config modelled;
-  if ((dtype == SK_F16 || dtype == SK_BF16 || dtype == SK_F8E4M3 || dtype == SK_F8E5M2 || dtype == SK_I8) && M > 64 &&
+  const bool model_applies =
+      (dtype == SK_F16 || dtype == SK_BF16 || dtype == SK_F8E4M3 || dtype == SK_F8E5M2 || dtype == SK_I8) && M > 64 &&
       !rows_65_to_96_stream(M, N, dtype, layout, num_cus) &&
       (!cfg || (cfg->bm == 0 && cfg->bn == 0 && cfg->bk == 0 && cfg->reserved[0] == 0 &&
-                cfg->schedule == SK_SCHED_AUTO && cfg->grid == 0))) {
+                cfg->schedule == SK_SCHED_AUTO && cfg->grid == 0));
+  if (model_applies) {
+    if (cfg) modelled = *cfg; else memset(&modelled, 0, sizeof(modelled));
+    if ((dtype == SK_F16 || dtype == SK_BF16) && layout == SK_LAYOUT_NT && M <= 128 && K >= 1536 &&
+        model_pick_ring(N, K, dtype, num_cus, &modelled))
+      cfg = &modelled;
+  }
+  if (cfg != &modelled && model_applies) {
     int split = 1, model_sched = SK_SCHED_AUTO;
     if (const KernelInfo *mk = model_pick(M, N, K, dtype, layout, num_cus, &split, &model_sched)) {
       if (cfg) modelled = *cfg; else memset(&modelled, 0, sizeof(modelled));

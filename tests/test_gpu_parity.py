@@ -2523,3 +2523,54 @@ def test_one_byte_weights_streamed_through_lds(sk, dtype):
     for M, N in ((1, 4096), (16, 8192), (16, 8224), (17, 8192), (32, 8224), (33, 4096), (64, 28672)):
         assert sk.kernel_name(sk.make_plan(M, N, 4096, dtype, "nt", sk.plan.operator_config(M, N, 4096, dtype, "nt"), cus=256).kernel_id).startswith("stream_"), (M, N)
     sk.workspace_status()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_ring_tile_kernels(sk, dtype):
+    """The tile kernels with rings of different depths for weights and A: rows and columns around the tiles' edges, K from
+    one 16-byte piece to more iterations than the rings have slots, every schedule and fix-up, bias and activation.
+    Integer operands keep every partial sum exact, so C must equal the host product rounded once; A's rows end in NaN,
+    C's in a marker."""
+    import torch
+    rng = np.random.default_rng(380)
+    kind = getattr(torch, dtype)
+    f = sk.streamk_fp16 if dtype == "float16" else sk.streamk_bf16
+    ran = set()
+    for bn in (64, 128):
+        for N, K in ((bn, 8), (bn - 3, 72), (bn + 5, 640), (3 * bn, 1544)):
+            A = rng.integers(-3, 4, (131, K)).astype(np.float32)
+            B = rng.integers(-3, 4, (N, K)).astype(np.float32)
+            bias = rng.integers(-8, 9, N).astype(np.float32)
+            full = A @ B.T
+            tB, tb = torch.from_numpy(B).to(kind).cuda(), torch.from_numpy(bias).to(kind).cuda()
+            for M in (1, 127, 128, 131):
+                Ap = torch.full((M, K + 8), float("nan"), device="cuda", dtype=kind)
+                Ap[:, :K] = torch.from_numpy(A[:M]).to(kind).cuda()
+                want = torch.from_numpy(full[:M]).to(kind)
+                act = torch.from_numpy(np.maximum(full[:M] + bias, 0)).to(kind)
+                Cp = torch.empty(M, N + 4, device="cuda", dtype=kind)
+                iters = -(-K // 64) * -(-N // bn) * -(-M // 128)
+                for sch in (dict(schedule="dp"), dict(schedule="dp", grid=2), dict(schedule="basic", fixup="reduce", grid=5),
+                            dict(schedule="basic", fixup="atomic", grid=7), dict(schedule="splitk", split=2)):
+                    if sch.get("grid", 0) > iters or (sch["schedule"] == "splitk" and -(-K // 64) % 2):
+                        continue   # (a CTA keeps at least one iteration)
+                    plan = sk.make_plan(M, N, K, dtype, "nt", dict(bm=128, bn=bn, bk=64, variant=10, **sch), cus=256)
+                    assert "_ring_" in sk.kernel_name(plan.kernel_id)
+                    Cp.fill_(7.0)
+                    f(Ap[:, :K], tB, out=Cp[:, :N], plan=plan)
+                    assert torch.equal(Cp[:, :N].cpu(), want) and (Cp[:, N:] == 7).all(), (M, N, K, bn, sch)
+                    assert torch.equal(f(Ap[:, :K], tB, plan=plan, bias=tb, activation="relu").cpu(), act), (M, N, K, bn, sch)
+                    ran.add(plan.kernel_id)
+    assert len(ran) == 2
+    for N, K, ring in ((4096, 11008, True), (28672, 8192, True), (1024, 1000, False), (777, 3000, True)):
+        plan = sk.make_plan(100, N, K, dtype, "nt", cus=256, use_tuned=False)
+        assert ("_ring_" in sk.kernel_name(plan.kernel_id)) == ring, (N, K)
+        if ring:
+            A, B = torch.randn(100, K, device="cuda").to(kind), (torch.randn(N, K, device="cuda") / K ** 0.5).to(kind)
+            ref = A.double().cpu() @ B.double().cpu().T if N <= 4096 else A.double() @ B.double().T
+            C = f(A, B, plan=plan).double().to(ref.device)
+            assert (C - ref).norm() / ref.norm() <= (2.5e-3 if dtype == "bfloat16" else 4e-4), (N, K)   # one rounding of C
+    # the tile alone names the kernels it named before
+    assert "_ring_" not in sk.kernel_name(sk.make_plan(100, 4096, 4096, dtype, "nt", dict(bm=128, bn=128, bk=64), cus=256).kernel_id)
+    sk.workspace_status()
