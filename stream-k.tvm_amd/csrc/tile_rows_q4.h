@@ -14,8 +14,11 @@
 //    piece p of a row of A at p ^ row: the 16 lanes served together then read 16 different bank groups.  Rows of A beyond
 //    the MR staged ones repeat them: they only reach rows of the result that are not stored.  TILED_: the weights come in
 //    tiles of 16 rows x 64 bytes (see tile_skinny.h), a load then reads one of them; everything else is the same.
-//  * The nibbles go into the MFMA as the exact integers q - zero (1024 + q and 64 + q minus 1024 + zero and 64 + zero in
-//    fp16) and the group's scale multiplies the fp32 group sum, so no weight is rounded.
+//  * The nibbles become the exact integers q - zero (1024 + q and 64 + q minus 1024 + zero and 64 + zero in fp16).  With
+//    one zero point for the matrix they go into the MFMA as they are and the group's scale multiplies the fp32 group sum,
+//    so no weight is rounded.  With per-group zero points (ZP_) the contract for more than one row is the rounded weights
+//    bit for bit -- what the dequantiser and the kernels for more rows give, blocks of one call among them: they are
+//    multiplied by the scale in fp16 first and the sums run on in the accumulators.
 //
 // What bounds it: launch, arguments and the first trip to memory are about 4 us, then the weights stream; without the
 // decode and the MFMAs 4 x 11008 x 4096 takes 9.0 us, without the loads of A 11.0, as it is 11.1 (one row: 7.2).  Weights
@@ -133,7 +136,8 @@ struct TileRowsQ4 : TileStreamPairs<1, 1, NB_, 1, 3, false> {
       const char *a_rd[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) a_rd[q] = smem + wave * RING + W_BYTES + (fi % MR) * 256 + 16 * ((4 * fg + q) ^ (fi % MR));
-      const half_t *s_rd = lds_s + 4 * fg, *z_rd = lds_z + fi;
+      // scales: of the four weight rows whose sums the lane holds, or of the weight row it decodes (ZP_)
+      const half_t *s_rd = lds_s + (ZP_ ? fi : 4 * fg), *z_rd = lds_z + fi;
       Q4Consts qc;
       q4_pin_patterns(qc);
       uint32_t magic_hi = 0x54005400u;   // fp16 64.0: 64 + q for the nibbles at bits 4..7 of a half
@@ -152,11 +156,15 @@ struct TileRowsQ4 : TileStreamPairs<1, 1, NB_, 1, 3, false> {
         for (int q = 0; q < 4; ++q) fa[q] = *reinterpret_cast<const half8v *>(a_rd[q] + sofs);
         const int g = group_of(t), gs = min(g, a.groups - 1) - g0;   // (a wave without a group reads zeros and any scale)
         half4v sc[NB];
-        half_t z[NB];
+        half_t z[NB], s[NB];
 #pragma unroll
         for (int j = 0; j < NB; ++j) {
-          sc[j] = *reinterpret_cast<const half4v *>(s_rd + gs * BN + 16 * j);
-          if constexpr (ZP_) z[j] = z_rd[gs * BN + 16 * j];
+          if constexpr (ZP_) {
+            s[j] = s_rd[gs * BN + 16 * j];
+            z[j] = z_rd[gs * BN + 16 * j];
+          } else {
+            sc[j] = *reinterpret_cast<const half4v *>(s_rd + gs * BN + 16 * j);
+          }
         }
         // the slot is read: refill it
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -177,7 +185,7 @@ struct TileRowsQ4 : TileStreamPairs<1, 1, NB_, 1, 3, false> {
             const half_t zero = ZP_ ? z[j] : (half_t)(float)a.zero;
             const half_t lo = (half_t)1024.f + zero, hi = (half_t)64.f + zero;   // exact
             const half2v lo2 = half2v{lo, lo}, hi2 = half2v{hi, hi};
-            AccV sum = AccV{0, 0, 0, 0};
+            AccV sum = ZP_ ? part[j] : AccV{0, 0, 0, 0};
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
               union {
@@ -194,10 +202,19 @@ struct TileRowsQ4 : TileStreamPairs<1, 1, NB_, 1, 3, false> {
               r.h[1] = r.h[1] - hi2;
               r.h[2] = r.h[2] - lo2;
               r.h[3] = r.h[3] - hi2;
+              if constexpr (ZP_) {
+                const half2v s2 = half2v{s[j], s[j]};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) r.h[e] = r.h[e] * s2;
+              }
               sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(r.v, fa[q], sum, 0, 0, 0);
             }
+            if constexpr (ZP_) {
+              part[j] = sum;
+            } else {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) part[j][r] = __builtin_fmaf(sum[r], (float)sc[j][r], part[j][r]);
+              for (int r = 0; r < 4; ++r) part[j][r] = __builtin_fmaf(sum[r], (float)sc[j][r], part[j][r]);
+            }
           }
         }
         slot = slot + 1 == S ? 0 : slot + 1;

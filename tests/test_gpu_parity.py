@@ -2475,6 +2475,45 @@ def test_q4_waves_streaming_k_on_their_own(sk, oracle, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["q4_zp", "q4_zp_tiled"])
+def test_q4_zero_point_kernels_multiply_the_rounded_weights(sk, oracle, dtype):
+    """Per-group zero points, more than one row of A: the product is that of the fp16-rounded weights, bit for bit.  Every
+    row of A holds one 1 and one -1 in different scale groups, so C is the difference of two rounded weights: exact in
+    fp32 (both are fp16 within 2^13 of each other) and rounded to fp16 once.  The unrounded (q - zero) * scale differ
+    from it where the two nearly cancel.  A call of more than 64 rows goes in blocks: its last rows equal the same rows in
+    the first block."""
+    import torch
+    rng = np.random.default_rng(311)
+    for N, K in ((200, 1152), (72, 4096)):
+        Wq = rng.integers(0, 256, (N, K // 2), dtype=np.uint8)
+        sc = rng.uniform(0.005, 0.02, (N, K // 128)).astype(np.float16)
+        zp = rng.integers(0, 16, (N, K // 128)).astype(np.float16)
+        W = oracle.dequant_q4_zp_np(Wq, sc, zp).astype(np.float64)
+        A = np.zeros((16, K), np.float16)
+        for m in range(16):
+            g1, g2 = rng.choice(K // 128, 2, replace=False)
+            A[m, g1 * 128 + rng.integers(128)], A[m, g2 * 128 + rng.integers(128)] = 1, -1
+        want = (A.astype(np.float64) @ W.T).astype(np.float16)
+        exact = A.astype(np.float64) @ ((oracle.unpack_q4_np(Wq).astype(np.float64) - np.repeat(zp, 128, axis=1).astype(np.float64))
+                                        * np.repeat(sc, 128, axis=1).astype(np.float64)).T
+        assert not np.array_equal(want, exact.astype(np.float16))   # (the two forms can be told apart)
+        dA, dW, dS, dZ = _t(A), _t(Wq), _t(sc), _t(zp)
+        kw = dict(zeros=dZ, tiled=dtype == "q4_zp_tiled")
+        if kw["tiled"]:
+            dW = sk.tile_q4(dW)
+        for M in (2, 4, 5, 8, 9, 16):
+            plan = sk.make_plan(M, N, K, dtype, "nt", use_tuned=False)
+            assert np.array_equal(sk.streamk_q4(dA[:M].contiguous(), dW, dS, plan=plan, **kw).cpu().numpy(), want[:M]), (M, N, K)
+            for bn in (16, 32, 48, 64):
+                plan = sk.make_plan(M, N, K, dtype, "nt", dict(bm=16, bn=bn, bk=1024, variant=6, schedule="dp"))
+                assert np.array_equal(sk.streamk_q4(dA[:M].contiguous(), dW, dS, plan=plan, **kw).cpu().numpy(), want[:M]), (M, N, K, bn)
+        A72 = torch.cat([dA, dA, dA, dA, dA[:8]])
+        C = sk.streamk_q4(A72, dW, dS, **kw).cpu().numpy()
+        assert np.array_equal(C, np.concatenate([want] * 4 + [want[:8]])), (N, K)
+    sk.workspace_status()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["float8_e4m3", "float8_e5m2", "int8"])
 def test_one_byte_weights_streamed_through_lds(sk, dtype):
     """The kernels that stream one-byte weights through LDS (16, 32 and 64 rows of A, tiles of 16 to 64 weight rows): M
