@@ -598,7 +598,11 @@ extern "C" int sk_make_plan(int64_t M, int64_t N, int64_t K, int dtype, int layo
                 cfg->schedule == SK_SCHED_AUTO && cfg->grid == 0));
   if (model_applies) {
     if (cfg) modelled = *cfg; else memset(&modelled, 0, sizeof(modelled));
+    // (the ring kernels add up fp32 partial tiles: a fix-up that adds packed 16-bit partials into C, or exchanges them in 16
+    // bits, is a matter of the other tile kernels)
+    const int fixup = modelled.fixup;
     if ((dtype == SK_F16 || dtype == SK_BF16) && layout == SK_LAYOUT_NT && M <= 128 && K >= 1536 &&
+        (fixup == SK_FIXUP_AUTO || fixup == SK_FIXUP_REDUCE || fixup == SK_FIXUP_ATOMIC) &&
         model_pick_ring(N, K, dtype, num_cus, &modelled))
       cfg = &modelled;
   }

@@ -131,6 +131,23 @@ def test_fp8_plans(sk):
         sk.make_plan(256, 256, 264, "float8_e4m3", "nt", cus=256)   # K not a multiple of 16
 
 
+def test_65_to_128_rows_take_every_fixup(sk):
+    """16-bit products of 65 to 128 rows with nothing but the fix-up given: each of the fix-ups that add up fp32 partials,
+    and the reference's packed atomics into C, get a plan (the ring kernels, which have no atomics into C, only for the
+    others)."""
+    for dtype in ("float16", "bfloat16"):
+        for layout in ("nt", "nn"):
+            for M in (65, 100, 128):
+                for N, K in ((4096, 4096), (11008, 4096), (1024, 16384), (520, 2048), (8, 2312), (28672, 8192)):
+                    for fixup in ("auto", "reduce", "atomic", "atomic_c"):
+                        streams = M <= 96 and layout == "nt" and 5 * -(-N // 32) >= 3 * 256 and -(-N // 32) <= 256
+                        if fixup == "atomic_c" and streams:
+                            continue   # (the 96-row weight-streaming kernels never had it)
+                        p = sk.make_plan(M, N, K, dtype, layout, cus=256, fixup=fixup)
+                        ring = "_ring_" in sk.kernel_name(p.kernel_id)
+                        assert ring == (layout == "nt" and fixup != "atomic_c" and not streams), (M, N, K, dtype, layout, fixup)
+
+
 def test_raster_is_a_permutation(sk):
     plan = sk.make_plan(3000, 5120, 4096, "float16", "nt", cus=256, bm=128, bn=128, bk=64, raster=8)
     seen = {sk.tile_coords(plan, t) for t in range(plan.total_tiles)}

@@ -350,6 +350,26 @@ def test_reference_fixup_packed_atomics_into_c(sk, oracle):
     sk.workspace_status()
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 1024, 8192), (100, 1000, 4096), (128, 4096, 4096)])
+def test_reference_fixup_with_65_to_128_rows(sk, oracle, M, N, K):
+    """The packed atomics into C asked for with nothing else, on rows that the ring kernels take otherwise: exact on
+    integer data (every partial and every sum below 2048), C handed over full of garbage; bfloat16 on data whose sums
+    stay below 256."""
+    import torch
+    rng = np.random.default_rng(290)
+    A, B = rng.integers(-1, 2, (M, K)).astype(np.float16), rng.integers(-1, 2, (N, K)).astype(np.float16)
+    A[:, 1500:] = 0
+    exact = A.astype(np.float32) @ B.astype(np.float32).T
+    assert np.abs(exact).max() < 2048
+    C = sk.streamk_fp16(_t(A), _t(B), fixup="atomic_c", out=torch.full((M, N), 777.0, dtype=torch.float16, device="cuda"))
+    assert np.array_equal(C.float().cpu().numpy(), exact)
+    A[:, 200:] = 0
+    exact = A.astype(np.float32) @ B.astype(np.float32).T
+    C = sk.streamk_bf16(_t(A).bfloat16(), _t(B).bfloat16(), fixup="atomic_c")
+    assert np.array_equal(C.float().cpu().numpy(), exact)
+    sk.workspace_status()
+
+
 def test_assembly_loop_tile_kernels(sk, oracle, golden_dir):
     """The four-wave 256 x 256 x 64 kernels whose K loop is hand-scheduled assembly (accumulators in the
     accumulation registers): fp16 and bfloat16, NT and NN, ragged M and N, K any multiple of 64 (odd and even iteration
