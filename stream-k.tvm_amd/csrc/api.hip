@@ -147,6 +147,8 @@ int check_plan(const sk_plan *plan, int64_t M, int64_t N, int64_t K, int dtype, 
 // is_static: ws is the library's own static workspace (no registry entry; prepared by its own kernel)
 int make_dev_plan(const sk_plan *plan, const KernelInfo *k, void *ws, size_t ws_bytes, int occupancy,
                   hipStream_t stream, DevPlan *dp, Workspace *w, bool is_static = false) {
+  // (a plan kept from a library in which this kernel had another tile: its partition would be of something else)
+  if (plan->bm != k->bm || plan->bn != k->bn || plan->bk != k->bk) return SK_ERR_CONFIG;
   if ((size_t)plan->workspace_bytes > ws_bytes) return SK_ERR_WORKSPACE;
   if (plan->workspace_bytes > 0 && !ws) return SK_ERR_WORKSPACE;
   if (plan->workspace_bytes > 0 && (reinterpret_cast<uintptr_t>(ws) & 255)) return SK_ERR_ALIGN;

@@ -12,18 +12,23 @@ __global__ __launch_bounds__(P::NT, P::WAVES_PER_EU) void sk_f32_kernel(typename
 }
 
 // X(id, B is [K,N], BM, BN, BK, WM, WN, stages, CTAs per CU); the reference's own fp32 run is 16 x 16384 x 8192
-// (streamk_fp32.py:10-12 with the values of :24-28)
+// (streamk_fp32.py:10-12 with the values of :24-28).  A tile without its K-iteration, or a schedule or grid without a tile,
+// names the first four: 16 K-values, two CTAs per CU.  The [N,K] tiles of 128 x 128 and 32 x 256 also exist with 32, which
+// the planner takes when everything is left to it (weights from HBM, 16 / 32 K-values, in us: 32 x 8192 x 8192 71.6 / 67.4,
+// 32 x 28672 x 4096 112 / 106, 32 x 11008 x 4096 53.5 / 52.7, 16 x 16384 x 8192 103 / 104).
 #define SK_F32_KERNELS(X)                    \
   X(200, true, 128, 128, 16, 2, 2, 4, 2)     \
-  X(201, false, 128, 128, 32, 2, 2, 2, 2)    \
-  X(202, true, 32, 256, 16, 1, 4, 8, 1)      \
-  X(203, false, 32, 256, 32, 1, 4, 4, 1)     \
+  X(201, false, 128, 128, 16, 2, 2, 4, 2)    \
+  X(202, true, 32, 256, 16, 1, 4, 4, 2)      \
+  X(203, false, 32, 256, 16, 1, 4, 4, 2)     \
   X(204, true, 64, 64, 32, 2, 2, 5, 2)       \
   X(205, false, 64, 64, 32, 2, 2, 5, 2)      \
   X(206, true, 64, 128, 32, 2, 2, 3, 2)      \
   X(207, false, 64, 128, 32, 2, 2, 3, 2)     \
   X(208, true, 32, 64, 32, 1, 4, 6, 2)       \
-  X(209, false, 32, 64, 64, 1, 4, 6, 1)
+  X(209, false, 32, 64, 64, 1, 4, 6, 1)      \
+  X(212, false, 128, 128, 32, 2, 2, 2, 2)    \
+  X(213, false, 32, 256, 32, 1, 4, 4, 1)
 
 int f32_kernel_infos(KernelInfo *out, int max) {
   int n = 0;

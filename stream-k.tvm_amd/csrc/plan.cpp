@@ -521,17 +521,20 @@ static const KernelInfo *model_pick_f32(int64_t M, int64_t N, int64_t K, int lay
     const bool tiny = M > 128 && N > 128 && M <= 256 && N <= 256;
     if (tiny && f.bm != 128) continue;
     const KernelInfo *k = nullptr;
-    for (int i = 0; i < count && !k; ++i)
-      if (t[i].dtype == SK_F32 && t[i].layout == layout && t[i].bm == f.bm && t[i].bn == f.bn) k = &t[i];
+    for (int i = 0; i < count; ++i)   // (the instance with the longest K-iteration: see kernels_f32.hip)
+      if (t[i].dtype == SK_F32 && t[i].layout == layout && t[i].bm == f.bm && t[i].bn == f.bn && (!k || t[i].bk > k->bk)) k = &t[i];
     if (!k) continue;
-    const int64_t tiles = cdiv(M, f.bm) * cdiv(N, f.bn), ipt = cdiv(K, k->bk), cap = (int64_t)num_cus * k->ctas_per_cu;
+    // (a tile that gains nothing from a second CTA on its CU is offered one: 16 x 16384 x 8192 on 256 CTAs of 32 x 256
+    // 99.7 us, on 512 110)
+    const int ctas = f.two > f.one ? k->ctas_per_cu : 1;
+    const int64_t tiles = cdiv(M, f.bm) * cdiv(N, f.bn), ipt = cdiv(K, k->bk), cap = (int64_t)num_cus * ctas;
     const double tile_us = (double)(f.bm == 32 && M <= 16 ? 16 : f.bm) * f.bn * K * 2 / 0.614e6;
     const double bytes_us = 4.0 * ((double)N * K + (double)M * K + (double)M * N) / 5.1e6 / (f.bn == 256 ? 1.05 : 1.0);
     auto consider = [&](int sched, int64_t grid, int split) {
       double comp, fix = 0;
       const double contributors = (double)grid / tiles;
       if (sched == SK_SCHED_DP) {
-        comp = (double)cdiv(tiles, num_cus) * tile_us / (tiles > num_cus && k->ctas_per_cu > 1 ? f.two : f.one);
+        comp = (double)cdiv(tiles, num_cus) * tile_us / (tiles > num_cus && ctas > 1 ? f.two : f.one);
       } else {
         comp = (double)cdiv(grid, num_cus) / contributors * tile_us / (grid > num_cus ? f.two : f.one);
         fix = 1.7 + 0.34 * f.bm * f.bn / 8192 * (contributors > 1 ? contributors : 1);

@@ -148,6 +148,31 @@ def test_65_to_128_rows_take_every_fixup(sk):
                         assert ring == (layout == "nt" and fixup != "atomic_c" and not streams), (M, N, K, dtype, layout, fixup)
 
 
+def test_fp32_tiles_keep_their_iterations_and_grids(sk):
+    """fp32 with a tile, a grid or a split of the caller's: K-iterations of 16 in both layouts, two CTAs per CU, split
+    factors of K / 16; what the planner takes by itself ([N,K]: iterations of 32) can be named as well."""
+    for layout in ("nn", "nt"):
+        for bm, bn in ((128, 128), (32, 256)):
+            for tile in (dict(bm=bm, bn=bn, bk=16), dict(bm=bm, bn=bn)):
+                p = sk.make_plan(24, 4096, 1040, "float32", layout, cus=256, **tile)
+                assert (p.bm, p.bn, p.bk, p.iters_per_tile) == (bm, bn, 16, 65)
+                p = sk.make_plan(24, 4096, 1040, "float32", layout, cus=256, schedule="basic", grid=512, **tile)
+                assert (p.grid, p.streamk_tiles) == (512, p.total_tiles)
+                p = sk.make_plan(24, 4096, 1040, "float32", layout, cus=256, schedule="splitk", split=13, **tile)
+                assert p.grid == 13 * p.total_tiles
+        for M, tile in ((16, (32, 256, 16)), (100, (128, 128, 16))):
+            p = sk.make_plan(M, 4096, 1040, "float32", layout, cus=256, schedule="sk1", grid=512)
+            assert (p.bm, p.bn, p.bk) == tile and p.grid == 512
+            p = sk.make_plan(M, 4096, 1040, "float32", layout, cus=256, schedule="splitk", split=5)
+            assert (p.bm, p.bn, p.bk) == tile and p.grid == 5 * p.total_tiles
+    assert [sk.kernel_name(i) for i in (200, 201, 202, 203)] == ["tile_f32_nn_128x128x16", "tile_f32_nt_128x128x16",
+                                                                 "tile_f32_nn_32x256x16", "tile_f32_nt_32x256x16"]
+    for M, N, K, tile in ((16, 16384, 8192, (32, 256, 32)), (4096, 4096, 4096, (128, 128, 32))):
+        p = sk.make_plan(M, N, K, "float32", "nt", cus=256)
+        assert (p.bm, p.bn, p.bk) == tile
+        assert sk.make_plan(M, N, K, "float32", "nt", cus=256, bm=tile[0], bn=tile[1], bk=32).kernel_id == p.kernel_id
+
+
 def test_raster_is_a_permutation(sk):
     plan = sk.make_plan(3000, 5120, 4096, "float16", "nt", cus=256, bm=128, bn=128, bk=64, raster=8)
     seen = {sk.tile_coords(plan, t) for t in range(plan.total_tiles)}

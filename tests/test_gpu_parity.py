@@ -2431,6 +2431,33 @@ def test_fp32_tile_edges(sk, bm, bn, layout):
     sk.workspace_status()
 
 
+@pytest.mark.parametrize("layout,bm,bn,bk", [("nn", 128, 128, 16), ("nt", 128, 128, 16), ("nt", 128, 128, 32), ("nn", 32, 256, 16),
+                                            ("nt", 32, 256, 16), ("nt", 32, 256, 32)])
+def test_fp32_tiles_by_their_k_iteration(sk, layout, bm, bn, bk):
+    """The fp32 tiles that exist with one or two lengths of the K-iteration, named with it: K around one iteration and over
+    more of them than the ring has slots, whole tiles and tiles split over more CTAs than there are CUs (two to a CU
+    where that many stay resident).  Integer operands: C equals the host product."""
+    import torch
+    rng = np.random.default_rng(bm + bk)
+    cus, per_cu = sk.num_cus(), 1 if (bm, bk) == (32, 32) else 2
+    for M, N, K in ((bm - 3, bn + 4, bk - 4), (bm + 1, 2 * bn, bk + 4), (7, 8 * bn, 96 * bk)):
+        A, B = rng.integers(-4, 5, (M, K)).astype(np.float32), rng.integers(-4, 5, (K, N)).astype(np.float32)
+        dA, dB = _t(A), _t(B if layout == "nn" else np.ascontiguousarray(B.T))
+        want = A.astype(np.float64) @ B.astype(np.float64)
+        schedules = [dict(schedule="dp")]
+        if K > 90 * bk:
+            schedules += [dict(schedule="basic", grid=per_cu * cus, fixup=f) for f in ("reduce", "atomic")] + [dict(schedule="splitk", split=6)]
+        for sch in schedules:
+            plan = sk.make_plan(M, N, K, "float32", layout, dict(bm=bm, bn=bn, bk=bk, **sch))
+            assert (plan.bm, plan.bn, plan.bk) == (bm, bn, bk)
+            assert np.array_equal(sk.streamk_fp32(dA, dB, layout=layout, plan=plan).double().cpu().numpy(), want), (M, N, K, sch)
+    # a plan whose tile is not the kernel's
+    plan.bk *= 2
+    with pytest.raises(sk.StreamKError):
+        sk.streamk_fp32(dA, dB, layout=layout, plan=plan)
+    sk.workspace_status()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["q4", "q4_zp", "q4_zp_tiled"])
 def test_q4_waves_streaming_k_on_their_own(sk, oracle, dtype):
