@@ -78,6 +78,16 @@ static bool accepts_shape(const KernelInfo &k, int64_t M, int64_t K) {
          (k.family != FAMILY_TILE || k.variant != 7 || K % k.k_align == 0);
 }
 
+// whether the kernel can run the grid or the fixed split that a configuration names
+static bool takes_partition(const KernelInfo &k, int64_t M, int64_t N, int64_t K, const sk_config *cfg, int num_cus) {
+  if (!cfg) return true;
+  const int64_t most = (int64_t)num_cus * k.ctas_per_cu;
+  if (cfg->grid > most) return false;
+  if (cfg->schedule != SK_SCHED_SPLIT_K) return true;
+  const int64_t split = cfg->reserved[1] > 0 ? cfg->reserved[1] : 1;
+  return cdiv(K, k.bk) % split == 0 && cdiv(M, k.bm) * cdiv(N, k.bn) * split <= most;
+}
+
 // 65 to 96 rows of fp16 / bfloat16 (NT) whose 96 x 32 tiles fill the device in one round: see pick_kernel
 static bool rows_65_to_96_stream(int64_t M, int64_t N, int dtype, int layout, int num_cus) {
   return (dtype == SK_F16 || dtype == SK_BF16) && layout == SK_LAYOUT_NT && M > 64 && M <= 96 && cdiv(N, 32) <= num_cus &&
@@ -93,12 +103,15 @@ static const KernelInfo *pick_kernel(int64_t M, int64_t N, int64_t K, int dtype,
   const int want_variant = cfg ? cfg->reserved[0] - 1 : -1;
   if (want_tile) {
     const KernelInfo *found = nullptr;
-    for (int i = 0; i < n; ++i)
-      if (t[i].dtype == dtype && t[i].layout == layout && t[i].bm == cfg->bm && t[i].bn == cfg->bn &&
-          (cfg->bk <= 0 || t[i].bk == cfg->bk) &&
-          (want_variant < 0 ? !by_variant_only(t[i]) : t[i].variant == want_variant) &&
-          accepts_shape(t[i], M, K) && (found == nullptr || variant_rank(t[i]) > variant_rank(*found)))
-        found = &t[i];
+    // (fp32 tiles that exist with two lengths of the K-iteration: the first that takes the caller's grid or split)
+    for (int pass = dtype == SK_F32 ? 0 : 1; pass < 2 && !found; ++pass)
+      for (int i = 0; i < n; ++i)
+        if (t[i].dtype == dtype && t[i].layout == layout && t[i].bm == cfg->bm && t[i].bn == cfg->bn &&
+            (cfg->bk <= 0 || t[i].bk == cfg->bk) &&
+            (want_variant < 0 ? !by_variant_only(t[i]) : t[i].variant == want_variant) &&
+            (pass > 0 || takes_partition(t[i], M, N, K, cfg, num_cus)) &&
+            accepts_shape(t[i], M, K) && (found == nullptr || variant_rank(t[i]) > variant_rank(*found)))
+          found = &t[i];
     return found;
   }
   // heuristic: small M -> weight-streaming kernels; otherwise the largest tile that still gives
@@ -198,7 +211,10 @@ static const KernelInfo *pick_kernel(int64_t M, int64_t N, int64_t K, int dtype,
     // rounds of 32 13.2).  With one zero point for the matrix up to 8 rows, where 64-row tiles run in one round (beyond,
     // 4 x 28672 x 8192: 31.9 us on the general kernel against 38); 5 to 8 rows on 32-row tiles stay with the kernel
     // that streams through shared LDS (8 x 5120 x 5120: 8.1 us against 8.7, 8 x 8192 x 8192: 11.8 / 11.9).
-    if ((dtype == SK_Q4_ZP || dtype == SK_Q4_ZP_TILED || (dtype == SK_Q4 && M <= 8 && cdiv(N, 64) <= num_cus)) && M > 1 && M <= 16 && want_variant < 0) {
+    // (a caller's grid or fixed split that they cannot take -- more CTAs than stay resident, a factor that does not divide
+    // their K-iterations -- goes to the kernels below)
+    if ((dtype == SK_Q4_ZP || dtype == SK_Q4_ZP_TILED || (dtype == SK_Q4 && M <= 8 && cdiv(N, 64) <= num_cus)) && M > 1 && M <= 16 &&
+        want_variant < 0) {
       int64_t least = 0;
       for (int i = 0; i < n; ++i) {
         if (t[i].family != FAMILY_SKINNY || t[i].dtype != dtype || t[i].variant != 5 || !accepts_shape(t[i], M, K)) continue;
@@ -209,7 +225,7 @@ static const KernelInfo *pick_kernel(int64_t M, int64_t N, int64_t K, int dtype,
           least = busiest;
         }
       }
-      if (best && !(dtype == SK_Q4 && M > 4 && best->bn == 32 && K % 256 == 0)) return best;
+      if (best && takes_partition(*best, M, N, K, cfg, num_cus) && !(dtype == SK_Q4 && M > 4 && best->bn == 32 && K % 256 == 0)) return best;
       best = nullptr;
     }
     // 2 <= M <= 16 with row-major Q4 weights (scalar zero point), weights from HBM.  Where 64-row tiles give three
@@ -265,8 +281,8 @@ static const KernelInfo *pick_kernel(int64_t M, int64_t N, int64_t K, int dtype,
     const int want_bm = M <= 32 ? 32 : 128;
     const KernelInfo *any = nullptr;
     for (int i = 0; i < n; ++i)
-      if (t[i].dtype == SK_F32 && t[i].layout == layout) {
-        if (t[i].bm == want_bm) return &t[i];
+      if (t[i].dtype == SK_F32 && t[i].layout == layout && t[i].bm == want_bm && t[i].bn == (want_bm == 32 ? 256 : 128)) {
+        if (takes_partition(t[i], M, N, K, cfg, num_cus)) return &t[i];
         if (!any) any = &t[i];
       }
     return any;

@@ -165,12 +165,29 @@ def test_fp32_tiles_keep_their_iterations_and_grids(sk):
             assert (p.bm, p.bn, p.bk) == tile and p.grid == 512
             p = sk.make_plan(M, 4096, 1040, "float32", layout, cus=256, schedule="splitk", split=5)
             assert (p.bm, p.bn, p.bk) == tile and p.grid == 5 * p.total_tiles
+    # (a split that only the iterations of 32 divide into)
+    assert sk.make_plan(100, 1920, 460, "float32", "nt", cus=256, schedule="splitk", split=3).bk == 32
+    assert sk.make_plan(100, 1920, 460, "float32", "nt", cus=256, bm=128, bn=128, schedule="splitk", split=3).bk == 32
     assert [sk.kernel_name(i) for i in (200, 201, 202, 203)] == ["tile_f32_nn_128x128x16", "tile_f32_nt_128x128x16",
                                                                  "tile_f32_nn_32x256x16", "tile_f32_nt_32x256x16"]
     for M, N, K, tile in ((16, 16384, 8192, (32, 256, 32)), (4096, 4096, 4096, (128, 128, 32))):
         p = sk.make_plan(M, N, K, "float32", "nt", cus=256)
         assert (p.bm, p.bn, p.bk) == tile
         assert sk.make_plan(M, N, K, "float32", "nt", cus=256, bm=tile[0], bn=tile[1], bk=32).kernel_id == p.kernel_id
+
+
+def test_few_rows_of_q4_take_a_callers_grid_and_split(sk):
+    """Q4 with few rows of A and a grid or a fixed split of the caller's: up to two CTAs per CU and split factors of the
+    general small-M kernels' K-iterations, as ever; what the kernels whose waves stream K on their own can run is theirs."""
+    for dtype, M, N, K, cfg in (("q4", 3, 15168, 2304, dict(schedule="basic", grid=512)), ("q4", 5, 11096, 512, dict(schedule="sk1", grid=300)),
+                                ("q4", 2, 11592, 1024, dict(schedule="dp", grid=300)),
+                                ("q4_zp_tiled", 10, 1024, 9344, dict(schedule="splitk", split=5))):
+        p = sk.make_plan(M, N, K, dtype, "nt", cus=256, **cfg)
+        assert p.grid == cfg.get("grid", p.grid) or p.schedule == 1
+        assert p.grid == 5 * p.total_tiles or "split" not in cfg
+        assert not sk.kernel_name(p.kernel_id).startswith("rows_q4")
+        for free in (dict(), dict(schedule="dp"), dict(schedule="basic", grid=200), dict(fixup="atomic"), dict(schedule="splitk", split=2)):
+            assert sk.kernel_name(sk.make_plan(4, 2048, 4096, dtype, "nt", cus=256, **free).kernel_id).startswith("rows_q4")
 
 
 def test_raster_is_a_permutation(sk):
