@@ -7,7 +7,9 @@
 // missing or too small, operands that have to be copied first or that the checks refuse -- goes, with its arguments as
 // they are, to the Python implementation (streamk::<name>_general), which answers it or raises.  Kept here are plans, by
 // shape, device and type, and the addresses of the workspaces that the Python layer owns, by device and stream; it tells
-// of both and takes both back (sk_torch_*), and the library refuses a workspace that has been released in between.
+// of both and takes both back (sk_torch_*).  A call holds the tables' lock, shared, from the look-up until its kernels are
+// enqueued; a workspace is taken back under the same lock, exclusively, before its memory goes to the allocator, which
+// orders whatever uses it next on that stream behind them.
 // (A call's host time now: 5.9 to 10 us, of which the launch is about 3.)
 #include <ATen/ATen.h>
 #include <ATen/core/dispatch/Dispatcher.h>
@@ -18,6 +20,7 @@
 
 #include <map>
 #include <mutex>
+#include <shared_mutex>
 #include <optional>
 #include <string>
 #include <tuple>
@@ -31,7 +34,7 @@ using torch::jit::Stack;
 // (M, N, K, dtype, layout, device)
 typedef std::tuple<int64_t, int64_t, int64_t, int, int, int> PlanKey;
 constexpr size_t MAX_PLANS = 4096;
-std::mutex g_mutex;
+std::shared_mutex g_mutex;
 struct Buffer {
   void *ptr = nullptr;
   size_t bytes = 0;
@@ -39,15 +42,17 @@ struct Buffer {
 std::map<PlanKey, sk_plan> g_plans;
 std::map<std::pair<int, void *>, Buffer> g_workspaces;
 
-// what a launch on the current stream takes beside the operands
+// what a launch on the current stream takes beside the operands; the workspace is there as long as this is.  (Nothing but
+// the launch happens while it lives: an allocation could run a caller's code, which may call an operator itself.)
 struct Launch {
+  std::shared_lock<std::shared_mutex> lock{g_mutex, std::defer_lock};
   sk_plan plan;
   Buffer ws;
   void *stream;
   bool find(int64_t M, int64_t N, int64_t K, int dtype, int layout) {
     const int device = (int)c10::hip::current_device();
     stream = (void *)c10::hip::getCurrentHIPStream().stream();
-    std::lock_guard<std::mutex> lock(g_mutex);
+    lock.lock();
     const auto it = g_plans.find(PlanKey(M, N, K, dtype, layout, device));
     if (it == g_plans.end()) return false;
     plan = it->second;
@@ -104,13 +109,13 @@ at::Tensor gemm_16bit(const at::Tensor &A, const at::Tensor &B, const at::Tensor
   const bool nt = layout == "nt";
   const int64_t M = A.size(0), K = A.size(1), N = B.size(nt ? 0 : 1);
   if (B.size(nt ? 1 : 0) != K) return {};
-  Launch l;
-  if (!l.find(M, N, K, dtype, nt ? SK_LAYOUT_NT : SK_LAYOUT_NN)) return {};
   sk_epilogue epi;
   bool used;
   if (!epilogue(a[2], a[3], A, N, type, &epi, &used)) return {};
   at::Tensor C = result(out, A, M, N, type);
   if (!C.defined()) return {};
+  Launch l;
+  if (!l.find(M, N, K, dtype, nt ? SK_LAYOUT_NT : SK_LAYOUT_NN)) return {};
   const int rc = (dtype == SK_F16 ? sk_gemm_f16_ex : sk_gemm_bf16_ex)(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, A.stride(0),
                                                                       B.stride(0), C.stride(0), &l.plan, l.ws.ptr, l.ws.bytes, l.stream,
                                                                       used ? &epi : nullptr);
@@ -125,10 +130,10 @@ at::Tensor gemm_f32(const at::Tensor &A, const at::Tensor &B, const at::Tensor *
   const bool nt = layout == "nt";
   const int64_t M = A.size(0), K = A.size(1), N = B.size(nt ? 0 : 1);
   if (B.size(nt ? 1 : 0) != K) return {};
-  Launch l;
-  if (!l.find(M, N, K, SK_F32, nt ? SK_LAYOUT_NT : SK_LAYOUT_NN)) return {};
   at::Tensor C = result(out, A, M, N, at::kFloat);
   if (!C.defined()) return {};
+  Launch l;
+  if (!l.find(M, N, K, SK_F32, nt ? SK_LAYOUT_NT : SK_LAYOUT_NN)) return {};
   const int rc = sk_gemm_f32(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, A.stride(0), B.stride(0), C.stride(0), &l.plan, l.ws.ptr, l.ws.bytes, l.stream);
   return rc == SK_OK ? C : at::Tensor();
 }
@@ -142,13 +147,13 @@ at::Tensor gemm_f8(const at::Tensor &A, const at::Tensor &B, const at::Tensor *o
   if (!is_matrix(A, type) || !is_matrix(B, type) || A.size(0) == 0) return {};
   const int64_t M = A.size(0), K = A.size(1), N = B.size(0);
   if (B.size(1) != K) return {};
-  Launch l;
-  if (!l.find(M, N, K, type == at::kFloat8_e5m2 ? SK_F8E5M2 : SK_F8E4M3, SK_LAYOUT_NT)) return {};
   sk_epilogue epi;
   bool used;
   if (!epilogue(a[3], a[4], A, N, at::kHalf, &epi, &used)) return {};
   at::Tensor C = result(out, A, M, N, at::kHalf);
   if (!C.defined()) return {};
+  Launch l;
+  if (!l.find(M, N, K, type == at::kFloat8_e5m2 ? SK_F8E5M2 : SK_F8E4M3, SK_LAYOUT_NT)) return {};
   const int rc = sk_gemm_f8_ex(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, A.stride(0), B.stride(0), C.stride(0),
                                (float)a[0].toDouble(), &l.plan, l.ws.ptr, l.ws.bytes, l.stream, used ? &epi : nullptr);
   return rc == SK_OK ? C : at::Tensor();
@@ -159,10 +164,10 @@ at::Tensor gemm_i8(const at::Tensor &A, const at::Tensor &B, const at::Tensor *o
   if (!a[0].toStringRef().empty() || !is_matrix(A, at::kChar) || !is_matrix(B, at::kChar) || A.size(0) == 0) return {};
   const int64_t M = A.size(0), K = A.size(1), N = B.size(0);
   if (B.size(1) != K) return {};
-  Launch l;
-  if (!l.find(M, N, K, SK_I8, SK_LAYOUT_NT)) return {};
   at::Tensor C = result(out, A, M, N, at::kInt);
   if (!C.defined()) return {};
+  Launch l;
+  if (!l.find(M, N, K, SK_I8, SK_LAYOUT_NT)) return {};
   const int rc = sk_gemm_i8(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, A.stride(0), B.stride(0), C.stride(0), &l.plan, l.ws.ptr, l.ws.bytes, l.stream);
   return rc == SK_OK ? C : at::Tensor();
 }
@@ -187,13 +192,13 @@ at::Tensor gemm_q4(const c10::IValue *operands, const at::Tensor *out, const c10
     zeros = z.data_ptr();
   }
   if (M > (zp ? 64 : 1024)) return {};
-  Launch l;
-  if (!l.find(M, N, K, zp ? SK_Q4_ZP : SK_Q4, SK_LAYOUT_NT)) return {};
   sk_epilogue epi;
   bool used;
   if (!epilogue(a[4], a[5], A, N, at::kHalf, &epi, &used)) return {};
   at::Tensor C = result(out, A, M, N, at::kHalf);
   if (!C.defined()) return {};
+  Launch l;
+  if (!l.find(M, N, K, zp ? SK_Q4_ZP : SK_Q4, SK_LAYOUT_NT)) return {};
   const int rc = sk_gemm_q4_ex(A.data_ptr(), Wq.data_ptr(), scales.data_ptr(), zeros, C.data_ptr(), M, N, K, A.stride(0), C.stride(0),
                                (int)group, zp ? 0 : (int)zero, &l.plan, l.ws.ptr, l.ws.bytes, l.stream, used ? &epi : nullptr);
   return rc == SK_OK ? C : at::Tensor();
@@ -242,19 +247,24 @@ TORCH_LIBRARY_IMPL(streamk, CUDA, m) {
 #undef IMPL
 }
 
-// plan of an operator call without a configuration of its own
-extern "C" __attribute__((visibility("default"))) void sk_torch_add_plan(const sk_plan *plan, int device) {
+// plan of an operator call without a configuration of its own.  (Nothing is thrown through these C entries: a plan or a
+// workspace that there is no memory to note is one that the general implementation serves.)
+extern "C" __attribute__((visibility("default"))) void sk_torch_add_plan(const sk_plan *plan, int device) try {
   if (plan == nullptr) return;
-  std::lock_guard<std::mutex> lock(g_mutex);
+  std::lock_guard<std::shared_mutex> lock(g_mutex);
   if (g_plans.size() < MAX_PLANS) g_plans[PlanKey(plan->M, plan->N, plan->K, plan->dtype, plan->layout, device)] = *plan;
+} catch (...) {
 }
-extern "C" __attribute__((visibility("default"))) void sk_torch_clear_plans(void) {
-  std::lock_guard<std::mutex> lock(g_mutex);
+extern "C" __attribute__((visibility("default"))) void sk_torch_clear_plans(void) try {
+  std::lock_guard<std::shared_mutex> lock(g_mutex);
   g_plans.clear();
+} catch (...) {
 }
 // the workspace that operator calls on a stream use, initialised (null: forget it); the caller keeps the memory alive
-extern "C" __attribute__((visibility("default"))) void sk_torch_set_workspace(int device, void *stream, void *ptr, size_t bytes) {
-  std::lock_guard<std::mutex> lock(g_mutex);
+// until it has taken it back here
+extern "C" __attribute__((visibility("default"))) void sk_torch_set_workspace(int device, void *stream, void *ptr, size_t bytes) try {
+  std::lock_guard<std::shared_mutex> lock(g_mutex);
   if (ptr != nullptr) g_workspaces[{device, stream}] = Buffer{ptr, bytes};
   else g_workspaces.erase({device, stream});
+} catch (...) {
 }

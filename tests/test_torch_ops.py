@@ -274,3 +274,87 @@ def test_native_operators_answer_like_the_general_ones(name):
         x = args[0].clone().requires_grad_()
         assert op(x, *args[1:]).requires_grad == general(x, *args[1:]).requires_grad
     streamk.workspace_status()
+
+
+# (two shapes per operator whose plans split tiles: one that the smallest workspace serves, one that it does not)
+_SPLIT_SHAPES = {"gemm_f16": ("float16", (64, 256, 4096), (100, 4096, 8192)), "gemm_bf16": ("bfloat16", (64, 256, 4096), (100, 4096, 8192)),
+                 "gemm_f32": ("float32", (16, 256, 2048), (512, 1024, 4096)), "gemm_f8": ("float8_e4m3", (100, 512, 8192), (300, 1024, 16384)),
+                 "gemm_i8": ("int8", (80, 256, 4096), (300, 1024, 8192)), "gemm_q4": ("q4", (64, 256, 4096), (300, 1024, 8192))}
+
+
+def test_split_shapes_need_the_workspaces_they_stand_for(sk):
+    for dtype, small, large in _SPLIT_SHAPES.values():
+        sizes = [sk.make_plan(*shape, dtype, "nt", sk.plan.operator_config(*shape, dtype, "nt"), cus=256).workspace_bytes for shape in (small, large)]
+        assert 0 < sizes[0] <= 1 << 20 < sizes[1], (dtype, sizes)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", sorted(_SPLIT_SHAPES))
+def test_native_operators_with_a_workspace(name):
+    """Calls whose plans split tiles: natively from the second call on, on the workspace that the Python layer owns -- after
+    it was taken back, after it grew and for the smaller plan on the grown one, on a stream of its own, replayed from a
+    graph between eager calls, and with another thread's calls on the same stream.  Bits as the general implementation."""
+    import sys
+    import threading
+    import torch
+    import streamk
+    dtype, *shapes = _SPLIT_SHAPES[name]
+    op, general = getattr(torch.ops.streamk, name), getattr(torch.ops.streamk, name + "_general")
+    torch.manual_seed(6)
+    kind = {"q4": torch.float16, "float8_e4m3": torch.float8_e4m3fn}.get(dtype, getattr(torch, dtype, None))
+    calls, wants = [], []
+    for M, N, K in shapes:
+        plan = sys.modules["streamk.ops"]._plan_for("", M, N, K, dtype, "nt")
+        assert plan.workspace_bytes > (0 if not calls else 1 << 20)
+        A = torch.randint(-3, 4, (M, K), device="cuda").float().to(kind)
+        if name == "gemm_q4":
+            args = (A, torch.randint(0, 256, (N, K // 2), device="cuda", dtype=torch.uint8), torch.rand(N, K // 128, device="cuda").half(), None)
+        else:
+            args = (A, torch.randint(-3, 4, (N, K), device="cuda").float().to(kind)) + (("nt",) if kind != torch.float8_e4m3fn and name != "gemm_i8" else ())
+        calls.append(args)
+    streamk.reset_workspaces()
+    wants = [general(*args) for args in calls]
+
+    def check(args, want, native):
+        names, got = _calls_of(lambda: op(*args))
+        assert names == ([name] if native else [name, name + "_general"]), names
+        assert torch.equal(got, want)
+
+    small, large = zip(calls, wants)
+    for _ in range(2):
+        streamk.reset_workspaces()
+        check(*small, False)    # nothing to launch with: the general implementation makes a workspace
+        check(*small, True)
+        check(*large, False)    # too small: it makes a larger one
+        check(*large, True)
+        check(*small, True)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        check(*large, False)
+        check(*small, True)
+    s.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        got = op(*small[0])
+    for _ in range(3):
+        got.zero_()
+        check(*large, True)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, small[1])
+    # two threads on one stream: both run natively on its workspace, one behind the other
+    wrong = []
+
+    def calls_of_a_thread(args, want):
+        for _ in range(20):
+            if not torch.equal(op(*args), want):
+                wrong.append(args[0].shape)
+
+    threads = [threading.Thread(target=calls_of_a_thread, args=pair) for pair in (small, large)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong, wrong
+    streamk.workspace_status()
