@@ -466,14 +466,20 @@ static const KernelInfo *model_pick(int64_t M, int64_t N, int64_t K, int dtype, 
 
 // ---- 65 to 128 rows of fp16 / bfloat16, NT: the ring kernels' tile and split of K ----
 // time = o + rounds * iterations * (t + u * busy CUs / CUs) + fix-up(split), fitted to 60 timings, weights from HBM
-// (within 6 % of each).  100 rows, the tile kernels of the table above / these, in us: 4096 x 11008 42.0 / 33.5,
+// (within 6 % of each); a split that does not divide the iterations costs 3 to 5 us more, as its CTAs cross from one tile into
+// the next (100 x 11008 x 4160, 65 iterations: 128-wide tiles in two 38.7, whole 64-wide ones 35.7).  100 rows, the tile kernels of the table above / these, in us: 4096 x 11008 42.0 / 33.5,
 // 2048 x 8192 29.1 / 21.4, 5120 x 5120 35.2 / 27.2, 8192 x 8192 48.9 / 40.2, 28672 x 8192 130 / 98, 11008 x 4096 37.4 / 34.4.
-// From K = 1536 on: 110 x 22712 x 1688 37.5 / 34.7, 110 x 1024 x 1024 8.8 / 10.3, 110 x 28672 x 1024 20.4 / 21.6.
 struct RingFamily {
   int bn;
-  double o, t, u, fix, per_log2;
+  double o, t, u, fix, per_log2, uneven;
 };
-static const RingFamily kFamiliesRing[] = {{64, 3.9, 0.395, 0.09, 2.6, 2.6}, {128, 2.4, 0.55, 0.22, 3.5, 4.3}};
+static const RingFamily kFamiliesRing[] = {{64, 3.9, 0.395, 0.09, 2.6, 2.6, 3.0}, {128, 2.4, 0.55, 0.22, 3.5, 4.3, 5.0}};
+// Short K and few columns give a CTA too few iterations for its deep ring to fill: there the tile kernels stay (100 rows, tile
+// kernels / these, in us: K = 1024: 1024 wide 8.8 / 10.3, 28672 20.4 / 21.6; K = 1536: 1024 wide 10.8 / 13.1, 4096 14.6 / 15.0,
+// 11008 20.0 / 17.5, 28672 29.2 / 29.0; K = 2048: 256 to 1024 wide 11.8 / 12.0, 1536 15.1 / 13.0, 4096 16.7 / 15.4; K = 2176:
+// 256 to 1024 wide 12.2 / 14.4; K = 2816: 777 wide 14.2 / 14.5, 1024 15.1 / 13.8; K = 3000: 777 wide 23.6 / 18.8; K = 3072:
+// 256 wide 14.2 / 13.3, 1024 16.4 / 14.5; 66 and 128 rows alike).
+static bool ring_pays(int64_t N, int64_t K) { return K >= 2880 || (K >= 2048 && N >= 1536) || (K >= 1536 && N >= 8192); }
 static const KernelInfo *model_pick_ring(int64_t N, int64_t K, int dtype, int num_cus, sk_config *out) {
   const KernelInfo *best = nullptr;
   double best_time = 0;
@@ -488,12 +494,12 @@ static const KernelInfo *model_pick_ring(int64_t N, int64_t K, int dtype, int nu
     for (int s = 1; s <= 8; s *= 2) {
       if (s > 1 && (tiles * s > num_cus || ipt / s < 8)) continue;
       const double busy = tiles * s < num_cus ? (double)(tiles * s) / num_cus : 1.0;
+      const bool even = ipt % s == 0;
       const double time = f.o + (double)cdiv(tiles * s, num_cus) * ((double)ipt / s) * (f.t + f.u * busy) +
-                          (s == 1 ? 0.0 : f.fix + f.per_log2 * (s == 2 ? 1 : (s == 4 ? 2 : 3)));
+                          (s == 1 ? 0.0 : f.fix + f.per_log2 * (s == 2 ? 1 : (s == 4 ? 2 : 3)) + (even ? 0 : f.uneven));
       if (best && time >= best_time) continue;
       best = k;
       best_time = time;
-      const bool even = ipt % s == 0;
       out->schedule = s == 1 ? SK_SCHED_DP : (even ? SK_SCHED_SPLIT_K : SK_SCHED_SK_BASIC);
       out->grid = s > 1 && !even ? (int)(tiles * s) : 0;
       out->reserved[1] = s > 1 && even ? s : 0;
@@ -620,7 +626,7 @@ extern "C" int sk_make_plan(int64_t M, int64_t N, int64_t K, int dtype, int layo
     // (the ring kernels add up fp32 partial tiles: a fix-up that adds packed 16-bit partials into C, or exchanges them in 16
     // bits, is a matter of the other tile kernels)
     const int fixup = modelled.fixup;
-    if ((dtype == SK_F16 || dtype == SK_BF16) && layout == SK_LAYOUT_NT && M <= 128 && K >= 1536 &&
+    if ((dtype == SK_F16 || dtype == SK_BF16) && layout == SK_LAYOUT_NT && M <= 128 && ring_pays(N, K) &&
         (fixup == SK_FIXUP_AUTO || fixup == SK_FIXUP_REDUCE || fixup == SK_FIXUP_ATOMIC) &&
         model_pick_ring(N, K, dtype, num_cus, &modelled))
       cfg = &modelled;

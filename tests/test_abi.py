@@ -145,7 +145,18 @@ def test_65_to_128_rows_take_every_fixup(sk):
                             continue   # (the 96-row weight-streaming kernels never had it)
                         p = sk.make_plan(M, N, K, dtype, layout, cus=256, fixup=fixup)
                         ring = "_ring_" in sk.kernel_name(p.kernel_id)
-                        assert ring == (layout == "nt" and fixup != "atomic_c" and not streams), (M, N, K, dtype, layout, fixup)
+                        long = K >= 2880 or (K >= 2048 and N >= 1536)   # (see test_short_k_of_65_to_128_rows...)
+                        assert ring == (layout == "nt" and fixup != "atomic_c" and not streams and long), (M, N, K, dtype, layout, fixup)
+
+
+def test_short_k_of_65_to_128_rows_stays_with_the_tile_kernels(sk):
+    """The ring kernels take 65 to 128 rows where they were measured to be the faster ones: K from 2880 on, from 2048 on with
+    1536 columns, from 1536 on with 8192."""
+    for dtype in ("float16", "bfloat16"):
+        for N, K, ring in ((256, 1536, False), (4096, 1536, False), (8192, 1528, False), (8192, 1536, True), (28672, 1536, True),
+                           (1024, 2048, False), (1528, 2048, False), (1536, 2040, False), (1536, 2048, True), (256, 2872, False), (256, 2880, True), (777, 3000, True)):
+            name = sk.kernel_name(sk.make_plan(100, N, K, dtype, "nt", cus=256).kernel_id)
+            assert ("_ring_" in name) == ring, (N, K, name)
 
 
 def test_fp32_tiles_keep_their_iterations_and_grids(sk):
