@@ -678,15 +678,16 @@ extern "C" int sk_make_plan(int64_t M, int64_t N, int64_t K, int dtype, int layo
     // fp16 / bfloat16: two fifths -- they run data-parallel rather than pay a fix-up; Q4 16 x 11008 x 4096: 11.5 us
     // against 14.3 us, fp16 16 x 2048 x 8192 on 128 tiles: 11.5 against 14.1, 32 x 11008 x 4096 on 172 tiles of 32 x 64:
     // 19.2 against 22.7; not the 64 x 32 tiles, where the split wins)
-    // (one-byte weights through LDS: always up to 32 rows -- 16 x 1024 x 16384 on 64 tiles 11.0 us against 11.4 -- and on
-    // 64 rows unless a CTA would run many iterations while others idle: 64 x 4096 x 4096 9.7 us against 11.9,
-    // 64 x 5120 x 5120 11.9 / 15.4, 64 x 4096 x 11008 20.2 / 18.9, 64 x 2048 x 8192 15.0 / 12.7)
+    // (one-byte weights through LDS: always up to 16 rows -- 16 x 1024 x 16384 on 64 tiles 11.2 us against 11.5, at worst
+    // 16 x 520 x 16384 10.8 / 10.0 -- and on 32 and 64 rows unless a CTA would run many iterations while others idle, data-parallel /
+    // split: 32 x 520 x 8192 9.2 us / 9.2, 32 x 2048 x 8192 11.9 / 11.8, 32 x 520 x 16384 18.5 / 13.6, 32 x 2048 x 16384 19.5 / 15.0,
+    // 64 x 4096 x 4096 9.7 / 11.9, 64 x 5120 x 5120 11.9 / 15.4, 64 x 4096 x 11008 20.2 / 18.9, 64 x 2048 x 8192 15.0 / 12.7)
     const bool stream_bytes = k->family == FAMILY_SKINNY && k->variant == 8;
     // (the Q4 kernels whose waves stream K on their own, variant 5: from two fifths on; 8 x 2048 x 8192 on 128 tiles 7.9 us
     // against 9.9, 16 x 1024 x 16384 on 64 tiles 14.8 / 11.7)
     const bool stream_dp =
         k->family == FAMILY_SKINNY &&
-        (stream_bytes ? k->bm <= 32 || total64 >= num_cus || out->iters_per_tile * (num_cus - total64) <= 8 * num_cus
+        (stream_bytes ? k->bm == 16 || total64 >= num_cus || out->iters_per_tile * (num_cus - total64) <= 8 * num_cus
          : k->variant == 5 ? total64 * 5 >= (int64_t)num_cus * 2
                          : (k->variant == 4 || k->dtype == SK_Q4) && k->max_m >= 16 &&
                                (k->bm == 16 || (k->variant == 4 && k->dtype != SK_Q4 && !(k->bm == 64 && k->bn == 32))) &&

@@ -201,6 +201,18 @@ def test_few_rows_of_q4_take_a_callers_grid_and_split(sk):
             assert sk.kernel_name(sk.make_plan(4, 2048, 4096, dtype, "nt", cus=256, **free).kernel_id).startswith("rows_q4")
 
 
+def test_long_k_of_few_one_byte_rows_is_split(sk):
+    """One-byte operands on the kernels that stream the weights through LDS: 17 to 64 rows on few tiles with a long K are
+    split over the CUs; up to 16 rows, and with few iterations per tile, a CTA takes a whole tile."""
+    for dtype in ("float8_e4m3", "float8_e5m2", "int8"):
+        for M, N, K, split in ((24, 520, 16384, True), (32, 1024, 16384, True), (32, 2048, 16384, True), (17, 64, 16384, True), (32, 2048, 12288, True),
+                               (32, 520, 8192, False), (32, 2048, 8192, False), (32, 4096, 16384, False), (16, 520, 16384, False), (1, 64, 16384, False)):
+            p = sk.make_plan(M, N, K, dtype, "nt", cus=256, variant=9)
+            assert (p.streamk_tiles > 0) == split and (p.grid > 2 * p.total_tiles) == split, (M, N, K, dtype, p.grid, p.total_tiles)
+            if split:   # (at least four iterations of a tile per CTA)
+                assert p.grid <= 256 and 4 * p.grid <= p.total_tiles * p.iters_per_tile
+
+
 def test_raster_is_a_permutation(sk):
     plan = sk.make_plan(3000, 5120, 4096, "float16", "nt", cus=256, bm=128, bn=128, bk=64, raster=8)
     seen = {sk.tile_coords(plan, t) for t in range(plan.total_tiles)}
