@@ -210,7 +210,8 @@ static const KernelInfo *pick_kernel(int64_t M, int64_t N, int64_t K, int dtype,
     // 40.9 us, three of 48 49.9, four of 32 50.0, seven of 16 60.4; 4 x 11008 x 4096: 48 rows 11.1, 64 rows 11.9, two
     // rounds of 32 13.2).  With one zero point for the matrix up to 8 rows, where 64-row tiles run in one round (beyond,
     // 4 x 28672 x 8192: 31.9 us on the general kernel against 38); 5 to 8 rows on 32-row tiles stay with the kernel
-    // that streams through shared LDS (8 x 5120 x 5120: 8.1 us against 8.7, 8 x 8192 x 8192: 11.8 / 11.9).
+    // that streams through shared LDS where that one is taken, from 16 MB of weights on (8 x 5120 x 5120: 8.1 us against
+    // 8.7, 8 x 8192 x 8192: 11.8 / 11.9; below, the general kernel / these: 8 x 5120 x 2048 5.4 / 4.9, 8 x 8192 x 1024 5.2 / 4.2).
     // (a caller's grid or fixed split that they cannot take -- more CTAs than stay resident, a factor that does not divide
     // their K-iterations -- goes to the kernels below)
     if ((dtype == SK_Q4_ZP || dtype == SK_Q4_ZP_TILED || (dtype == SK_Q4 && M <= 8 && cdiv(N, 64) <= num_cus)) && M > 1 && M <= 16 &&
@@ -225,7 +226,8 @@ static const KernelInfo *pick_kernel(int64_t M, int64_t N, int64_t K, int dtype,
           least = busiest;
         }
       }
-      if (best && takes_partition(*best, M, N, K, cfg, num_cus) && !(dtype == SK_Q4 && M > 4 && best->bn == 32 && K % 256 == 0)) return best;
+      const bool shared_lds = dtype == SK_Q4 && M > 4 && best && best->bn == 32 && K % 256 == 0 && N * K >= ((int64_t)16 << 20);
+      if (best && takes_partition(*best, M, N, K, cfg, num_cus) && !shared_lds) return best;
       best = nullptr;
     }
     // 2 <= M <= 16 with row-major Q4 weights (scalar zero point), weights from HBM.  Where 64-row tiles give three

@@ -213,6 +213,14 @@ def test_long_k_of_few_one_byte_rows_is_split(sk):
                 assert p.grid <= 256 and 4 * p.grid <= p.total_tiles * p.iters_per_tile
 
 
+def test_five_to_eight_rows_of_q4_without_a_hole(sk):
+    """5 to 8 rows with one zero point for the matrix: on 32-row tiles the kernel that streams through shared LDS from 16 MB of
+    weights on, the kernels whose waves stream K on their own below."""
+    for M, N, K, name in ((8, 5120, 2048, "rows_q4"), (8, 4352, 3840, "rows_q4"), (5, 8192, 1920, "rows_q4"), (8, 8192, 2048, "stream_q4"),
+                          (8, 5120, 5120, "stream_q4"), (8, 5120, 5248, "rows_q4"), (4, 5120, 2048, "rows_q4")):
+        assert sk.kernel_name(sk.make_plan(M, N, K, "q4", "nt", cus=256).kernel_id).startswith(name), (M, N, K)
+
+
 def test_raster_is_a_permutation(sk):
     plan = sk.make_plan(3000, 5120, 4096, "float16", "nt", cus=256, bm=128, bn=128, bk=64, raster=8)
     seen = {sk.tile_coords(plan, t) for t in range(plan.total_tiles)}
