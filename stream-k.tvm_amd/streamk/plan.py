@@ -74,13 +74,17 @@ def tuned_generation():
     return _tuned_generation
 
 
-def tuned_config(M, N, K, dtype="float16", layout="nt"):
-    """Configuration the autotuner recorded for exactly this problem, or None."""
+def _tuned_entry(M, N, K, dtype, layout):
     global _tuned
     if _tuned is None:
         from .autotune import load_cache
         _tuned = load_cache()
-    hit = _tuned.get(f"gfx950/{dtype}/{layout}/{M}x{N}x{K}")
+    return _tuned.get(f"gfx950/{dtype}/{layout}/{M}x{N}x{K}")
+
+
+def tuned_config(M, N, K, dtype="float16", layout="nt"):
+    """Configuration the autotuner recorded for exactly this problem, or None."""
+    hit = _tuned_entry(M, N, K, dtype, layout)
     if not hit:
         return None
     cfg = dict(hit["config"])
@@ -92,14 +96,22 @@ def tuned_config(M, N, K, dtype="float16", layout="nt"):
 _TWIN_OF = {"bfloat16": "float16", "float8_e5m2": "float8_e4m3"}
 
 
+# search space of the autotuner that has the kernels which stream one-byte weights through LDS; entries carry theirs
+SEARCH_WITH_BYTE_STREAMS = 2
+
+
 def operator_config(M, N, K, dtype, layout):
     """Configuration of an operator call that names none: the tuned one (None: make_plan finds it), else, for up to 64
     rows of one-byte operands, the kernels that stream the weights through LDS (16 x 4096 x 4096 6.5 us against 9.8 on
-    the general small-M kernel that the library's heuristic takes, 64 x 28672 x 8192 56.5 / 67.5)."""
+    the general small-M kernel that the library's heuristic takes, 64 x 28672 x 8192 56.5 / 67.5).  A tuned entry from a
+    search that did not have these kernels does not speak for them: it configures the plans that make_plan gives, and
+    an operator call takes the faster kernel (16 x 8192 x 8192 14.3 us, by the entry 16.7)."""
     if M > 64 or dtype not in ("float8_e4m3", "float8_e5m2", "int8"):
         return None
-    if tuned_config(M, N, K, dtype, layout) or tuned_config(M, N, K, _TWIN_OF.get(dtype, dtype), layout):
-        return None
+    for d in dict.fromkeys((dtype, _TWIN_OF.get(dtype, dtype))):
+        hit = _tuned_entry(M, N, K, d, layout)
+        if hit and hit.get("search", 1) >= SEARCH_WITH_BYTE_STREAMS:
+            return None
     return {"variant": 9}
 
 

@@ -447,3 +447,32 @@ def test_operator_plans_follow_the_tuned_cache(monkeypatch):
     assert (p2.bm, p2.bn) == (256, 256)
     monkeypatch.undo()
     P.invalidate_tuned_cache()
+
+
+def test_one_byte_plans_keep_their_tuned_entries(monkeypatch):
+    """Up to 64 rows of fp8 / int8: a plan made without a configuration is the tuned one where there is an entry (by the
+    e4m3 entry for e5m2); an operator call takes the kernels that stream the weights through LDS unless the entry comes from
+    a search that had them."""
+    import streamk
+    from streamk import ops
+    from streamk import plan as P
+    autotune = sys.modules["streamk.autotune"]
+    monkeypatch.setattr(P, "num_cus", lambda: 256)
+    P.invalidate_tuned_cache()
+    for dtype in ("float8_e4m3", "float8_e5m2", "int8"):
+        p = streamk.make_plan(16, 8192, 8192, dtype)
+        assert (p.bm, p.bn, p.bk, p.schedule) == (16, 32, 1024, 1), dtype
+        p = streamk.make_plan(1, 4096, 11008, dtype)
+        assert (p.bm, p.bn, p.bk) == (16, 16, 1024), dtype
+        for M, N, K in ((16, 8192, 8192), (1, 4096, 11008), (24, 8192, 8192)):
+            assert streamk.kernel_name(ops._plan_for("", M, N, K, dtype, "nt").kernel_id).startswith("stream_"), (dtype, M, N, K)
+    for search, streams in ((None, True), (1, True), (2, False)):
+        entry = {"config": dict(bm=16, bn=64, bk=256, schedule="dp"), **({"search": search} if search else {})}
+        monkeypatch.setattr(autotune, "load_cache", lambda path=None: {"gfx950/float8_e4m3/nt/16x4096x4096": entry})
+        P.invalidate_tuned_cache()
+        for dtype in ("float8_e4m3", "float8_e5m2"):
+            assert streamk.kernel_name(streamk.make_plan(16, 4096, 4096, dtype).kernel_id).startswith("skinny_f8")
+            name = streamk.kernel_name(ops._plan_for("", 16, 4096, 4096, dtype, "nt").kernel_id)
+            assert name.startswith("stream_" if streams else "skinny_"), (search, dtype, name)
+    monkeypatch.undo()
+    P.invalidate_tuned_cache()
