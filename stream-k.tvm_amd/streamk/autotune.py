@@ -16,7 +16,7 @@ import os
 import torch
 
 from . import ops, plan as _plan
-from ._lib import StreamKError
+from ._lib import SCHEDULES, StreamKError
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 DEFAULT_CACHE = os.path.join(_HERE, "tuned", "gfx950.json")
@@ -31,8 +31,15 @@ _STREAM_F16 = [(16, 16, 1024), (16, 32, 512), (16, 64, 256), (32, 32, 256), (32,
                (96, 32, 256)]
 _SKINNY_F8 = [(16, 64, 256), (32, 64, 256), (16, 16, 1024), (16, 32, 512), (16, 32, 1024), (16, 64, 512), (32, 64, 512),
               (64, 64, 256), (64, 64, 512)]
+# one-byte weights streamed through LDS in contiguous loads (variant 9 of these shapes)
+_STREAM_BYTES = [(16, 16, 2048), (16, 32, 1024), (16, 64, 512), (32, 32, 1024), (32, 64, 512), (64, 32, 512), (64, 64, 512)]
 _SKINNY_Q4 = [(16, 64, 256), (32, 64, 256), (64, 64, 256), (16, 16, 1024), (16, 32, 512), (16, 16, 256),
               (16, 32, 256), (16, 32, 1024), (16, 16, 2048), (16, 64, 512), (16, 16, 512)]
+
+
+# which kernels a search had, kept in the entries it writes: 2 has the one-byte kernels that stream the weights through LDS,
+# the Q4 ones whose waves stream K on their own and the ring kernels of 65 to 128 rows
+SEARCH = 2
 
 
 def _key(dtype, layout, M, N, K):
@@ -55,11 +62,43 @@ def save_cache(cache, path=None):
         json.dump(cache, f, indent=1, sort_keys=True)
 
 
-def candidate_configs(M, N, K, dtype="float16", cus=None, reduce16=True):
+def untuned_config(M, N, K, dtype, layout="nt", cus=None):
+    """The configuration that names the plan an operator call runs where nothing has been tuned, or None if no
+    configuration does."""
+    cus = cus or _plan.num_cus()
+    try:
+        untuned = {"variant": 9} if M <= 64 and dtype in ("float8_e4m3", "float8_e5m2", "int8") else None
+        p = _plan.make_plan(M, N, K, dtype, layout, untuned, cus=cus, use_tuned=False)
+    except StreamKError:
+        return None
+    schedule = {v: k for k, v in SCHEDULES.items()}[p.schedule]
+    cfg = dict(bm=p.bm, bn=p.bn, bk=p.bk, schedule=schedule)
+    if schedule == "splitk":
+        cfg["split"] = p.grid // p.total_tiles
+    elif schedule != "dp" or p.grid != p.total_tiles:
+        cfg["grid"] = p.grid
+    if schedule != "dp":
+        cfg["fixup"] = "reduce"
+    if p.raster > 0:
+        cfg["raster"] = p.raster
+    if p.interleave > 1:
+        cfg["interleave"] = 1
+    for variant in range(1, 11):
+        try:
+            q = _plan.make_plan(M, N, K, dtype, layout, dict(cfg, variant=variant), cus=cus)
+        except StreamKError:
+            continue
+        if all(getattr(q, f) == getattr(p, f) for f in ("kernel_id", "grid", "streamk_tiles", "streamk_iters", "schedule", "fixup", "raster", "interleave")):
+            return dict(cfg, variant=variant)
+    return None
+
+
+def candidate_configs(M, N, K, dtype="float16", cus=None, reduce16=True, layout="nt"):
     """The search space.  The reference multiplies out warp/chunk/stage lists
     (autotune/streamk_fp16_autotune.py:38-53); here the axes are tile shape, kernel variant,
     schedule, grid and fix-up.  reduce16=False leaves out the candidates that exchange partial sums rounded to 16
-    bits (fixup 'reduce16': within the 1e-2 every candidate is held to, but not the fp32 sums of the other fix-ups)."""
+    bits (fixup 'reduce16': within the 1e-2 every candidate is held to, but not the fp32 sums of the other fix-ups).  The
+    last candidate is the plan of an untuned call, so that a search never ends behind it."""
     cus = cus or _plan.num_cus()
     out = []
     f8 = dtype in ("float8_e4m3", "float8_e5m2", "int8")  # one-byte operands
@@ -86,6 +125,28 @@ def candidate_configs(M, N, K, dtype="float16", cus=None, reduce16=True):
             out.append(dict(base, schedule="dp"))
             for sched, fixup in (("sk2", "reduce"), ("basic", "reduce"), ("basic", "atomic")):
                 out.append(dict(base, schedule=sched, grid=cus, fixup=fixup))
+    if f8 and M <= 64:
+        for (bm, bn, bk) in _STREAM_BYTES:
+            if bm < M or (bm >= 2 * M and bm > 16):
+                continue
+            base = dict(bm=bm, bn=bn, bk=bk, variant=9)
+            out.append(dict(base, schedule="dp"))
+            tiles = -(-N // bn)
+            for grid in sorted({g for g in (2 * tiles, 4 * tiles, cus) if tiles < g <= cus} | {cus}):
+                out.extend(dict(base, schedule="basic", grid=grid, fixup=fixup) for fixup in ("reduce", "atomic"))
+    if dtype in ("q4", "q4_zp") and 2 <= M <= 16:
+        # Q4 kernels whose waves stream K on their own (variant 6)
+        for bn in (16, 32, 48, 64):
+            base = dict(bm=16, bn=bn, bk=1024, variant=6)
+            out.append(dict(base, schedule="dp"))
+            out.extend(dict(base, schedule="basic", grid=cus, fixup=fixup) for fixup in ("reduce", "atomic"))
+    if dtype in ("float16", "bfloat16") and 64 < M <= 128:
+        # rings of different depths for weights and A (variant 10; NT)
+        for bn in (64, 128):
+            base = dict(bm=128, bn=bn, bk=64, variant=10)
+            out.append(dict(base, schedule="dp"))
+            out.extend(dict(base, schedule="splitk", split=split, fixup="reduce") for split in (2, 4, 8))
+            out.extend(dict(base, schedule="basic", grid=cus, fixup=fixup) for fixup in ("reduce", "atomic"))
     if dtype in ("float16", "bfloat16") and M <= 96:
         for (bm, bn, bk) in _STREAM_F16:
             if bm < M or (bm >= 2 * M and bm > 16):
@@ -136,6 +197,9 @@ def candidate_configs(M, N, K, dtype="float16", cus=None, reduce16=True):
             if -(-M // bm) * -(-N // bn) < cus:
                 out.extend(dict(base, schedule="splitk", fixup=fixup) for fixup in ("reduce", "atomic"))
                 out.append(dict(base, schedule="splitk", split=2, fixup="reduce"))
+    untuned = untuned_config(M, N, K, dtype, layout, cus)
+    if untuned is not None and untuned not in out:
+        out.append(untuned)
     return out
 
 
@@ -243,7 +307,7 @@ def autotune(M, N, K, dtype="float16", layout="nt", *, configs=None, warmup=5, r
         as_b = (lambda b: b.T) if layout == "nt" else (lambda b: b)
         ref_ms = _time_ms(lambda: torch.matmul(A, as_b(rotate(Bs)), out=C), warmup, rep, small)
     small = 2.0 * M * N * K < 5e11  # microsecond kernels: time graph-captured batches
-    configs = configs if configs is not None else candidate_configs(M, N, K, dtype, reduce16=reduce16)
+    configs = configs if configs is not None else candidate_configs(M, N, K, dtype, reduce16=reduce16, layout=layout)
     best, golden, results = None, None, []
     for cfg in configs:
         try:
@@ -296,7 +360,7 @@ def autotune(M, N, K, dtype="float16", layout="nt", *, configs=None, warmup=5, r
         best = min(near, key=lambda r: r[0])
     if cache:
         c = load_cache(cache_path)
-        c[_key(dtype, layout, M, N, K)] = {"config": best[1], "latency_ms": best[0], "ref_latency_ms": ref_ms,
+        c[_key(dtype, layout, M, N, K)] = {"config": best[1], "latency_ms": best[0], "ref_latency_ms": ref_ms, "search": SEARCH,
                                            "box_reference_tflops": box_reference_tflops()}
         save_cache(c, cache_path)
         _plan.invalidate_tuned_cache()

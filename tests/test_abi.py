@@ -476,3 +476,33 @@ def test_one_byte_plans_keep_their_tuned_entries(monkeypatch):
             assert name.startswith("stream_" if streams else "skinny_"), (search, dtype, name)
     monkeypatch.undo()
     P.invalidate_tuned_cache()
+
+
+def test_autotune_offers_what_an_untuned_call_runs():
+    """The search space holds the kernels that operator calls take by themselves -- the byte-streaming, the Q4 rows and the
+    ring ones -- and, as its last resort, the very plan of an untuned call."""
+    import streamk
+    at = sys.modules["streamk.autotune"]
+
+    def named(p):
+        return (streamk.kernel_name(p.kernel_id), p.grid, p.streamk_tiles, p.streamk_iters, p.interleave)
+
+    for dtype, kinds, shapes in (("float8_e4m3", ("stream_f8",), ((1, 4096, 4096), (24, 520, 16384), (64, 28672, 8192))), ("int8", ("stream_i8",), ((16, 8192, 8192),)),
+                                 ("q4_zp", ("rows_q4zp",), ((4, 11008, 4096), (16, 1024, 16384))), ("q4", ("rows_q4", "stream_q4"), ((4, 11008, 4096), (8, 8192, 8192))),
+                                 ("float16", ("_ring_",), ((100, 11008, 4096), (128, 28672, 8192), (100, 777, 3000))), ("bfloat16", ("_ring_",), ((100, 4096, 11008),)),
+                                 ("float16", ("_nt_",), ((1024, 1024, 8192), (3000, 5120, 12288), (8192, 8192, 8192))), ("float32", ("_f32_",), ((16, 4096, 4096),))):
+        for M, N, K in shapes:
+            plans = []
+            for c in at.candidate_configs(M, N, K, dtype, cus=256):
+                try:
+                    plans.append(streamk.make_plan(M, N, K, dtype, "nt", c, cus=256))
+                except streamk.StreamKError:
+                    pass
+            want = streamk.make_plan(M, N, K, dtype, "nt", streamk.plan.operator_config(M, N, K, dtype, "nt") if "8" in dtype else None, cus=256, use_tuned=False)
+            assert named(want) in [named(p) for p in plans], (dtype, M, N, K, named(want))
+            for kind in kinds:
+                assert any(kind in streamk.kernel_name(p.kernel_id) for p in plans), (dtype, M, N, K, kind)
+    for layout in ("nt", "nn"):   # ([K,N] weights: the last candidate is of that layout)
+        c = at.untuned_config(1000, 1000, 1000, "float16", layout, 256)
+        p, want = (streamk.make_plan(1000, 1000, 1000, "float16", layout, x, cus=256, use_tuned=False) for x in (c, None))
+        assert named(p) == named(want)
