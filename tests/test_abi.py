@@ -506,3 +506,15 @@ def test_autotune_offers_what_an_untuned_call_runs():
         c = at.untuned_config(1000, 1000, 1000, "float16", layout, 256)
         p, want = (streamk.make_plan(1000, 1000, 1000, "float16", layout, x, cus=256, use_tuned=False) for x in (c, None))
         assert named(p) == named(want)
+
+
+def test_tuned_cache_leaves_the_faster_untuned_plans_alone(monkeypatch):
+    """128 rows of fp16 / bfloat16 and four rows of Q4 at the sizes that had tuned entries for older kernels: the ring and
+    the rows kernels."""
+    import streamk
+    from streamk import plan as P
+    monkeypatch.setattr(P, "num_cus", lambda: 256)
+    for N, K in ((4096, 4096), (11008, 4096), (4096, 11008), (8192, 8192), (28672, 8192), (8192, 28672)):
+        for dtype in ("float16", "bfloat16"):
+            assert "_ring_" in streamk.kernel_name(streamk.make_plan(128, N, K, dtype).kernel_id), (N, K, dtype)
+    assert streamk.kernel_name(streamk.make_plan(4, 8192, 8192, "q4").kernel_id).startswith("rows_q4")
