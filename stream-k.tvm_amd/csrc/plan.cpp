@@ -541,9 +541,6 @@ static const KernelInfo *model_pick_f32(int64_t M, int64_t N, int64_t K, int lay
   const KernelInfo *t = kernel_table(&count);
   for (const F32Family &f : kFamiliesF32) {
     if ((f.bm == 32 && M > 64) || (f.bm == 128 && M <= 32)) continue;
-    // (one 128 x 128 tile per 128 rows and columns of a problem of 2 x 2 of them: a handful of CTAs either way)
-    const bool tiny = M > 128 && N > 128 && M <= 256 && N <= 256;
-    if (tiny && f.bm != 128) continue;
     const KernelInfo *k = nullptr;
     for (int i = 0; i < count; ++i)   // (the instance with the longest K-iteration: see kernels_f32.hip)
       if (t[i].dtype == SK_F32 && t[i].layout == layout && t[i].bm == f.bm && t[i].bn == f.bn && (!k || t[i].bk > k->bk)) k = &t[i];

@@ -68,8 +68,11 @@ def test_schedules(sk):
     assert (one.total_tiles, one.streamk_tiles, one.blocking_tiles) == (960, 192, 768)
     f32 = sk.make_plan(16, 16384, 8192, "float32", "nn", cus=256)
     assert (f32.bm, f32.bn, f32.bk, f32.kernel_id) == (32, 256, 16, 202)  # M <= 32: the 32-row tile
-    f32 = sk.make_plan(256, 256, 1024, "float32", "nn", cus=256)
+    f32 = sk.make_plan(4096, 4096, 4096, "float32", "nn", cus=256)
     assert (f32.bm, f32.bn, f32.bk, f32.kernel_id) == (128, 128, 16, 200)
+    # (16 tiles of 64 x 64 on 128 CTAs: 10.6 us; the four of 128 x 128 split over 32: 20.1)
+    f32 = sk.make_plan(256, 256, 1024, "float32", "nn", cus=256)
+    assert (f32.bm, f32.bn, f32.bk, f32.kernel_id) == (64, 64, 32, 204)
     auto = sk.make_plan(8192, 8192, 8192, "float16", "nt", cus=256)
     assert (auto.bm, auto.bn, auto.schedule, auto.streamk_tiles) == (256, 256, 1, 0)
 
@@ -185,6 +188,16 @@ def test_fp32_tiles_keep_their_iterations_and_grids(sk):
         p = sk.make_plan(M, N, K, "float32", "nt", cus=256)
         assert (p.bm, p.bn, p.bk) == tile
         assert sk.make_plan(M, N, K, "float32", "nt", cus=256, bm=tile[0], bn=tile[1], bk=32).kernel_id == p.kernel_id
+
+
+def test_fp32_rule_has_no_size_window(sk):
+    """fp32 with everything left to the planner: a column or a row more or less around 2 x 2 tiles of 128 does not change the
+    tile or how many CTAs share the work by multiples."""
+    for layout in ("nn", "nt"):
+        for K in (512, 1024, 4096, 16384):
+            plans = [sk.make_plan(M, N, K, "float32", layout, cus=256) for M, N in ((128, 128), (132, 132), (200, 200), (256, 256), (256, 260), (260, 260))]
+            assert len({(p.bm, p.bn) for p in plans}) == 1, [(p.bm, p.bn, p.grid) for p in plans]
+            assert max(p.grid for p in plans[3:]) <= 2 * min(p.grid for p in plans[3:])
 
 
 def test_few_rows_of_q4_take_a_callers_grid_and_split(sk):
