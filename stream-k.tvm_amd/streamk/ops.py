@@ -44,13 +44,13 @@ def _workspace(nbytes, device):
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
         if ws is not None:  # the library must not take a later allocation at this address for this workspace
-            _lib.torch_lib().sk_torch_set_workspace(*key, None, 0)
+            _lib.tell_native_operators("sk_torch_set_workspace", *key, None, 0)
             _lib.lib().sk_workspace_release(ws.data_ptr())
         ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         _lib.check(_lib.lib().sk_workspace_init(ws.data_ptr(), ws.numel(), _stream_ptr()),
                    "sk_workspace_init")
         _workspaces[key] = ws
-        _lib.torch_lib().sk_torch_set_workspace(*key, ws.data_ptr(), ws.numel())
+        _lib.tell_native_operators("sk_torch_set_workspace", *key, ws.data_ptr(), ws.numel())
     return ws
 
 
@@ -65,7 +65,7 @@ def reset_workspaces():
     with status SK_ERR_TIMEOUT: the library refuses a workspace on which a fix-up wait gave up until it
     has been initialised again, which the next call on a fresh workspace does."""
     for key, ws in _workspaces.items():
-        _lib.torch_lib().sk_torch_set_workspace(*key, None, 0)
+        _lib.tell_native_operators("sk_torch_set_workspace", *key, None, 0)
         _lib.lib().sk_workspace_release(ws.data_ptr())
     _workspaces.clear()
 
@@ -160,7 +160,7 @@ def _plan_for(config, M, N, K, dtype, layout):
             if config == "":   # from now on the native implementation answers calls of this shape
                 with _plan_mod.tuned_lock:
                     if generation == _plan_mod.tuned_generation():
-                        _lib.torch_lib().sk_torch_add_plan(ctypes.byref(plan), device)
+                        _lib.tell_native_operators("sk_torch_add_plan", ctypes.byref(plan), device)
     return plan
 
 
@@ -415,8 +415,10 @@ def _register(name, before_out, after_out, run, out_meta):
         if args[out_pos].numel() > 0 or args[0].shape[0] > 0:
             run(*args)
 
-    _LIBRARY.impl(name + general, functional, "CUDA")
-    _LIBRARY.impl(f"{name}_out{general}", out_variant, "CUDA")
+    # (without the native library the Python implementation stands under both names)
+    for suffix in {general} if native and _lib.torch_lib() is not None else {"", general}:
+        _LIBRARY.impl(name + suffix, functional, "CUDA")
+        _LIBRARY.impl(f"{name}_out{suffix}", out_variant, "CUDA")
     torch.library.register_fake(f"streamk::{name}", functional_fake, lib=_LIBRARY)
     torch.library.register_fake(f"streamk::{name}_out", lambda *args: None, lib=_LIBRARY)
 
@@ -452,7 +454,6 @@ _register("dequant_q4", "Tensor Wq, Tensor scales, Tensor? zeros", "int zero=8, 
           lambda Wq, scales, zeros, W, zero=8, group=128: _run_dequant_q4(Wq, scales, zeros, W, zero, group),
           lambda Wq, scales, *rest: ((Wq.shape[0], Wq.shape[1] * 2), torch.float16))
 
-_lib.torch_lib()
 _ops = torch.ops.streamk
 
 

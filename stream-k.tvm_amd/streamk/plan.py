@@ -66,7 +66,7 @@ def invalidate_tuned_cache():
     with tuned_lock:
         _tuned = None
         _tuned_generation += 1
-        _lib.torch_lib().sk_torch_clear_plans()
+        _lib.tell_native_operators("sk_torch_clear_plans")
 
 
 def tuned_generation():

@@ -358,3 +358,46 @@ def test_native_operators_with_a_workspace(name):
         t.join()
     assert not wrong, wrong
     streamk.workspace_status()
+
+
+_WITHOUT_NATIVE = """
+import ctypes, sys, warnings
+import torch
+load = ctypes.CDLL
+def refuse(name, *args, **kwargs):
+    if str(name).endswith("libstreamk_torch.so"):
+        raise OSError("undefined symbol: of another libtorch")
+    return load(name, *args, **kwargs)
+ctypes.CDLL = refuse
+with warnings.catch_warnings(record=True) as caught:
+    warnings.simplefilter("always")
+    sys.path.insert(0, sys.argv[1])
+    import streamk
+assert [w for w in caught if w.category is RuntimeWarning and "another libtorch" in str(w.message)], caught
+for name in ("gemm_f16", "gemm_bf16", "gemm_f32", "gemm_f8", "gemm_i8", "gemm_q4"):
+    for op in (name, name + "_out", name + "_general", name + "_out_general"):
+        assert torch._C._dispatch_has_kernel_for_dispatch_key("streamk::" + op, "CUDA"), op
+assert streamk.make_plan(100, 512, 8192, "float16", "nt", cus=256).workspace_bytes > 0
+streamk.plan.invalidate_tuned_cache()
+streamk.reset_workspaces()
+if sys.argv[2:] == ["gpu"]:
+    A = torch.randint(-3, 4, (100, 8192), device="cuda").half()
+    B = torch.randint(-1, 2, (512, 8192), device="cuda").half()
+    for _ in range(2):
+        assert torch.equal(streamk.streamk_fp16(A, B), (A.float() @ B.float().T).half())
+    streamk.reset_workspaces()
+    assert torch.equal(streamk.streamk_fp16(A, B, out=torch.empty(100, 512, device="cuda").half()), (A.float() @ B.float().T).half())
+print("answered")
+"""
+
+
+@pytest.mark.parametrize("where", ["host", pytest.param("gpu", marks=pytest.mark.gpu)])
+def test_operators_without_their_native_library(where):
+    """libstreamk_torch.so built against another libtorch: the package imports with a warning and the operators answer from
+    their Python implementations, on the kernels as ever."""
+    import os
+    import subprocess
+    import sys
+    package = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "stream-k.tvm_amd")
+    done = subprocess.run([sys.executable, "-c", _WITHOUT_NATIVE, package] + (["gpu"] if where == "gpu" else []), capture_output=True, text=True, timeout=100)
+    assert done.returncode == 0 and done.stdout.strip().endswith("answered"), done.stderr[-2000:]
