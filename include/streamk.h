@@ -163,6 +163,9 @@ int sk_device_info(int *num_cus, int *clock_khz, int *lds_bytes_per_cu);
  * Host partitioner (pure integer arithmetic, no GPU needed when num_cus > 0 is given).
  * Replaces streamk_fp32.py:30-54 / streamk_fp16.py:92-113.
  *   dtype/layout select the kernel family; cfg may be NULL (all heuristic).
+ * fp8 / int8 with up to 64 rows: all heuristic means the general small-M kernels.  The kernels that stream the weights
+ * through LDS are faster on every size measured (16 x 8192 x 8192 14.3 us against 22.5, 64 x 28672 x 8192 56.5 / 67.5) and
+ * are planned for a cfg whose only field is reserved[0] = 9, as the Python operators do.
  */
 int sk_make_plan(int64_t M, int64_t N, int64_t K, int dtype, int layout, const sk_config *cfg,
                  int num_cus, sk_plan *out);
@@ -333,8 +336,8 @@ int sk_gemm_q4(const void *A, const void *Wq, const void *scales, void *C, int64
  * quantisers (min/max per group), which the reference's unsigned nibbles with one implied zero point do
  * not cover.  The plan is made with dtype SK_Q4_ZP; at most 64 rows per call.  M == 1 takes matrix-vector kernels
  * that, like sk_gemm_q4's, multiply the nibbles undecoded and apply zero point and scale to fp32 group sums (the
- * unrounded (q - zero) * scale); 2 <= M <= 64, and M == 1 with an explicit variant-0 plan, the general small-M
- * kernels, which form the rounded weights bit for bit.
+ * unrounded (q - zero) * scale); 2 <= M <= 64, and M == 1 with an explicit variant-0 plan, kernels that form the
+ * rounded weights bit for bit.
  * A plan made with dtype SK_Q4_ZP_TILED takes Wq in the tiled layout (sk_q4_tile_host / sk_q4_tile; scales and
  * zeros stay row-major): the same kernels with the tiled loads, results bit for bit those of SK_Q4_ZP. */
 int sk_gemm_q4_zp(const void *A, const void *Wq, const void *scales, const void *zeros, void *C, int64_t M,

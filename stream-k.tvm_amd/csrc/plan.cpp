@@ -207,8 +207,8 @@ static const KernelInfo *pick_kernel(int64_t M, int64_t N, int64_t K, int dtype,
     // 2 <= M <= 16 with Q4 weights and per-group zero points: the kernels whose waves stream K on their own
     // (tile_rows_q4.h), as many rows of A staged as M needs, and the tile that gives the busiest CU the least to do -- a
     // round of tiles costs about 24 weight rows' time beside its own rows (ZP 16 x 28672 x 8192: two rounds of 64 rows
-    // 40.9 us, three of 48 49.9, four of 32 50.0, seven of 16 60.4; 4 x 11008 x 4096: 48 rows 11.1, 64 rows 11.9, two
-    // rounds of 32 13.2).  With one zero point for the matrix up to 8 rows, where 64-row tiles run in one round (beyond,
+    // 40.7 us, three of 48 48.1, four of 32 49.3, seven of 16 61.0; 4 x 11008 x 4096: 48 rows 11.4, 64 rows 11.7, two
+    // rounds of 32 12.5).  With one zero point for the matrix up to 8 rows, where 64-row tiles run in one round (beyond,
     // 4 x 28672 x 8192: 31.9 us on the general kernel against 38); 5 to 8 rows on 32-row tiles stay with the kernel
     // that streams through shared LDS where that one is taken, from 16 MB of weights on (8 x 5120 x 5120: 8.1 us against
     // 8.7, 8 x 8192 x 8192: 11.8 / 11.9; below, the general kernel / these: 8 x 5120 x 2048 5.4 / 4.9, 8 x 8192 x 1024 5.2 / 4.2).
@@ -470,7 +470,7 @@ static const KernelInfo *model_pick(int64_t M, int64_t N, int64_t K, int dtype, 
 // time = o + rounds * iterations * (t + u * busy CUs / CUs) + fix-up(split), fitted to 60 timings, weights from HBM
 // (within 6 % of each); a split that does not divide the iterations costs 3 to 5 us more, as its CTAs cross from one tile into
 // the next (100 x 11008 x 4160, 65 iterations: 128-wide tiles in two 38.7, whole 64-wide ones 35.7).  100 rows, the tile kernels of the table above / these, in us: 4096 x 11008 42.0 / 33.5,
-// 2048 x 8192 29.1 / 21.4, 5120 x 5120 35.2 / 27.2, 8192 x 8192 48.9 / 40.2, 28672 x 8192 130 / 98, 11008 x 4096 37.4 / 34.4.
+// 2048 x 8192 29.1 / 21.4, 5120 x 5120 35.2 / 27.2, 8192 x 8192 48.9 / 40.2, 28672 x 8192 130 / 98, 11008 x 4096 36.7 / 33.0.
 struct RingFamily {
   int bn;
   double o, t, u, fix, per_log2, uneven;
@@ -519,8 +519,8 @@ static const KernelInfo *model_pick_ring(int64_t N, int64_t K, int dtype, int nu
 // ---- fp32: tile, schedule and grid, when the caller leaves all three open ----
 // The matrix pipe is slow enough (64 FLOP per cycle and SIMD) that tiles of 64 x 64 keep it busy; what decides is how
 // many CTAs there are and whether two of them share a CU (one computes while the other waits at its barrier).  Model,
-// fitted to 590 timings of every tile and schedule on 18 shapes in both layouts, weights from HBM (mean |log error|
-// 4 %; its choice is 0.9 % behind the fastest candidate on average, 17 % at worst; the rule before -- 128 x 128 tiles,
+// fitted to 590 timings of every tile and schedule on 18 shapes in both layouts, weights from HBM, on one device with the
+// 32 x 256 tiles' ring eight slots deep (mean |log error| 4 %; its choice is 0.9 % behind the fastest candidate on average, 17 % at worst; the rule before -- 128 x 128 tiles,
 // 32 x 256 up to 32 rows, split in two or four -- was 1.1 to 5.8 times behind):
 //     time = o + (compute^4 + memory^4)^(1/4) + fix-up
 //   compute  tiles of the busiest CU x the tile's FLOP at 0.614 TFLOP/s per CU, over `one` (a CTA alone on its CU) or
@@ -682,8 +682,8 @@ extern "C" int sk_make_plan(int64_t M, int64_t N, int64_t K, int dtype, int layo
     // split: 32 x 520 x 8192 9.2 us / 9.2, 32 x 2048 x 8192 11.9 / 11.8, 32 x 520 x 16384 18.5 / 13.6, 32 x 2048 x 16384 19.5 / 15.0,
     // 64 x 4096 x 4096 9.7 / 11.9, 64 x 5120 x 5120 11.9 / 15.4, 64 x 4096 x 11008 20.2 / 18.9, 64 x 2048 x 8192 15.0 / 12.7)
     const bool stream_bytes = k->family == FAMILY_SKINNY && k->variant == 8;
-    // (the Q4 kernels whose waves stream K on their own, variant 5: from two fifths on; 8 x 2048 x 8192 on 128 tiles 7.9 us
-    // against 9.9, 16 x 1024 x 16384 on 64 tiles 14.8 / 11.7)
+    // (the Q4 kernels whose waves stream K on their own, variant 5: from two fifths on; ZP 8 x 2048 x 8192 on 128 tiles
+    // 8.8 us against 10.2, 16 x 1024 x 16384 on 64 tiles 15.0 / 11.3)
     const bool stream_dp =
         k->family == FAMILY_SKINNY &&
         (stream_bytes ? k->bm == 16 || total64 >= num_cus || out->iters_per_tile * (num_cus - total64) <= 8 * num_cus

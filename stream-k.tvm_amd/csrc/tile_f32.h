@@ -10,7 +10,8 @@
 // M <= 32 (see the planner's kFamiliesF32).  Measured (B [K,N], weights from HBM) against the register-staged two-slot
 // kernels this replaced, in us: 16 x 16384 x 8192 120 -> 92 (5.8 TB/s), 16 x 4096 x 4096 59.8 -> 20.7, 64 x 4096 x 4096
 // 97 -> 28, 256 x 1024 x 512 23.1 -> 10.0, 512 x 4096 x 4096 163 -> 133, 4096^3 1019 -> 961 (143 TFLOP/s); as [N,K]
-// 149 -> 97, 64.8 -> 20.2, 98 -> 28, 23.4 -> 10.8, 167 -> 131, 1061 -> 933 (147 TFLOP/s).
+// 149 -> 97, 64.8 -> 20.2, 98 -> 28, 23.4 -> 10.8, 167 -> 131, 1061 -> 933 (147 TFLOP/s).  (One device; between devices and
+// runs the first varies from 92 to 95, those the matrix pipe bounds by up to 12 %; profiles/f32_M16_N16384_K8192.md.)
 //
 // LDS layout of a slot: BM rows of A of BK * 4 bytes, then B: [N,K] BN rows like A's, [K,N] BK rows of BN * 4 bytes.
 // 16-byte piece p of a row of 4 / 8 / 16 pieces is kept at position p ^ swizzle(row) ((row >> 2) & 3, (row >> 1) & 7,

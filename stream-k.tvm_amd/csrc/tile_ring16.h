@@ -12,11 +12,15 @@
 //    through LDS at the end of the segment), which keeps two waves on a SIMD without more fragment reads.
 //  * Partial tiles travel with device-scope accesses, the owner of a tile adds them up.
 //
-// What bounds it: the direct loads of a CU, which bring 45 to 65 GB/s of A and weights together whatever the depths of the
-// rings (128 x 64 tiles: 12 + 3, 9 + 5 and 7 + 6 slots within 2 % of each other; 128 K-values per iteration with four
-// waves per K sub-block 6 % slower; all tiles starting at the same K no faster).  Weights from HBM, bfloat16, 100 rows,
-// the four-stage tile kernels -> these: 4096 x 11008 42.0 -> 33.5 us, 28672 x 8192 130 -> 98 (4.8 TB/s), 2048 x 8192
-// 29.1 -> 21.4, 11008 x 4096 37.4 -> 34.4.  128 x 32 tiles are not built (11008 x 4096 57 us).
+// What bounds it: a CU gets 30 to 65 GB/s of A and weights together, where its direct loads reach 107 GB/s on rows of 128
+// bytes in the L2 and 25 on every CU at once from HBM (profiles/lds_direct_load_rate.md), so neither limit is met: the waves
+// wait (two fifths of their cycles for a counter or the barrier, profiles/ring_bf16_M100_N11008_K4096.md) on iterations that
+// start with the slowest wave's loads, and widths that are no multiple of the CUs leave some idle.  The depths of the rings do
+// not matter much (128 x 64 tiles: 12 + 3, 9 + 5 and 7 + 6 slots within 2 % of each other; 128 K-values per iteration with
+// four waves per K sub-block 6 % slower; all tiles starting at the same K no faster).  Weights from HBM, bfloat16, 100 rows,
+// the four-stage tile kernels -> these: 4096 x 11008 41.9 -> 33.5 us, 28672 x 8192 135 -> 99 (4.7 TB/s), 2048 x 8192
+// 29.2 -> 21.8, 5120 x 5120 35.0 -> 28.1, 11008 x 4096 36.7 -> 33.0; with bias and GELU 44.0 -> 36.6, 140 -> 108,
+// 31.3 -> 25.3, 36.9 -> 31.0, 39.9 -> 39.1.  128 x 32 tiles are not built (11008 x 4096 57 us).
 #pragma once
 #include <type_traits>
 
@@ -171,7 +175,7 @@ struct TileRing16 {
     if (wave >= WM * WN) return;
     const int wm = wave % WM, wn = wave / WM;
     const bool vec_ok = (a.ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(a.C) & 7) == 0);
-    // (the bias once per column block, all loads at once: fetched per element it cost 7 us at 100 x 11008 x 4096)
+    // (the bias once per column block, all loads at once: fetched per element it cost 7 us at 100 x 11008 x 4096, so 2 to 3)
     float bcol[FN][4];
     if constexpr (BIAS) {
 #pragma unroll

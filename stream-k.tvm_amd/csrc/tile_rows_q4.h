@@ -20,12 +20,13 @@
 //    bit for bit -- what the dequantiser and the kernels for more rows give, blocks of one call among them: they are
 //    multiplied by the scale in fp16 first and the sums run on in the accumulators.
 //
-// What bounds it: launch, arguments and the first trip to memory are about 4 us, then the weights stream; without the
-// decode and the MFMAs 4 x 11008 x 4096 takes 9.0 us, without the loads of A 11.0, as it is 11.1 (one row: 7.2).  Weights
-// from HBM, in us, the kernels that ran these shapes before (tile_skinny.h, with a zero point for the matrix
-// tile_stream_q4.h) -> these: per-group zero points 4 x 11008 x 4096 17.1 -> 11.1, 4 x 4096 x 11008 18.8 -> 10.8,
-// 16 x 4096 x 4096 9.5 -> 7.2, 16 x 14336 x 4096 21.2 -> 13.0, 16 x 16384 x 16384 52.5 -> 47.9; one zero point
-// 4 x 4096 x 11008 15.3 -> 10.5, 4 x 4096 x 4096 6.9 -> 6.2, 8 x 2048 x 8192 11.1 -> 7.9, 8 x 16384 x 16384 40.0 -> 36.8.
+// What bounds it: launch, arguments and the first trip to memory are about 4 us, then the weights stream; with zero points
+// 4 x 11008 x 4096 takes 11.5 us (11.1 with unrounded weights; of these 9.0 without the decode and the MFMAs, 11.0 without
+// the loads of A; one row: 7.2).  Weights from HBM, in us, the kernels that ran these shapes before (tile_skinny.h, with a
+// zero point for the matrix tile_stream_q4.h) -> these: per-group zero points 4 x 11008 x 4096 16.9 -> 11.5,
+// 4 x 4096 x 11008 18.4 -> 10.6, 16 x 4096 x 4096 9.3 -> 7.3, 16 x 14336 x 4096 20.9 -> 12.9, 16 x 16384 x 16384 52 -> 47;
+// one zero point 4 x 4096 x 11008 15.3 -> 10.2, 4 x 4096 x 4096 6.9 -> 6.2, 8 x 2048 x 8192 11.1 -> 7.9,
+// 8 x 16384 x 16384 40.0 -> 36.7.  Counters: profiles/rows_q4zp_M4_N11008_K4096.md.
 // (Sixteen waves do not fit a workgroup beside the staging ones; twelve with 64 weight rows 11.8 against 12.0, eight
 // slots instead of four for 16 weight rows 12.8 against 11.9 at 4 x 4096 x 11008.)
 //

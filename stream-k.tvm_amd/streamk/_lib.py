@@ -137,7 +137,7 @@ _torch_lib = None
 def torch_lib():
     """libstreamk_torch.so, whose static initialisers register the operators' native implementations
     (csrc/torch_ops.cpp).  It is built against one libtorch; where it is missing or does not load, None, with a warning:
-    the operators' Python implementations then answer every call, at 20 to 28 us of host time instead of 6 to 12."""
+    the operators' Python implementations then answer every call, at 16 us of host time instead of 5 to 6."""
     global _torch_lib
     if _torch_lib is None:
         try:

@@ -318,7 +318,8 @@ def _run_q4(A, Wq, scales, zeros, C, zero, group, tiled, config, bias, activatio
         # The weight-streaming kernels take at most 64 rows of A; beyond that row-major weights with a scalar zero
         # point go to the Q4 tile kernels (below, like any other plan).  Per-group zero points and the tiled
         # layout have no tile kernel: up to 256 rows one launch per block of 64 rows, beyond that the weights are
-        # dequantised once (bit-exact device function) for the fp16 tile kernels.
+        # dequantised once (bit-exact device function) for the fp16 tile kernels.  (Blocks of two rows and more multiply
+        # the rounded weights alike; a last block of one row takes the matrix-vector kernels and the unrounded ones.)
         if M <= 4 * Q4_MAX_M:
             for m0 in range(0, M, Q4_MAX_M):
                 _run_q4(A[m0:m0 + Q4_MAX_M], Wq, scales, zeros, C[m0:m0 + Q4_MAX_M], zero, group, tiled, config,
