@@ -520,8 +520,9 @@ static const KernelInfo *model_pick_ring(int64_t N, int64_t K, int dtype, int nu
 // The matrix pipe is slow enough (64 FLOP per cycle and SIMD) that tiles of 64 x 64 keep it busy; what decides is how
 // many CTAs there are and whether two of them share a CU (one computes while the other waits at its barrier).  Model,
 // fitted to 590 timings of every tile and schedule on 18 shapes in both layouts, weights from HBM, on one device with the
-// 32 x 256 tiles' ring eight slots deep (mean |log error| 4 %; its choice is 0.9 % behind the fastest candidate on average, 17 % at worst; the rule before -- 128 x 128 tiles,
-// 32 x 256 up to 32 rows, split in two or four -- was 1.1 to 5.8 times behind):
+// 32 x 256 tiles' ring eight slots deep (mean |log error| 4 %).  On the kernels as they are its choice is 2.1 % behind the
+// fastest candidate on average over 20 shapes in both layouts, 12 % at worst (profiles/planner_f32_choice.md); the rule
+// before -- 128 x 128 tiles, 32 x 256 up to 32 rows, split in two or four -- was 1.1 to 5.8 times behind:
 //     time = o + (compute^4 + memory^4)^(1/4) + fix-up
 //   compute  tiles of the busiest CU x the tile's FLOP at 0.614 TFLOP/s per CU, over `one` (a CTA alone on its CU) or
 //            `two`; up to 16 rows a 32-row tile computes 16 rows only
