@@ -249,9 +249,9 @@ int make_dev_plan(const sk_plan *plan, const KernelInfo *k, void *ws, size_t ws_
 
 // family: 0 tile kernels, 1 small-M kernels, 2 fp32 kernels
 int cached_occupancy(int id, int family) {
-  static int cache[512];
-  static bool have[512];
-  const int slot = id & 511;  // kernel ids stay below 512
+  static int cache[1024];
+  static bool have[1024];
+  const int slot = id & 1023;  // kernel ids stay below 1024
   std::lock_guard<std::mutex> lock(g_mutex);
   if (!have[slot]) {
     cache[slot] = family == 1 ? occupancy_skinny(id) : (family == 2 ? occupancy_f32(id) : occupancy_tile(id));
@@ -529,11 +529,13 @@ static int gemm_q4_any(const void *A, const void *Wq, const void *scales, const 
   if (k->family == FAMILY_TILE) {
     // more than 64 rows of A: the tile kernels that dequantise B on its way into LDS (scalar zero point,
     // row-major nibbles)
-    if (dtype != SK_Q4) return SK_ERR_CONFIG;
+    const bool wavek = k->variant == 10;   // (these take per-group zero points as well)
+    if (dtype != SK_Q4 && !wavek) return SK_ERR_CONFIG;
     rc = make_dev_plan(plan, k, ws, ws_bytes, cached_occupancy(k->id, 0), (hipStream_t)stream, &dp, &w);
     if (rc) return rc;
     GemmArgs g{(const half_t *)A, (const half_t *)Wq, (half_t *)C, (int)M, (int)N, (int)K, lda, K / 2, ldc, 1.f,
                (const half_t *)scales, zero, (int)(K / group)};
+    if (wavek) return launch_wavek_q4(k->id, g, zeros, dp, w, (hipStream_t)stream, bias) == 0 ? SK_OK : SK_ERR_LAUNCH;
     return launch_tile_f16(k->id, g, dp, w, (hipStream_t)stream, bias) == 0 ? SK_OK : SK_ERR_LAUNCH;
   }
   if (k->family != FAMILY_SKINNY) return SK_ERR_CONFIG;

@@ -304,6 +304,33 @@ struct KernelInfo {
   X(382, 128, 128, 64, 2, 2, 2, 6, 4, false)    \
   X(383, 128, 128, 64, 2, 2, 2, 6, 4, true)
 
+// Tiles whose waves stream K on their own (tile_wavek.h; variant 10), every one for each type; ids from 400 + 20 type on
+// (types: WaveKType):  X(type, id, blocks of 16 rows of A, of 16 weight rows)
+#define SK_TILE_WAVEK_KERNELS(X, T, BASE) \
+  X(T, BASE + 0, 2, 2) \
+  X(T, BASE + 1, 2, 4) \
+  X(T, BASE + 2, 4, 2) \
+  X(T, BASE + 3, 4, 3) \
+  X(T, BASE + 4, 4, 4) \
+  X(T, BASE + 5, 4, 5) \
+  X(T, BASE + 6, 4, 6) \
+  X(T, BASE + 7, 4, 7) \
+  X(T, BASE + 8, 4, 8) \
+  X(T, BASE + 9, 6, 2) \
+  X(T, BASE + 10, 6, 4) \
+  X(T, BASE + 11, 8, 2) \
+  X(T, BASE + 12, 8, 3) \
+  X(T, BASE + 13, 8, 4)
+
+// the same for Q4 weights (tile_wavek_q4.h; dtypes SK_Q4 id, SK_Q4_ZP id + 20):  X(id, blocks of 16 rows of A, of 16 weight rows)
+#define SK_TILE_WAVEK_Q4_KERNELS(X) \
+  X(520, 2, 2) \
+  X(521, 2, 4) \
+  X(522, 4, 2) \
+  X(523, 4, 4) \
+  X(524, 4, 6) \
+  X(525, 8, 2)
+
 // Up to 16 rows of A, Q4 weights, every wave streaming K on its own (tile_rows_q4.h; dtypes SK_Q4, SK_Q4_ZP and
 // SK_Q4_ZP_TILED, variant 5; taken when asked for by variant or by the planner's rule):
 // X(id, rows of A staged, blocks of 16 weight rows, slots, per-group zero points, scale groups in LDS, tiled weights)

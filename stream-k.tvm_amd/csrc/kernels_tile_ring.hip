@@ -39,7 +39,7 @@ int launch_tile_ring(int id, const GemmArgs &a, const DevPlan &p, const Workspac
     SK_TILE_RING_KERNELS(X)
 #undef X
   }
-  return launch_tile_q4(id, a, p, ws, s, bias);
+  return launch_tile_wavek(id, a, p, ws, s, bias);
 }
 
 int occupancy_tile_ring(int id) {
@@ -53,7 +53,7 @@ int occupancy_tile_ring(int id) {
     SK_TILE_RING_KERNELS(X)
 #undef X
   }
-  return occupancy_tile_q4(id);
+  return occupancy_tile_wavek(id);
 }
 
 }  // namespace sk

@@ -1,0 +1,7 @@
+// The tiles whose waves stream K on their own (tile_wavek.h) for one type of operands.
+#define WAVEK_NAME "wavek_f8e5m2"
+#include "wavek_launch.h"
+
+namespace sk {
+SK_WAVEK_UNIT(WK_F8E5M2, 8, WAVEK_NAME)
+}  // namespace sk

@@ -1,0 +1,7 @@
+// The tiles whose waves stream K on their own (tile_wavek.h) for one type of operands.
+#define WAVEK_NAME "wavek_i8"
+#include "wavek_launch.h"
+
+namespace sk {
+SK_WAVEK_UNIT(WK_I8, 6, WAVEK_NAME)
+}  // namespace sk

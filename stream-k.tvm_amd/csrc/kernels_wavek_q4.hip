@@ -1,0 +1,73 @@
+// Tiles for Q4 weights whose waves stream K on their own (tile_wavek_q4.h).
+#include "launch.h"
+#include "sk_persistent.h"
+#include "tile_wavek_q4.h"
+
+namespace sk {
+
+template <class P, bool FIXUP>
+__global__ __launch_bounds__(P::NT, P::WAVES_PER_EU) void sk_tile_wavek_q4_kernel(typename P::Args a, DevPlan plan, Workspace ws,
+                                                                                  const void *bias) {
+  __shared__ __attribute__((aligned(1024))) char smem[P::LDS_BYTES];
+  run_persistent<P, FIXUP, true>(a, plan, ws, smem, bias);
+}
+
+int wavek_q4_kernel_infos(KernelInfo *out, int max) {
+  int n = 0;
+#define INFO(id, DT, TYPE, NAME, FM, FN)                                                                                          \
+  if (n < max) {                                                                                                                  \
+    typedef TileWaveKQ4<TYPE, FM, FN> P;                                                                                          \
+    out[n++] = KernelInfo{id, FAMILY_TILE, DT, 0, 10, P::BM, P::BN, P::BK, P::NT, P::LDS_TOTAL, P::CTAS_PER_CU, P::TILE_ELEMS, 0, \
+                          0, 128, NAME "_" #FM "x" #FN};                                                                          \
+  }
+#define X(id, FM, FN)                        \
+  INFO(id, 2, WK_Q4, "wavek_q4", FM, FN)     \
+  INFO(id + 20, 7, WK_Q4ZP, "wavek_q4zp", FM, FN)
+  SK_TILE_WAVEK_Q4_KERNELS(X)
+#undef X
+#undef INFO
+  return n;
+}
+
+template <class P>
+static int launch(const WaveKQ4Args &a, const DevPlan &p, const Workspace &ws, hipStream_t s, const void *bias) {
+  if (p.sk_tiles == 0)
+    hipLaunchKernelGGL((sk_tile_wavek_q4_kernel<P, false>), dim3(p.grid), dim3(P::NT), 0, s, a, p, ws, bias);
+  else
+    hipLaunchKernelGGL((sk_tile_wavek_q4_kernel<P, true>), dim3(p.grid), dim3(P::NT), 0, s, a, p, ws, bias);
+  return (int)hipGetLastError();
+}
+
+int launch_wavek_q4(int id, const GemmArgs &g, const void *zeros, const DevPlan &p, const Workspace &ws, hipStream_t s, const void *bias) {
+  WaveKQ4Args a;
+  static_cast<GemmArgs &>(a) = g;
+  a.zeros = static_cast<const half_t *>(zeros);
+  switch (id) {
+#define X(id_, FM, FN)                                                               \
+  case id_: return launch<TileWaveKQ4<WK_Q4, FM, FN>>(a, p, ws, s, bias);            \
+  case id_ + 20: return launch<TileWaveKQ4<WK_Q4ZP, FM, FN>>(a, p, ws, s, bias);
+    SK_TILE_WAVEK_Q4_KERNELS(X)
+#undef X
+  }
+  return (int)hipErrorInvalidValue;
+}
+
+int occupancy_wavek_q4(int id) {
+  int occ = 0;
+  switch (id) {
+#define OCC(id_, TYPE, FM, FN)                                                                                                     \
+  case id_: {                                                                                                                      \
+    typedef TileWaveKQ4<TYPE, FM, FN> P;                                                                                           \
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, sk_tile_wavek_q4_kernel<P, true>, P::NT, 0) == hipSuccess ? occ : -1; \
+  }
+#define X(id_, FM, FN)          \
+  OCC(id_, WK_Q4, FM, FN)       \
+  OCC(id_ + 20, WK_Q4ZP, FM, FN)
+    SK_TILE_WAVEK_Q4_KERNELS(X)
+#undef X
+#undef OCC
+  }
+  return -1;
+}
+
+}  // namespace sk

@@ -14,7 +14,8 @@
 
 namespace sk {
 
-static KernelInfo g_table[400];
+constexpr int TABLE_MAX = 512;
+static KernelInfo g_table[TABLE_MAX];
 static int g_count = 0;
 static std::once_flag g_table_once;
 
@@ -27,20 +28,22 @@ int skinny_kernel_infos(KernelInfo *out, int max);
 int rows_q4_kernel_infos(KernelInfo *out, int max);
 int stream_bytes_kernel_infos(KernelInfo *out, int max);
 int tile_ring_kernel_infos(KernelInfo *out, int max);
+int tile_wavek_kernel_infos(KernelInfo *out, int max);
 int f32_kernel_infos(KernelInfo *out, int max);
 
 const KernelInfo *kernel_table(int *count) {
   std::call_once(g_table_once, [] {
-    int n = tile_kernel_infos(g_table, 400);
-    n += tile_8bit_kernel_infos(g_table + n, 400 - n);
-    n += tile_asm_kernel_infos(g_table + n, 400 - n);
-    n += tile_asm8_kernel_infos(g_table + n, 400 - n);
-    n += tile_q4_kernel_infos(g_table + n, 400 - n);
-    n += skinny_kernel_infos(g_table + n, 400 - n);
-    n += rows_q4_kernel_infos(g_table + n, 400 - n);
-    n += stream_bytes_kernel_infos(g_table + n, 400 - n);
-    n += tile_ring_kernel_infos(g_table + n, 400 - n);
-    n += f32_kernel_infos(g_table + n, 400 - n);
+    int n = tile_kernel_infos(g_table, TABLE_MAX);
+    n += tile_8bit_kernel_infos(g_table + n, TABLE_MAX - n);
+    n += tile_asm_kernel_infos(g_table + n, TABLE_MAX - n);
+    n += tile_asm8_kernel_infos(g_table + n, TABLE_MAX - n);
+    n += tile_q4_kernel_infos(g_table + n, TABLE_MAX - n);
+    n += skinny_kernel_infos(g_table + n, TABLE_MAX - n);
+    n += rows_q4_kernel_infos(g_table + n, TABLE_MAX - n);
+    n += stream_bytes_kernel_infos(g_table + n, TABLE_MAX - n);
+    n += tile_ring_kernel_infos(g_table + n, TABLE_MAX - n);
+    n += tile_wavek_kernel_infos(g_table + n, TABLE_MAX - n);
+    n += f32_kernel_infos(g_table + n, TABLE_MAX - n);
     g_count = n;
   });
   if (count) *count = g_count;
@@ -54,6 +57,9 @@ const KernelInfo *kernel_by_id(int id) {
     if (t[i].id == id) return &t[i];
   return nullptr;
 }
+
+// sk_config.reserved[0] of the operators' calls that name nothing: the fastest kernel there is, see sk_make_plan
+constexpr int SK_VARIANT_OPERATOR = 12;
 
 static int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
@@ -70,7 +76,7 @@ static int variant_rank(const KernelInfo &k) {
 // kernels that a tile alone does not name: the Q4 ones whose waves stream K on their own, and the ones that stream one-byte
 // weights through LDS, and the tile kernels for 65 to 128 rows
 static bool by_variant_only(const KernelInfo &k) {
-  return k.variant == 9 || (k.family == FAMILY_SKINNY && (k.variant == 5 || k.variant == 8));
+  return k.variant >= 9 || (k.family == FAMILY_SKINNY && (k.variant == 5 || k.variant == 8));
 }
 static bool accepts_shape(const KernelInfo &k, int64_t M, int64_t K) {
   // (the assembly-loop tile kernels have no K tail: other K go to the next-best variant of the tile)
@@ -406,7 +412,7 @@ static const TileFamily kFamiliesI8[] = {
 };
 
 static const KernelInfo *model_pick(int64_t M, int64_t N, int64_t K, int dtype, int layout, int num_cus, int *split,
-                                    int *sched) {
+                                    int *sched, double *time_us) {
   const TileFamily *fams = kFamilies16;
   int nfams = (int)(sizeof(kFamilies16) / sizeof(kFamilies16[0]));
   if (dtype == SK_F8E4M3 || dtype == SK_F8E5M2) {
@@ -463,6 +469,7 @@ static const KernelInfo *model_pick(int64_t M, int64_t N, int64_t K, int dtype, 
       }
     }
   }
+  *time_us = best_time;
   return best;
 }
 
@@ -482,7 +489,7 @@ static const RingFamily kFamiliesRing[] = {{64, 3.9, 0.395, 0.09, 2.6, 2.6, 3.0}
 // 256 to 1024 wide 12.2 / 14.4; K = 2816: 777 wide 14.2 / 14.5, 1024 15.1 / 13.8; K = 3000: 777 wide 23.6 / 18.8; K = 3072:
 // 256 wide 14.2 / 13.3, 1024 16.4 / 14.5; 66 and 128 rows alike).
 static bool ring_pays(int64_t N, int64_t K) { return K >= 2880 || (K >= 2048 && N >= 1536) || (K >= 1536 && N >= 8192); }
-static const KernelInfo *model_pick_ring(int64_t N, int64_t K, int dtype, int num_cus, sk_config *out) {
+static const KernelInfo *model_pick_ring(int64_t N, int64_t K, int dtype, int num_cus, sk_config *out, double *time_us) {
   const KernelInfo *best = nullptr;
   double best_time = 0;
   int count;
@@ -512,8 +519,141 @@ static const KernelInfo *model_pick_ring(int64_t N, int64_t K, int dtype, int nu
     out->bn = best->bn;
     out->bk = best->bk;
     out->reserved[0] = best->variant + 1;
+    *time_us = best_time;
   }
   return best;
+}
+
+// ---- a middling number of rows: the tiles whose waves stream K on their own (tile_wavek.h, tile_wavek_q4.h) ----
+// Model, fitted to 7 000 timings of every tile and split (16-bit, one-byte and Q4 operands, 20 to 2048 rows, 27 shapes, three sets of
+// operands in turn; mean |log error| 3 to 6 %):
+//     time = start + round (rounds - 1) + (core^4 + memory^4)^(1/4) + split + log2 (log2 of the split)
+//   core    rounds x iterations x (iter + busy x busy CUs / CUs): one CTA per CU, every tile of a round side by side
+//   memory  the operands and C once at 5.9 TB/s, slower where less than five eighths of the CUs are busy
+// The tile it chooses is within 1 % of the fastest of them on average.
+struct WaveKFamily {
+  int bm, bn;
+  float start, round, iter, busy, split, log2;
+};
+static const WaveKFamily kFamiliesWaveK16[] = {
+    {32, 32, 3.37f, 1.31f, 0.280f, 0.101f, 1.88f, 0.47f},
+    {32, 64, 3.76f, 1.48f, 0.394f, 0.182f, 1.90f, 0.61f},
+    {64, 32, 3.87f, 1.52f, 0.384f, 0.160f, 1.83f, 0.68f},
+    {64, 48, 4.22f, 1.56f, 0.462f, 0.187f, 1.93f, 0.82f},
+    {64, 64, 4.67f, 1.68f, 0.505f, 0.298f, 1.90f, 0.90f},
+    {64, 80, 5.23f, 2.16f, 0.622f, 0.280f, 1.81f, 1.05f},
+    {64, 96, 5.57f, 2.34f, 0.684f, 0.393f, 1.90f, 1.10f},
+    {64, 112, 6.43f, 2.82f, 0.867f, 0.416f, 2.07f, 1.14f},
+    {64, 128, 6.87f, 3.05f, 0.958f, 0.497f, 1.99f, 1.19f},
+    {96, 32, 4.32f, 1.54f, 0.482f, 0.225f, 1.92f, 0.82f},
+    {96, 64, 5.77f, 2.44f, 0.664f, 0.337f, 1.91f, 1.10f},
+    {128, 32, 4.81f, 1.78f, 0.597f, 0.310f, 1.80f, 1.02f},
+    {128, 48, 6.37f, 2.60f, 0.784f, 0.343f, 1.89f, 1.01f},
+    {128, 64, 7.08f, 2.95f, 0.960f, 0.428f, 2.08f, 1.21f},
+};
+static const WaveKFamily kFamiliesWaveK8[] = {
+    {32, 32, 3.41f, 1.19f, 0.319f, 0.082f, 1.87f, 0.47f},
+    {32, 64, 3.94f, 1.74f, 0.439f, 0.117f, 1.86f, 0.64f},
+    {64, 32, 4.03f, 1.67f, 0.401f, 0.134f, 1.95f, 0.62f},
+    {64, 48, 4.51f, 2.02f, 0.475f, 0.121f, 1.86f, 0.75f},
+    {64, 64, 5.03f, 2.45f, 0.539f, 0.187f, 1.76f, 0.88f},
+    {64, 80, 5.57f, 3.01f, 0.685f, 0.115f, 1.53f, 1.02f},
+    {64, 96, 5.96f, 3.45f, 0.747f, 0.198f, 1.73f, 1.01f},
+    {64, 112, 6.84f, 4.31f, 0.940f, 0.200f, 1.74f, 1.14f},
+    {64, 128, 7.32f, 4.24f, 0.983f, 0.344f, 1.78f, 1.15f},
+    {96, 32, 4.60f, 1.90f, 0.478f, 0.189f, 1.82f, 0.77f},
+    {96, 64, 6.07f, 3.46f, 0.705f, 0.217f, 1.74f, 1.05f},
+    {128, 32, 5.16f, 2.34f, 0.612f, 0.227f, 1.86f, 0.88f},
+    {128, 48, 6.54f, 3.52f, 0.838f, 0.198f, 1.91f, 0.93f},
+    {128, 64, 7.43f, 4.08f, 0.968f, 0.322f, 1.94f, 1.17f},
+};
+static const WaveKFamily kFamiliesWaveKQ4[] = {
+    {32, 32, 3.84f, 1.43f, 0.629f, 0.086f, 1.93f, 0.63f},
+    {32, 64, 4.46f, 1.88f, 0.973f, 0.115f, 1.85f, 0.79f},
+    {64, 32, 4.48f, 1.77f, 0.830f, 0.118f, 2.06f, 0.71f},
+    {64, 64, 5.32f, 2.28f, 1.222f, 0.237f, 2.05f, 0.93f},
+    {64, 96, 5.99f, 3.12f, 1.837f, 0.164f, 2.32f, 1.06f},
+    {128, 32, 5.41f, 1.72f, 1.224f, 0.307f, 2.15f, 0.83f},
+};
+static const KernelInfo *model_pick_wavek(int64_t M, int64_t N, int64_t K, int dtype, int num_cus, sk_config *out, double *time_us) {
+  const bool q4 = dtype == SK_Q4 || dtype == SK_Q4_ZP, one_byte = dtype == SK_F8E4M3 || dtype == SK_F8E5M2 || dtype == SK_I8;
+  const WaveKFamily *fams = q4 ? kFamiliesWaveKQ4 : (one_byte ? kFamiliesWaveK8 : kFamiliesWaveK16);
+  const int nfams = q4 ? (int)(sizeof(kFamiliesWaveKQ4) / sizeof(kFamiliesWaveKQ4[0]))
+                       : (one_byte ? (int)(sizeof(kFamiliesWaveK8) / sizeof(kFamiliesWaveK8[0])) : (int)(sizeof(kFamiliesWaveK16) / sizeof(kFamiliesWaveK16[0])));
+  const double weight_bytes = q4 ? 0.52 : (one_byte ? 1 : 2), a_bytes = one_byte ? 1 : 2, c_bytes = dtype == SK_I8 ? 4 : 2;
+  const double memory_us = (weight_bytes * N * K + a_bytes * M * K + c_bytes * M * N) / 5.9e6;
+  const KernelInfo *best = nullptr;
+  double best_time = 0;
+  int count;
+  const KernelInfo *t = kernel_table(&count);
+  for (int fi = 0; fi < nfams; ++fi) {
+    const WaveKFamily &f = fams[fi];
+    const KernelInfo *k = nullptr;
+    for (int i = 0; i < count && !k; ++i)
+      if (t[i].family == FAMILY_TILE && t[i].variant == 10 && t[i].dtype == dtype && t[i].bm == f.bm && t[i].bn == f.bn) k = &t[i];
+    if (!k || K % k->k_align != 0) continue;
+    const int64_t tiles = cdiv(M, f.bm) * cdiv(N, f.bn), ipt = cdiv(K, k->bk);
+    for (int s = 1; s <= 8; s *= 2) {
+      if (s > 1 && (ipt % s != 0 || tiles * s > num_cus)) continue;
+      const double busy = tiles * s < num_cus ? (double)(tiles * s) / num_cus : 1.0;
+      const double rounds = (double)cdiv(tiles * s, num_cus);
+      const double core = rounds * ((double)ipt / s) * (f.iter + f.busy * busy), memory = memory_us / (1.6 * busy < 1 ? 1.6 * busy : 1.0);
+      const double c2 = core * core, m2 = memory * memory;
+      const double time = f.start + f.round * (rounds - 1) + sqrt(sqrt(c2 * c2 + m2 * m2)) +
+                          (s == 1 ? 0.0 : f.split + f.log2 * (s == 2 ? 1 : (s == 4 ? 2 : 3)));
+      // (within 2 % the larger tile: fewer bytes of the operands through the caches)
+      if (best && time >= best_time * (f.bm * f.bn > best->bm * best->bn ? 1.02 : (f.bm * f.bn < best->bm * best->bn ? 0.98 : 1.0))) continue;
+      best = k;
+      best_time = time;
+      out->schedule = s == 1 ? SK_SCHED_DP : SK_SCHED_SPLIT_K;
+      out->reserved[1] = s > 1 ? s : 0;
+    }
+  }
+  if (best) {
+    out->bm = best->bm;
+    out->bn = best->bn;
+    out->bk = best->bk;
+    out->reserved[0] = best->variant + 1;
+    *time_us = best_time;
+  }
+  return best;
+}
+// Whether a problem whose tile, variant, schedule and grid are open goes to them; `other_us`: the time the other tile kernels'
+// model gives (0: none of them runs it).
+static bool wavek_pays(int64_t M, int64_t N, int64_t K, int dtype, int num_cus, double wavek_us, double other_us) {
+  if (dtype == SK_Q4 || dtype == SK_Q4_ZP) {
+    // up to 64 rows the general small-M kernels: behind everywhere but with up to 32 rows on more than one round of 64-row tiles
+    // (20 x 28672 x 1280 10.4 us against 13.1, 20 x 20480 x 3072 15.8 / 19.1; 20 x 8192 x 8192 18.4 / 14.9, 64 x 4096 x 4096
+    // 16.0 / 9.4, 64 x 28672 x 1280 25.0 / 17.2)
+    if (M <= 64) return M > 32 || cdiv(N, 64) <= num_cus;
+    if (dtype == SK_Q4_ZP) return true;   // (nothing else runs them in one launch)
+    // the tile kernels that decode into LDS: fitted like the others, 128 x 128 tiles up to 128 rows, 256 x 128 beyond (mean
+    // |log error| 6 and 4 %; by this choice 35 % faster on average over 197 shapes, none slower: 512 x 4096 x 4096 33.4 us / 30.1,
+    // 128 x 8192 x 8192 41.9 / 27.5, 512 x 8192 x 8192 76.0 on the tile kernels, 103 here)
+    const int bm = M > 128 ? 256 : 128, occ = bm == 256 ? 1 : 2;
+    const int64_t tiles = cdiv(M, bm) * cdiv(N, 128), ipt = K / 64;
+    int split = 1;
+    for (int s = 2; tiles < num_cus && s <= 4; s *= 2)
+      if (tiles * s <= (int64_t)num_cus * occ && ipt % s == 0 && ipt / s >= 8) split = s;
+    const double busy = tiles * split < num_cus ? (double)(tiles * split) / num_cus : 1.0;
+    const double per = bm == 256 ? 0.667 + 0.316 * busy : 0.664 + 0.105 * busy;
+    const double tile_us = (bm == 256 ? 5.24 : 2.45) + (double)cdiv(tiles * split, num_cus) * ((double)ipt / split) * per +
+                           (split == 1 ? 0.0 : (bm == 256 ? 4.8 : 5.0) * (split == 2 ? 1 : 2));
+    return wavek_us < 0.95 * tile_us;
+  }
+  if (M > 64) return other_us <= 0 || wavek_us < 0.95 * other_us;
+  // 33 to 64 rows against the kernels that stream the weights through LDS: K long enough for a ring to fill, and few columns
+  // (in us, those / these, 64 rows: fp16 2048 x 2048 9.5 / 6.2, 4096 x 4096 14.0 / 9.9, 5120 x 5120 17.8 / 15.9, 6144 x 2048
+  // 12.7 / 9.0, 1024 x 8192 13.8 / 10.4; int8 4096 x 11008 16.4 / 13.1, 2048 x 8192 11.7 / 9.3; but fp16 4096 x 11008 25.9 / 27.1,
+  // 8192 x 8192 29.7 / 31.4, 4096 x 1024 5.9 / 5.0, 1024 x 1024 5.8 / 6.4; int8 8192 x 16384 29.7 / 34.7) or more than a round of
+  // their 64-row tiles where 112-row tiles need one (20480 x 3072 fp16 37.6 / 27.9, 28672 x 8192 88.3 / 85.4, of fp8 50.4 / 47.5).
+  // One-byte operands of fewer than 6144 K-values stay with the streaming kernels throughout: there the gain is 1 to 2 us
+  // (4096 x 4096 8.8 / 7.4, 2048 x 2048 5.8 / 5.0), and those are the kernels their plans are known by.  Up to 32 rows there is
+  // nothing to gain (20 x 4096 x 4096 9.4 / 9.1 and 6.6 / 6.7).
+  const bool one_byte = dtype == SK_F8E4M3 || dtype == SK_F8E5M2 || dtype == SK_I8;
+  if (M <= 32 || (one_byte && K < 6144)) return false;
+  if (cdiv(N, 64) > num_cus && cdiv(N, 112) <= num_cus) return K >= 2048;
+  return N <= (one_byte ? 4096 : 6144) && K >= 1536 && N * K <= (one_byte ? (int64_t)48 << 20 : (int64_t)32 << 20);
 }
 
 // ---- fp32: tile, schedule and grid, when the caller leaves all three open ----
@@ -594,9 +734,9 @@ using namespace sk;
 extern "C" int sk_selfcheck(void) {
   int n;
   const KernelInfo *t = kernel_table(&n);
-  if (n <= 0 || n >= 400) return SK_ERR_CONFIG;  // (400: the table's capacity)
+  if (n <= 0 || n >= TABLE_MAX) return SK_ERR_CONFIG;
   for (int i = 0; i < n; ++i) {
-    if (t[i].id < 0 || t[i].id >= 512 || !t[i].name || !t[i].name[0]) return SK_ERR_CONFIG;
+    if (t[i].id < 0 || t[i].id >= 1024 || !t[i].name || !t[i].name[0]) return SK_ERR_CONFIG;
     for (int j = 0; j < i; ++j)
       if (t[j].id == t[i].id) return SK_ERR_CONFIG;
   }
@@ -614,32 +754,52 @@ extern "C" int sk_make_plan(int64_t M, int64_t N, int64_t K, int dtype, int layo
   if (layout != SK_LAYOUT_NT && layout != SK_LAYOUT_NN) return SK_ERR_CONFIG;
   if (num_cus <= 0) return SK_ERR_DEVICE;
   // tile, variant, schedule and grid all left open for a 16-bit or one-byte problem with more rows than the
-  // weight-streaming kernels take: the cost model chooses kernel and split
-  sk_config modelled;
-  const bool model_applies =
-      (dtype == SK_F16 || dtype == SK_BF16 || dtype == SK_F8E4M3 || dtype == SK_F8E5M2 || dtype == SK_I8) && M > 64 &&
-      !rows_65_to_96_stream(M, N, dtype, layout, num_cus) &&
-      (!cfg || (cfg->bm == 0 && cfg->bn == 0 && cfg->bk == 0 && cfg->reserved[0] == 0 &&
-                cfg->schedule == SK_SCHED_AUTO && cfg->grid == 0));
-  if (model_applies) {
-    if (cfg) modelled = *cfg; else memset(&modelled, 0, sizeof(modelled));
-    // (the ring kernels add up fp32 partial tiles: a fix-up that adds packed 16-bit partials into C, or exchanges them in 16
-    // bits, is a matter of the other tile kernels)
-    const int fixup = modelled.fixup;
-    if ((dtype == SK_F16 || dtype == SK_BF16) && layout == SK_LAYOUT_NT && M <= 128 && ring_pays(N, K) &&
-        (fixup == SK_FIXUP_AUTO || fixup == SK_FIXUP_REDUCE || fixup == SK_FIXUP_ATOMIC) &&
-        model_pick_ring(N, K, dtype, num_cus, &modelled))
-      cfg = &modelled;
+  // weight-streaming kernels take: the cost models choose kernel and split.  The kernels whose waves stream K on their own and
+  // the ring kernels add up fp32 partial tiles: a fix-up that adds packed 16-bit partials into C, or exchanges them in 16 bits,
+  // is a matter of the other tile kernels.  The former are for a caller who asks for SK_VARIANT_OPERATOR: a plan without it
+  // takes the kernels that plans have taken so far.  (So do products of fewer than 768 columns, for the workspaces their callers
+  // have sized -- 100 x 512 x 8192 of fp8 would take 9 us instead of 17 -- except where nothing else runs them in one launch.)
+  sk_config modelled, wavek;
+  const bool q4_rows = dtype == SK_Q4 || dtype == SK_Q4_ZP, b16 = dtype == SK_F16 || dtype == SK_BF16;
+  const bool one_byte = dtype == SK_F8E4M3 || dtype == SK_F8E5M2 || dtype == SK_I8;
+  const bool by_operator = cfg && cfg->reserved[0] == SK_VARIANT_OPERATOR && cfg->bm == 0 && cfg->bn == 0;
+  const bool open = !cfg || (cfg->bm == 0 && cfg->bn == 0 && cfg->bk == 0 && (cfg->reserved[0] == 0 || by_operator) &&
+                             cfg->schedule == SK_SCHED_AUTO && cfg->grid == 0);
+  const bool few = M <= 64;
+  if (by_operator) {
+    modelled = *cfg;
+    modelled.reserved[0] = one_byte && few ? 9 : 0;
+    cfg = &modelled;
   }
-  if (cfg != &modelled && model_applies) {
-    int split = 1, model_sched = SK_SCHED_AUTO;
-    if (const KernelInfo *mk = model_pick(M, N, K, dtype, layout, num_cus, &split, &model_sched)) {
-      if (cfg) modelled = *cfg; else memset(&modelled, 0, sizeof(modelled));
-      modelled.bm = mk->bm; modelled.bn = mk->bn; modelled.bk = mk->bk;
-      modelled.reserved[0] = mk->variant + 1;
-      modelled.schedule = model_sched;
-      if (split > 1) modelled.reserved[1] = split;
+  const int want_fixup = cfg ? cfg->fixup : SK_FIXUP_AUTO;
+  const bool fp32_partials = want_fixup == SK_FIXUP_AUTO || want_fixup == SK_FIXUP_REDUCE || want_fixup == SK_FIXUP_ATOMIC;
+  if (open && layout == SK_LAYOUT_NT && fp32_partials && by_operator && M > 16 && (N >= 768 || (dtype == SK_Q4_ZP && !few)) && (b16 || q4_rows || one_byte)) {
+    double wavek_us = 0, other_us = 0;
+    if (cfg) wavek = *cfg; else memset(&wavek, 0, sizeof(wavek));
+    const KernelInfo *k = model_pick_wavek(M, N, K, dtype, num_cus, &wavek, &wavek_us);
+    if (k && !few && !q4_rows) {
+      sk_config ring;
+      int split, sched;
+      if (!(b16 && M <= 128 && ring_pays(N, K) && model_pick_ring(N, K, dtype, num_cus, &ring, &other_us)))
+        model_pick(M, N, K, dtype, layout, num_cus, &split, &sched, &other_us);
+    }
+    if (k && wavek_pays(M, N, K, dtype, num_cus, wavek_us, other_us)) cfg = &wavek;
+  }
+  if (open && cfg != &wavek && (b16 || one_byte) && !few && !rows_65_to_96_stream(M, N, dtype, layout, num_cus)) {
+    double model_us = 0;
+    if (cfg) modelled = *cfg; else memset(&modelled, 0, sizeof(modelled));
+    if (b16 && layout == SK_LAYOUT_NT && M <= 128 && ring_pays(N, K) && fp32_partials &&
+        model_pick_ring(N, K, dtype, num_cus, &modelled, &model_us)) {
       cfg = &modelled;
+    } else {
+      int split = 1, model_sched = SK_SCHED_AUTO;
+      if (const KernelInfo *mk = model_pick(M, N, K, dtype, layout, num_cus, &split, &model_sched, &model_us)) {
+        modelled.bm = mk->bm; modelled.bn = mk->bn; modelled.bk = mk->bk;
+        modelled.reserved[0] = mk->variant + 1;
+        modelled.schedule = model_sched;
+        if (split > 1) modelled.reserved[1] = split;
+        cfg = &modelled;
+      }
     }
   }
   if (dtype == SK_F32 && (!cfg || (cfg->bm == 0 && cfg->bn == 0 && cfg->bk == 0 && cfg->reserved[0] == 0 &&

@@ -1,0 +1,384 @@
+// Tiles for a middling number of rows of A (NT): every wave of a CTA multiplies the whole tile with its own share of K.
+//
+//  * CTA = four waves, one per SIMD.  An iteration is four chunks of 128 bytes of K per row (64 16-bit or 128 one-byte
+//    K-values), one per wave.  A wave fetches the BM + BN rows of its chunk straight into a ring of LDS of its own (loads of
+//    8 rows x 128 bytes), reads the fragments back, refills what it has read and multiplies.  What orders a ring's loads, reads
+//    and refills is the wave's own vmcnt / lgkmcnt: the main loop has no barrier, no wave waits for another one's loads, and
+//    the CTA has most of its 160 KB of LDS in flight all the time.  Every fragment is read from LDS once per CTA.
+//  * The fragments of a chunk are read beside the MFMAs of the first half of the chunk before, its place is refilled beside those
+//    of the second half: a wave that has its SIMD for itself issues one instruction in four cycles, a quarter of an MFMA.
+//  * The ring is a ring of loads, R KB long, a chunk being L of them: for tiles whose chunks are larger than 20 KB, R is no
+//    multiple of L, and part of the chunk after next is in flight.
+//  * When the segment ends the four waves' sums are added by a butterfly through LDS, halving what each holds: a wave ends up
+//    with a quarter of the tile's 16 x 16 blocks, and all four take part in the epilogue and the fix-up.
+//
+// What bounds it: a CU takes 75 to 85 GB/s of operands (its direct loads alone 107, profiles/lds_direct_load_rate.md), whether
+// they come through LDS or registers (a variant that loads to registers and writes the chunk to LDS: 77 to 80 GB/s), and 3 us
+// pass before and 1 to 3 us, by the tile, behind the loop.  So it serves what fits one or two rounds of tiles.  Without the
+// interleaving of reads and refills 64 x 64 tiles took 18.3 us at 256 x 4096 x 4096, with it 16.9; every XCD walks K from a start of
+// its own, because all CTAs of one share A as well as the weights (a start per column of tiles: 2048 x 1024 x 4096 45 us, so 28).
+// Weights from HBM and the Infinity Cache in turn (three sets of operands), the kernels before / these, in us: fp16
+// 128 x 4096 x 4096 17.7 / 12.9, 256 x 4096 x 4096 22.0 / 17.0, 64 x 4096 x 4096 14.0 / 9.9, 128 x 2048 x 2048 13.0 / 6.6,
+// 1024 x 1024 x 8192 32.6 / 26.0 (eager), bf16 100 x 11008 x 4096 with bias and GELU 34.6 / 28.1 (eager); int8 100 x 4096 x 4096
+// 13.1 / 8.9, 128 x 8192 x 8192 21.6 / 17.0; fp8 256 x 1024 x 8192 24.9 / 10.2, 64 x 28672 x 8192 with bias and SiLU 57.0 / 51.3 (eager).
+#pragma once
+#include <type_traits>
+
+#include "sk_device.h"
+#include "tile_f16.h"
+
+namespace sk {
+
+enum WaveKType { WK_F16 = 0, WK_BF16 = 1, WK_F8E4M3 = 2, WK_F8E5M2 = 3, WK_I8 = 4, WK_Q4 = 5, WK_Q4ZP = 6 };
+
+// Q4 weights: with the array of zero points where every group has its own
+struct WaveKQ4Args : GemmArgs {
+  const half_t *zeros;
+};
+
+// what the kernels of this file share: who holds which block of the tile, the sums over the waves, epilogue, partial tiles
+template <int TYPE_, int FM_, int FN_>
+struct WaveKTile {
+  typedef typename std::conditional<(TYPE_ >= WK_Q4), WaveKQ4Args, GemmArgs>::type Args;
+  static constexpr bool LEAN_ENTRY = true;            // see run_persistent
+  static constexpr bool COHERENT_PARTIALS = true;
+  static constexpr bool FIXUP_WORD_IN_LDS = true;     // the rings are dead between two calls of mac
+  static constexpr int TYPE = TYPE_, FM = FM_, FN = FN_, BM = 16 * FM_, BN = 16 * FN_, WAVES = 4, NT = 256;
+  static constexpr int TILE_ELEMS = BM * BN, NB = FM * FN, NQ = NB / WAVES;   // blocks of the tile, of a wave's quarter
+  static_assert(NB % WAVES == 0, "the waves share out the blocks evenly");
+  static constexpr bool I8 = TYPE_ == WK_I8, BF16 = TYPE_ == WK_BF16, F8 = TYPE_ == WK_F8E4M3 || TYPE_ == WK_F8E5M2;
+  typedef int intx4 __attribute__((ext_vector_type(4)));
+  typedef typename std::conditional<I8, intx4, floatx4>::type AccV;
+  typedef typename std::conditional<I8, int, float>::type AccT;
+
+  // c[u]: block v = first_block() + u, that is C[pm*BM + (v / FN)*16 + lane%16][pn*BN + (v % FN)*16 + 4*(lane/16) + e]
+  struct Acc {
+    AccV c[NQ];
+  };
+  static __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
+  static __device__ __forceinline__ int first_block(int wave) { return (wave & 1) * (NB / 2) + (wave >> 1) * NQ; }
+
+  // c: the wave's sums of all blocks.  (w0 + w1) + (w2 + w3) in every wave, whatever it keeps.
+  static __device__ __forceinline__ void add_waves(AccV (&c)[NB], Acc &acc, char *smem) {
+    const int lane = threadIdx.x & 63, wave = wave_id();
+    AccV *mine = reinterpret_cast<AccV *>(smem) + (wave * (NB / 2)) * 64 + lane;
+    const AccV *theirs = reinterpret_cast<const AccV *>(smem) + ((wave ^ 1) * (NB / 2)) * 64 + lane;
+    __syncthreads();   // the rings are read
+    // (values are selected, not branches taken: two branches that differ in the block they name become one that indexes c)
+    const bool odd = wave & 1, high = wave & 2;
+    static_for<0, NB / 2>([&](auto v) {
+      const AccV lo = c[v], hi = c[NB / 2 + v];
+      mine[v * 64] = odd ? lo : hi;
+      c[v] = odd ? hi : lo;
+    });
+    __syncthreads();
+    static_for<0, NB / 2>([&](auto v) { c[v] += theirs[v * 64]; });
+    __syncthreads();
+    AccV *mine2 = reinterpret_cast<AccV *>(smem) + (wave * NQ) * 64 + lane;
+    const AccV *theirs2 = reinterpret_cast<const AccV *>(smem) + ((wave ^ 2) * NQ) * 64 + lane;
+    static_for<0, NQ>([&](auto v) {
+      const AccV lo = c[v], hi = c[NQ + v];
+      mine2[v * 64] = high ? lo : hi;
+      acc.c[v] = high ? hi : lo;
+    });
+    __syncthreads();
+    static_for<0, NQ>([&](auto v) { acc.c[v] += theirs2[v * 64]; });
+    __syncthreads();   // the rings may be filled again
+  }
+
+  // (two copies behind one uniform branch: the epilogue without a bias carries none of its code)
+  static __device__ __forceinline__ void store_c(const Args &a, const Acc &acc, int pm, int pn, char *, const void *bias) {
+    if (bias == nullptr)
+      store_c_impl<false>(a, acc, pm, pn, nullptr);
+    else
+      store_c_impl<true>(a, acc, pm, pn, bias);
+  }
+  template <bool BIAS>
+  static __device__ __forceinline__ void store_c_impl(const Args &a, const Acc &acc, int pm, int pn, const void *epi) {
+    const half_t *bias = BIAS ? epi_bias(epi) : nullptr;
+    const int act = BIAS ? epi_act(epi) : 0;
+    const int lane = threadIdx.x & 63, first = first_block(wave_id());
+    const bool vec_ok = (a.ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(a.C) & (I8 ? 15 : 7)) == 0);
+    floatx4 b4[NQ];
+    if constexpr (BIAS && !I8) {   // all loads at once
+#pragma unroll
+      for (int u = 0; u < NQ; ++u) b4[u] = bias4_at<BF16>(bias, pn * BN + ((first + u) % FN) * 16 + 4 * (lane >> 4), a.N);
+    }
+#pragma unroll
+    for (int u = 0; u < NQ; ++u) {
+      const int row = pm * BM + ((first + u) / FN) * 16 + (lane & 15);
+      const int col = pn * BN + ((first + u) % FN) * 16 + 4 * (lane >> 4);
+      if (row >= a.M || col >= a.N) continue;
+      if constexpr (I8) {   // int32 C straight from the accumulators (ldc counts int32 elements)
+        int *dst = reinterpret_cast<int *>(a.C) + (int64_t)row * a.ldc + col;
+        if (vec_ok && col + 4 <= a.N) {
+          *reinterpret_cast<intx4 *>(dst) = acc.c[u];
+        } else {
+          for (int e = 0; e < 4 && col + e < a.N; ++e) dst[e] = acc.c[u][e];
+        }
+      } else {
+        half4v h;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float x = acc.c[u][e];
+          if constexpr (F8) x *= a.alpha;
+          if constexpr (BIAS) x = activate(x + b4[u][e], act);
+          if constexpr (BF16) {
+            const __bf16 b = (__bf16)x;
+            h[e] = __builtin_bit_cast(half_t, b);  // C carries 16-bit patterns
+          } else {
+            h[e] = (half_t)x;
+          }
+        }
+        half_t *dst = a.C + (int64_t)row * a.ldc + col;
+        if (vec_ok && col + 4 <= a.N) {
+          *reinterpret_cast<half4v *>(dst) = h;
+        } else {
+          for (int e = 0; e < 4 && col + e < a.N; ++e) dst[e] = h[e];
+        }
+      }
+    }
+  }
+
+  // Partial tiles: block u of thread t at (u NT + t) 4; the accumulating form keeps element e of it at (u 4 + e) NT + t.
+  static __device__ __forceinline__ void store_partial(const Acc &acc, float *dst) {
+    const BufferRsrc r = make_rsrc(dst, TILE_ELEMS * 4);
+#pragma unroll
+    for (int u = 0; u < NQ; ++u) st_coherent16(r, threadIdx.x * 16, u * NT * 16, __builtin_bit_cast(uint4v, acc.c[u]));
+  }
+  static __device__ __forceinline__ void add_partial(Acc &acc, const float *src) {
+    const BufferRsrc r = make_rsrc(src, TILE_ELEMS * 4);
+    AccV x[NQ];
+#pragma unroll
+    for (int u = 0; u < NQ; ++u) x[u] = __builtin_bit_cast(AccV, ld_coherent16(r, threadIdx.x * 16, u * NT * 16));
+#pragma unroll
+    for (int u = 0; u < NQ; ++u) acc.c[u] += x[u];
+  }
+  static __device__ __forceinline__ void atomic_partial(const Acc &acc, float *dst_) {
+    AccT *dst = reinterpret_cast<AccT *>(dst_);
+#pragma unroll
+    for (int u = 0; u < NQ; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (I8)
+          atomic_add_i32(dst + (size_t)(u * 4 + e) * NT + threadIdx.x, acc.c[u][e]);
+        else
+          atomic_add_f32(dst + (size_t)(u * 4 + e) * NT + threadIdx.x, acc.c[u][e]);
+      }
+  }
+  static __device__ __forceinline__ void take_partial(Acc &acc, float *src_) {
+    AccT *src = reinterpret_cast<AccT *>(src_);
+#pragma unroll
+    for (int u = 0; u < NQ; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        AccT *p = src + (size_t)(u * 4 + e) * NT + threadIdx.x;
+        acc.c[u][e] = ld_coherent_scalar(p);
+        st_coherent(p, (AccT)0);
+      }
+  }
+};
+
+// dma_load_16 (sk_device.h) to lds_base + IMM: one scalar instruction for the address.  A wave has its SIMD for itself in these
+// kernels and issues one instruction in four cycles, so what a load costs in them is what it takes from the MFMAs.
+template <int IMM>
+static __device__ __forceinline__ void wavek_dma_16(uint4v rsrc, uint32_t lds_base, uint32_t lane_off, uint32_t uniform_off) {
+  asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :
+               : "s"(lds_base), "v"(lane_off), "s"(rsrc), "s"(uniform_off), "n"(IMM)
+               : "memory", "m0", "scc");
+}
+// two bytes per lane, zero-extended to four: lane l's value lands at lds_base + IMM + 4 l
+template <int IMM>
+static __device__ __forceinline__ void wavek_dma_2(uint4v rsrc, uint32_t lds_base, uint32_t lane_off, uint32_t uniform_off) {
+  asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_ushort %1, %2, %3 offen lds"
+               :
+               : "s"(lds_base), "v"(lane_off), "s"(rsrc), "s"(uniform_off), "n"(IMM)
+               : "memory", "m0", "scc");
+}
+
+template <int N>
+static __device__ __forceinline__ void wavek_wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N < 63 ? N : 63) : "memory");
+}
+
+template <int TYPE_, int FM_, int FN_>
+struct TileWaveK : WaveKTile<TYPE_, FM_, FN_> {
+  typedef WaveKTile<TYPE_, FM_, FN_> Base;
+  typedef typename Base::Args Args;
+  typedef typename Base::Acc Acc;
+  typedef typename Base::AccV AccV;
+  static constexpr int FM = FM_, FN = FN_, BM = Base::BM, BN = Base::BN, WAVES = Base::WAVES, NT = Base::NT, NB = Base::NB;
+  static constexpr int KV = 64, BK = KV * WAVES;      // 16-bit units of K: of a chunk, of an iteration
+  static constexpr int L = 2 * (FM + FN);             // loads of a chunk
+  static constexpr int R = L > 20 ? 40 : (L * 4 < 40 ? L * 4 : 40 / L * L);   // loads of a wave's ring (at most 160 KB / 4 waves, four chunks)
+  static constexpr int S = R / L, PART = R % L;       // whole chunks in the ring, loads of one more
+  static_assert(S >= 1 && (L % 2) == 0 && (R % 2) == 0, "a 16-row block of a chunk stays together in the ring");
+  static constexpr int RING = R * 1024, LDS_RINGS = WAVES * RING, LDS_SUMS = WAVES * (NB / 2) * 1024;
+  static constexpr int LDS_BYTES = LDS_RINGS > LDS_SUMS ? LDS_RINGS : LDS_SUMS, LDS_TOTAL = LDS_BYTES;
+  static_assert(LDS_BYTES <= 160 * 1024, "LDS of a CU");
+  static constexpr int CTAS_PER_CU = 1, WAVES_PER_EU = 1;
+  static constexpr int NMFMA = Base::F8 ? NB : 2 * NB;   // MFMAs of a chunk
+  static constexpr int H = NMFMA / 2, HR = H - (H + 3) / 4;   // of a phase, of those that have fragments read beside them
+
+  // the loads of a chunk behind which `left` more chunks of the segment follow (the last PART loads of a segment fetch nothing)
+  static __device__ __forceinline__ void wait_chunk(int left) {
+    if (left >= S - 1) wavek_wait_loads<R - L>();
+    else if (left == 0) wavek_wait_loads<PART>();
+    else if (left == 1) wavek_wait_loads<L + PART>();
+    else wavek_wait_loads<2 * L + PART>();
+  }
+  struct Frags {
+    half8v a[FM][2], b[FN][2];   // [K-step]
+  };
+  // MFMA m of a chunk
+  template <int m>
+  static __device__ __forceinline__ void mfma(AccV (&c)[NB], const Frags &f) {
+    constexpr int v = m % NB, s = m / NB, i = v / FN, j = v % FN;
+    if constexpr (Base::F8) {
+      typedef int intx8 __attribute__((ext_vector_type(8)));
+      struct Pair { half8v v[2]; };
+      const intx8 b = __builtin_bit_cast(intx8, Pair{{f.b[j][0], f.b[j][1]}}), x = __builtin_bit_cast(intx8, Pair{{f.a[i][0], f.a[i][1]}});
+      constexpr int FMT = TYPE_ == WK_F8E4M3 ? 0 : 1;
+      c[v] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b, x, c[v], FMT, FMT, 0, 0, 0, 0);
+    } else if constexpr (Base::I8) {
+      typedef typename Base::intx4 intx4;
+      c[v] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(intx4, f.b[j][s]), __builtin_bit_cast(intx4, f.a[i][s]), c[v], 0, 0, 0);
+    } else if constexpr (Base::BF16) {
+      typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+      c[v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, f.b[j][s]), __builtin_bit_cast(bf16x8, f.a[i][s]), c[v], 0, 0, 0);
+    } else {
+      c[v] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.b[j][s], f.a[i][s], c[v], 0, 0, 0);
+    }
+  }
+
+  static __device__ __forceinline__ void mac(const Args &a, Acc &acc, int pm, int pn, int k0, int n, char *smem) {
+    const int lane = threadIdx.x & 63, wave = Base::wave_id();
+    AccV c[NB];
+    static_for<0, NB>([&](auto v) { c[v] = AccV{0, 0, 0, 0}; });
+    // ---- descriptors: rows past M / N read as zero ----
+    const uint32_t lda_bytes = (uint32_t)a.lda * 2, ldb_bytes = (uint32_t)a.ldb * 2;
+    const uint4v rsrc_a = uniform_rsrc(make_rsrc_words(a.A + (int64_t)pm * BM * a.lda, (uint32_t)min(BM, a.M - pm * BM) * lda_bytes));
+    const uint4v rsrc_b = uniform_rsrc(make_rsrc_words(a.B + (int64_t)pn * BN * a.ldb, (uint32_t)min(BN, a.N - pn * BN) * ldb_bytes));
+    // load l of a chunk: rows 8 l .. 8 l + 7 (A's first), lane's row lane / 8, piece p (16 bytes) of row r of a block at position
+    // p ^ ((r >> 1) & 7)
+    const int row8 = lane >> 3;
+    uint32_t off[L];
+    int kp[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) kp[e] = ((lane & 7) ^ (4 * e + (row8 >> 1))) * 8;
+    static_for<0, L>([&](auto l) {
+      off[l] = l < 2 * FM ? (uint32_t)(8 * l + row8) * lda_bytes + (uint32_t)kp[l & 1] * 2
+                          : (uint32_t)(8 * (l - 2 * FM) + row8) * ldb_bytes + (uint32_t)kp[l & 1] * 2;
+    });
+    const uint32_t ring = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_address(smem) + wave * RING);
+    // one row of tiles: see rotation_of.  Several: the CTAs of an XCD share A as well as the weights and stay on the same K
+    const int rot = a.M <= BM ? rotation_of(pn, n) : (int)((blockIdx.x & 7) * (uint32_t)n) >> 3;
+    // load l of a chunk that starts kbytes into the rows and `left` 16-bit units before K's end, pos: where the chunk starts in
+    // the ring.  (Pieces past K fetch nothing: zeros arrive and the wait counts stay exact.)
+    struct Chunk {
+      uint32_t kbytes;
+      int left, pos;
+      uint32_t base;   // LDS address of load 0, were the ring long enough
+    };
+    auto chunk = [&](int t, int pos) {
+      const int kk = ((k0 + rotated_iteration(t, rot, n)) * WAVES + wave) * KV, left = t < n ? a.K - kk : 0;
+      // (a chunk past K or past the segment must not carry its offset either)
+      return Chunk{(uint32_t)__builtin_amdgcn_readfirstlane(left > 0 ? kk * 2 : 0), left, pos, ring + (uint32_t)pos * 1024};
+    };
+    auto issue = [&](auto li, const Chunk &q) {
+      constexpr int l = decltype(li)::value;
+      uint32_t base = q.base;
+      if (R % L != 0) base = q.pos >= R - l ? base - R * 1024 : base;
+      wavek_dma_16<l * 1024>(l < 2 * FM ? rsrc_a : rsrc_b, base, q.left >= KV || kp[l & 1] < q.left ? off[l] : OOB_OFFSET, q.kbytes);
+    };
+#pragma unroll
+    for (int t = 0; t < S; ++t)
+      if (t < n) {
+        const Chunk q = chunk(t, t * L);
+        static_for<0, L>([&](auto l) { issue(l, q); });
+      }
+    {
+      const Chunk q = chunk(S, S * L);
+      static_for<0, PART>([&](auto l) { issue(l, q); });
+    }
+
+    // fragments: lane (i, g) takes piece 4 s + g of its row for K-step s
+    const int fi = lane & 15, fg = lane >> 4;
+    const char *rd0 = smem + wave * RING + fi * 128 + ((fg ^ ((fi >> 1) & 7)) * 16), *rd1 = smem + wave * RING + fi * 128 + (((4 + fg) ^ ((fi >> 1) & 7)) * 16);
+    auto read = [&](auto ri, Frags &f, int pos) {
+      constexpr int r = decltype(ri)::value, s = r / (FM + FN), b = r % (FM + FN);   // block b of the chunk: A's, then the weights'
+      const char *from = (s ? rd1 : rd0) + pos * 1024;
+      if (R % L != 0) from = pos >= R - 2 * b ? from - R * 1024 : from;
+      const half8v x = *reinterpret_cast<const half8v *>(from + 2 * b * 1024);
+      if constexpr (b < FM) f.a[b][s] = x;
+      else f.b[b - FM][s] = x;
+    };
+    int pos = 0;   // of the chunk that is read next
+    auto advance = [&] {
+      pos += L;
+      if (pos >= R) pos -= R;
+    };
+    // the place of the chunk just read (t) takes the rest of chunk t + S and the first PART loads of chunk t + S + 1
+    Chunk q0, q1;
+    auto refill_begin = [&](int t) {
+      int p = pos + S * L;
+      if (p >= R) p -= R;
+      q0 = chunk(t + S, p);
+      p += L;
+      if (p >= R) p -= R;
+      if (PART > 0) q1 = chunk(t + S + 1, p);
+    };
+    auto refill = [&](auto xi) {
+      constexpr int x = decltype(xi)::value;
+      if constexpr (x < L - PART) issue(std::integral_constant<int, x + PART>{}, q0);
+      else issue(std::integral_constant<int, x - (L - PART)>{}, q1);
+    };
+    // X: fragments of chunk t, Y: of chunk t + 1, read while the first half of chunk t is multiplied; their place is refilled
+    // during the second half
+    auto body = [&](int t, const Frags &x, Frags &y) {
+      if (t + 1 < n) {
+        wait_chunk(n - 2 - t);
+        static_for<0, H>([&](auto m) {
+          mfma<m>(c, x);
+          // (none beside the last MFMAs: they are waited for behind those)
+          static_for<(m * L / HR < L ? m * L / HR : L), ((m + 1) * L / HR < L ? (m + 1) * L / HR : L)>([&](auto r) { read(r, y, pos); });
+          __builtin_amdgcn_sched_barrier(0);
+        });
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      } else {
+        static_for<0, H>([&](auto m) { mfma<m>(c, x); });
+      }
+      if (t + 1 + S < n) {
+        refill_begin(t + 1);
+        static_for<0, NMFMA - H>([&](auto m) {
+          mfma<H + m>(c, x);
+          static_for<m * L / (NMFMA - H), (m + 1) * L / (NMFMA - H)>([&](auto l) { refill(l); });
+          __builtin_amdgcn_sched_barrier(0);
+        });
+      } else {
+        static_for<H, NMFMA>([&](auto m) { mfma<m>(c, x); });
+      }
+      advance();
+    };
+    Frags x, y;
+    wait_chunk(n - 1);
+    static_for<0, L>([&](auto r) { read(r, x, pos); });
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (S < n) {
+      refill_begin(0);
+      static_for<0, L>([&](auto l) { refill(l); });
+    }
+    advance();
+    for (int t = 0;;) {
+      body(t, x, y);
+      if (++t == n) break;
+      body(t, y, x);
+      if (++t == n) break;
+    }
+    wavek_wait_loads<0>();   // the loads past the segment write LDS too
+    Base::add_waves(c, acc, smem);
+  }
+};
+
+}  // namespace sk

@@ -173,9 +173,9 @@ at::Tensor gemm_i8(const at::Tensor &A, const at::Tensor &B, const at::Tensor *o
   return rc == SK_OK ? C : at::Tensor();
 }
 
-// operands A, Wq, scales, zeros; (zero, group, tiled, config, bias, activation).  One launch, row-major weights: up to 64
-// rows, or with one zero point for the matrix as many as the Q4 tile kernels serve -- a shape that the general
-// implementation answers with several launches never has a plan here under these types.
+// operands A, Wq, scales, zeros; (zero, group, tiled, config, bias, activation).  One launch, row-major weights, as many rows as
+// the Q4 tile kernels serve -- a shape that the general implementation answers with several launches never has a plan here
+// under these types.
 at::Tensor gemm_q4(const c10::IValue *operands, const at::Tensor *out, const c10::IValue *a) {
   const at::Tensor &A = operands[0].toTensor(), &Wq = operands[1].toTensor(), &scales = operands[2].toTensor();
   const int64_t zero = a[0].toInt(), group = a[1].toInt();
@@ -192,7 +192,8 @@ at::Tensor gemm_q4(const c10::IValue *operands, const at::Tensor *out, const c10
     if (!is_matrix(z, at::kHalf) || !z.is_contiguous() || z.sizes() != scales.sizes()) return {};
     zeros = z.data_ptr();
   }
-  if (M > (zp ? 64 : 1024)) return {};
+  // (per-group zero points and few columns: the general implementation, as before there were kernels for these rows)
+  if (M > 1024 || (zp && M > 64 && N < 768)) return {};
   sk_epilogue epi;
   bool used;
   if (!epilogue(a[4], a[5], A, N, at::kHalf, &epi, &used)) return {};

@@ -33,13 +33,17 @@ _SKINNY_F8 = [(16, 64, 256), (32, 64, 256), (16, 16, 1024), (16, 32, 512), (16, 
               (64, 64, 256), (64, 64, 512)]
 # one-byte weights streamed through LDS in contiguous loads (variant 9 of these shapes)
 _STREAM_BYTES = [(16, 16, 2048), (16, 32, 1024), (16, 64, 512), (32, 32, 1024), (32, 64, 512), (64, 32, 512), (64, 64, 512)]
+# tiles whose waves stream K on their own (variant 11)
+_WAVEK = [(32, 32), (32, 64), (64, 32), (64, 48), (64, 64), (64, 80), (64, 96), (64, 112), (64, 128), (96, 32), (96, 64), (128, 32),
+          (128, 48), (128, 64)]
+_WAVEK_Q4 = [(32, 32), (32, 64), (64, 32), (64, 64), (64, 96), (128, 32)]
 _SKINNY_Q4 = [(16, 64, 256), (32, 64, 256), (64, 64, 256), (16, 16, 1024), (16, 32, 512), (16, 16, 256),
               (16, 32, 256), (16, 32, 1024), (16, 16, 2048), (16, 64, 512), (16, 16, 512)]
 
 
 # which kernels a search had, kept in the entries it writes: 2 has the one-byte kernels that stream the weights through LDS,
-# the Q4 ones whose waves stream K on their own and the ring kernels of 65 to 128 rows
-SEARCH = 2
+# the Q4 ones whose waves stream K on their own and the ring kernels of 65 to 128 rows, 3 the tiles whose waves stream K on their own
+SEARCH = 3
 
 
 def _key(dtype, layout, M, N, K):
@@ -67,7 +71,7 @@ def untuned_config(M, N, K, dtype, layout="nt", cus=None):
     configuration does."""
     cus = cus or _plan.num_cus()
     try:
-        untuned = {"variant": 9} if M <= 64 and dtype in ("float8_e4m3", "float8_e5m2", "int8") else None
+        untuned = {"variant": _plan.OPERATOR_VARIANT} if M <= 64 and dtype in ("float8_e4m3", "float8_e5m2", "int8") else None
         p = _plan.make_plan(M, N, K, dtype, layout, untuned, cus=cus, use_tuned=False)
     except StreamKError:
         return None
@@ -83,7 +87,7 @@ def untuned_config(M, N, K, dtype, layout="nt", cus=None):
         cfg["raster"] = p.raster
     if p.interleave > 1:
         cfg["interleave"] = 1
-    for variant in range(1, 11):
+    for variant in range(1, 12):
         try:
             q = _plan.make_plan(M, N, K, dtype, layout, dict(cfg, variant=variant), cus=cus)
         except StreamKError:
@@ -140,6 +144,15 @@ def candidate_configs(M, N, K, dtype="float16", cus=None, reduce16=True, layout=
             base = dict(bm=16, bn=bn, bk=1024, variant=6)
             out.append(dict(base, schedule="dp"))
             out.extend(dict(base, schedule="basic", grid=cus, fixup=fixup) for fixup in ("reduce", "atomic"))
+    if layout == "nt" and M > 16:
+        # tiles whose waves stream K on their own (variant 11)
+        for (bm, bn) in _WAVEK_Q4 if dtype in ("q4", "q4_zp") else (_WAVEK if dtype != "float32" else ()):
+            if bm >= 2 * M or -(-M // bm) * -(-N // bn) > 3 * cus:
+                continue
+            base = dict(bm=bm, bn=bn, variant=11, raster=8 if M > bm else 0)
+            out.append(dict(base, schedule="dp"))
+            out.extend(dict(base, schedule="splitk", split=split, fixup="reduce") for split in (2, 4, 8)
+                       if -(-M // bm) * -(-N // bn) * split <= cus)
     if dtype in ("float16", "bfloat16") and 64 < M <= 128:
         # rings of different depths for weights and A (variant 10; NT)
         for bn in (64, 128):

@@ -300,6 +300,15 @@ def _zero_points(zeros, scales):
     return zeros
 
 
+def _has_plan(config, M, N, K, dtype):
+    """Whether some kernel runs the configuration for all the rows at once."""
+    try:
+        _plan_for(config, M, N, K, dtype, "nt")
+        return True
+    except _lib.StreamKError:
+        return False
+
+
 def _run_q4(A, Wq, scales, zeros, C, zero, group, tiled, config, bias, activation):
     if zeros is not None:
         zeros = _zero_points(zeros, scales)  # (row-major like the scales also where the weights are tiled)
@@ -314,12 +323,11 @@ def _run_q4(A, Wq, scales, zeros, C, zero, group, tiled, config, bias, activatio
     if tuple(scales.shape) != (N, K // group) or not scales.is_contiguous():
         raise ValueError(f"scales must be contiguous [N, K/group]; got {tuple(scales.shape)}")
     _check_out(C, M, N, torch.float16)
-    if M > Q4_MAX_M and (zeros is not None or tiled) and not config.startswith("#"):
-        # The weight-streaming kernels take at most 64 rows of A; beyond that row-major weights with a scalar zero
-        # point go to the Q4 tile kernels (below, like any other plan).  Per-group zero points and the tiled
-        # layout have no tile kernel: up to 256 rows one launch per block of 64 rows, beyond that the weights are
-        # dequantised once (bit-exact device function) for the fp16 tile kernels.  (Blocks of two rows and more multiply
-        # the rounded weights alike; a last block of one row takes the matrix-vector kernels and the unrounded ones.)
+    if M > Q4_MAX_M and (tiled or (zeros is not None and config and not _has_plan(config, M, N, K, "q4_zp"))) \
+            and not config.startswith("#"):
+        # The kernels for the tiled layout take at most 64 rows of A: up to 256 rows one launch per block of 64, and so do
+        # configurations that name kernels for few rows.  (Blocks of two rows and more multiply the rounded weights alike; a
+        # last block of one row takes the matrix-vector kernels and the unrounded ones.)
         if M <= 4 * Q4_MAX_M:
             for m0 in range(0, M, Q4_MAX_M):
                 _run_q4(A[m0:m0 + Q4_MAX_M], Wq, scales, zeros, C[m0:m0 + Q4_MAX_M], zero, group, tiled, config,
@@ -327,18 +335,21 @@ def _run_q4(A, Wq, scales, zeros, C, zero, group, tiled, config, bias, activatio
             return
         if tiled:
             raise ValueError("more than 256 rows of A need the row-major weights (they are dequantised once)")
-        W = torch.empty((N, K), dtype=torch.float16, device=Wq.device)
+        config = ""
+        dequantise = True
+    else:
+        # (with per-group zero points the kernels for many rows have 64 x 64 tiles: beyond 256 rows and three rounds of them the
+        # pass pays; 512 x 8192 x 8192 97 us against 103, 512 x 4096 x 4096 41 against 30)
+        dequantise = config == "" and (M > Q4_FUSED_MAX_M or (
+            zeros is not None and M > 4 * Q4_MAX_M and -(-M // 64) * -(-N // 64) > 3 * _plan_mod.num_cus()))
+    if dequantise:
+        # Prefill-sized calls: one pass that dequantises the weights (bit-exact device function), then the fp16 tile kernels
+        # on them.  The pass costs 26 us for 8192 x 8192 weights, under 7 % of the product from 4096 rows on, where the
+        # fused Q4 tile kernels are behind the four-wave fp16 kernel.  The buffer is kept per stream, allocated on first use;
+        # with per-group zero points it is the call's own.
+        W = (_staging(N * K * 2, A.device).view(torch.float16)[:N * K].view(N, K) if zeros is None
+             else torch.empty((N, K), dtype=torch.float16, device=Wq.device))
         _run_dequant_q4(Wq, scales, zeros, W, zero, group)
-        _run_16bit(A, W, C, "nt", "", bias, activation, torch.float16, "float16")
-        return
-    if M > Q4_FUSED_MAX_M and config == "":
-        # Prefill-sized calls: one pass that dequantises the weights (bit-exact device function) into a staging
-        # buffer kept per stream, then the fp16 tile kernels on it.  The pass costs 26 us for 8192 x 8192 weights,
-        # under 7 % of the product from 4096 rows on, where the fused Q4 tile kernels (the register-limited
-        # eight-wave form) are 20-25 % behind the four-wave fp16 kernel.  The buffer is allocated on first use and
-        # kept: no allocation per call.
-        W = _staging(N * K * 2, A.device).view(torch.float16)[:N * K].view(N, K)
-        _run_dequant_q4(Wq, scales, None, W, zero, group)
         _run_16bit(A, W, C, "nt", "", bias, activation, torch.float16, "float16")
         return
     name = ("q4_zp_tiled" if tiled else "q4_zp") if zeros is not None else ("q4_tiled" if tiled else "q4")

@@ -26,7 +26,8 @@ def num_cus():
 def make_config(config=None, **kw):
     """dict / kwargs -> SkConfig.  Keys: bm, bn, bk, grid, schedule ('auto'|'dp'|'sk2'|'sk1'|
     'basic'|'splitk'), split, fixup ('auto'|'atomic'|'reduce'|'atomic_c'|'reduce16'), raster, spin_limit, variant, interleave.
-    variant 9 with up to 64 rows of one-byte operands and no tile: the kernels that stream the weights through LDS."""
+    variant 9 with up to 64 rows of one-byte operands and no tile: the kernels that stream the weights through LDS;
+    variant 11 with a tile: the kernels whose waves stream K on their own."""
     d = dict(config or {})
     d.update(kw)
     c = SkConfig()
@@ -96,23 +97,29 @@ def tuned_config(M, N, K, dtype="float16", layout="nt"):
 _TWIN_OF = {"bfloat16": "float16", "float8_e5m2": "float8_e4m3"}
 
 
-# search space of the autotuner that has the kernels which stream one-byte weights through LDS; entries carry theirs
+# What the operators ask sk_make_plan for: the fastest kernels it knows, the ones that stream one-byte weights through LDS
+# (variant 9) and the ones whose waves stream K on their own (variant 11) among them.  Without it a plan takes one of the
+# kernels that plans have always taken.
+OPERATOR_VARIANT = 12
+_WAVEK_DTYPES = ("float16", "bfloat16", "float8_e4m3", "float8_e5m2", "int8", "q4", "q4_zp")
+# search space of the autotuner that has the former; entries carry theirs
 SEARCH_WITH_BYTE_STREAMS = 2
 
 
 def operator_config(M, N, K, dtype, layout):
-    """Configuration of an operator call that names none: the tuned one (None: make_plan finds it), else, for up to 64
-    rows of one-byte operands, the kernels that stream the weights through LDS (16 x 4096 x 4096 6.5 us against 9.8 on
-    the general small-M kernel that the library's heuristic takes, 64 x 28672 x 8192 56.5 / 67.5).  A tuned entry from a
-    search that did not have these kernels does not speak for them: it configures the plans that make_plan gives, and
-    an operator call takes the faster kernel (16 x 8192 x 8192 14.3 us, by the entry 16.7)."""
-    if M > 64 or dtype not in ("float8_e4m3", "float8_e5m2", "int8"):
+    """Configuration of an operator call that names none: the tuned one (None: make_plan finds it), else what
+    OPERATOR_VARIANT says, for weights [N, K] and the types that have those kernels.  Up to 64 rows of one-byte operands a tuned
+    entry from a search that did not have the kernels which stream the weights through LDS does not speak for them: it
+    configures the plans that make_plan gives, and an operator call takes the kernels the library chooses (16 x 8192 x 8192 of
+    fp8 14.3 us, by the entry 16.7)."""
+    few_bytes = M <= 64 and dtype in ("float8_e4m3", "float8_e5m2", "int8")
+    if layout != "nt" or not (few_bytes or (M > 16 and dtype in _WAVEK_DTYPES)):
         return None
     for d in dict.fromkeys((dtype, _TWIN_OF.get(dtype, dtype))):
         hit = _tuned_entry(M, N, K, d, layout)
-        if hit and hit.get("search", 1) >= SEARCH_WITH_BYTE_STREAMS:
+        if hit and hit.get("search", 1) >= (SEARCH_WITH_BYTE_STREAMS if few_bytes else 0):
             return None
-    return {"variant": 9}
+    return {"variant": OPERATOR_VARIANT}
 
 
 def make_plan(M, N, K, dtype="float16", layout="nt", config=None, cus=None, use_tuned=True, **kw):

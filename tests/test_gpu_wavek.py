@@ -1,0 +1,137 @@
+"""Tiles whose waves stream K on their own (tile_wavek.h, tile_wavek_q4.h): every tile of every type on operands whose sums are
+exact in fp32, so that results are equal to the bit whatever the order of the sums; and the operators' choice of them against
+the kernels that plans take."""
+import numpy as np
+import pytest
+
+_TILES = [(32, 32), (32, 64), (64, 32), (64, 48), (64, 64), (64, 80), (64, 96), (64, 112), (64, 128), (96, 32), (96, 64), (128, 32),
+          (128, 48), (128, 64)]
+_TILES_Q4 = [(32, 32), (32, 64), (64, 32), (64, 64), (64, 96), (128, 32)]
+
+
+@pytest.fixture(scope="module")
+def sk():
+    import streamk
+    return streamk
+
+
+def _small(rng, shape, most=2):
+    return rng.integers(-most, most + 1, shape).astype(np.float64)
+
+
+def _operands(torch, dtype, rng, M, N, K, pad=0):
+    """A (rows `pad` elements further apart), weights, a call, the exact product and the type of C."""
+    if dtype.startswith("q4"):
+        A = _small(rng, (M, K))
+        q = rng.integers(0, 16, (N, K))
+        zeros = rng.integers(0, 16, (N, K // 128)) if dtype == "q4_zp" else np.full((N, K // 128), 8)
+        scales = 2.0 ** rng.integers(-4, -1, (N, K // 128))
+        W = (q - np.repeat(zeros, 128, 1)) * np.repeat(scales, 128, 1)
+        Wq = torch.from_numpy((q[:, 0::2] | q[:, 1::2] << 4).astype(np.uint8)).cuda()
+        ds, dz = torch.from_numpy(scales).half().cuda(), torch.from_numpy(zeros).half().cuda() if dtype == "q4_zp" else None
+        kind, rest = torch.float16, (Wq, ds)
+    else:
+        A, W = _small(rng, (M, K)), _small(rng, (N, K))
+        kind = {"float8_e4m3": torch.float8_e4m3fn, "float8_e5m2": torch.float8_e5m2}.get(dtype) or getattr(torch, dtype)
+        rest = (torch.from_numpy(W).float().cuda().to(kind),)
+    dA = torch.zeros(M, K + pad, device="cuda").to(kind) if kind != torch.int8 else torch.zeros(M, K + pad, device="cuda", dtype=kind)
+    dA[:, :K].copy_(torch.from_numpy(A).float().cuda().to(kind))
+    import streamk
+    f = {"float16": streamk.streamk_fp16, "bfloat16": streamk.streamk_bf16, "int8": streamk.streamk_int8}.get(dtype)
+    if dtype in ("float16", "bfloat16"):
+        call = lambda **kw: f(dA[:, :K], rest[0], layout="nt", **kw)   # noqa: E731
+    elif dtype == "int8":
+        call = lambda **kw: f(dA[:, :K], rest[0], **kw)   # noqa: E731
+    elif dtype.startswith("float8"):
+        call = lambda **kw: streamk.streamk_fp8(dA[:, :K], rest[0], **kw)   # noqa: E731
+    else:
+        call = lambda **kw: streamk.streamk_q4(dA[:, :K], rest[0], rest[1], zeros=dz, **kw)   # noqa: E731
+    return call, A @ W.T
+
+
+def _rounded(torch, exact, dtype):
+    if dtype == "int8":
+        return torch.from_numpy(exact).to(torch.int32)
+    return torch.from_numpy(exact).float().to(torch.bfloat16 if dtype == "bfloat16" else torch.float16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16", "float8_e4m3", "float8_e5m2", "int8", "q4", "q4_zp"])
+def test_every_tile_is_exact(sk, dtype):
+    import torch
+    rng = np.random.default_rng(41)
+    step = 128 if dtype.startswith("q4") else (16 if "8" in dtype and dtype != "bfloat16" and dtype != "float16" else 8)
+    long = {128: 6528, 16: 5136, 8: 2568}[step]   # rings full, iterations that K does not fill, odd numbers of them
+    for bm, bn in _TILES_Q4 if dtype.startswith("q4") else _TILES:
+        for M, N, K in ((bm + 1, 2 * bn + 8, long), (1, 1, step), (2 * bm - 3, bn + 5, 3 * step + (128 if step < 128 else 0)), (bm, 3 * bn, 2048)):
+            call, exact = _operands(torch, dtype, rng, M, N, K, pad=8 if dtype in ("float16", "bfloat16") or step == 128 else 16)
+            want = _rounded(torch, exact, dtype)
+            for sched in (dict(schedule="dp"), dict(schedule="splitk", split=2, fixup="reduce"), dict(schedule="basic", grid=7, fixup="reduce"),
+                          dict(schedule="basic", grid=5, fixup="atomic")):
+                try:
+                    plan = sk.make_plan(M, N, K, dtype, "nt", dict(sched, bm=bm, bn=bn, variant=11))
+                except sk.StreamKError:
+                    assert sched["schedule"] == "splitk"   # (a split that does not divide the iterations)
+                    continue
+                assert sk.kernel_name(plan.kernel_id).startswith("wavek_")
+                got = call(plan=plan).cpu()
+                assert torch.equal(got, want), (dtype, bm, bn, M, N, K, sched, (got != want).sum().item())
+            if dtype != "int8":
+                kind = torch.bfloat16 if dtype == "bfloat16" else torch.float16
+                bias = torch.from_numpy(rng.integers(-8, 9, N).astype(np.float32)).to(kind)
+                plan = sk.make_plan(M, N, K, dtype, "nt", dict(bm=bm, bn=bn, variant=11, schedule="dp"))
+                got = call(plan=plan, bias=bias.cuda(), activation="relu").cpu()
+                want = _rounded(torch, np.maximum(exact + bias.double().numpy(), 0), dtype)
+                assert torch.equal(got, want), (dtype, bm, bn, M, N, K)
+    sk.workspace_status()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16", "float8_e4m3", "int8", "q4", "q4_zp"])
+def test_operator_calls_equal_the_plans_they_replace(sk, dtype):
+    """What an operator call takes by itself against the plan that make_plan gives (per-group zero points beyond 64 rows: the
+    exact product alone), sizes around the limits of the rule, rows of A and C further apart than they are long, C at an odd
+    element."""
+    import torch
+    rng = np.random.default_rng(42)
+    step = 128 if dtype.startswith("q4") else (16 if dtype in ("float8_e4m3", "int8") else 8)
+    seen = set()
+    for M, N, K in ((17, 768, 1536), (33, 770, 6144), (40, 2049, 2048), (64, 1000, 8192), (65, 775, 512), (100, 3001, 1664), (128, 768, 4096),
+                    (129, 1031, 640), (257, 2050, 1152), (300, 769, 2304), (513, 801, 384)):
+        K = K // step * step
+        call, exact = _operands(torch, dtype, rng, M, N, K, pad=8 * (2 if step == 16 else 1))
+        want = _rounded(torch, exact, dtype)
+        plan = sk.make_plan(M, N, K, dtype, "nt", sk.plan.operator_config(M, N, K, dtype, "nt"))
+        seen.add(sk.kernel_name(plan.kernel_id).split("_")[0])
+        for _ in range(2):   # (the first call through Python, the second natively)
+            assert torch.equal(call().cpu(), want), (dtype, M, N, K, sk.kernel_name(plan.kernel_id))
+        if not (dtype == "q4_zp" and M > 64):
+            assert torch.equal(call(plan=sk.make_plan(M, N, K, dtype, "nt", use_tuned=False)).cpu(), want), (dtype, M, N, K)
+        buf = torch.zeros(M * (N + 3) + 1, dtype=want.dtype, device="cuda")
+        out = buf[1:].view(M, N + 3)[:, :N]
+        call(out=out)
+        assert torch.equal(out.cpu(), want) and not buf[1:].view(M, N + 3)[:, N:].any() and not buf[:1].any(), (dtype, M, N, K)
+    assert "wavek" in seen, dtype
+    sk.workspace_status()
+
+
+def test_the_operators_rule(sk):
+    """Plans keep the kernels they had; an operator call takes these where the model says so, never for [K, N] weights, few
+    columns or fix-ups that they do not have."""
+    wavek = lambda *a, **k: sk.kernel_name(sk.make_plan(*a, cus=256, use_tuned=False, **k).kernel_id).startswith("wavek_")   # noqa: E731
+    for dtype in ("float16", "bfloat16", "float8_e4m3", "float8_e5m2", "int8", "q4", "q4_zp"):
+        for M, N, K in ((100, 4096, 4096), (256, 4096, 4096), (128, 2048, 2048)):
+            assert wavek(M, N, K, dtype, "nt", variant=12), (dtype, M, N, K)
+            if dtype == "q4_zp":   # (a plain plan of them has 64 rows at most)
+                with pytest.raises(sk.StreamKError):
+                    sk.make_plan(M, N, K, dtype, "nt", cus=256, use_tuned=False)
+            else:
+                assert not wavek(M, N, K, dtype, "nt"), (dtype, M, N, K)
+        assert not wavek(16, 4096, 4096, dtype, "nt", variant=12)
+        assert wavek(100, 760, 4096, dtype, "nt", variant=12) == (dtype == "q4_zp")
+        assert wavek(4096, 8192, 8192, dtype, "nt", variant=12) == (dtype == "q4_zp")
+    for dtype in ("float16", "bfloat16"):
+        assert not wavek(100, 4096, 4096, dtype, "nn", variant=12)
+        assert not wavek(100, 4096, 4096, dtype, "nt", variant=12, fixup="atomic_c")
+        assert sk.plan.operator_config(100, 4096, 4096, dtype, "nn") is None
+    assert sk.make_plan(40, 4096, 4096, "q4_zp", "nt", cus=256, use_tuned=False).kernel_id < 400
