@@ -322,6 +322,16 @@ struct KernelInfo {
   X(T, BASE + 12, 8, 3) \
   X(T, BASE + 13, 8, 4)
 
+// the same for [K, N] weights (NN_; types WK_F16 and WK_BF16, ids from 600 + 20 type on)
+#define SK_TILE_WAVEK_NN_KERNELS(X, T, BASE) \
+  X(T, BASE + 0, 2, 2) \
+  X(T, BASE + 1, 2, 4) \
+  X(T, BASE + 2, 2, 8) \
+  X(T, BASE + 3, 4, 2) \
+  X(T, BASE + 4, 4, 4) \
+  X(T, BASE + 5, 6, 4) \
+  X(T, BASE + 6, 8, 2)
+
 // the same for Q4 weights (tile_wavek_q4.h; dtypes SK_Q4 id, SK_Q4_ZP id + 20):  X(id, blocks of 16 rows of A, of 16 weight rows)
 #define SK_TILE_WAVEK_Q4_KERNELS(X) \
   X(520, 2, 2) \

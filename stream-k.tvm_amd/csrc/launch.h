@@ -43,12 +43,12 @@ int occupancy_tile_q4(int id);
 // tile kernels for 65 to 128 rows of 16-bit operands (translation unit kernels_tile_ring.hip)
 int launch_tile_ring(int id, const GemmArgs &a, const DevPlan &p, const Workspace &ws, hipStream_t s, const void *bias);
 int occupancy_tile_ring(int id);
-// tile kernels whose waves stream K on their own (tile_wavek.h), a translation unit per type (WaveKType)
-template <int TYPE>
+// tile kernels whose waves stream K on their own (tile_wavek.h), a translation unit per type (WaveKType) and layout
+template <int TYPE, bool NN>
 int wavek_kernel_infos(KernelInfo *out, int max);
-template <int TYPE>
+template <int TYPE, bool NN>
 int wavek_launch(int id, const GemmArgs &a, const DevPlan &p, const Workspace &ws, hipStream_t s, const void *bias);
-template <int TYPE>
+template <int TYPE, bool NN>
 int wavek_occupancy(int id);
 // (Q4 weights: zeros null where one zero point, in the arguments, serves the matrix)
 int wavek_q4_kernel_infos(KernelInfo *out, int max);

@@ -311,7 +311,7 @@ static const KernelInfo *pick_kernel(int64_t M, int64_t N, int64_t K, int dtype,
       for (int i = 0; i < n; ++i) {
         if (t[i].family != FAMILY_TILE || t[i].dtype != dtype || t[i].layout != layout) continue;
         if (t[i].bm != pref[pi][0] || t[i].bn != pref[pi][1]) continue;
-        if (want_variant >= 0 && t[i].variant != want_variant) continue;
+        if (want_variant >= 0 ? t[i].variant != want_variant : by_variant_only(t[i])) continue;
         if (pass == 0 && want_variant < 0 && (t[i].bk != pref[pi][2] || t[i].variant != pref[pi][3])) continue;
         if (!accepts_shape(t[i], M, K)) continue;
         if (best == nullptr || variant_rank(t[i]) > variant_rank(*best)) best = &t[i];
@@ -551,6 +551,16 @@ static const WaveKFamily kFamiliesWaveK16[] = {
     {128, 48, 6.37f, 2.60f, 0.784f, 0.343f, 1.89f, 1.01f},
     {128, 64, 7.08f, 2.95f, 0.960f, 0.428f, 2.08f, 1.21f},
 };
+// [K, N] weights: 2 000 timings, 1 to 1024 rows, 18 shapes (mean |log error| 7 to 10 %)
+static const WaveKFamily kFamiliesWaveKNN[] = {
+    {32, 32, 3.13f, 1.08f, 0.448f, 0.154f, 1.71f, 0.62f},
+    {32, 64, 3.58f, 1.44f, 0.549f, 0.163f, 1.57f, 0.76f},
+    {32, 128, 4.54f, 2.03f, 0.815f, 0.256f, 1.85f, 0.78f},
+    {64, 32, 3.56f, 1.56f, 0.589f, 0.159f, 1.54f, 0.90f},
+    {64, 64, 4.52f, 1.67f, 0.649f, 0.268f, 1.63f, 1.06f},
+    {96, 64, 5.79f, 2.26f, 0.684f, 0.427f, 1.67f, 1.16f},
+    {128, 32, 4.37f, 1.72f, 0.799f, 0.299f, 1.80f, 1.15f},
+};
 static const WaveKFamily kFamiliesWaveK8[] = {
     {32, 32, 3.41f, 1.19f, 0.319f, 0.082f, 1.87f, 0.47f},
     {32, 64, 3.94f, 1.74f, 0.439f, 0.117f, 1.86f, 0.64f},
@@ -575,11 +585,21 @@ static const WaveKFamily kFamiliesWaveKQ4[] = {
     {64, 96, 5.99f, 3.12f, 1.837f, 0.164f, 2.32f, 1.06f},
     {128, 32, 5.41f, 1.72f, 1.224f, 0.307f, 2.15f, 0.83f},
 };
-static const KernelInfo *model_pick_wavek(int64_t M, int64_t N, int64_t K, int dtype, int num_cus, sk_config *out, double *time_us) {
+static const KernelInfo *model_pick_wavek(int64_t M, int64_t N, int64_t K, int dtype, int layout, int num_cus, sk_config *out,
+                                          double *time_us) {
   const bool q4 = dtype == SK_Q4 || dtype == SK_Q4_ZP, one_byte = dtype == SK_F8E4M3 || dtype == SK_F8E5M2 || dtype == SK_I8;
-  const WaveKFamily *fams = q4 ? kFamiliesWaveKQ4 : (one_byte ? kFamiliesWaveK8 : kFamiliesWaveK16);
-  const int nfams = q4 ? (int)(sizeof(kFamiliesWaveKQ4) / sizeof(kFamiliesWaveKQ4[0]))
-                       : (one_byte ? (int)(sizeof(kFamiliesWaveK8) / sizeof(kFamiliesWaveK8[0])) : (int)(sizeof(kFamiliesWaveK16) / sizeof(kFamiliesWaveK16[0])));
+  const WaveKFamily *fams = kFamiliesWaveK16;
+  int nfams = (int)(sizeof(kFamiliesWaveK16) / sizeof(kFamiliesWaveK16[0]));
+  if (layout == SK_LAYOUT_NN) {
+    fams = kFamiliesWaveKNN;
+    nfams = (int)(sizeof(kFamiliesWaveKNN) / sizeof(kFamiliesWaveKNN[0]));
+  } else if (q4) {
+    fams = kFamiliesWaveKQ4;
+    nfams = (int)(sizeof(kFamiliesWaveKQ4) / sizeof(kFamiliesWaveKQ4[0]));
+  } else if (one_byte) {
+    fams = kFamiliesWaveK8;
+    nfams = (int)(sizeof(kFamiliesWaveK8) / sizeof(kFamiliesWaveK8[0]));
+  }
   const double weight_bytes = q4 ? 0.52 : (one_byte ? 1 : 2), a_bytes = one_byte ? 1 : 2, c_bytes = dtype == SK_I8 ? 4 : 2;
   const double memory_us = (weight_bytes * N * K + a_bytes * M * K + c_bytes * M * N) / 5.9e6;
   const KernelInfo *best = nullptr;
@@ -590,7 +610,7 @@ static const KernelInfo *model_pick_wavek(int64_t M, int64_t N, int64_t K, int d
     const WaveKFamily &f = fams[fi];
     const KernelInfo *k = nullptr;
     for (int i = 0; i < count && !k; ++i)
-      if (t[i].family == FAMILY_TILE && t[i].variant == 10 && t[i].dtype == dtype && t[i].bm == f.bm && t[i].bn == f.bn) k = &t[i];
+      if (t[i].family == FAMILY_TILE && t[i].variant == 10 && t[i].dtype == dtype && t[i].layout == layout && t[i].bm == f.bm && t[i].bn == f.bn) k = &t[i];
     if (!k || K % k->k_align != 0) continue;
     const int64_t tiles = cdiv(M, f.bm) * cdiv(N, f.bn), ipt = cdiv(K, k->bk);
     for (int s = 1; s <= 8; s *= 2) {
@@ -620,7 +640,7 @@ static const KernelInfo *model_pick_wavek(int64_t M, int64_t N, int64_t K, int d
 }
 // Whether a problem whose tile, variant, schedule and grid are open goes to them; `other_us`: the time the other tile kernels'
 // model gives (0: none of them runs it).
-static bool wavek_pays(int64_t M, int64_t N, int64_t K, int dtype, int num_cus, double wavek_us, double other_us) {
+static bool wavek_pays(int64_t M, int64_t N, int64_t K, int dtype, int layout, int num_cus, double wavek_us, double other_us) {
   if (dtype == SK_Q4 || dtype == SK_Q4_ZP) {
     // up to 64 rows the general small-M kernels: behind everywhere but with up to 32 rows on more than one round of 64-row tiles
     // (20 x 28672 x 1280 10.4 us against 13.1, 20 x 20480 x 3072 15.8 / 19.1; 20 x 8192 x 8192 18.4 / 14.9, 64 x 4096 x 4096
@@ -635,25 +655,39 @@ static bool wavek_pays(int64_t M, int64_t N, int64_t K, int dtype, int num_cus, 
     int split = 1;
     for (int s = 2; tiles < num_cus && s <= 4; s *= 2)
       if (tiles * s <= (int64_t)num_cus * occ && ipt % s == 0 && ipt / s >= 8) split = s;
+    int skt;
+    const bool even = tiles > num_cus && auto_tile_schedule(tiles, num_cus * occ, (int)ipt, &skt) != SK_SCHED_DP;
+    const double rounds = even ? (double)tiles / num_cus : (double)cdiv(tiles * split, num_cus);
     const double busy = tiles * split < num_cus ? (double)(tiles * split) / num_cus : 1.0;
     const double per = bm == 256 ? 0.667 + 0.316 * busy : 0.664 + 0.105 * busy;
-    const double tile_us = (bm == 256 ? 5.24 : 2.45) + (double)cdiv(tiles * split, num_cus) * ((double)ipt / split) * per +
+    const double tile_us = (bm == 256 ? 5.24 : 2.45) + rounds * ((double)ipt / split) * per +
                            (split == 1 ? 0.0 : (bm == 256 ? 4.8 : 5.0) * (split == 2 ? 1 : 2));
     return wavek_us < 0.95 * tile_us;
   }
-  if (M > 64) return other_us <= 0 || wavek_us < 0.95 * other_us;
+  const bool one_byte = dtype == SK_F8E4M3 || dtype == SK_F8E5M2 || dtype == SK_I8;
+  // (weights that the Infinity Cache does not keep between calls come in slower than the fit's average of both says: 80 to 128 x
+  // 4096 x 11008 of fp16 29.5 to 31.0 us on the ring kernels, 32 to 36 here against a predicted 28)
+  if (M > 64) {
+    const bool from_hbm = (one_byte ? 1 : 2) * N * K > ((int64_t)(layout == SK_LAYOUT_NN ? 48 : 64) << 20);
+    return other_us <= 0 || wavek_us < (from_hbm ? 0.85 : (one_byte ? 0.95 : 0.92)) * other_us;
+  }
+  // [K, N] weights and up to 64 rows, against the 64 x 64 and larger tiles of tile_f16_dma.h (in us, those / these): behind where
+  // the weights come from HBM through pieces of 64 bytes, or in a second round of 64-wide ones (16 rows: 8192 x 8192 34.8 / 38.2,
+  // 5120 x 5120 16.9 / 18.0, but 1024 x 8192 13.6 / 10.9, 4096 x 11008 40 / 34, 28672 x 1280 23.4 / 15.8, 4096 x 4096 13.6 / 12.2;
+  // 64 rows: 28672 x 8192 104 / 122, 20480 x 3072 41 / 50, 11008 x 4096 23.4 / 23.5, but 4096 x 11008 50 / 35, 2048 x 2048 9.5 / 6.6,
+  // 6144 x 2048 12.4 / 10.6, 28672 x 1280 26.3 / 20.4)
+  if (layout == SK_LAYOUT_NN) return M <= 32 ? !(N > 4608 && N <= 8192 && K >= 4096) : N <= 4608 || K < 3000;
   // 33 to 64 rows against the kernels that stream the weights through LDS: K long enough for a ring to fill, and few columns
-  // (in us, those / these, 64 rows: fp16 2048 x 2048 9.5 / 6.2, 4096 x 4096 14.0 / 9.9, 5120 x 5120 17.8 / 15.9, 6144 x 2048
+  // (in us, those / these, 64 rows: fp16 2048 x 2048 9.5 / 6.2, 4096 x 4096 14.0 / 9.9, 6144 x 2048
   // 12.7 / 9.0, 1024 x 8192 13.8 / 10.4; int8 4096 x 11008 16.4 / 13.1, 2048 x 8192 11.7 / 9.3; but fp16 4096 x 11008 25.9 / 27.1,
-  // 8192 x 8192 29.7 / 31.4, 4096 x 1024 5.9 / 5.0, 1024 x 1024 5.8 / 6.4; int8 8192 x 16384 29.7 / 34.7) or more than a round of
+  // 5120 x 5120 from HBM 21.1 / 23.2, 8192 x 8192 29.7 / 31.4, 4096 x 1024 5.9 / 5.0, 1024 x 1024 5.8 / 6.4; int8 8192 x 16384 29.7 / 34.7) or more than a round of
   // their 64-row tiles where 112-row tiles need one (20480 x 3072 fp16 37.6 / 27.9, 28672 x 8192 88.3 / 85.4, of fp8 50.4 / 47.5).
   // One-byte operands of fewer than 6144 K-values stay with the streaming kernels throughout: there the gain is 1 to 2 us
   // (4096 x 4096 8.8 / 7.4, 2048 x 2048 5.8 / 5.0), and those are the kernels their plans are known by.  Up to 32 rows there is
   // nothing to gain (20 x 4096 x 4096 9.4 / 9.1 and 6.6 / 6.7).
-  const bool one_byte = dtype == SK_F8E4M3 || dtype == SK_F8E5M2 || dtype == SK_I8;
   if (M <= 32 || (one_byte && K < 6144)) return false;
   if (cdiv(N, 64) > num_cus && cdiv(N, 112) <= num_cus) return K >= 2048;
-  return N <= (one_byte ? 4096 : 6144) && K >= 1536 && N * K <= (one_byte ? (int64_t)48 << 20 : (int64_t)32 << 20);
+  return N <= (one_byte ? 4096 : 6144) && K >= 1536 && N * K <= (one_byte ? (int64_t)48 << 20 : (int64_t)24 << 20);
 }
 
 // ---- fp32: tile, schedule and grid, when the caller leaves all three open ----
@@ -773,17 +807,17 @@ extern "C" int sk_make_plan(int64_t M, int64_t N, int64_t K, int dtype, int layo
   }
   const int want_fixup = cfg ? cfg->fixup : SK_FIXUP_AUTO;
   const bool fp32_partials = want_fixup == SK_FIXUP_AUTO || want_fixup == SK_FIXUP_REDUCE || want_fixup == SK_FIXUP_ATOMIC;
-  if (open && layout == SK_LAYOUT_NT && fp32_partials && by_operator && M > 16 && (N >= 768 || (dtype == SK_Q4_ZP && !few)) && (b16 || q4_rows || one_byte)) {
+  if (open && fp32_partials && by_operator && (layout == SK_LAYOUT_NT ? M > 16 : b16) && (N >= 768 || (dtype == SK_Q4_ZP && !few)) && (b16 || q4_rows || one_byte)) {
     double wavek_us = 0, other_us = 0;
     if (cfg) wavek = *cfg; else memset(&wavek, 0, sizeof(wavek));
-    const KernelInfo *k = model_pick_wavek(M, N, K, dtype, num_cus, &wavek, &wavek_us);
+    const KernelInfo *k = model_pick_wavek(M, N, K, dtype, layout, num_cus, &wavek, &wavek_us);
     if (k && !few && !q4_rows) {
       sk_config ring;
       int split, sched;
-      if (!(b16 && M <= 128 && ring_pays(N, K) && model_pick_ring(N, K, dtype, num_cus, &ring, &other_us)))
+      if (!(b16 && layout == SK_LAYOUT_NT && M <= 128 && ring_pays(N, K) && model_pick_ring(N, K, dtype, num_cus, &ring, &other_us)))
         model_pick(M, N, K, dtype, layout, num_cus, &split, &sched, &other_us);
     }
-    if (k && wavek_pays(M, N, K, dtype, num_cus, wavek_us, other_us)) cfg = &wavek;
+    if (k && wavek_pays(M, N, K, dtype, layout, num_cus, wavek_us, other_us)) cfg = &wavek;
   }
   if (open && cfg != &wavek && (b16 || one_byte) && !few && !rows_65_to_96_stream(M, N, dtype, layout, num_cus)) {
     double model_us = 0;

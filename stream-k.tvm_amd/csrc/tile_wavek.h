@@ -202,7 +202,11 @@ static __device__ __forceinline__ void wavek_wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N < 63 ? N : 63) : "memory");
 }
 
-template <int TYPE_, int FM_, int FN_>
+// NN_: the weights are [K, N] (16-bit operands).  A chunk's weights are 64 rows of K of BN columns, and their fragments are read
+// with ds_read_b64_tr_b16: a 16-lane group that points at a 4 (K) x 16 (N) patch receives, per lane, 4 consecutive K of one column.
+// 16-byte piece c of K-row k stands at position c ^ 2 f(k) of the row, so that the 32 lanes served together -- 2 groups x 4
+// rows x 32 bytes, the groups 8 rows apart -- read 8 different 32-byte slots of the 256 bytes of banks; f by the length of a row.
+template <int TYPE_, int FM_, int FN_, bool NN_ = false>
 struct TileWaveK : WaveKTile<TYPE_, FM_, FN_> {
   typedef WaveKTile<TYPE_, FM_, FN_> Base;
   typedef typename Base::Args Args;
@@ -211,7 +215,9 @@ struct TileWaveK : WaveKTile<TYPE_, FM_, FN_> {
   static constexpr int FM = FM_, FN = FN_, BM = Base::BM, BN = Base::BN, WAVES = Base::WAVES, NT = Base::NT, NB = Base::NB;
   static constexpr int KV = 64, BK = KV * WAVES;      // 16-bit units of K: of a chunk, of an iteration
   static constexpr int L = 2 * (FM + FN);             // loads of a chunk
-  static constexpr int R = L > 20 ? 40 : (L * 4 < 40 ? L * 4 : 40 / L * L);   // loads of a wave's ring (at most 160 KB / 4 waves, four chunks)
+  static constexpr bool NN = NN_;
+  static_assert(!NN || ((TYPE_ == WK_F16 || TYPE_ == WK_BF16) && (BN == 32 || BN == 64 || BN == 128)), "[K, N] weights: 16-bit, loads of whole rows");
+  static constexpr int R = L > 20 && !NN ? 40 : (L * 4 < 40 ? L * 4 : 40 / L * L);   // loads of a wave's ring (at most 160 KB / 4 waves, four chunks)
   static constexpr int S = R / L, PART = R % L;       // whole chunks in the ring, loads of one more
   static_assert(S >= 1 && (L % 2) == 0 && (R % 2) == 0, "a 16-row block of a chunk stays together in the ring");
   static constexpr int RING = R * 1024, LDS_RINGS = WAVES * RING, LDS_SUMS = WAVES * (NB / 2) * 1024;
@@ -231,6 +237,9 @@ struct TileWaveK : WaveKTile<TYPE_, FM_, FN_> {
   struct Frags {
     half8v a[FM][2], b[FN][2];   // [K-step]
   };
+  static __device__ __forceinline__ int nn_swizzle(int k) {   // 2 f(k)
+    return BN == 32 ? (k >> 2) & 2 : (BN == 64 ? (k & 2) | ((k >> 1) & 4) : 2 * (k & 3) | (k & 8));
+  }
   // MFMA m of a chunk
   template <int m>
   static __device__ __forceinline__ void mfma(AccV (&c)[NB], const Frags &f) {
@@ -259,7 +268,10 @@ struct TileWaveK : WaveKTile<TYPE_, FM_, FN_> {
     // ---- descriptors: rows past M / N read as zero ----
     const uint32_t lda_bytes = (uint32_t)a.lda * 2, ldb_bytes = (uint32_t)a.ldb * 2;
     const uint4v rsrc_a = uniform_rsrc(make_rsrc_words(a.A + (int64_t)pm * BM * a.lda, (uint32_t)min(BM, a.M - pm * BM) * lda_bytes));
-    const uint4v rsrc_b = uniform_rsrc(make_rsrc_words(a.B + (int64_t)pn * BN * a.ldb, (uint32_t)min(BN, a.N - pn * BN) * ldb_bytes));
+    const int rows_b = min(BN, a.N - pn * BN);
+    // (NN: to the tile's last element of row K - 1, so that rows past K read as zero)
+    const uint4v rsrc_b = NN ? uniform_rsrc(make_rsrc_words(a.B + (int64_t)pn * BN, (uint32_t)(((int64_t)(a.K - 1) * a.ldb + rows_b) * 2)))
+                             : uniform_rsrc(make_rsrc_words(a.B + (int64_t)pn * BN * a.ldb, (uint32_t)rows_b * ldb_bytes));
     // load l of a chunk: rows 8 l .. 8 l + 7 (A's first), lane's row lane / 8, piece p (16 bytes) of row r of a block at position
     // p ^ ((r >> 1) & 7)
     const int row8 = lane >> 3;
@@ -270,27 +282,36 @@ struct TileWaveK : WaveKTile<TYPE_, FM_, FN_> {
     static_for<0, L>([&](auto l) {
       off[l] = l < 2 * FM ? (uint32_t)(8 * l + row8) * lda_bytes + (uint32_t)kp[l & 1] * 2
                           : (uint32_t)(8 * (l - 2 * FM) + row8) * ldb_bytes + (uint32_t)kp[l & 1] * 2;
+      if constexpr (NN && l >= 2 * FM) {   // 512 / BN rows of K, BN / 8 lanes to a row
+        const int k = (l - 2 * FM) * (512 / BN) + lane / (BN / 8), c = lane % (BN / 8) ^ nn_swizzle(k);
+        off[l] = 8 * c < rows_b ? (uint32_t)k * ldb_bytes + (uint32_t)c * 16 : OOB_OFFSET;
+      }
     });
     const uint32_t ring = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_address(smem) + wave * RING);
     // one row of tiles: see rotation_of.  Several: the CTAs of an XCD share A as well as the weights and stay on the same K
-    const int rot = a.M <= BM ? rotation_of(pn, n) : (int)((blockIdx.x & 7) * (uint32_t)n) >> 3;
+    // ([K, N] weights: the CTAs of a row of tiles read neighbouring pieces of the same rows and stay together too)
+    const int rot = a.M <= BM && !NN ? rotation_of(pn, n) : (int)((blockIdx.x & 7) * (uint32_t)n) >> 3;
     // load l of a chunk that starts kbytes into the rows and `left` 16-bit units before K's end, pos: where the chunk starts in
     // the ring.  (Pieces past K fetch nothing: zeros arrive and the wait counts stay exact.)
     struct Chunk {
-      uint32_t kbytes;
+      uint32_t kbytes, kbytes_b;
       int left, pos;
       uint32_t base;   // LDS address of load 0, were the ring long enough
     };
     auto chunk = [&](int t, int pos) {
       const int kk = ((k0 + rotated_iteration(t, rot, n)) * WAVES + wave) * KV, left = t < n ? a.K - kk : 0;
       // (a chunk past K or past the segment must not carry its offset either)
-      return Chunk{(uint32_t)__builtin_amdgcn_readfirstlane(left > 0 ? kk * 2 : 0), left, pos, ring + (uint32_t)pos * 1024};
+      const uint32_t kbytes = (uint32_t)__builtin_amdgcn_readfirstlane(left > 0 ? kk * 2 : 0);
+      return Chunk{kbytes, NN ? kbytes * (uint32_t)a.ldb : kbytes, left, pos, ring + (uint32_t)pos * 1024};
     };
     auto issue = [&](auto li, const Chunk &q) {
       constexpr int l = decltype(li)::value;
       uint32_t base = q.base;
       if (R % L != 0) base = q.pos >= R - l ? base - R * 1024 : base;
-      wavek_dma_16<l * 1024>(l < 2 * FM ? rsrc_a : rsrc_b, base, q.left >= KV || kp[l & 1] < q.left ? off[l] : OOB_OFFSET, q.kbytes);
+      if constexpr (NN && l >= 2 * FM)   // (the descriptor ends with K)
+        wavek_dma_16<l * 1024>(rsrc_b, base, q.left > 0 ? off[l] : OOB_OFFSET, q.kbytes_b);
+      else
+        wavek_dma_16<l * 1024>(l < 2 * FM ? rsrc_a : rsrc_b, base, q.left >= KV || kp[l & 1] < q.left ? off[l] : OOB_OFFSET, q.kbytes);
     };
 #pragma unroll
     for (int t = 0; t < S; ++t)
@@ -306,8 +327,26 @@ struct TileWaveK : WaveKTile<TYPE_, FM_, FN_> {
     // fragments: lane (i, g) takes piece 4 s + g of its row for K-step s
     const int fi = lane & 15, fg = lane >> 4;
     const char *rd0 = smem + wave * RING + fi * 128 + ((fg ^ ((fi >> 1) & 7)) * 16), *rd1 = smem + wave * RING + fi * 128 + (((4 + fg) ^ ((fi >> 1) & 7)) * 16);
+    // (NN: lane L of group g points at row 8 g + L / 4 of K, columns 4 (L % 4) .. of the block; four rows further on the other half)
+    const char *rd_nn[FN];
+    if constexpr (NN) {
+      const int k = 8 * fg + (fi >> 2);
+      static_for<0, FN>([&](auto j) {
+        rd_nn[j] = smem + wave * RING + 2 * FM * 1024 + k * (BN * 2) + ((2 * j + ((fi & 3) >> 1)) ^ nn_swizzle(k)) * 16 + (fi & 1) * 8;
+      });
+    }
     auto read = [&](auto ri, Frags &f, int pos) {
       constexpr int r = decltype(ri)::value, s = r / (FM + FN), b = r % (FM + FN);   // block b of the chunk: A's, then the weights'
+      if constexpr (NN && b >= FM) {
+        typedef short short4v __attribute__((ext_vector_type(4)));
+        typedef __attribute__((address_space(3))) short4v *lds_s4;
+        const char *from = rd_nn[b - FM] + pos * 1024 + 32 * s * (BN * 2);
+        union { short4v s[2]; half8v h; } u;
+        u.s[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)from);
+        u.s[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(from + 4 * (BN * 2)));
+        f.b[b - FM][s] = u.h;
+        return;
+      }
       const char *from = (s ? rd1 : rd0) + pos * 1024;
       if (R % L != 0) from = pos >= R - 2 * b ? from - R * 1024 : from;
       const half8v x = *reinterpret_cast<const half8v *>(from + 2 * b * 1024);

@@ -1,5 +1,5 @@
 // Kernel entry, table entries and launcher of the tiles whose waves stream K on their own, shared by the units that compile them
-// for one type each.
+// for one type each (WAVEK_NAME: what the kernels are called, WAVEK_NN: whether the weights are [K, N]).
 #pragma once
 #include "launch.h"
 #include "sk_persistent.h"
@@ -15,37 +15,37 @@ __global__ __launch_bounds__(P::NT, P::WAVES_PER_EU) void sk_tile_wavek_kernel(t
 }
 
 // ids of a type
-constexpr int wavek_base(int type) { return 400 + 20 * type; }
+constexpr int wavek_base(int type, bool nn = false) { return (nn ? 600 : 400) + 20 * type; }
 
-#define SK_WAVEK_UNIT(TYPE, SK_DTYPE, NAME)                                                                                    \
+#define SK_WAVEK_UNIT(TYPE, SK_DTYPE, NN, LIST)                                                                                \
   template <>                                                                                                                  \
-  int wavek_kernel_infos<TYPE>(KernelInfo * out, int max) {                                                                    \
+  int wavek_kernel_infos<TYPE, NN>(KernelInfo * out, int max) {                                                                    \
     int n = 0;                                                                                                                 \
-    SK_TILE_WAVEK_KERNELS(SK_WAVEK_INFO, TYPE, wavek_base(TYPE))                                                               \
-    for (int i = 0; i < n; ++i) out[i].dtype = SK_DTYPE;                                                                       \
+    LIST(SK_WAVEK_INFO, TYPE, wavek_base(TYPE, NN))                                                               \
+    for (int i = 0; i < n; ++i) out[i].dtype = SK_DTYPE, out[i].layout = NN;                                                                       \
     return n;                                                                                                                  \
   }                                                                                                                            \
   template <>                                                                                                                  \
-  int wavek_launch<TYPE>(int id, const GemmArgs &a, const DevPlan &p, const Workspace &ws, hipStream_t s, const void *bias) {  \
-    switch (id) { SK_TILE_WAVEK_KERNELS(SK_WAVEK_LAUNCH, TYPE, wavek_base(TYPE)) }                                             \
+  int wavek_launch<TYPE, NN>(int id, const GemmArgs &a, const DevPlan &p, const Workspace &ws, hipStream_t s, const void *bias) {  \
+    switch (id) { LIST(SK_WAVEK_LAUNCH, TYPE, wavek_base(TYPE, NN)) }                                             \
     return (int)hipErrorInvalidValue;                                                                                          \
   }                                                                                                                            \
   template <>                                                                                                                  \
-  int wavek_occupancy<TYPE>(int id) {                                                                                          \
+  int wavek_occupancy<TYPE, NN>(int id) {                                                                                          \
     int occ = 0;                                                                                                               \
-    switch (id) { SK_TILE_WAVEK_KERNELS(SK_WAVEK_OCC, TYPE, wavek_base(TYPE)) }                                                \
+    switch (id) { LIST(SK_WAVEK_OCC, TYPE, wavek_base(TYPE, NN)) }                                                \
     return -1;                                                                                                                 \
   }
 #define SK_WAVEK_INFO(TYPE, ID, FM, FN)                                                                                          \
   if (n < max) {                                                                                                                 \
-    typedef TileWaveK<TYPE, FM, FN> P;                                                                                           \
+    typedef TileWaveK<TYPE, FM, FN, WAVEK_NN> P;                                                                                           \
     constexpr bool one_byte = TYPE >= WK_F8E4M3;                                                                                 \
     out[n++] = KernelInfo{ID, FAMILY_TILE, 0, 0, 10, P::BM, P::BN, one_byte ? 2 * P::BK : P::BK, P::NT, P::LDS_TOTAL,            \
                           P::CTAS_PER_CU, P::TILE_ELEMS, 0, 0, one_byte ? 16 : 8, WAVEK_NAME "_" #FM "x" #FN};                   \
   }
 #define SK_WAVEK_LAUNCH(TYPE, ID, FM, FN)                                                                    \
   case ID: {                                                                                                 \
-    typedef TileWaveK<TYPE, FM, FN> P;                                                                       \
+    typedef TileWaveK<TYPE, FM, FN, WAVEK_NN> P;                                                                       \
     if (p.sk_tiles == 0)                                                                                     \
       hipLaunchKernelGGL((sk_tile_wavek_kernel<P, false>), dim3(p.grid), dim3(P::NT), 0, s, a, p, ws, bias); \
     else                                                                                                     \
@@ -54,7 +54,7 @@ constexpr int wavek_base(int type) { return 400 + 20 * type; }
   }
 #define SK_WAVEK_OCC(TYPE, ID, FM, FN)                                                                                          \
   case ID: {                                                                                                                    \
-    typedef TileWaveK<TYPE, FM, FN> P;                                                                                          \
+    typedef TileWaveK<TYPE, FM, FN, WAVEK_NN> P;                                                                                          \
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, sk_tile_wavek_kernel<P, true>, P::NT, 0) == hipSuccess ? occ : -1; \
   }
 

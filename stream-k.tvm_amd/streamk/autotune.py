@@ -36,6 +36,7 @@ _STREAM_BYTES = [(16, 16, 2048), (16, 32, 1024), (16, 64, 512), (32, 32, 1024), 
 # tiles whose waves stream K on their own (variant 11)
 _WAVEK = [(32, 32), (32, 64), (64, 32), (64, 48), (64, 64), (64, 80), (64, 96), (64, 112), (64, 128), (96, 32), (96, 64), (128, 32),
           (128, 48), (128, 64)]
+_WAVEK_NN = [(32, 32), (32, 64), (32, 128), (64, 32), (64, 64), (96, 64), (128, 32)]
 _WAVEK_Q4 = [(32, 32), (32, 64), (64, 32), (64, 64), (64, 96), (128, 32)]
 _SKINNY_Q4 = [(16, 64, 256), (32, 64, 256), (64, 64, 256), (16, 16, 1024), (16, 32, 512), (16, 16, 256),
               (16, 32, 256), (16, 32, 1024), (16, 16, 2048), (16, 64, 512), (16, 16, 512)]
@@ -144,10 +145,10 @@ def candidate_configs(M, N, K, dtype="float16", cus=None, reduce16=True, layout=
             base = dict(bm=16, bn=bn, bk=1024, variant=6)
             out.append(dict(base, schedule="dp"))
             out.extend(dict(base, schedule="basic", grid=cus, fixup=fixup) for fixup in ("reduce", "atomic"))
-    if layout == "nt" and M > 16:
+    if dtype != "float32" and (M > 16 or layout == "nn"):
         # tiles whose waves stream K on their own (variant 11)
-        for (bm, bn) in _WAVEK_Q4 if dtype in ("q4", "q4_zp") else (_WAVEK if dtype != "float32" else ()):
-            if bm >= 2 * M or -(-M // bm) * -(-N // bn) > 3 * cus:
+        for (bm, bn) in _WAVEK_NN if layout == "nn" else (_WAVEK_Q4 if dtype in ("q4", "q4_zp") else _WAVEK):
+            if (bm >= 2 * M and bm > 32) or -(-M // bm) * -(-N // bn) > 3 * cus:
                 continue
             base = dict(bm=bm, bn=bn, variant=11, raster=8 if M > bm else 0)
             out.append(dict(base, schedule="dp"))

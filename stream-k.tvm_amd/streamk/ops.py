@@ -338,10 +338,12 @@ def _run_q4(A, Wq, scales, zeros, C, zero, group, tiled, config, bias, activatio
         config = ""
         dequantise = True
     else:
-        # (with per-group zero points the kernels for many rows have 64 x 64 tiles: beyond 256 rows and three rounds of them the
-        # pass pays; 512 x 8192 x 8192 97 us against 103, 512 x 4096 x 4096 41 against 30)
+        # (with per-group zero points the kernels for many rows have 64 x 64 tiles: beyond 256 rows the pass pays from three
+        # rounds of them on, beyond 512 from two; 512 x 8192 x 8192 97 us against 103, 768 x 4096 x 11008 93 / 117,
+        # but 512 x 4096 x 4096 41 / 30, 320 x 8192 x 8192 99 / 76)
         dequantise = config == "" and (M > Q4_FUSED_MAX_M or (
-            zeros is not None and M > 4 * Q4_MAX_M and -(-M // 64) * -(-N // 64) > 3 * _plan_mod.num_cus()))
+            zeros is not None and M > 4 * Q4_MAX_M and
+            -(-M // 64) * -(-N // 64) > (3 if M <= 8 * Q4_MAX_M else 2) * _plan_mod.num_cus()))
     if dequantise:
         # Prefill-sized calls: one pass that dequantises the weights (bit-exact device function), then the fp16 tile kernels
         # on them.  The pass costs 26 us for 8192 x 8192 weights, under 7 % of the product from 4096 rows on, where the

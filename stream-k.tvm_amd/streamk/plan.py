@@ -108,12 +108,12 @@ SEARCH_WITH_BYTE_STREAMS = 2
 
 def operator_config(M, N, K, dtype, layout):
     """Configuration of an operator call that names none: the tuned one (None: make_plan finds it), else what
-    OPERATOR_VARIANT says, for weights [N, K] and the types that have those kernels.  Up to 64 rows of one-byte operands a tuned
+    OPERATOR_VARIANT says, for the types and layouts that have those kernels.  Up to 64 rows of one-byte operands a tuned
     entry from a search that did not have the kernels which stream the weights through LDS does not speak for them: it
     configures the plans that make_plan gives, and an operator call takes the kernels the library chooses (16 x 8192 x 8192 of
     fp8 14.3 us, by the entry 16.7)."""
     few_bytes = M <= 64 and dtype in ("float8_e4m3", "float8_e5m2", "int8")
-    if layout != "nt" or not (few_bytes or (M > 16 and dtype in _WAVEK_DTYPES)):
+    if not (few_bytes or (dtype in _WAVEK_DTYPES if layout == "nt" and M > 16 else layout == "nn" and dtype in ("float16", "bfloat16"))):
         return None
     for d in dict.fromkeys((dtype, _TWIN_OF.get(dtype, dtype))):
         hit = _tuned_entry(M, N, K, d, layout)

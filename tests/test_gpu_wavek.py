@@ -6,6 +6,7 @@ import pytest
 
 _TILES = [(32, 32), (32, 64), (64, 32), (64, 48), (64, 64), (64, 80), (64, 96), (64, 112), (64, 128), (96, 32), (96, 64), (128, 32),
           (128, 48), (128, 64)]
+_TILES_NN = [(32, 32), (32, 64), (32, 128), (64, 32), (64, 64), (96, 64), (128, 32)]
 _TILES_Q4 = [(32, 32), (32, 64), (64, 32), (64, 64), (64, 96), (128, 32)]
 
 
@@ -19,8 +20,8 @@ def _small(rng, shape, most=2):
     return rng.integers(-most, most + 1, shape).astype(np.float64)
 
 
-def _operands(torch, dtype, rng, M, N, K, pad=0):
-    """A (rows `pad` elements further apart), weights, a call, the exact product and the type of C."""
+def _operands(torch, dtype, rng, M, N, K, pad=0, layout="nt"):
+    """A call on A (rows `pad` elements further apart) and weights, and the exact product."""
     if dtype.startswith("q4"):
         A = _small(rng, (M, K))
         q = rng.integers(0, 16, (N, K))
@@ -33,13 +34,13 @@ def _operands(torch, dtype, rng, M, N, K, pad=0):
     else:
         A, W = _small(rng, (M, K)), _small(rng, (N, K))
         kind = {"float8_e4m3": torch.float8_e4m3fn, "float8_e5m2": torch.float8_e5m2}.get(dtype) or getattr(torch, dtype)
-        rest = (torch.from_numpy(W).float().cuda().to(kind),)
+        rest = (torch.from_numpy(W if layout == "nt" else W.T.copy()).float().cuda().to(kind),)
     dA = torch.zeros(M, K + pad, device="cuda").to(kind) if kind != torch.int8 else torch.zeros(M, K + pad, device="cuda", dtype=kind)
     dA[:, :K].copy_(torch.from_numpy(A).float().cuda().to(kind))
     import streamk
     f = {"float16": streamk.streamk_fp16, "bfloat16": streamk.streamk_bf16, "int8": streamk.streamk_int8}.get(dtype)
     if dtype in ("float16", "bfloat16"):
-        call = lambda **kw: f(dA[:, :K], rest[0], layout="nt", **kw)   # noqa: E731
+        call = lambda **kw: f(dA[:, :K], rest[0], layout=layout, **kw)   # noqa: E731
     elif dtype == "int8":
         call = lambda **kw: f(dA[:, :K], rest[0], **kw)   # noqa: E731
     elif dtype.startswith("float8"):
@@ -56,20 +57,21 @@ def _rounded(torch, exact, dtype):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("dtype", ["float16", "bfloat16", "float8_e4m3", "float8_e5m2", "int8", "q4", "q4_zp"])
-def test_every_tile_is_exact(sk, dtype):
+@pytest.mark.parametrize("dtype,layout", [("float16", "nt"), ("bfloat16", "nt"), ("float8_e4m3", "nt"), ("float8_e5m2", "nt"), ("int8", "nt"),
+                                          ("q4", "nt"), ("q4_zp", "nt"), ("float16", "nn"), ("bfloat16", "nn")])
+def test_every_tile_is_exact(sk, dtype, layout):
     import torch
     rng = np.random.default_rng(41)
     step = 128 if dtype.startswith("q4") else (16 if "8" in dtype and dtype != "bfloat16" and dtype != "float16" else 8)
     long = {128: 6528, 16: 5136, 8: 2568}[step]   # rings full, iterations that K does not fill, odd numbers of them
-    for bm, bn in _TILES_Q4 if dtype.startswith("q4") else _TILES:
-        for M, N, K in ((bm + 1, 2 * bn + 8, long), (1, 1, step), (2 * bm - 3, bn + 5, 3 * step + (128 if step < 128 else 0)), (bm, 3 * bn, 2048)):
-            call, exact = _operands(torch, dtype, rng, M, N, K, pad=8 if dtype in ("float16", "bfloat16") or step == 128 else 16)
+    for bm, bn in _TILES_Q4 if dtype.startswith("q4") else (_TILES if layout == "nt" else _TILES_NN):
+        for M, N, K in ((bm + 1, 2 * bn + 8, long), (1, 1 if layout == "nt" else 8, step), (2 * bm - 3, bn + (5 if layout == "nt" else 8), 3 * step + (128 if step < 128 else 0)), (bm, 3 * bn, 2048)):
+            call, exact = _operands(torch, dtype, rng, M, N, K, pad=8 if dtype in ("float16", "bfloat16") or step == 128 else 16, layout=layout)
             want = _rounded(torch, exact, dtype)
             for sched in (dict(schedule="dp"), dict(schedule="splitk", split=2, fixup="reduce"), dict(schedule="basic", grid=7, fixup="reduce"),
                           dict(schedule="basic", grid=5, fixup="atomic")):
                 try:
-                    plan = sk.make_plan(M, N, K, dtype, "nt", dict(sched, bm=bm, bn=bn, variant=11))
+                    plan = sk.make_plan(M, N, K, dtype, layout, dict(sched, bm=bm, bn=bn, variant=11))
                 except sk.StreamKError:
                     assert sched["schedule"] == "splitk"   # (a split that does not divide the iterations)
                     continue
@@ -79,7 +81,7 @@ def test_every_tile_is_exact(sk, dtype):
             if dtype != "int8":
                 kind = torch.bfloat16 if dtype == "bfloat16" else torch.float16
                 bias = torch.from_numpy(rng.integers(-8, 9, N).astype(np.float32)).to(kind)
-                plan = sk.make_plan(M, N, K, dtype, "nt", dict(bm=bm, bn=bn, variant=11, schedule="dp"))
+                plan = sk.make_plan(M, N, K, dtype, layout, dict(bm=bm, bn=bn, variant=11, schedule="dp"))
                 got = call(plan=plan, bias=bias.cuda(), activation="relu").cpu()
                 want = _rounded(torch, np.maximum(exact + bias.double().numpy(), 0), dtype)
                 assert torch.equal(got, want), (dtype, bm, bn, M, N, K)
@@ -87,8 +89,9 @@ def test_every_tile_is_exact(sk, dtype):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("dtype", ["float16", "bfloat16", "float8_e4m3", "int8", "q4", "q4_zp"])
-def test_operator_calls_equal_the_plans_they_replace(sk, dtype):
+@pytest.mark.parametrize("dtype,layout", [("float16", "nt"), ("bfloat16", "nt"), ("float8_e4m3", "nt"), ("int8", "nt"), ("q4", "nt"), ("q4_zp", "nt"),
+                                          ("float16", "nn"), ("bfloat16", "nn")])
+def test_operator_calls_equal_the_plans_they_replace(sk, dtype, layout):
     """What an operator call takes by itself against the plan that make_plan gives (per-group zero points beyond 64 rows: the
     exact product alone), sizes around the limits of the rule, rows of A and C further apart than they are long, C at an odd
     element."""
@@ -96,17 +99,17 @@ def test_operator_calls_equal_the_plans_they_replace(sk, dtype):
     rng = np.random.default_rng(42)
     step = 128 if dtype.startswith("q4") else (16 if dtype in ("float8_e4m3", "int8") else 8)
     seen = set()
-    for M, N, K in ((17, 768, 1536), (33, 770, 6144), (40, 2049, 2048), (64, 1000, 8192), (65, 775, 512), (100, 3001, 1664), (128, 768, 4096),
+    for M, N, K in ((1, 2048, 1024), (17, 768, 1536), (33, 770, 6144), (40, 2049, 2048), (64, 1000, 8192), (65, 775, 512), (100, 3001, 1664), (128, 768, 4096),
                     (129, 1031, 640), (257, 2050, 1152), (300, 769, 2304), (513, 801, 384)):
-        K = K // step * step
-        call, exact = _operands(torch, dtype, rng, M, N, K, pad=8 * (2 if step == 16 else 1))
+        K, N = K // step * step, N if layout == "nt" else N // 8 * 8
+        call, exact = _operands(torch, dtype, rng, M, N, K, pad=8 * (2 if step == 16 else 1), layout=layout)
         want = _rounded(torch, exact, dtype)
-        plan = sk.make_plan(M, N, K, dtype, "nt", sk.plan.operator_config(M, N, K, dtype, "nt"))
+        plan = sk.make_plan(M, N, K, dtype, layout, sk.plan.operator_config(M, N, K, dtype, layout))
         seen.add(sk.kernel_name(plan.kernel_id).split("_")[0])
         for _ in range(2):   # (the first call through Python, the second natively)
             assert torch.equal(call().cpu(), want), (dtype, M, N, K, sk.kernel_name(plan.kernel_id))
         if not (dtype == "q4_zp" and M > 64):
-            assert torch.equal(call(plan=sk.make_plan(M, N, K, dtype, "nt", use_tuned=False)).cpu(), want), (dtype, M, N, K)
+            assert torch.equal(call(plan=sk.make_plan(M, N, K, dtype, layout, use_tuned=False)).cpu(), want), (dtype, M, N, K)
         buf = torch.zeros(M * (N + 3) + 1, dtype=want.dtype, device="cuda")
         out = buf[1:].view(M, N + 3)[:, :N]
         call(out=out)
@@ -116,8 +119,8 @@ def test_operator_calls_equal_the_plans_they_replace(sk, dtype):
 
 
 def test_the_operators_rule(sk):
-    """Plans keep the kernels they had; an operator call takes these where the model says so, never for [K, N] weights, few
-    columns or fix-ups that they do not have."""
+    """Plans keep the kernels they had; an operator call takes these where the model says so, never for few columns or fix-ups
+    that they do not have."""
     wavek = lambda *a, **k: sk.kernel_name(sk.make_plan(*a, cus=256, use_tuned=False, **k).kernel_id).startswith("wavek_")   # noqa: E731
     for dtype in ("float16", "bfloat16", "float8_e4m3", "float8_e5m2", "int8", "q4", "q4_zp"):
         for M, N, K in ((100, 4096, 4096), (256, 4096, 4096), (128, 2048, 2048)):
@@ -131,7 +134,8 @@ def test_the_operators_rule(sk):
         assert wavek(100, 760, 4096, dtype, "nt", variant=12) == (dtype == "q4_zp")
         assert wavek(4096, 8192, 8192, dtype, "nt", variant=12) == (dtype == "q4_zp")
     for dtype in ("float16", "bfloat16"):
-        assert not wavek(100, 4096, 4096, dtype, "nn", variant=12)
-        assert not wavek(100, 4096, 4096, dtype, "nt", variant=12, fixup="atomic_c")
-        assert sk.plan.operator_config(100, 4096, 4096, dtype, "nn") is None
+        for layout in ("nt", "nn"):
+            assert not wavek(100, 4096, 4096, dtype, layout, variant=12, fixup="atomic_c")
+        assert wavek(1, 4096, 4096, dtype, "nn", variant=12) and wavek(100, 4096, 4096, dtype, "nn", variant=12)
+        assert not wavek(1, 4096, 4096, dtype, "nn") and not wavek(64, 8192, 8192, dtype, "nn", variant=12)
     assert sk.make_plan(40, 4096, 4096, "q4_zp", "nt", cus=256, use_tuned=False).kernel_id < 400
