@@ -671,12 +671,10 @@ static bool wavek_pays(int64_t M, int64_t N, int64_t K, int dtype, int layout, i
     const bool from_hbm = (one_byte ? 1 : 2) * N * K > ((int64_t)(layout == SK_LAYOUT_NN ? 48 : 64) << 20);
     return other_us <= 0 || wavek_us < (from_hbm ? 0.85 : (one_byte ? 0.95 : 0.92)) * other_us;
   }
-  // [K, N] weights and up to 64 rows, against the 64 x 64 and larger tiles of tile_f16_dma.h (in us, those / these): behind where
-  // the weights come from HBM through pieces of 64 bytes, or in a second round of 64-wide ones (16 rows: 8192 x 8192 34.8 / 38.2,
-  // 5120 x 5120 16.9 / 18.0, but 1024 x 8192 13.6 / 10.9, 4096 x 11008 40 / 34, 28672 x 1280 23.4 / 15.8, 4096 x 4096 13.6 / 12.2;
-  // 64 rows: 28672 x 8192 104 / 122, 20480 x 3072 41 / 50, 11008 x 4096 23.4 / 23.5, but 4096 x 11008 50 / 35, 2048 x 2048 9.5 / 6.6,
-  // 6144 x 2048 12.4 / 10.6, 28672 x 1280 26.3 / 20.4)
-  if (layout == SK_LAYOUT_NN) return M <= 32 ? !(N > 4608 && N <= 8192 && K >= 4096) : N <= 4608 || K < 3000;
+  // [K, N] weights and up to 64 rows, against tiles of 128 rows and more (in us, those / these: 16 rows 4096 x 4096 21.5 / 12.0,
+  // 11008 x 4096 32.3 / 19.8, 8192 x 8192 43 / 36, 64 rows 4096 x 11008 44 / 35, 2048 x 2048 15.2 / 6.6): behind only where more than 32
+  // rows take two rounds of 64-wide tiles (33 x 20480 x 3072 40.0 / 46.8, 64 x 28672 x 8192 107 / 125, but 64 x 28672 x 1280 24 / 20)
+  if (layout == SK_LAYOUT_NN) return M <= 32 || cdiv(N, 64) <= num_cus || K < 2048;
   // 33 to 64 rows against the kernels that stream the weights through LDS: K long enough for a ring to fill, and few columns
   // (in us, those / these, 64 rows: fp16 2048 x 2048 9.5 / 6.2, 4096 x 4096 14.0 / 9.9, 6144 x 2048
   // 12.7 / 9.0, 1024 x 8192 13.8 / 10.4; int8 4096 x 11008 16.4 / 13.1, 2048 x 8192 11.7 / 9.3; but fp16 4096 x 11008 25.9 / 27.1,

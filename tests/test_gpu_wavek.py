@@ -137,5 +137,6 @@ def test_the_operators_rule(sk):
         for layout in ("nt", "nn"):
             assert not wavek(100, 4096, 4096, dtype, layout, variant=12, fixup="atomic_c")
         assert wavek(1, 4096, 4096, dtype, "nn", variant=12) and wavek(100, 4096, 4096, dtype, "nn", variant=12)
-        assert not wavek(1, 4096, 4096, dtype, "nn") and not wavek(64, 8192, 8192, dtype, "nn", variant=12)
+        assert not wavek(1, 4096, 4096, dtype, "nn") and wavek(64, 8192, 8192, dtype, "nn", variant=12)
+        assert not wavek(64, 28672, 8192, dtype, "nn", variant=12)
     assert sk.make_plan(40, 4096, 4096, "q4_zp", "nt", cus=256, use_tuned=False).kernel_id < 400
