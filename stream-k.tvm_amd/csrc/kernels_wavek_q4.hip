@@ -2,6 +2,7 @@
 #include "launch.h"
 #include "sk_persistent.h"
 #include "tile_wavek_q4.h"
+#include "wavek_launch.h"
 
 namespace sk {
 
@@ -10,6 +11,22 @@ __global__ __launch_bounds__(P::NT, P::WAVES_PER_EU) void sk_tile_wavek_q4_kerne
                                                                                   const void *bias) {
   __shared__ __attribute__((aligned(1024))) char smem[P::LDS_BYTES];
   run_persistent<P, FIXUP, true>(a, plan, ws, smem, bias);
+}
+
+// (what the loop begins with leads the arguments; the last two and the epilogue's are read later)
+template <class P>
+__global__ __launch_bounds__(P::NT, P::WAVES_PER_EU) void sk_tile_wavek_q4_flat_kernel(const half_t *A, const half_t *B, const half_t *scales,
+                                                                                       const half_t *zeros, int M, int N, int K, int lda,
+                                                                                       int tiles_m, int zero, half_t *C, int ldc,
+                                                                                       const void *bias) {
+  __shared__ __attribute__((aligned(1024))) char smem[P::LDS_BYTES];
+  WaveKQ4Args a;
+  a.A = A; a.B = B; a.C = C;
+  a.M = M; a.N = N; a.K = K;
+  a.lda = lda; a.ldb = K / 2; a.ldc = ldc;
+  a.alpha = 1.f; a.scales = scales; a.zero = zero; a.groups = K / 128;
+  a.zeros = zeros;
+  flat_run<P>(a, tiles_m, bias, smem);
 }
 
 int wavek_q4_kernel_infos(KernelInfo *out, int max) {
@@ -31,7 +48,10 @@ int wavek_q4_kernel_infos(KernelInfo *out, int max) {
 
 template <class P>
 static int launch(const WaveKQ4Args &a, const DevPlan &p, const Workspace &ws, hipStream_t s, const void *bias) {
-  if (p.sk_tiles == 0)
+  if (flat_plan(a, p, P::BK) && a.ldb == a.K / 2 && a.groups == a.K / 128)
+    hipLaunchKernelGGL((sk_tile_wavek_q4_flat_kernel<P>), dim3(p.grid), dim3(P::NT), 0, s, a.A, a.B, a.scales, a.zeros, a.M, a.N, a.K,
+                       (int)a.lda, p.tiles_m, a.zero, a.C, (int)a.ldc, bias);
+  else if (p.sk_tiles == 0)
     hipLaunchKernelGGL((sk_tile_wavek_q4_kernel<P, false>), dim3(p.grid), dim3(P::NT), 0, s, a, p, ws, bias);
   else
     hipLaunchKernelGGL((sk_tile_wavek_q4_kernel<P, true>), dim3(p.grid), dim3(P::NT), 0, s, a, p, ws, bias);

@@ -65,6 +65,11 @@ template <class P, class = void>
 struct has_prefetch { static constexpr bool value = false; };
 template <class P>
 struct has_prefetch<P, std::void_t<decltype(P::CROSS_TILE_PREFETCH)>> { static constexpr bool value = P::CROSS_TILE_PREFETCH; };
+// prefetch_bias: the policy fetches its bias before a tile's loop
+template <class P, class = void>
+struct has_prefetch_bias { static constexpr bool value = false; };
+template <class P>
+struct has_prefetch_bias<P, std::void_t<decltype(&P::prefetch_bias)>> { static constexpr bool value = true; };
 template <class P, class = void>
 struct has_halves { static constexpr bool value = false; };
 template <class P>
@@ -133,6 +138,9 @@ __device__ __forceinline__ void run_persistent(const typename P::Args &a, const 
     }
     int pm, pn;
     tile_coords(plan, tile, pm, pn);
+    if constexpr (has_prefetch_bias<P>::value && BIAS) {
+      if (bias != nullptr) P::prefetch_bias(a, acc, pn, bias);
+    }
     if constexpr (has_prefetch<P>::value) {
       P::mac(a, acc, pm, pn, k0, n, smem, first_stage_requested);
       first_stage_requested = false;

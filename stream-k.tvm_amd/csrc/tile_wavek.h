@@ -9,18 +9,21 @@
 //    of the second half: a wave that has its SIMD for itself issues one instruction in four cycles, a quarter of an MFMA.
 //  * The ring is a ring of loads, R KB long, a chunk being L of them: for tiles whose chunks are larger than 20 KB, R is no
 //    multiple of L, and part of the chunk after next is in flight.
-//  * When the segment ends the four waves' sums are added by a butterfly through LDS, halving what each holds: a wave ends up
-//    with a quarter of the tile's 16 x 16 blocks, and all four take part in the epilogue and the fix-up.
+//  * When the segment ends every wave puts its sums into its own ring and every thread adds the four waves' values of its share
+//    of the tile: pieces of 16 bytes along the rows of C, whose stores fill whole lines.
 //
 // What bounds it: a CU takes 75 to 85 GB/s of operands (its direct loads alone 107, profiles/lds_direct_load_rate.md), whether
-// they come through LDS or registers (a variant that loads to registers and writes the chunk to LDS: 77 to 80 GB/s), and 3 us
-// pass before and 1 to 3 us, by the tile, behind the loop.  So it serves what fits one or two rounds of tiles.  Without the
+// they come through LDS or registers (a variant that loads to registers and writes the chunk to LDS: 77 to 80 GB/s), and what
+// passes before and behind the loop.  So it serves what fits one or two rounds of tiles.  Without the
 // interleaving of reads and refills 64 x 64 tiles took 18.3 us at 256 x 4096 x 4096, with it 16.9; every XCD walks K from a start of
 // its own, because all CTAs of one share A as well as the weights (a start per column of tiles: 2048 x 1024 x 4096 45 us, so 28).
 // Weights from HBM and the Infinity Cache in turn (three sets of operands), the kernels before / these, in us: fp16
 // 128 x 4096 x 4096 17.7 / 12.9, 256 x 4096 x 4096 22.0 / 17.0, 64 x 4096 x 4096 14.0 / 9.9, 128 x 2048 x 2048 13.0 / 6.6,
 // 1024 x 1024 x 8192 32.6 / 26.0 (eager), bf16 100 x 11008 x 4096 with bias and GELU 34.6 / 28.1 (eager); int8 100 x 4096 x 4096
 // 13.1 / 8.9, 128 x 8192 x 8192 21.6 / 17.0; fp8 256 x 1024 x 8192 24.9 / 10.2, 64 x 28672 x 8192 with bias and SiLU 57.0 / 51.3 (eager).
+// Those figures are of a first form: with preloaded arguments (wavek_launch.h), one barrier in the sums over the waves in place of
+// five, stores of 16 bytes in place of 8 and the bias fetched ahead the three eager ones take 24.1, 26.0 and 48.0, and 300
+// sizes of 33 to 512 rows 3.5 % less on average, the smallest 0.5 to 1 us.
 #pragma once
 #include <type_traits>
 
@@ -51,39 +54,55 @@ struct WaveKTile {
   typedef typename std::conditional<I8, intx4, floatx4>::type AccV;
   typedef typename std::conditional<I8, int, float>::type AccT;
 
-  // c[u]: block v = first_block() + u, that is C[pm*BM + (v / FN)*16 + lane%16][pn*BN + (v % FN)*16 + 4*(lane/16) + e]
+  // What a thread ends up with: pieces of PW columns of one row, 16 bytes of C where the tile's size allows.  Piece u of thread t is
+  // number u NT + t of the tile's, along its rows.
+  static constexpr int PV = !I8 && NQ % 2 == 0 ? 2 : 1, PW = 4 * PV, PIECES = NQ / PV, PPR = BN / PW;   // PPR pieces make a row
   struct Acc {
     AccV c[NQ];
+    half_t bias __attribute__((ext_vector_type(PW)));   // (prefetch_bias)
   };
   static __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
-  static __device__ __forceinline__ int first_block(int wave) { return (wave & 1) * (NB / 2) + (wave >> 1) * NQ; }
+  static __device__ __forceinline__ int piece_row(int u, int tid) { return (int)((unsigned)(u * NT + tid) / (unsigned)PPR); }
+  static __device__ __forceinline__ int piece_col(int u, int tid) { return (int)((unsigned)(u * NT + tid) % (unsigned)PPR); }
+  static constexpr bool ONE_COL = NT % PPR == 0;        // the thread's pieces stand below each other
 
-  // c: the wave's sums of all blocks.  (w0 + w1) + (w2 + w3) in every wave, whatever it keeps.
-  static __device__ __forceinline__ void add_waves(AccV (&c)[NB], Acc &acc, char *smem) {
-    const int lane = threadIdx.x & 63, wave = wave_id();
-    AccV *mine = reinterpret_cast<AccV *>(smem) + (wave * (NB / 2)) * 64 + lane;
-    const AccV *theirs = reinterpret_cast<const AccV *>(smem) + ((wave ^ 1) * (NB / 2)) * 64 + lane;
-    __syncthreads();   // the rings are read
-    // (values are selected, not branches taken: two branches that differ in the block they name become one that indexes c)
-    const bool odd = wave & 1, high = wave & 2;
-    static_for<0, NB / 2>([&](auto v) {
-      const AccV lo = c[v], hi = c[NB / 2 + v];
-      mine[v * 64] = odd ? lo : hi;
-      c[v] = odd ? hi : lo;
+  // c: the wave's sums of all blocks, lane l of block v holding C[16 (v / FN) + l % 16][16 (v % FN) + 4 (l / 16) + e].  Every wave
+  // puts them into its own ring -- row r of a block's 16 at place r ^ key, so that the eight pieces along a row that are read
+  // together stand in eight different 16-byte places -- and after one barrier every thread adds the four waves' values of its
+  // pieces, (w0 + w1) + (w2 + w3).
+  template <int RING>
+  static __device__ __forceinline__ void add_waves(const AccV (&c)[NB], Acc &acc, char *smem) {
+    static_assert(NB * 1024 <= RING, "a wave's sums fit its ring");
+    constexpr int KM = PPR >= 8 ? 1 : (PPR >= 4 ? 2 : 4);
+    const int tid = pin_here((int)threadIdx.x), lane = tid & 63;   // (pinned: no address is held through the loop)
+    char *mine = smem + wave_id() * RING + (lane >> 4) * 256;
+    static_for<0, NB>([&](auto v) {
+      constexpr int j = v % FN;
+      const int key = ((PV == 2 ? 2 * j + (lane >> 5) : 4 * j + (lane >> 4)) * KM) & 7;
+      *reinterpret_cast<AccV *>(mine + v * 1024 + ((lane & 15) ^ key) * 16) = c[v];
     });
     __syncthreads();
-    static_for<0, NB / 2>([&](auto v) { c[v] += theirs[v * 64]; });
-    __syncthreads();
-    AccV *mine2 = reinterpret_cast<AccV *>(smem) + (wave * NQ) * 64 + lane;
-    const AccV *theirs2 = reinterpret_cast<const AccV *>(smem) + ((wave ^ 2) * NQ) * 64 + lane;
-    static_for<0, NQ>([&](auto v) {
-      const AccV lo = c[v], hi = c[NQ + v];
-      mine2[v * 64] = high ? lo : hi;
-      acc.c[v] = high ? hi : lo;
+    static_for<0, PIECES>([&](auto u) {
+      const int row = piece_row(u, tid), p = piece_col(u, tid);
+      static_for<0, PV>([&](auto h) {
+        const int col4 = p * PV + h;
+        const char *from = smem + (((row >> 4) * FN + (col4 >> 2)) * 64 + (col4 & 3) * 16 + ((row & 15) ^ ((p * KM) & 7))) * 16;
+        const AccV w0 = *reinterpret_cast<const AccV *>(from), w1 = *reinterpret_cast<const AccV *>(from + RING);
+        const AccV w2 = *reinterpret_cast<const AccV *>(from + 2 * RING), w3 = *reinterpret_cast<const AccV *>(from + 3 * RING);
+        acc.c[u * PV + h] = (w0 + w1) + (w2 + w3);
+      });
     });
-    __syncthreads();
-    static_for<0, NQ>([&](auto v) { acc.c[v] += theirs2[v * 64]; });
     __syncthreads();   // the rings may be filled again
+  }
+
+  // The bias of the thread's pieces, requested before the tile's loop: behind it the trip to memory would be waited for.  Whole
+  // aligned pieces of one column only; the others are read in the epilogue.
+  static __device__ __forceinline__ bool whole_bias(const Args &a, const half_t *bias) {
+    return ONE_COL && !I8 && bias != nullptr && a.N % PW == 0 && (reinterpret_cast<uintptr_t>(bias) & (2 * PW - 1)) == 0;
+  }
+  static __device__ __forceinline__ void prefetch_bias(const Args &a, Acc &acc, int pn, const void *epi) {
+    const half_t *bias = epi_bias(epi);
+    if (whole_bias(a, bias)) acc.bias = *reinterpret_cast<const decltype(acc.bias) *>(bias + min(pn * BN + piece_col(0, threadIdx.x) * PW, a.N - PW));
   }
 
   // (two copies behind one uniform branch: the epilogue without a bias carries none of its code)
@@ -96,18 +115,28 @@ struct WaveKTile {
   template <bool BIAS>
   static __device__ __forceinline__ void store_c_impl(const Args &a, const Acc &acc, int pm, int pn, const void *epi) {
     const half_t *bias = BIAS ? epi_bias(epi) : nullptr;
-    const int act = BIAS ? epi_act(epi) : 0;
-    const int lane = threadIdx.x & 63, first = first_block(wave_id());
-    const bool vec_ok = (a.ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(a.C) & (I8 ? 15 : 7)) == 0);
+    const int act = BIAS ? epi_act(epi) : 0, tid = pin_here((int)threadIdx.x);
+    typedef half_t HalfP __attribute__((ext_vector_type(PW)));
+    const uintptr_t at = reinterpret_cast<uintptr_t>(a.C);
+    const bool wide = a.ldc % PW == 0 && (at & (I8 ? 15 : 2 * PW - 1)) == 0, vec_ok = a.ldc % 4 == 0 && (at & (I8 ? 15 : 7)) == 0;
     floatx4 b4[NQ];
-    if constexpr (BIAS && !I8) {   // all loads at once
+    if constexpr (BIAS && !I8) {
+      if (whole_bias(a, bias)) {
 #pragma unroll
-      for (int u = 0; u < NQ; ++u) b4[u] = bias4_at<BF16>(bias, pn * BN + ((first + u) % FN) * 16 + 4 * (lane >> 4), a.N);
+        for (int x = 0; x < PW; ++x) {
+          const half_t h = acc.bias[x];
+          const float f = BF16 ? __builtin_bit_cast(float, (uint32_t)__builtin_bit_cast(uint16_t, h) << 16) : (float)h;
+#pragma unroll
+          for (int u = 0; u < PIECES; ++u) b4[u * PV + x / 4][x % 4] = f;
+        }
+      } else {   // all loads at once
+#pragma unroll
+        for (int u = 0; u < NQ; ++u) b4[u] = bias4_at<BF16>(bias, pn * BN + piece_col(u / PV, tid) * PW + 4 * (u % PV), a.N);
+      }
     }
 #pragma unroll
-    for (int u = 0; u < NQ; ++u) {
-      const int row = pm * BM + ((first + u) / FN) * 16 + (lane & 15);
-      const int col = pn * BN + ((first + u) % FN) * 16 + 4 * (lane >> 4);
+    for (int u = 0; u < PIECES; ++u) {
+      const int row = pm * BM + piece_row(u, tid), col = pn * BN + piece_col(u, tid) * PW;
       if (row >= a.M || col >= a.N) continue;
       if constexpr (I8) {   // int32 C straight from the accumulators (ldc counts int32 elements)
         int *dst = reinterpret_cast<int *>(a.C) + (int64_t)row * a.ldc + col;
@@ -117,12 +146,12 @@ struct WaveKTile {
           for (int e = 0; e < 4 && col + e < a.N; ++e) dst[e] = acc.c[u][e];
         }
       } else {
-        half4v h;
+        HalfP h;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float x = acc.c[u][e];
+        for (int e = 0; e < PW; ++e) {
+          float x = acc.c[u * PV + e / 4][e % 4];
           if constexpr (F8) x *= a.alpha;
-          if constexpr (BIAS) x = activate(x + b4[u][e], act);
+          if constexpr (BIAS) x = activate(x + b4[u * PV + e / 4][e % 4], act);
           if constexpr (BF16) {
             const __bf16 b = (__bf16)x;
             h[e] = __builtin_bit_cast(half_t, b);  // C carries 16-bit patterns
@@ -131,16 +160,25 @@ struct WaveKTile {
           }
         }
         half_t *dst = a.C + (int64_t)row * a.ldc + col;
-        if (vec_ok && col + 4 <= a.N) {
-          *reinterpret_cast<half4v *>(dst) = h;
+        if (wide && col + PW <= a.N) {
+          *reinterpret_cast<HalfP *>(dst) = h;
         } else {
-          for (int e = 0; e < 4 && col + e < a.N; ++e) dst[e] = h[e];
+#pragma unroll
+          for (int q = 0; q < PW; q += 4) {
+            if (vec_ok && col + q + 4 <= a.N) {
+              *reinterpret_cast<half4v *>(dst + q) = half4v{h[q], h[q + 1], h[q + 2], h[q + 3]};
+            } else {
+#pragma unroll
+              for (int e = q; e < q + 4; ++e)
+                if (col + e < a.N) dst[e] = h[e];
+            }
+          }
         }
       }
     }
   }
 
-  // Partial tiles: block u of thread t at (u NT + t) 4; the accumulating form keeps element e of it at (u 4 + e) NT + t.
+  // Partial tiles: four columns u of thread t at (u NT + t) 4; the accumulating form keeps element e of it at (u 4 + e) NT + t.
   static __device__ __forceinline__ void store_partial(const Acc &acc, float *dst) {
     const BufferRsrc r = make_rsrc(dst, TILE_ELEMS * 4);
 #pragma unroll
@@ -220,8 +258,7 @@ struct TileWaveK : WaveKTile<TYPE_, FM_, FN_> {
   static constexpr int R = L > 20 && !NN ? 40 : (L * 4 < 40 ? L * 4 : 40 / L * L);   // loads of a wave's ring (at most 160 KB / 4 waves, four chunks)
   static constexpr int S = R / L, PART = R % L;       // whole chunks in the ring, loads of one more
   static_assert(S >= 1 && (L % 2) == 0 && (R % 2) == 0, "a 16-row block of a chunk stays together in the ring");
-  static constexpr int RING = R * 1024, LDS_RINGS = WAVES * RING, LDS_SUMS = WAVES * (NB / 2) * 1024;
-  static constexpr int LDS_BYTES = LDS_RINGS > LDS_SUMS ? LDS_RINGS : LDS_SUMS, LDS_TOTAL = LDS_BYTES;
+  static constexpr int RING = R * 1024, LDS_BYTES = WAVES * RING, LDS_TOTAL = LDS_BYTES;
   static_assert(LDS_BYTES <= 160 * 1024, "LDS of a CU");
   static constexpr int CTAS_PER_CU = 1, WAVES_PER_EU = 1;
   static constexpr int NMFMA = Base::F8 ? NB : 2 * NB;   // MFMAs of a chunk
@@ -416,7 +453,7 @@ struct TileWaveK : WaveKTile<TYPE_, FM_, FN_> {
       if (++t == n) break;
     }
     wavek_wait_loads<0>();   // the loads past the segment write LDS too
-    Base::add_waves(c, acc, smem);
+    Base::template add_waves<RING>(c, acc, smem);
   }
 };
 

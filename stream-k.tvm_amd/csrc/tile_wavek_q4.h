@@ -41,8 +41,8 @@ struct TileWaveKQ4 : WaveKTile<TYPE_, FM_, FN_> {
   }
   static constexpr int DA = rings() / 10, DW = rings() % 10;
   static_assert(DA >= 2 && DW == (DA + 1) / 2, "two halves of A and a group of weights at least");
-  static constexpr int RING_W = DA * A_SLOT, RING = RING_W + DW * W_SLOT, LDS_RINGS = WAVES * RING, LDS_SUMS = WAVES * (NB / 2) * 1024;
-  static constexpr int LDS_BYTES = LDS_RINGS > LDS_SUMS ? LDS_RINGS : LDS_SUMS, LDS_TOTAL = LDS_BYTES;
+  static constexpr int RING_W = DA * A_SLOT, RING = RING_W + DW * W_SLOT;
+  static constexpr int LDS_BYTES = WAVES * RING, LDS_TOTAL = LDS_BYTES;
   static_assert(LDS_BYTES <= 160 * 1024, "LDS of a CU");
   static constexpr int CTAS_PER_CU = 1, WAVES_PER_EU = 1;
   static constexpr bool PERM_W = FM >= FN;   // the four permutations of a fragment on the side that has fewer of them
@@ -268,7 +268,7 @@ struct TileWaveKQ4 : WaveKTile<TYPE_, FM_, FN_> {
     if constexpr (DA == 2 * DW)
       if (t + DW < n) iteration(t++, std::true_type{}, std::false_type{}, std::false_type{});
     for (; t < n; ++t) iteration(t, std::false_type{}, std::false_type{}, std::false_type{});
-    Base::add_waves(c, acc, smem);
+    Base::template add_waves<RING>(c, acc, smem);
   }
 };
 

@@ -89,6 +89,36 @@ def test_every_tile_is_exact(sk, dtype, layout):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16", "float8_e4m3", "int8", "q4"])
+def test_alignments_of_the_epilogue(sk, dtype):
+    """C and the bias at every alignment that decides how they are accessed, by tiles with pieces of eight and of four columns,
+    as whole tiles in one round and through the fix-up."""
+    import torch
+    rng = np.random.default_rng(43)
+    for bm, bn in ((64, 64), (32, 32), (96, 64)) if dtype != "q4" else ((64, 64), (32, 32), (64, 96)):
+        for N in (4 * bn, bn + 4, bn + 13):
+            M, K = bm + 5, 2048
+            call, exact = _operands(torch, dtype, rng, M, N, K)
+            kind = torch.bfloat16 if dtype == "bfloat16" else torch.float16
+            values = torch.from_numpy(rng.integers(-8, 9, N).astype(np.float32)).to(kind)
+            for sched in (dict(schedule="dp"), dict(schedule="basic", grid=5, fixup="reduce")):
+                plan = sk.make_plan(M, N, K, dtype, "nt", dict(sched, bm=bm, bn=bn, variant=11))
+                for at, ldc in ((0, N), (0, (N + 7) // 8 * 8), (4, (N + 7) // 8 * 8 + 4), (1, N + 1), (8, (N + 7) // 8 * 8 + 1)):
+                    for bias_at in (0, 4, 1) if dtype != "int8" else (None,):
+                        bias = None
+                        if bias_at is not None:
+                            bias = torch.zeros(N + bias_at, dtype=kind, device="cuda")[bias_at:]
+                            bias.copy_(values)
+                        want = _rounded(torch, exact if bias is None else exact + values.double().numpy(), dtype)
+                        buf = torch.zeros(at + M * ldc, dtype=want.dtype, device="cuda")
+                        out = buf[at:].view(M, ldc)[:, :N]
+                        call(plan=plan, out=out, **({} if bias is None else {"bias": bias}))
+                        assert torch.equal(out.cpu(), want), (dtype, bm, bn, N, sched, at, ldc, bias_at)
+                        assert not buf[:at].any() and not buf[at:].view(M, ldc)[:, N:].any(), (dtype, bm, bn, N, sched, at, ldc, bias_at)
+    sk.workspace_status()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype,layout", [("float16", "nt"), ("bfloat16", "nt"), ("float8_e4m3", "nt"), ("int8", "nt"), ("q4", "nt"), ("q4_zp", "nt"),
                                           ("float16", "nn"), ("bfloat16", "nn")])
 def test_operator_calls_equal_the_plans_they_replace(sk, dtype, layout):
