@@ -672,7 +672,9 @@ static bool wavek_pays(int64_t M, int64_t N, int64_t K, int dtype, int layout, i
     // ([K, N] weights and 97 to 128 rows, which fill the others' tiles: 128 x 5120 x 5120 29.8 us on those, 35.2 here against a
     // predicted 24; 72 rows 29.2 / 28.2, 160 rows 34.8 / 31.9)
     const bool full_rows = layout == SK_LAYOUT_NN && M > 96 && M <= 128;
-    return other_us <= 0 || wavek_us < (from_hbm ? (full_rows ? 0.7 : 0.85) : (one_byte ? 0.95 : 0.92)) * other_us;
+    // (More rows than one 128-row tile has: 320 x 4096 x 11008 of fp16 66 us on the kernels before, 50 here, 160 rows 43.4 / 40.6.)
+    const bool one_row = M <= 128 || layout == SK_LAYOUT_NN;
+    return other_us <= 0 || wavek_us < (from_hbm && one_row ? (full_rows ? 0.7 : 0.85) : (one_byte ? 0.95 : 0.92)) * other_us;
   }
   // [K, N] weights and up to 64 rows, against tiles of 128 rows and more (in us, those / these: 16 rows 4096 x 4096 21.5 / 12.0,
   // 11008 x 4096 32.3 / 19.8, 8192 x 8192 43 / 36, 64 rows 4096 x 11008 44 / 35, 2048 x 2048 15.2 / 6.6): behind only where more than 32
