@@ -665,16 +665,21 @@ static bool wavek_pays(int64_t M, int64_t N, int64_t K, int dtype, int layout, i
     return wavek_us < 0.95 * tile_us;
   }
   const bool one_byte = dtype == SK_F8E4M3 || dtype == SK_F8E5M2 || dtype == SK_I8;
-  // (weights that the Infinity Cache does not keep between calls come in slower than the fit's average of both says: 80 to 128 x
-  // 4096 x 11008 of fp16 29.5 to 31.0 us on the ring kernels, 32 to 36 here against a predicted 28)
+  // (16-bit weights that the Infinity Cache does not keep between calls come in slower than the fit's average of both says: 80 to
+  // 128 x 4096 x 11008 of fp16 29.5 to 31.0 us on the ring kernels, 32 to 36 here against a predicted 28)
   if (M > 64) {
-    const bool from_hbm = (one_byte ? 1 : 2) * N * K > ((int64_t)(layout == SK_LAYOUT_NN ? 48 : 64) << 20);
+    const bool from_hbm = !one_byte && 2 * N * K > ((int64_t)(layout == SK_LAYOUT_NN ? 48 : 64) << 20);
     // ([K, N] weights and 97 to 128 rows, which fill the others' tiles: 128 x 5120 x 5120 29.8 us on those, 35.2 here against a
     // predicted 24; 72 rows 29.2 / 28.2, 160 rows 34.8 / 31.9)
     const bool full_rows = layout == SK_LAYOUT_NN && M > 96 && M <= 128;
     // (More rows than one 128-row tile has: 320 x 4096 x 11008 of fp16 66 us on the kernels before, 50 here, 160 rows 43.4 / 40.6.)
     const bool one_row = M <= 128 || layout == SK_LAYOUT_NN;
-    return other_us <= 0 || wavek_us < (from_hbm && one_row ? (full_rows ? 0.7 : 0.85) : (one_byte ? 0.95 : 0.92)) * other_us;
+    if (from_hbm && one_row) return other_us <= 0 || wavek_us < (full_rows ? 0.7 : 0.85) * other_us;
+    // The fit is of a form of these kernels that took 0.5 to 1.8 us longer to add up and store, so a tie is theirs: over 201 sizes
+    // each 22.5 % off fp8's times by this choice, 21.2 % with a margin of 5 %, no size slower (600 x 1500 x 3008 15.6 us / 9.9,
+    // 128 x 8192 x 16384 56.3 / 37.8, 128 x 6144 x 2048 9.7 / 7.0; 1024 x 1024 x 8192 of fp16 34.5 / 26.6); at 1.04 int8
+    // 320 x 11008 x 4096 would go from 25.3 to 29.6.
+    return other_us <= 0 || wavek_us < (one_byte ? 1.0 : (layout == SK_LAYOUT_NN ? 0.92 : 0.97)) * other_us;
   }
   // [K, N] weights and up to 64 rows, against tiles of 128 rows and more (in us, those / these: 16 rows 4096 x 4096 21.5 / 12.0,
   // 11008 x 4096 32.3 / 19.8, 8192 x 8192 43 / 36, 64 rows 4096 x 11008 44 / 35, 2048 x 2048 15.2 / 6.6): behind only where more than 32

@@ -169,4 +169,17 @@ def test_the_operators_rule(sk):
         assert wavek(1, 4096, 4096, dtype, "nn", variant=12) and wavek(100, 4096, 4096, dtype, "nn", variant=12)
         assert not wavek(1, 4096, 4096, dtype, "nn") and wavek(64, 8192, 8192, dtype, "nn", variant=12)
         assert not wavek(64, 28672, 8192, dtype, "nn", variant=12)
+        # weights from HBM: a wide margin while one row of the others' tiles holds them
+        assert wavek(320, 4096, 11008, dtype, "nt", variant=12) and not wavek(100, 4096, 11008, dtype, "nt", variant=12)
+        assert wavek(80, 5120, 5120, dtype, "nn", variant=12) and not wavek(128, 5120, 5120, dtype, "nn", variant=12)
     assert sk.make_plan(40, 4096, 4096, "q4_zp", "nt", cus=256, use_tuned=False).kernel_id < 400
+
+
+@pytest.mark.gpu
+def test_rows_too_long_for_the_preferred_tiles_take_the_plain_plan(sk):
+    """128 rows of 2 GiB and more are refused by the tiles that operators prefer; kernels for fewer rows take them."""
+    import sys
+    plan_for = sys.modules["streamk.ops"]._plan_for
+    name = lambda *pitches: sk.kernel_name(plan_for("", 100, 3840, 4096, "float16", "nt", *pitches).kernel_id)   # noqa: E731
+    assert name(8192, 8192).startswith("wavek_") and name(8192, (1 << 24) - 2).startswith("wavek_")
+    assert not name(8192, 1 << 24).startswith("wavek_") and not name(1 << 24, 8192).startswith("wavek_")
