@@ -140,9 +140,18 @@ def _parse_config(text):
     return out
 
 
-def _plan_for(config, M, N, K, dtype, layout):
+def _too_long(*pitches):
+    """Whether 128 rows of any of these lengths in bytes reach 2 GiB: the kernels for few rows, whose tiles have fewer, take
+    longer rows than those that operators prefer."""
+    return any(p * 128 >= 1 << 31 for p in pitches)
+
+
+def _plan_for(config, M, N, K, dtype, layout, *pitches):
     """The plan an operator call runs: the registered plan object, or one made from the configuration
-    string for this shape (made once per (shape, type, layout, configuration))."""
+    string for this shape (made once per (shape, type, layout, configuration)).  `pitches`: lengths in bytes of the rows
+    that a tile reads; beyond what every kernel takes, the plain plan."""
+    if config == "" and _too_long(*pitches):
+        config = "raster=0"
     if config.startswith("#"):
         plan = _plan_registry.get(config)
         if plan is None:
@@ -199,7 +208,7 @@ def _run_16bit(A, B, C, layout, config, bias, activation, tdtype, name):
     if K != Kb:
         raise ValueError(f"K mismatch: A is {tuple(A.shape)}, B is {tuple(B.shape)}")
     _check_out(C, M, N, tdtype)
-    plan = _plan_for(config, M, N, K, name, layout)
+    plan = _plan_for(config, M, N, K, name, layout, 2 * A.stride(0), 2 * B.stride(0) if layout == "nt" else 0)
     epi = _epilogue(bias, N, tdtype, A.device, _act(activation))
     args = (A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, A.stride(0), B.stride(0), C.stride(0),
             *_ws_args(plan, A.device))
@@ -250,7 +259,7 @@ def _run_f8(A, B, C, alpha, fmt, config, bias, activation):
     if K != Kb:
         raise ValueError(f"K mismatch: A is {tuple(A.shape)}, B is {tuple(B.shape)}")
     _check_out(C, M, N, torch.float16)
-    plan = _plan_for(config, M, N, K, "float8_" + fmt, "nt")
+    plan = _plan_for(config, M, N, K, "float8_" + fmt, "nt", A.stride(0), B.stride(0))
     if plan.dtype != (_lib.SK_F8E5M2 if fmt == "e5m2" else _lib.SK_F8E4M3):
         raise ValueError("the plan was made for the other fp8 format")
     epi = _epilogue(bias, N, torch.float16, A.device, _act(activation))
@@ -268,7 +277,7 @@ def _run_i8(A, B, C, config):
     if K != Kb:
         raise ValueError(f"K mismatch: A is {tuple(A.shape)}, B is {tuple(B.shape)}")
     _check_out(C, M, N, torch.int32)
-    plan = _plan_for(config, M, N, K, "int8", "nt")
+    plan = _plan_for(config, M, N, K, "int8", "nt", A.stride(0), B.stride(0))
     rc = _lib.lib().sk_gemm_i8(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, A.stride(0), B.stride(0),
                                C.stride(0), *_ws_args(plan, A.device))
     _lib.check(rc, "sk_gemm_i8")
@@ -323,7 +332,7 @@ def _run_q4(A, Wq, scales, zeros, C, zero, group, tiled, config, bias, activatio
     if tuple(scales.shape) != (N, K // group) or not scales.is_contiguous():
         raise ValueError(f"scales must be contiguous [N, K/group]; got {tuple(scales.shape)}")
     _check_out(C, M, N, torch.float16)
-    if M > Q4_MAX_M and (tiled or (zeros is not None and config and not _has_plan(config, M, N, K, "q4_zp"))) \
+    if M > Q4_MAX_M and (tiled or (zeros is not None and (_too_long(2 * A.stride(0), K // 2) if config == "" else not _has_plan(config, M, N, K, "q4_zp")))) \
             and not config.startswith("#"):
         # The kernels for the tiled layout take at most 64 rows of A: up to 256 rows one launch per block of 64, and so do
         # configurations that name kernels for few rows.  (Blocks of two rows and more multiply the rounded weights alike; a
@@ -355,7 +364,7 @@ def _run_q4(A, Wq, scales, zeros, C, zero, group, tiled, config, bias, activatio
         _run_16bit(A, W, C, "nt", "", bias, activation, torch.float16, "float16")
         return
     name = ("q4_zp_tiled" if tiled else "q4_zp") if zeros is not None else ("q4_tiled" if tiled else "q4")
-    plan = _plan_for(config, M, N, K, name, "nt")
+    plan = _plan_for(config, M, N, K, name, "nt", 2 * A.stride(0), K // 2)
     if (plan.dtype in (_lib.SK_Q4_TILED, _lib.SK_Q4_ZP_TILED)) != bool(tiled):
         raise ValueError("the plan was made for the other weight layout")
     if (plan.dtype in (_lib.SK_Q4_ZP, _lib.SK_Q4_ZP_TILED)) != (zeros is not None):
