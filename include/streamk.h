@@ -113,6 +113,9 @@ typedef struct sk_config {
   int32_t reserved[4];    /* reserved[0]: 0 = preferred kernel variant of the tile, v > 0 = variant v - 1
                              (9 without a tile, fp8 / int8 up to 64 rows: weights streamed through LDS)
                              (implementation alternatives of one tile shape, for the autotuner);
+                             11: the tiles whose waves stream K on their own (bm, bn: 32..128); 12 without a
+                             tile, schedule or grid: what an operator call takes, those tiles or else the
+                             kernel that 0 means;
                              reserved[1]: split factor of SK_SCHED_SPLIT_K, 0 = choose;
                              reserved[2]: 1 = interleaved order of the Stream-K tiles (see sk_plan.interleave); with 0 the
                              automatic schedule still chooses it for 256 x 256 tiles whose CTA ranges would start
@@ -334,7 +337,8 @@ int sk_gemm_q4(const void *A, const void *Wq, const void *scales, void *C, int64
 /* The same with one zero point per scale group and row: zeros [N, K/group] fp16 holding integers 0..15,
  * w = fp16_rn((fp16(q) - zeros[n][k/group]) * scales[n][k/group]) -- the asymmetric formats of weight-only
  * quantisers (min/max per group), which the reference's unsigned nibbles with one implied zero point do
- * not cover.  The plan is made with dtype SK_Q4_ZP; at most 64 rows per call.  M == 1 takes matrix-vector kernels
+ * not cover.  The plan is made with dtype SK_Q4_ZP; at most 64 rows per call, any
+ * number with a plan of reserved[0] = 11 or 12 (sk_config).  M == 1 takes matrix-vector kernels
  * that, like sk_gemm_q4's, multiply the nibbles undecoded and apply zero point and scale to fp32 group sums (the
  * unrounded (q - zero) * scale); 2 <= M <= 64, and M == 1 with an explicit variant-0 plan, kernels that form the
  * rounded weights bit for bit.

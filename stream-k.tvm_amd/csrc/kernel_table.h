@@ -25,7 +25,8 @@ struct KernelInfo {
                 // swizzled rows; 2: as 1 with four waves per CTA (one per SIMD, accumulators in AGPRs);
                 // 3: as 1 with BK = 32 and four LDS stages (loads three iterations ahead);
                 // 4: as 1 with 16x16x32 MFMAs; 5: as 3 with 16x16x32 MFMAs; 6: as 1 for fp8 operands (32x32x64 MFMAs);
-                // 7: as 4 with four waves per CTA, the K loop in assembly and the accumulators in a[0:255]
+                // 7: as 4 with four waves per CTA, the K loop in assembly and the accumulators in a[0:255];
+                // 9: rings of different depths for weights and A; 10: waves that stream K on their own
                 // small-M kernels -- 0: up to 16*MB rows of A; 1: M == 1; 2: M == 1, matrix-vector on 4x4x4 MFMA;
                 // 3: the matrix-vector form with up to four rows of A; 4: weights streamed through LDS in contiguous loads
   int bm, bn, bk;  // CTA tile; bk is the K extent of one CTA iteration
