@@ -685,17 +685,27 @@ static bool wavek_pays(int64_t M, int64_t N, int64_t K, int dtype, int layout, i
   // 11008 x 4096 32.3 / 19.8, 8192 x 8192 43 / 36, 64 rows 4096 x 11008 44 / 35, 2048 x 2048 15.2 / 6.6): behind only where more than 32
   // rows take two rounds of 64-wide tiles (33 x 20480 x 3072 40.0 / 46.8, 64 x 28672 x 8192 107 / 125, but 64 x 28672 x 1280 24 / 20)
   if (layout == SK_LAYOUT_NN) return M <= 32 || cdiv(N, 64) <= num_cus || K < 2048;
-  // 33 to 64 rows against the kernels that stream the weights through LDS: K long enough for a ring to fill, and few columns
-  // (in us, those / these, 64 rows: fp16 2048 x 2048 9.5 / 6.2, 4096 x 4096 14.0 / 9.9, 6144 x 2048
-  // 12.7 / 9.0, 1024 x 8192 13.8 / 10.4; int8 4096 x 11008 16.4 / 13.1, 2048 x 8192 11.7 / 9.3; but fp16 4096 x 11008 25.9 / 27.1,
-  // 5120 x 5120 from HBM 21.1 / 23.2, 8192 x 8192 29.7 / 31.4, 4096 x 1024 5.9 / 5.0, 1024 x 1024 5.8 / 6.4; int8 8192 x 16384 29.7 / 34.7) or more than a round of
-  // their 64-row tiles where 112-row tiles need one (20480 x 3072 fp16 37.6 / 27.9, 28672 x 8192 88.3 / 85.4, of fp8 50.4 / 47.5).
-  // One-byte operands of fewer than 6144 K-values stay with the streaming kernels throughout: there the gain is 1 to 2 us
-  // (4096 x 4096 8.8 / 7.4, 2048 x 2048 5.8 / 5.0), and those are the kernels their plans are known by.  Up to 32 rows there is
-  // nothing to gain (20 x 4096 x 4096 9.4 / 9.1 and 6.6 / 6.7).
-  if (M <= 32 || (one_byte && K < 6144)) return false;
-  if (cdiv(N, 64) > num_cus && cdiv(N, 112) <= num_cus) return K >= 2048;
-  return N <= (one_byte ? 4096 : 6144) && K >= 1536 && N * K <= (one_byte ? (int64_t)48 << 20 : (int64_t)24 << 20);
+  // 17 to 64 rows against the kernels that stream the weights through LDS.  Times over theirs with the weights from HBM / three sets
+  // in turn, 29 shapes at 17 to 64 rows each:
+  //   more than a round of 64-wide tiles where wider ones need one   20480 x 3072 .86 / .86 (17 to 32 rows, of fp8 .86 / .82; 33 to 64 rows
+  //     of fp16 37.6 us / 27.9, of fp8 .76 / .74), 28672 x 1280 .91 / .94 and .87 / .88 from 33 rows on, 1.01 / .99 before
+  //   33 to 64 rows, few columns   fp16 768 x 1024 .80 / .79, 2048 x 1280 .52 / .49, 4096 x 1024 .85 / .79, 4096 x 8192 .95 / .81; fp8
+  //     1024 x 1024 .81 / .81, 2048 x 5120 .67 / .67, 4096 x 3584 .75 / .75; but fp16 5120 x 5120 1.05 / .83, 4096 x 11008 .97 / .96,
+  //     8192 x 3072 1.10 / .95; fp8 5120 x 5120 1.12 / .90, 14336 x 3072 1.03 / 1.02
+  //   17 to 32 rows   fp16 1504 x 3072 .86 / .84, 2048 x 1280 .65 / .62, 2048 x 8192 .93 / .92; but 1024 x 1024 1.0 / 1.0, 4096 x 1024
+  //     1.06 / .99, 1280 x 16384 1.04 / .86, 5632 x 3072 1.06 / 1.03; fp8 1024 x 1024 .89 / .91, 4096 x 2048 .96 / .90, 8192 x 1280 .87 / .82, 8192 x 3072 .93 / .93; but
+  //     11008 x 2048 1.02 / 1.03, 4096 x 8192 1.08 / .89
+  // One-byte operands of 4096 K-values and a little more stay with the streaming kernels: those are the kernels that operator calls
+  // of that length are known by (4096 x 4096 8.8 us / 7.0).
+  if (one_byte && K >= 4096 && K < 4608) return false;
+  const bool rounds = cdiv(N, 64) > num_cus;
+  if (M <= 32) {
+    if (rounds) return K >= 2048 && cdiv(N, 80) <= num_cus;
+    return one_byte ? K >= 1024 && K < 4096 && N <= 8192 : K >= 1280 && N >= 1280 && N <= 2560 && N * K <= (int64_t)16 << 20;
+  }
+  if (rounds && cdiv(N, 112) <= num_cus) return K >= 1024;
+  if (N <= 4096) return K >= 1024 && N * K <= (int64_t)(one_byte ? 48 : 36) << 20;
+  return !one_byte && N <= 6144 && K >= 1536 && N * K <= (int64_t)24 << 20;
 }
 
 // ---- fp32: tile, schedule and grid, when the caller leaves all three open ----

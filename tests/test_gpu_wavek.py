@@ -129,7 +129,7 @@ def test_operator_calls_equal_the_plans_they_replace(sk, dtype, layout):
     rng = np.random.default_rng(42)
     step = 128 if dtype.startswith("q4") else (16 if dtype in ("float8_e4m3", "int8") else 8)
     seen = set()
-    for M, N, K in ((1, 2048, 1024), (17, 768, 1536), (33, 770, 6144), (40, 2049, 2048), (64, 1000, 8192), (65, 775, 512), (100, 3001, 1664), (128, 768, 4096),
+    for M, N, K in ((1, 2048, 1024), (17, 768, 1536), (24, 1290, 1408), (31, 2056, 3200), (33, 770, 6144), (40, 2049, 2048), (64, 1000, 8192), (65, 775, 512), (100, 3001, 1664), (128, 768, 4096),
                     (129, 1031, 640), (257, 2050, 1152), (300, 769, 2304), (513, 801, 384)):
         K, N = K // step * step, N if layout == "nt" else N // 8 * 8
         call, exact = _operands(torch, dtype, rng, M, N, K, pad=8 * (2 if step == 16 else 1), layout=layout)
@@ -163,6 +163,12 @@ def test_the_operators_rule(sk):
         assert not wavek(16, 4096, 4096, dtype, "nt", variant=12)
         assert wavek(100, 760, 4096, dtype, "nt", variant=12) == (dtype == "q4_zp")
         assert wavek(4096, 8192, 8192, dtype, "nt", variant=12) == (dtype == "q4_zp")
+    # 17 to 64 rows: few columns, or more than one round of 64-wide tiles where wider ones need one
+    for dtype in ("float8_e4m3", "int8", "float16"):
+        assert wavek(48, 2048, 5120, dtype, "nt", variant=12) and wavek(24, 20480, 3072, dtype, "nt", variant=12)
+        assert wavek(24, 2048, 2048, dtype, "nt", variant=12) and not wavek(24, 11008, 2048, dtype, "nt", variant=12)
+        assert wavek(24, 1024, 1024, dtype, "nt", variant=12) == wavek(24, 4096, 2048, dtype, "nt", variant=12) == (dtype != "float16")
+        assert wavek(48, 4096, 4096, dtype, "nt", variant=12) == (dtype == "float16")
     for dtype in ("float16", "bfloat16"):
         for layout in ("nt", "nn"):
             assert not wavek(100, 4096, 4096, dtype, layout, variant=12, fixup="atomic_c")
