@@ -13,20 +13,22 @@ __global__ __launch_bounds__(P::NT, P::WAVES_PER_EU) void sk_tile_wavek_q4_kerne
   run_persistent<P, FIXUP, true>(a, plan, ws, smem, bias);
 }
 
-// (what the loop begins with leads the arguments; the last two and the epilogue's are read later)
+// (what the loop needs leads the arguments, as many as are preloaded -- hence the tiles, at most eight, and the zero point in one; the
+// others are read later)
 template <class P>
 __global__ __launch_bounds__(P::NT, P::WAVES_PER_EU) void sk_tile_wavek_q4_flat_kernel(const half_t *A, const half_t *B, const half_t *scales,
                                                                                        const half_t *zeros, int M, int N, int K, int lda,
-                                                                                       int tiles_m, int zero, half_t *C, int ldc,
+                                                                                       int tiles_zero, uint32_t start_scale, half_t *C, int ldc,
                                                                                        const void *bias) {
   __shared__ __attribute__((aligned(1024))) char smem[P::LDS_BYTES];
   WaveKQ4Args a;
   a.A = A; a.B = B; a.C = C;
   a.M = M; a.N = N; a.K = K;
   a.lda = lda; a.ldb = K / 2; a.ldc = ldc;
-  a.alpha = 1.f; a.scales = scales; a.zero = zero; a.groups = K / 128;
+  a.alpha = 1.f; a.scales = scales; a.zero = tiles_zero >> 8; a.groups = K / 128;
+  a.start_scale = start_scale;
   a.zeros = zeros;
-  flat_run<P>(a, tiles_m, bias, smem);
+  flat_run<P>(a, tiles_zero & 255, bias, smem);
 }
 
 int wavek_q4_kernel_infos(KernelInfo *out, int max) {
@@ -50,7 +52,7 @@ template <class P>
 static int launch(const WaveKQ4Args &a, const DevPlan &p, const Workspace &ws, hipStream_t s, const void *bias) {
   if (flat_plan(a, p, P::BK) && a.ldb == a.K / 2 && a.groups == a.K / 128)
     hipLaunchKernelGGL((sk_tile_wavek_q4_flat_kernel<P>), dim3(p.grid), dim3(P::NT), 0, s, a.A, a.B, a.scales, a.zeros, a.M, a.N, a.K,
-                       (int)a.lda, p.tiles_m, a.zero, a.C, (int)a.ldc, bias);
+                       (int)a.lda, p.tiles_m | a.zero << 8, a.start_scale, a.C, (int)a.ldc, bias);
   else if (p.sk_tiles == 0)
     hipLaunchKernelGGL((sk_tile_wavek_q4_kernel<P, false>), dim3(p.grid), dim3(P::NT), 0, s, a, p, ws, bias);
   else
@@ -61,6 +63,7 @@ static int launch(const WaveKQ4Args &a, const DevPlan &p, const Workspace &ws, h
 int launch_wavek_q4(int id, const GemmArgs &g, const void *zeros, const DevPlan &p, const Workspace &ws, hipStream_t s, const void *bias) {
   WaveKQ4Args a;
   static_cast<GemmArgs &>(a) = g;
+  a.start_scale = start_scale(p);
   a.zeros = static_cast<const half_t *>(zeros);
   switch (id) {
 #define X(id_, FM, FN)                                                               \

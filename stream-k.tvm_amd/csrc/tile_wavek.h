@@ -16,7 +16,8 @@
 // they come through LDS or registers (a variant that loads to registers and writes the chunk to LDS: 77 to 80 GB/s), and what
 // passes before and behind the loop.  So it serves what fits one or two rounds of tiles.  Without the
 // interleaving of reads and refills 64 x 64 tiles took 18.3 us at 256 x 4096 x 4096, with it 16.9; every XCD walks K from a start of
-// its own, because all CTAs of one share A as well as the weights (a start per column of tiles: 2048 x 1024 x 4096 45 us, so 28).
+// its own (start_of), because all CTAs of one share A as well as the weights (a start per column of tiles: 2048 x 1024 x 4096 45 us,
+// so 28).
 // Weights from HBM and the Infinity Cache in turn (three sets of operands), the kernels before / these, in us: fp16
 // 128 x 4096 x 4096 17.7 / 12.9, 256 x 4096 x 4096 22.0 / 17.0, 64 x 4096 x 4096 14.0 / 9.9, 128 x 2048 x 2048 13.0 / 6.6,
 // 1024 x 1024 x 8192 32.6 / 26.0 (eager), bf16 100 x 11008 x 4096 with bias and GELU 34.6 / 28.1 (eager); int8 100 x 4096 x 4096
@@ -34,15 +35,18 @@ namespace sk {
 
 enum WaveKType { WK_F16 = 0, WK_BF16 = 1, WK_F8E4M3 = 2, WK_F8E5M2 = 3, WK_I8 = 4, WK_Q4 = 5, WK_Q4ZP = 6 };
 
+struct WaveKArgs : GemmArgs {
+  uint32_t start_scale;   // 2^32 / tiles of a round of the launch, rounded up (start_of)
+};
 // Q4 weights: with the array of zero points where every group has its own
-struct WaveKQ4Args : GemmArgs {
+struct WaveKQ4Args : WaveKArgs {
   const half_t *zeros;
 };
 
 // what the kernels of this file share: who holds which block of the tile, the sums over the waves, epilogue, partial tiles
 template <int TYPE_, int FM_, int FN_>
 struct WaveKTile {
-  typedef typename std::conditional<(TYPE_ >= WK_Q4), WaveKQ4Args, GemmArgs>::type Args;
+  typedef typename std::conditional<(TYPE_ >= WK_Q4), WaveKQ4Args, WaveKArgs>::type Args;
   static constexpr bool LEAN_ENTRY = true;            // see run_persistent
   static constexpr bool COHERENT_PARTIALS = true;
   static constexpr bool FIXUP_WORD_IN_LDS = true;     // the rings are dead between two calls of mac
@@ -65,6 +69,15 @@ struct WaveKTile {
   static __device__ __forceinline__ int piece_row(int u, int tid) { return (int)((unsigned)(u * NT + tid) / (unsigned)PPR); }
   static __device__ __forceinline__ int piece_col(int u, int tid) { return (int)((unsigned)(u * NT + tid) % (unsigned)PPR); }
   static constexpr bool ONE_COL = NT % PPR == 0;        // the thread's pieces stand below each other
+
+  // The iteration of a segment of n that a tile of column pn starts with: the XCDs' starts are spread over the segment, and a tile takes
+  // that of the XCD which holds the first tile of its column -- its own XCD's but where a column straddles two, or goes on in another
+  // group of eight rows.  So all tiles of a column add up K in one order: equal rows of A give equal bits, wherever they stand in it.
+  // (first * start_scale: how far the first tile is into its round of the launch, as a fraction of 2^32)
+  static __device__ __forceinline__ int start_of(const Args &a, int pn, int n) {
+    const uint32_t first = (uint32_t)(pn * min((a.M + BM - 1) / BM, 8));
+    return (int)(((first * a.start_scale) >> 29) * (uint32_t)n >> 3);
+  }
 
   // c: the wave's sums of all blocks, lane l of block v holding C[16 (v / FN) + l % 16][16 (v % FN) + 4 (l / 16) + e].  Every wave
   // puts them into its own ring -- row r of a block's 16 at place r ^ key, so that the eight pieces along a row that are read
@@ -327,7 +340,7 @@ struct TileWaveK : WaveKTile<TYPE_, FM_, FN_> {
     const uint32_t ring = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_address(smem) + wave * RING);
     // one row of tiles: see rotation_of.  Several: the CTAs of an XCD share A as well as the weights and stay on the same K
     // ([K, N] weights: the CTAs of a row of tiles read neighbouring pieces of the same rows and stay together too)
-    const int rot = a.M <= BM && !NN ? rotation_of(pn, n) : (int)((blockIdx.x & 7) * (uint32_t)n) >> 3;
+    const int rot = a.M <= BM && !NN ? rotation_of(pn, n) : Base::start_of(a, pn, n);
     // load l of a chunk that starts kbytes into the rows and `left` 16-bit units before K's end, pos: where the chunk starts in
     // the ring.  (Pieces past K fetch nothing: zeros arrive and the wait counts stay exact.)
     struct Chunk {

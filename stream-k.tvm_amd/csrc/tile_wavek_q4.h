@@ -94,7 +94,7 @@ struct TileWaveKQ4 : WaveKTile<TYPE_, FM_, FN_> {
     static_for<0, LW>([&](auto l) { off_w[l] = (uint32_t)(16 * l + (lane >> 2)) * ldb_bytes + (uint32_t)((lane & 3) ^ (lane >> 4)) * 16; });
     static_for<0, LS>([&](auto l) { off_s[l] = 64 * l + lane < BN ? (uint32_t)(64 * l + lane) * groups_bytes : OOB_OFFSET; });
     const uint32_t ring = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_address(smem) + wave * RING);
-    const int rot = a.M <= BM ? rotation_of(pn, n) : (int)((blockIdx.x & 7) * (uint32_t)n) >> 3;   // see tile_wavek.h
+    const int rot = a.M <= BM ? rotation_of(pn, n) : Base::start_of(a, pn, n);
     auto group_of = [&](int t) { return (k0 + rotated_iteration(t, rot, n)) * WAVES + wave; };
     // (a group past K fetches nothing: zeros arrive and the wait counts stay exact; it must not carry its offset either)
     struct Where {

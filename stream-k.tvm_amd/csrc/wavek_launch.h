@@ -21,14 +21,14 @@ __global__ __launch_bounds__(P::NT, P::WAVES_PER_EU) void sk_tile_wavek_kernel(t
 struct FlatTile {
   int pm, pn;
 };
-static __device__ __forceinline__ FlatTile flat_tile(int tiles_m) {
-  const int b = blockIdx.x, grid = gridDim.x, x = b & 7, id = x * (grid >> 3) + min(x, grid & 7) + (b >> 3);
+static __device__ __forceinline__ FlatTile flat_tile(int tiles_m, int tiles_n) {
+  const int b = blockIdx.x, grid = tiles_m * tiles_n, x = b & 7, id = x * (grid >> 3) + min(x, grid & 7) + (b >> 3);
   const int pn = (int)((uint32_t)id / (uint32_t)tiles_m);
   return FlatTile{id - pn * tiles_m, pn};
 }
 template <class P>
 static __device__ __forceinline__ void flat_run(const typename P::Args &a, int tiles_m, const void *bias, char *smem) {
-  const FlatTile t = flat_tile(tiles_m);
+  const FlatTile t = flat_tile(tiles_m, (a.N + P::BN - 1) / P::BN);   // (gridDim would be a load from memory)
   typename P::Acc acc;
   if (bias != nullptr) P::prefetch_bias(a, acc, t.pn, bias);
   P::mac(a, acc, t.pm, t.pn, 0, (a.K + P::BK - 1) / P::BK, smem);
@@ -37,19 +37,25 @@ static __device__ __forceinline__ void flat_run(const typename P::Args &a, int t
 template <class P>
 __global__ __launch_bounds__(P::NT, P::WAVES_PER_EU) void sk_tile_wavek_flat_kernel(const half_t *A, const half_t *B, half_t *C, int M, int N,
                                                                                     int K, int lda, int ldb, int ldc, int tiles_m,
-                                                                                    const void *bias, float alpha) {
+                                                                                    uint32_t start_scale, const void *bias, float alpha) {
   __shared__ __attribute__((aligned(1024))) char smem[P::LDS_BYTES];
-  GemmArgs a;
+  WaveKArgs a;
   a.A = A; a.B = B; a.C = C;
   a.M = M; a.N = N; a.K = K;
   a.lda = lda; a.ldb = ldb; a.ldc = ldc;
   a.alpha = alpha; a.scales = nullptr; a.zero = 0; a.groups = 0;
+  a.start_scale = start_scale;
   flat_run<P>(a, tiles_m, bias, smem);
 }
 // the plans it runs
 static inline bool flat_plan(const GemmArgs &a, const DevPlan &p, int bk) {
   return p.sk_tiles == 0 && p.grid == p.total_tiles && p.tiles_m <= 8 && (p.tiles_m == 1 || p.raster == 8) && p.xcd_remap == 1 &&
          p.ipt == (a.K + bk - 1) / bk && a.lda <= 0x7fffffff && a.ldb <= 0x7fffffff && a.ldc <= 0x7fffffff;
+}
+
+static inline uint32_t start_scale(const DevPlan &p) {
+  const uint64_t round = (uint64_t)(p.grid < p.total_tiles ? p.grid : p.total_tiles);
+  return (uint32_t)((((uint64_t)1 << 32) + round - 1) / round);
 }
 
 // ids of a type
@@ -83,14 +89,17 @@ constexpr int wavek_base(int type, bool nn = false) { return (nn ? 600 : 400) + 
   }
 #define SK_WAVEK_LAUNCH(TYPE, ID, FM, FN)                                                                    \
   case ID: {                                                                                                 \
-    typedef TileWaveK<TYPE, FM, FN, WAVEK_NN> P;                                                                       \
+    typedef TileWaveK<TYPE, FM, FN, WAVEK_NN> P;                                                             \
+    WaveKArgs w;                                                                                             \
+    static_cast<GemmArgs &>(w) = a;                                                                          \
+    w.start_scale = start_scale(p);                                                                          \
     if (flat_plan(a, p, P::BK))                                                                              \
       hipLaunchKernelGGL((sk_tile_wavek_flat_kernel<P>), dim3(p.grid), dim3(P::NT), 0, s, a.A, a.B, a.C, a.M, a.N, a.K, (int)a.lda, \
-                         (int)a.ldb, (int)a.ldc, p.tiles_m, bias, a.alpha);                                  \
+                         (int)a.ldb, (int)a.ldc, p.tiles_m, w.start_scale, bias, a.alpha);                    \
     else if (p.sk_tiles == 0)                                                                                \
-      hipLaunchKernelGGL((sk_tile_wavek_kernel<P, false>), dim3(p.grid), dim3(P::NT), 0, s, a, p, ws, bias); \
+      hipLaunchKernelGGL((sk_tile_wavek_kernel<P, false>), dim3(p.grid), dim3(P::NT), 0, s, w, p, ws, bias); \
     else                                                                                                     \
-      hipLaunchKernelGGL((sk_tile_wavek_kernel<P, true>), dim3(p.grid), dim3(P::NT), 0, s, a, p, ws, bias);  \
+      hipLaunchKernelGGL((sk_tile_wavek_kernel<P, true>), dim3(p.grid), dim3(P::NT), 0, s, w, p, ws, bias);  \
     return (int)hipGetLastError();                                                                           \
   }
 #define SK_WAVEK_OCC(TYPE, ID, FM, FN)                                                                                          \

@@ -148,6 +148,33 @@ def test_operator_calls_equal_the_plans_they_replace(sk, dtype, layout):
     sk.workspace_status()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,layout", [("float16", "nt"), ("bfloat16", "nt"), ("float8_e4m3", "nt"), ("q4", "nt"), ("q4_zp", "nt"), ("float16", "nn")])
+def test_equal_rows_give_equal_bits(sk, dtype, layout):
+    """Rows of A that repeat from one row of tiles to the next, on values whose sums round: every tile of a column adds up K in one
+    order, also where a column straddles two XCDs, has more than eight tiles, or a launch several rounds or a fixed split."""
+    import torch
+    gen = torch.Generator(device="cuda").manual_seed(44)
+    normal = lambda *shape: torch.randn(*shape, generator=gen, device="cuda")   # noqa: E731
+    kind = {"float8_e4m3": torch.float8_e4m3fn}.get(dtype) or getattr(torch, dtype, torch.float16)
+    for bm, bn in ((32, 64), (64, 64), (128, 32)):
+        for rows, N, K, split in ((2, 115 * bn, 2048, 1), (3, 41 * bn, 4096, 2), (5, 61 * bn - 8, 1536, 1), (11, 21 * bn, 1024, 1), (7, 90 * bn, 1024, 1)):
+            A = normal(bm, K).to(torch.float16).to(kind).repeat(rows, 1) if kind != torch.float8_e4m3fn else normal(bm, K).repeat(rows, 1).to(kind)
+            plan = sk.make_plan(rows * bm, N, K, dtype, layout, dict(bm=bm, bn=bn, variant=11, schedule="splitk" if split > 1 else "dp", split=split))
+            if dtype.startswith("q4"):
+                Wq = torch.randint(0, 256, (N, K // 2), generator=gen, device="cuda", dtype=torch.uint8)
+                zeros = torch.randint(0, 16, (N, K // 128), generator=gen, device="cuda").half() if dtype == "q4_zp" else None
+                C = sk.streamk_q4(A, Wq, normal(N, K // 128).half(), zeros=zeros, plan=plan)
+            elif kind == torch.float8_e4m3fn:
+                C = sk.streamk_fp8(A, normal(N, K).to(kind), plan=plan, alpha=0.01)
+            else:
+                f = sk.streamk_fp16 if kind == torch.float16 else sk.streamk_bf16
+                C = f(A, normal(*((N, K) if layout == "nt" else (K, N))).to(kind), layout=layout, plan=plan)
+            C = C.view(rows, bm, N)
+            assert (C == C[:1]).all(), (dtype, layout, bm, bn, rows, N, K, split, [(C[r] != C[0]).any(0).sum().item() for r in range(rows)])
+    sk.workspace_status()
+
+
 def test_the_operators_rule(sk):
     """Plans keep the kernels they had; an operator call takes these where the model says so, never for few columns or fix-ups
     that they do not have."""
