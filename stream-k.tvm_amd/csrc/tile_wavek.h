@@ -334,7 +334,8 @@ struct TileWaveK : WaveKTile<TYPE_, FM_, FN_> {
                           : (uint32_t)(8 * (l - 2 * FM) + row8) * ldb_bytes + (uint32_t)kp[l & 1] * 2;
       if constexpr (NN && l >= 2 * FM) {   // 512 / BN rows of K, BN / 8 lanes to a row
         const int k = (l - 2 * FM) * (512 / BN) + lane / (BN / 8), c = lane % (BN / 8) ^ nn_swizzle(k);
-        off[l] = 8 * c < rows_b ? (uint32_t)k * ldb_bytes + (uint32_t)c * 16 : OOB_OFFSET;
+        // (a row past K of a problem shorter than a chunk: k * ldb_bytes may wrap around into the descriptor)
+        off[l] = 8 * c < rows_b && k < a.K ? (uint32_t)k * ldb_bytes + (uint32_t)c * 16 : OOB_OFFSET;
       }
     });
     const uint32_t ring = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_address(smem) + wave * RING);

@@ -175,6 +175,28 @@ def test_equal_rows_give_equal_bits(sk, dtype, layout):
     sk.workspace_status()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("bm,bn", _TILES_NN)
+def test_short_k_over_rows_far_apart(sk, bm, bn):
+    """[K, N] weights with fewer K than a chunk has rows and rows so far apart that 32 of them span 4 GiB: what lies past K is not
+    read, so infinities of the weights reach only the sums that they belong to."""
+    import torch
+    rng = np.random.default_rng(45)
+    ldb, N = 1 << 26, 2 * bn + 8
+    base = torch.zeros(7 * ldb + N, dtype=torch.float16, device="cuda")
+    K = 8
+    B = base.as_strided((K, N), (ldb, 1))
+    values = _small(rng, (K, N))
+    values[0, 3], values[2, bn + 1], values[7, N - 1] = np.inf, -np.inf, np.nan
+    B.copy_(torch.from_numpy(values).half())
+    A = np.abs(_small(rng, (bm + 1, K))) + 1
+    want = torch.from_numpy(A @ values).half()
+    for sched in (dict(schedule="dp"), dict(schedule="dp", grid=2)):
+        plan = sk.make_plan(bm + 1, N, K, "float16", "nn", dict(sched, bm=bm, bn=bn, variant=11))
+        got = sk.streamk_fp16(torch.from_numpy(A).half().cuda(), B, layout="nn", plan=plan).cpu()
+        assert torch.equal(got.nan_to_num(99.0, 98.0, 97.0), want.nan_to_num(99.0, 98.0, 97.0)), (bm, bn, sched)
+
+
 def test_the_operators_rule(sk):
     """Plans keep the kernels they had; an operator call takes these where the model says so, never for few columns or fix-ups
     that they do not have."""
