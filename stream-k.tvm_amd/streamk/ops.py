@@ -140,36 +140,46 @@ def _parse_config(text):
     return out
 
 
-def _too_long(*pitches):
-    """Whether 128 rows of any of these lengths in bytes reach 2 GiB: the kernels for few rows, whose tiles have fewer, take
-    longer rows than those that operators prefer."""
-    return any(p * 128 >= 1 << 31 for p in pitches)
+def _takes_rows(plan, pitch_a, pitch_b):
+    """Whether the plan's tiles take rows of A and of the weights that are so many bytes apart (the library refuses a tile
+    whose rows span 2 GiB)."""
+    return plan.bm * pitch_a < 1 << 31 and plan.bn * pitch_b < 1 << 31
 
 
-def _plan_for(config, M, N, K, dtype, layout, *pitches):
-    """The plan an operator call runs: the registered plan object, or one made from the configuration
-    string for this shape (made once per (shape, type, layout, configuration)).  `pitches`: lengths in bytes of the rows
-    that a tile reads; beyond what every kernel takes, the plain plan."""
-    if config == "" and _too_long(*pitches):
-        config = "raster=0"
-    if config.startswith("#"):
-        plan = _plan_registry.get(config)
-        if plan is None:
-            raise ValueError(f"unknown plan handle {config!r}")
-        return plan
+_LONG_ROWS = "long rows"   # configuration of a call that names none and whose rows are too far apart for the plan of "": see operator_config
+
+
+def _plan_of(config, M, N, K, dtype, layout):
+    """The plan of a configuration string for this shape (made once per (shape, type, layout, configuration))."""
     # (a plan depends on the tuned cache it was made from and on the device it was made for)
     generation, device = _plan_mod.tuned_generation(), torch.cuda.current_device() if torch.cuda.is_available() else -1
     key = (M, N, K, dtype, layout, config, generation, device)
     plan = _plan_cache.get(key)
     if plan is None:
+        named = config not in ("", _LONG_ROWS)
         plan = make_plan(M, N, K, dtype, layout,
-                         _parse_config(config) if config else _plan_mod.operator_config(M, N, K, dtype, layout))
+                         _parse_config(config) if named else _plan_mod.operator_config(M, N, K, dtype, layout, config == _LONG_ROWS))
         if len(_plan_cache) < 4096:
             _plan_cache[key] = plan
             if config == "":   # from now on the native implementation answers calls of this shape
                 with _plan_mod.tuned_lock:
                     if generation == _plan_mod.tuned_generation():
                         _lib.tell_native_operators("sk_torch_add_plan", ctypes.byref(plan), device)
+    return plan
+
+
+def _plan_for(config, M, N, K, dtype, layout, pitch_a=0, pitch_b=0):
+    """The plan an operator call runs: the registered plan object, or the one of the configuration string.  Where rows of A or of
+    the weights (pitch_a, pitch_b bytes apart) are too long for the tile that a call without a configuration takes, the kernel
+    that it takes otherwise, whose tile may have fewer rows."""
+    if config.startswith("#"):
+        plan = _plan_registry.get(config)
+        if plan is None:
+            raise ValueError(f"unknown plan handle {config!r}")
+        return plan
+    plan = _plan_of(config, M, N, K, dtype, layout)
+    if config == "" and not _takes_rows(plan, pitch_a, pitch_b):
+        plan = _plan_of(_LONG_ROWS, M, N, K, dtype, layout)
     return plan
 
 
@@ -309,11 +319,10 @@ def _zero_points(zeros, scales):
     return zeros
 
 
-def _has_plan(config, M, N, K, dtype):
-    """Whether some kernel runs the configuration for all the rows at once."""
+def _has_plan(config, M, N, K, dtype, pitch_a, pitch_b):
+    """Whether some kernel runs the configuration, on rows so far apart, for all the rows at once."""
     try:
-        _plan_for(config, M, N, K, dtype, "nt")
-        return True
+        return _takes_rows(_plan_for(config, M, N, K, dtype, "nt", pitch_a, pitch_b), pitch_a, pitch_b)
     except _lib.StreamKError:
         return False
 
@@ -332,8 +341,14 @@ def _run_q4(A, Wq, scales, zeros, C, zero, group, tiled, config, bias, activatio
     if tuple(scales.shape) != (N, K // group) or not scales.is_contiguous():
         raise ValueError(f"scales must be contiguous [N, K/group]; got {tuple(scales.shape)}")
     _check_out(C, M, N, torch.float16)
-    if M > Q4_MAX_M and (tiled or (zeros is not None and (_too_long(2 * A.stride(0), K // 2) if config == "" else not _has_plan(config, M, N, K, "q4_zp")))) \
-            and not config.startswith("#"):
+    # Prefill-sized calls dequantise first, see below: beyond 1024 rows, and with per-group zero points, whose kernels for many rows
+    # have 64 x 64 tiles, beyond 256 rows from three rounds of them on, beyond 512 from two; 512 x 8192 x 8192 97 us against 103,
+    # 768 x 4096 x 11008 93 / 117, but 512 x 4096 x 4096 41 / 30, 320 x 8192 x 8192 99 / 76.
+    dequantise = config == "" and not tiled and (M > Q4_FUSED_MAX_M or (
+        zeros is not None and M > 4 * Q4_MAX_M and
+        -(-M // 64) * -(-N // 64) > (3 if M <= 8 * Q4_MAX_M else 2) * _plan_mod.num_cus()))
+    if M > Q4_MAX_M and not dequantise and not config.startswith("#") and \
+            (tiled or (zeros is not None and not _has_plan(config, M, N, K, "q4_zp", 2 * A.stride(0), K // 2))):
         # The kernels for the tiled layout take at most 64 rows of A: up to 256 rows one launch per block of 64, and so do
         # configurations that name kernels for few rows.  (Blocks of two rows and more multiply the rounded weights alike; a
         # last block of one row takes the matrix-vector kernels and the unrounded ones.)
@@ -344,15 +359,7 @@ def _run_q4(A, Wq, scales, zeros, C, zero, group, tiled, config, bias, activatio
             return
         if tiled:
             raise ValueError("more than 256 rows of A need the row-major weights (they are dequantised once)")
-        config = ""
-        dequantise = True
-    else:
-        # (with per-group zero points the kernels for many rows have 64 x 64 tiles: beyond 256 rows the pass pays from three
-        # rounds of them on, beyond 512 from two; 512 x 8192 x 8192 97 us against 103, 768 x 4096 x 11008 93 / 117,
-        # but 512 x 4096 x 4096 41 / 30, 320 x 8192 x 8192 99 / 76)
-        dequantise = config == "" and (M > Q4_FUSED_MAX_M or (
-            zeros is not None and M > 4 * Q4_MAX_M and
-            -(-M // 64) * -(-N // 64) > (3 if M <= 8 * Q4_MAX_M else 2) * _plan_mod.num_cus()))
+        config, dequantise = "", True
     if dequantise:
         # Prefill-sized calls: one pass that dequantises the weights (bit-exact device function), then the fp16 tile kernels
         # on them.  The pass costs 26 us for 8192 x 8192 weights, under 7 % of the product from 4096 rows on, where the

@@ -106,20 +106,22 @@ _WAVEK_DTYPES = ("float16", "bfloat16", "float8_e4m3", "float8_e5m2", "int8", "q
 SEARCH_WITH_BYTE_STREAMS = 2
 
 
-def operator_config(M, N, K, dtype, layout):
+def operator_config(M, N, K, dtype, layout, long_rows=False):
     """Configuration of an operator call that names none: the tuned one (None: make_plan finds it), else what
     OPERATOR_VARIANT says, for the types and layouts that have those kernels.  Up to 64 rows of one-byte operands a tuned
     entry from a search that did not have the kernels which stream the weights through LDS does not speak for them: it
     configures the plans that make_plan gives, and an operator call takes the kernels the library chooses (16 x 8192 x 8192 of
-    fp8 14.3 us, by the entry 16.7)."""
+    fp8 14.3 us, by the entry 16.7).  long_rows: without the kernels whose waves stream K on their own, whose tiles may have more
+    rows than the others'."""
     few_bytes = M <= 64 and dtype in ("float8_e4m3", "float8_e5m2", "int8")
-    if not (few_bytes or (dtype in _WAVEK_DTYPES if layout == "nt" and M > 16 else layout == "nn" and dtype in ("float16", "bfloat16"))):
+    wavek = not long_rows and (dtype in _WAVEK_DTYPES if layout == "nt" and M > 16 else layout == "nn" and dtype in ("float16", "bfloat16"))
+    if not (few_bytes or wavek):
         return None
     for d in dict.fromkeys((dtype, _TWIN_OF.get(dtype, dtype))):
         hit = _tuned_entry(M, N, K, d, layout)
         if hit and hit.get("search", 1) >= (SEARCH_WITH_BYTE_STREAMS if few_bytes else 0):
             return None
-    return {"variant": OPERATOR_VARIANT}
+    return {"variant": OPERATOR_VARIANT if wavek else 9}
 
 
 def make_plan(M, N, K, dtype="float16", layout="nt", config=None, cus=None, use_tuned=True, **kw):

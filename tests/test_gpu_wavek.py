@@ -231,10 +231,31 @@ def test_the_operators_rule(sk):
 
 
 @pytest.mark.gpu
-def test_rows_too_long_for_the_preferred_tiles_take_the_plain_plan(sk):
-    """128 rows of 2 GiB and more are refused by the tiles that operators prefer; kernels for fewer rows take them."""
+@pytest.mark.parametrize("dtype", ["float16", "float8_e4m3", "int8"])
+def test_rows_far_apart(sk, dtype):
+    """Rows of A up to 2 GiB of them to a tile run on the plan of the call's shape, natively from the second call on -- one row
+    whatever its stride -- and rows further apart on the kernel that the call takes otherwise, whose tile has fewer of them."""
     import sys
+    import torch
+    from test_torch_ops import _calls_of
+    rng = np.random.default_rng(46)
     plan_for = sys.modules["streamk.ops"]._plan_for
-    name = lambda *pitches: sk.kernel_name(plan_for("", 100, 3840, 4096, "float16", "nt", *pitches).kernel_id)   # noqa: E731
-    assert name(8192, 8192).startswith("wavek_") and name(8192, (1 << 24) - 2).startswith("wavek_")
-    assert not name(8192, 1 << 24).startswith("wavek_") and not name(1 << 24, 8192).startswith("wavek_")
+    kind = {"float8_e4m3": torch.float8_e4m3fn}.get(dtype) or getattr(torch, dtype)
+    size, op = torch.empty(0, dtype=kind).element_size(), getattr(torch.ops.streamk, {"float16": "gemm_f16", "int8": "gemm_i8"}.get(dtype, "gemm_f8"))
+    for M, N, K in ((1, 1024, 1024), (24, 20480, 3072)):
+        A, B = _small(rng, (M, K)), _small(rng, (N, K))
+        want, dB = _rounded(torch, A @ B.T, dtype), torch.from_numpy(B).float().cuda().to(kind)
+        usual = plan_for("", M, N, K, dtype, "nt")
+        most = (1 << 31) // (usual.bm * size)
+        for lda, native in ((most - 16, True), (most, M == 1)):
+            lda -= 16 if M == 1 else 0   # (the library looks at the stride of a single row too)
+            dA = torch.empty((M - 1) * lda + K, dtype=torch.uint8 if size == 1 else kind, device="cuda").view(kind).as_strided((M, K), (lda, 1))
+            dA.copy_(torch.from_numpy(A).float().cuda().to(kind))
+            args = (dA, dB) + (("nt",) if dtype == "float16" else ())
+            assert torch.equal(op(*args).cpu(), want), (dtype, M, lda)
+            names, got = _calls_of(lambda: op(*args))
+            assert torch.equal(got.cpu(), want) and (len(names) == 1) == native, (dtype, M, lda, names)
+            plan = plan_for("", M, N, K, dtype, "nt", lda * size, K * size)
+            other = sk.make_plan(M, N, K, dtype, "nt", None if dtype == "float16" else {"variant": 9})
+            assert plan.kernel_id == (usual if native else other).kernel_id, (dtype, M, lda)
+            del dA, args, got
