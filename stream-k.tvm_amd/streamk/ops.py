@@ -319,12 +319,23 @@ def _zero_points(zeros, scales):
     return zeros
 
 
+_without_plan = set()   # (configuration, shape, type, generation of the tuned cache) that no kernel runs at once
+
+
 def _has_plan(config, M, N, K, dtype, pitch_a, pitch_b):
-    """Whether some kernel runs the configuration, on rows so far apart, for all the rows at once."""
-    try:
-        return _takes_rows(_plan_for(config, M, N, K, dtype, "nt", pitch_a, pitch_b), pitch_a, pitch_b)
-    except _lib.StreamKError:
+    """Whether some kernel runs the configuration, on rows so far apart, for all the rows at once.  (Asked on every call, and a plan
+    that the library refuses is an exception: where the configuration names none, status -4, is remembered.)"""
+    generation = _plan_mod.tuned_generation()
+    key = (config, M, N, K, dtype, generation)
+    if key in _without_plan:
         return False
+    try:
+        plan = _plan_of(config, M, N, K, dtype, "nt")
+    except _lib.StreamKError as e:
+        if e.status == -4 and len(_without_plan) < 4096:
+            _without_plan.add(key)
+        return False
+    return _takes_rows(plan, pitch_a, pitch_b)
 
 
 def _run_q4(A, Wq, scales, zeros, C, zero, group, tiled, config, bias, activation):

@@ -276,6 +276,23 @@ def test_native_operators_answer_like_the_general_ones(name):
     streamk.workspace_status()
 
 
+def test_a_configuration_without_a_plan_is_asked_for_once(sk, monkeypatch):
+    """Per-group zero points with more than 64 rows ask on every call whether one launch runs the configuration."""
+    import sys
+    ops = sys.modules["streamk.ops"]
+    asked = []
+
+    def make_plan(*args):
+        asked.append(args)
+        raise sk.StreamKError(-4, "no kernel")
+    monkeypatch.setattr(ops, "make_plan", make_plan)
+    monkeypatch.setattr(ops, "_without_plan", set())
+    for _ in range(3):
+        assert not ops._has_plan("schedule=dp", 100, 1024, 1024, "q4_zp", 2048, 512)
+    assert len(asked) == 1
+    assert not ops._has_plan("schedule=dp", 101, 1024, 1024, "q4_zp", 2048, 512) and len(asked) == 2
+
+
 # (two shapes per operator whose plans split tiles: one that the smallest workspace serves, one that it does not)
 _SPLIT_SHAPES = {"gemm_f16": ("float16", (64, 256, 4096), (100, 4096, 8192)), "gemm_bf16": ("bfloat16", (64, 256, 4096), (100, 4096, 8192)),
                  "gemm_f32": ("float32", (16, 256, 2048), (512, 1024, 4096)), "gemm_f8": ("float8_e4m3", (100, 512, 8192), (300, 1024, 16384)),
