@@ -10,7 +10,7 @@ is in it.  Inference only: the GEMM is not recorded by autograd.
 import torch
 
 from . import ops
-from .plan import make_plan
+from .plan import make_plan, operator_config
 
 
 class StreamKLinear(torch.nn.Module):
@@ -39,7 +39,6 @@ class StreamKLinear(torch.nn.Module):
             if weight_format == "q4_zp":
                 self.register_buffer("zeros", torch.zeros(N, K // group, dtype=torch.float16, device=device))
         self.register_buffer("bias", torch.zeros(N, dtype=self.dtype, device=device) if bias else None)
-        self._plans = {}
 
     @classmethod
     def from_linear(cls, linear, *, weight_format="float16", group=128, zero=8, activation=None):
@@ -65,12 +64,12 @@ class StreamKLinear(torch.nn.Module):
         return m
 
     def plan_for(self, M):
-        """The plan a call with M rows runs (what forward's operator call resolves to)."""
-        p = self._plans.get(M)
-        if p is None:
-            dtype = self.weight_format
-            p = self._plans[M] = make_plan(M, self.out_features, self.in_features, dtype, "nt")
-        return p
+        """The plan a call with M rows runs (what forward's operator call resolves to); where that dequantises Q4 weights first,
+        a plan of one launch on the packed ones."""
+        N, K, dtype = self.out_features, self.in_features, self.weight_format
+        if dtype in ("q4", "q4_zp") and ops._dequantises(M, N, dtype == "q4_zp"):
+            return make_plan(M, N, K, dtype, "nt", operator_config(M, N, K, dtype, "nt") if dtype == "q4_zp" else None)
+        return ops._plan_for("", M, N, K, dtype, "nt")
 
     @torch.no_grad()
     def forward(self, x):

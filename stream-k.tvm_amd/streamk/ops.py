@@ -338,6 +338,15 @@ def _has_plan(config, M, N, K, dtype, pitch_a, pitch_b):
     return _takes_rows(plan, pitch_a, pitch_b)
 
 
+def _dequantises(M, N, zero_points):
+    """Whether a call on row-major Q4 weights without a configuration dequantises them first (prefill-sized calls): beyond 1024
+    rows, and with per-group zero points, whose kernels for many rows have 64 x 64 tiles, beyond 256 rows from three rounds of them
+    on, beyond 512 from two; 512 x 8192 x 8192 97 us against 103, 768 x 4096 x 11008 93 / 117, but 512 x 4096 x 4096 41 / 30,
+    320 x 8192 x 8192 99 / 76."""
+    return M > Q4_FUSED_MAX_M or (zero_points and M > 4 * Q4_MAX_M and
+                                  -(-M // 64) * -(-N // 64) > (3 if M <= 8 * Q4_MAX_M else 2) * _plan_mod.num_cus())
+
+
 def _run_q4(A, Wq, scales, zeros, C, zero, group, tiled, config, bias, activation):
     if zeros is not None:
         zeros = _zero_points(zeros, scales)  # (row-major like the scales also where the weights are tiled)
@@ -352,12 +361,7 @@ def _run_q4(A, Wq, scales, zeros, C, zero, group, tiled, config, bias, activatio
     if tuple(scales.shape) != (N, K // group) or not scales.is_contiguous():
         raise ValueError(f"scales must be contiguous [N, K/group]; got {tuple(scales.shape)}")
     _check_out(C, M, N, torch.float16)
-    # Prefill-sized calls dequantise first, see below: beyond 1024 rows, and with per-group zero points, whose kernels for many rows
-    # have 64 x 64 tiles, beyond 256 rows from three rounds of them on, beyond 512 from two; 512 x 8192 x 8192 97 us against 103,
-    # 768 x 4096 x 11008 93 / 117, but 512 x 4096 x 4096 41 / 30, 320 x 8192 x 8192 99 / 76.
-    dequantise = config == "" and not tiled and (M > Q4_FUSED_MAX_M or (
-        zeros is not None and M > 4 * Q4_MAX_M and
-        -(-M // 64) * -(-N // 64) > (3 if M <= 8 * Q4_MAX_M else 2) * _plan_mod.num_cus()))
+    dequantise = config == "" and not tiled and _dequantises(M, N, zeros is not None)
     if M > Q4_MAX_M and not dequantise and not config.startswith("#") and \
             (tiled or (zeros is not None and not _has_plan(config, M, N, K, "q4_zp", 2 * A.stride(0), K // 2))):
         # The kernels for the tiled layout take at most 64 rows of A: up to 256 rows one launch per block of 64, and so do
@@ -372,8 +376,7 @@ def _run_q4(A, Wq, scales, zeros, C, zero, group, tiled, config, bias, activatio
             raise ValueError("more than 256 rows of A need the row-major weights (they are dequantised once)")
         config, dequantise = "", True
     if dequantise:
-        # Prefill-sized calls: one pass that dequantises the weights (bit-exact device function), then the fp16 tile kernels
-        # on them.  The pass costs 26 us for 8192 x 8192 weights, under 7 % of the product from 4096 rows on, where the
+        # One pass that dequantises the weights (bit-exact device function), then the fp16 tile kernels on them.  The pass costs 26 us for 8192 x 8192 weights, under 7 % of the product from 4096 rows on, where the
         # fused Q4 tile kernels are behind the four-wave fp16 kernel.  The buffer is kept per stream, allocated on first use;
         # with per-group zero points it is the call's own.
         W = (_staging(N * K * 2, A.device).view(torch.float16)[:N * K].view(N, K) if zeros is None

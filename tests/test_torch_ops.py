@@ -276,6 +276,41 @@ def test_native_operators_answer_like_the_general_ones(name):
     streamk.workspace_status()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ["float16", "bfloat16", "q4", "q4_zp"])
+def test_a_layers_plan_is_what_its_call_runs(sk, fmt, monkeypatch):
+    """StreamKLinear.plan_for against the plan that forward's operator call asks for, on either side of 16, 64, 128, 256 and 512
+    rows; a plan of the layer's own type also where forward dequantises the weights first."""
+    import sys
+    import torch
+    ops = sys.modules["streamk.ops"]
+    layer = sk.StreamKLinear(1024, 3584, weight_format=fmt, device="cuda")
+    sk.plan.invalidate_tuned_cache()   # (a call goes through Python until its plan is known)
+    asked, plan_for = [], ops._plan_for
+
+    def recorded(*args):
+        asked.append(plan_for(*args))
+        return asked[-1]
+    for M in (1, 4, 17, 40, 64, 65, 128, 200, 257, 520, 1100):
+        with monkeypatch.context() as m:
+            m.setattr(ops, "_plan_for", recorded)
+            layer(torch.zeros(M, 1024, dtype=layer.dtype, device="cuda"))
+        plan, ran = layer.plan_for(M), asked[-1]
+        if M == 1100 and fmt in ("q4", "q4_zp"):
+            assert ran.dtype != plan.dtype and (plan.M, plan.N, plan.K) == (M, 3584, 1024)
+        else:
+            assert (plan.kernel_id, plan.grid, plan.dtype) == (ran.kernel_id, ran.grid, ran.dtype), (fmt, M)
+    # the plan of a launch with zero points that the operator would not take leaves its way alone
+    if fmt == "q4_zp":
+        x = torch.randn(520, 1024, device="cuda").half()
+        wide = sk.StreamKLinear(1024, 64 * 300, weight_format=fmt, device="cuda")
+        wide.scales.fill_(1.0)
+        first = wide(x)
+        wide.plan_for(520)
+        names, again = _calls_of(lambda: wide(x))
+        assert "gemm_q4_general" in names and torch.equal(first, again)
+
+
 def test_a_configuration_without_a_plan_is_asked_for_once(sk, monkeypatch):
     """Per-group zero points with more than 64 rows ask on every call whether one launch runs the configuration."""
     import sys
