@@ -378,41 +378,48 @@ static int auto_tile_schedule(int64_t total, int grid, int ipt, int *sk_tiles, i
   return sched;
 }
 
+// A time of the model is of warm weights.  `measured`: what the times of 1 600 sizes of 65 to 1100 rows, their rows multiples of 128
+// bytes, are of it, with the weights from the Infinity Cache (three sets of operands in turn) and from HBM (600 MB of them)
+// (standard deviations 5 to 10 % and 5 to 20 %).
+enum { FROM_CACHE, FROM_HBM };
+struct Times {
+  double us[2];
+};
 struct TileFamily {
   int bm, bn, bk, variant, occ, max_split;  // variant -1: the preferred variant of the tile
-  float tau, gamma, o, phi;
+  float tau, gamma, o, phi, measured[2];
 };
 static const TileFamily kFamilies16[] = {
-    {256, 256, 64, 7, 1, 4, 0.919f, 0.20f, 6.4f, 6.9f},   // four waves, K loop in assembly (K % 64 == 0)
-    {256, 256, 64, 4, 1, 2, 1.080f, 0.20f, 9.3f, 10.0f},  // eight waves, for the other K
-    {128, 128, 64, 4, 2, 4, 0.497f, 0.47f, 4.9f, 5.1f},
-    {128, 128, 32, 5, 2, 4, 0.218f, 0.89f, 3.8f, 4.5f},   // four stages of 32 (NT only)
-    {64, 128, 32, 5, 3, 4, 0.154f, 0.89f, 3.5f, 3.2f},
-    {128, 256, 64, 4, 1, 4, 0.689f, 1.00f, 6.0f, 5.9f},
-    {256, 128, 64, 4, 1, 4, 0.685f, 0.20f, 5.3f, 5.8f},
+    {256, 256, 64, 7, 1, 4, 0.919f, 0.20f, 6.4f, 6.9f, {1.08f, 1.12f}},   // four waves, K loop in assembly (K % 64 == 0)
+    {256, 256, 64, 4, 1, 2, 1.080f, 0.20f, 9.3f, 10.0f, {1.08f, 1.12f}},  // eight waves, for the other K
+    {128, 128, 64, 4, 2, 4, 0.497f, 0.47f, 4.9f, 5.1f, {0.93f, 1.06f}},
+    {128, 128, 32, 5, 2, 4, 0.218f, 0.89f, 3.8f, 4.5f, {1.00f, 1.21f}},   // four stages of 32 (NT only)
+    {64, 128, 32, 5, 3, 4, 0.154f, 0.89f, 3.5f, 3.2f, {1.01f, 1.17f}},
+    {128, 256, 64, 4, 1, 4, 0.689f, 1.00f, 6.0f, 5.9f, {1.06f, 1.25f}},
+    {256, 128, 64, 4, 1, 4, 0.685f, 0.20f, 5.3f, 5.8f, {1.02f, 1.13f}},
 };
 // one-byte operands (BK = 128), fitted the same way to 36 shapes each (64 x 128: to 42 shapes with M <= 1024)
 static const TileFamily kFamiliesF8[] = {
-    {256, 256, 128, -1, 1, 4, 0.934f, 1.00f, 8.8f, 6.1f},
-    {128, 128, 128, -1, 2, 2, 0.435f, 0.52f, 6.3f, 6.6f},
-    {128, 256, 128, -1, 1, 2, 0.580f, 0.20f, 9.3f, 6.7f},
-    {256, 128, 128, -1, 1, 2, 0.608f, 1.00f, 7.2f, 7.8f},
-    {64, 128, 128, -1, 2, 2, 0.335f, 0.46f, 4.3f, 6.5f},
-    {128, 128, 64, 5, 2, 4, 0.218f, 0.88f, 2.3f, 11.0f},  // four stages of 64 (fitted to 48 shapes with M <= 1024)
-    {64, 128, 64, 5, 3, 4, 0.135f, 1.00f, 2.9f, 8.6f},
+    {256, 256, 128, -1, 1, 4, 0.934f, 1.00f, 8.8f, 6.1f, {1.05f, 1.14f}},
+    {128, 128, 128, -1, 2, 2, 0.435f, 0.52f, 6.3f, 6.6f, {1.00f, 1.20f}},
+    {128, 256, 128, -1, 1, 2, 0.580f, 0.20f, 9.3f, 6.7f, {1.10f, 1.34f}},
+    {256, 128, 128, -1, 1, 2, 0.608f, 1.00f, 7.2f, 7.8f, {0.95f, 1.17f}},
+    {64, 128, 128, -1, 2, 2, 0.335f, 0.46f, 4.3f, 6.5f, {0.89f, 1.08f}},
+    {128, 128, 64, 5, 2, 4, 0.218f, 0.88f, 2.3f, 11.0f, {1.06f, 1.33f}},  // four stages of 64 (fitted to 48 shapes with M <= 1024)
+    {64, 128, 64, 5, 3, 4, 0.135f, 1.00f, 2.9f, 8.6f, {1.10f, 1.37f}},
 };
 static const TileFamily kFamiliesI8[] = {
-    {256, 256, 128, -1, 1, 4, 0.876f, 0.20f, 13.3f, 4.2f},
-    {128, 128, 128, -1, 2, 2, 0.531f, 0.52f, 2.3f, 6.4f},
-    {128, 256, 128, -1, 1, 2, 0.674f, 0.20f, 6.5f, 6.5f},
-    {256, 128, 128, -1, 1, 2, 0.700f, 1.00f, 4.9f, 6.5f},
-    {64, 128, 128, -1, 2, 2, 0.392f, 0.39f, 3.3f, 4.0f},
-    {128, 128, 64, 5, 2, 4, 0.222f, 0.77f, 4.7f, 3.9f},   // four stages of 64 (fitted to 48 shapes with M <= 1024)
-    {64, 128, 64, 5, 3, 4, 0.143f, 0.88f, 4.0f, 4.1f},
+    {256, 256, 128, -1, 1, 4, 0.876f, 0.20f, 13.3f, 4.2f, {1.06f, 1.09f}},
+    {128, 128, 128, -1, 2, 2, 0.531f, 0.52f, 2.3f, 6.4f, {1.33f, 1.53f}},
+    {128, 256, 128, -1, 1, 2, 0.674f, 0.20f, 6.5f, 6.5f, {1.16f, 1.40f}},
+    {256, 128, 128, -1, 1, 2, 0.700f, 1.00f, 4.9f, 6.5f, {1.13f, 1.35f}},
+    {64, 128, 128, -1, 2, 2, 0.392f, 0.39f, 3.3f, 4.0f, {0.95f, 1.15f}},
+    {128, 128, 64, 5, 2, 4, 0.222f, 0.77f, 4.7f, 3.9f, {0.98f, 1.25f}},   // four stages of 64 (fitted to 48 shapes with M <= 1024)
+    {64, 128, 64, 5, 3, 4, 0.143f, 0.88f, 4.0f, 4.1f, {1.01f, 1.19f}},
 };
 
 static const KernelInfo *model_pick(int64_t M, int64_t N, int64_t K, int dtype, int layout, int num_cus, int *split,
-                                    int *sched, double *time_us) {
+                                    int *sched, Times *times = nullptr) {
   const TileFamily *fams = kFamilies16;
   int nfams = (int)(sizeof(kFamilies16) / sizeof(kFamilies16[0]));
   if (dtype == SK_F8E4M3 || dtype == SK_F8E5M2) {
@@ -423,6 +430,7 @@ static const KernelInfo *model_pick(int64_t M, int64_t N, int64_t K, int dtype, 
     nfams = (int)(sizeof(kFamiliesI8) / sizeof(kFamiliesI8[0]));
   }
   const KernelInfo *best = nullptr;
+  const TileFamily *best_family = nullptr;
   double best_time = 0;
   bool have_asm = false;
   for (int fi = 0; fi < nfams; ++fi) {
@@ -448,6 +456,7 @@ static const KernelInfo *model_pick(int64_t M, int64_t N, int64_t K, int dtype, 
       const double time = eff * ((double)(ipt / s) * f.tau * clock + f.o) + (s == 1 ? 0.0 : (s == 2 ? f.phi : 2.0 * f.phi));
       if (!best || time < best_time) {
         best = k;
+        best_family = &f;
         best_time = time;
         *split = s;
         *sched = s > 1 ? SK_SCHED_SPLIT_K : SK_SCHED_DP;
@@ -463,13 +472,14 @@ static const KernelInfo *model_pick(int64_t M, int64_t N, int64_t K, int dtype, 
       const double time = (double)tiles * ipt / num_cus * f.tau * 1.4 + f.o * (double)cdiv(tiles, num_cus) + 2.0 * f.phi;
       if (!best || time < best_time) {
         best = k;
+        best_family = &f;
         best_time = time;
         *split = 1;
         *sched = SK_SCHED_AUTO;
       }
     }
   }
-  *time_us = best_time;
+  for (int from = FROM_CACHE; times && best && from <= FROM_HBM; ++from) times->us[from] = best_time * best_family->measured[from];
   return best;
 }
 
@@ -489,7 +499,7 @@ static const RingFamily kFamiliesRing[] = {{64, 3.9, 0.395, 0.09, 2.6, 2.6, 3.0}
 // 256 to 1024 wide 12.2 / 14.4; K = 2816: 777 wide 14.2 / 14.5, 1024 15.1 / 13.8; K = 3000: 777 wide 23.6 / 18.8; K = 3072:
 // 256 wide 14.2 / 13.3, 1024 16.4 / 14.5; 66 and 128 rows alike).
 static bool ring_pays(int64_t N, int64_t K) { return K >= 2880 || (K >= 2048 && N >= 1536) || (K >= 1536 && N >= 8192); }
-static const KernelInfo *model_pick_ring(int64_t N, int64_t K, int dtype, int num_cus, sk_config *out, double *time_us) {
+static const KernelInfo *model_pick_ring(int64_t N, int64_t K, int dtype, int num_cus, sk_config *out, Times *times = nullptr) {
   const KernelInfo *best = nullptr;
   double best_time = 0;
   int count;
@@ -519,89 +529,119 @@ static const KernelInfo *model_pick_ring(int64_t N, int64_t K, int dtype, int nu
     out->bn = best->bn;
     out->bk = best->bk;
     out->reserved[0] = best->variant + 1;
-    *time_us = best_time;
+    // (measured as in TileFamily; whatever the rows' alignment)
+    if (times) *times = Times{{0.90 * best_time, 0.97 * best_time}};
   }
   return best;
 }
 
 // ---- a middling number of rows: the tiles whose waves stream K on their own (tile_wavek.h, tile_wavek_q4.h) ----
-// Model, fitted to 7 000 timings of every tile and split (16-bit, one-byte and Q4 operands, 20 to 2048 rows, 27 shapes, three sets of
-// operands in turn; mean |log error| 3 to 6 %):
-//     time = start + round (rounds - 1) + (core^4 + memory^4)^(1/4) + split + log2 (log2 of the split)
-//   core    rounds x iterations x (iter + busy x busy CUs / CUs): one CTA per CU, every tile of a round side by side
-//   memory  the operands and C once at 5.9 TB/s, slower where less than five eighths of the CUs are busy
-// The tile it chooses is within 1 % of the fastest of them on average.
+// Model, fitted to 33 000 timings each with the weights from the Infinity Cache (three sets of operands in turn; weights below 85 MB)
+// and from HBM (600 MB of them): 16-bit, one-byte, Q4 and [K, N] weights, 1 to 1100 rows, 200 to 28672 columns, K from 512 to 16384;
+// mean |log error| 4 to 5 and 5 to 9 %:
+//     time = start + round (rounds - 1) + (core^1.6 + memory^1.6)^(1/1.6) + split + log2 (log2 of the split)
+//   core    rounds x iterations x (iter + busy x busy CUs / CUs): one CTA per CU, every tile of a round side by side; longer where
+//           rows of operands are no multiple of 128 bytes, because a wave's pieces then share lines with its neighbours', who drift
+//           away from it in the course of K: `off` of it for rows of 16 KB and proportionally less for shorter ones (half of it for
+//           odd multiples of 64 bytes), and `line` wherever that is so (fp16 63 x 1408 x 15096 on 32 x 32 tiles 49.6 us from HBM
+//           and 34.0 from the cache, 35.9 and 22.4 with K = 15104); shorter by `empty` of the share of its operands that are rows of A past M, which are not fetched
+//   memory  the operands and C once at `rate` TB/s, from HBM the higher the more weight rows a CTA has
 struct WaveKFamily {
   int bm, bn;
-  float start, round, iter, busy, split, log2;
+  float start, round, split, log2;
+  struct {
+    float iter, busy, rate;
+  } k[2];
+};
+struct WaveKRows {
+  float off, line, empty;
 };
 static const WaveKFamily kFamiliesWaveK16[] = {
-    {32, 32, 3.37f, 1.31f, 0.280f, 0.101f, 1.88f, 0.47f},
-    {32, 64, 3.76f, 1.48f, 0.394f, 0.182f, 1.90f, 0.61f},
-    {64, 32, 3.87f, 1.52f, 0.384f, 0.160f, 1.83f, 0.68f},
-    {64, 48, 4.22f, 1.56f, 0.462f, 0.187f, 1.93f, 0.82f},
-    {64, 64, 4.67f, 1.68f, 0.505f, 0.298f, 1.90f, 0.90f},
-    {64, 80, 5.23f, 2.16f, 0.622f, 0.280f, 1.81f, 1.05f},
-    {64, 96, 5.57f, 2.34f, 0.684f, 0.393f, 1.90f, 1.10f},
-    {64, 112, 6.43f, 2.82f, 0.867f, 0.416f, 2.07f, 1.14f},
-    {64, 128, 6.87f, 3.05f, 0.958f, 0.497f, 1.99f, 1.19f},
-    {96, 32, 4.32f, 1.54f, 0.482f, 0.225f, 1.92f, 0.82f},
-    {96, 64, 5.77f, 2.44f, 0.664f, 0.337f, 1.91f, 1.10f},
-    {128, 32, 4.81f, 1.78f, 0.597f, 0.310f, 1.80f, 1.02f},
-    {128, 48, 6.37f, 2.60f, 0.784f, 0.343f, 1.89f, 1.01f},
-    {128, 64, 7.08f, 2.95f, 0.960f, 0.428f, 2.08f, 1.21f},
+    {32, 32, 2.48f, 1.50f, 2.32f, 0.47f, {{0.317f, 0.043f, 9.3f}, {0.419f, 0.018f, 5.8f}}},
+    {32, 64, 2.87f, 1.69f, 2.34f, 0.61f, {{0.431f, 0.111f, 9.0f}, {0.573f, 0.105f, 5.8f}}},
+    {64, 32, 2.98f, 1.74f, 2.27f, 0.68f, {{0.427f, 0.095f, 10.4f}, {0.539f, 0.046f, 5.1f}}},
+    {64, 48, 3.33f, 1.78f, 2.37f, 0.82f, {{0.511f, 0.099f, 9.8f}, {0.676f, 0.019f, 5.7f}}},
+    {64, 64, 3.78f, 1.92f, 2.34f, 0.90f, {{0.553f, 0.133f, 10.0f}, {0.700f, 0.126f, 6.2f}}},
+    {64, 80, 4.34f, 2.47f, 2.25f, 1.05f, {{0.664f, 0.127f, 9.2f}, {0.844f, 0.106f, 6.1f}}},
+    {64, 96, 4.68f, 2.68f, 2.34f, 1.10f, {{0.724f, 0.129f, 9.5f}, {1.056f, 0.000f, 6.5f}}},
+    {64, 112, 5.54f, 3.23f, 2.51f, 1.14f, {{0.782f, 0.295f, 9.2f}, {1.270f, 0.000f, 7.1f}}},
+    {64, 128, 5.98f, 3.49f, 2.43f, 1.19f, {{0.840f, 0.298f, 10.7f}, {1.350f, 0.000f, 7.1f}}},
+    {96, 32, 3.43f, 1.76f, 2.36f, 0.82f, {{0.536f, 0.141f, 11.4f}, {0.687f, 0.030f, 4.8f}}},
+    {96, 64, 4.88f, 2.79f, 2.35f, 1.10f, {{0.704f, 0.126f, 10.0f}, {0.956f, 0.000f, 6.0f}}},
+    {128, 32, 3.92f, 2.04f, 2.24f, 1.02f, {{0.698f, 0.117f, 10.2f}, {0.856f, 0.032f, 4.9f}}},
+    {128, 48, 5.48f, 2.97f, 2.33f, 1.01f, {{0.877f, 0.095f, 9.9f}, {1.016f, 0.106f, 6.0f}}},
+    {128, 64, 6.19f, 3.37f, 2.52f, 1.21f, {{0.824f, 0.276f, 8.9f}, {1.241f, 0.000f, 6.0f}}},
 };
-// [K, N] weights: 2 000 timings, 1 to 1024 rows, 18 shapes (mean |log error| 7 to 10 %)
+// [K, N] weights
 static const WaveKFamily kFamiliesWaveKNN[] = {
-    {32, 32, 3.13f, 1.08f, 0.448f, 0.154f, 1.71f, 0.62f},
-    {32, 64, 3.58f, 1.44f, 0.549f, 0.163f, 1.57f, 0.76f},
-    {32, 128, 4.54f, 2.03f, 0.815f, 0.256f, 1.85f, 0.78f},
-    {64, 32, 3.56f, 1.56f, 0.589f, 0.159f, 1.54f, 0.90f},
-    {64, 64, 4.52f, 1.67f, 0.649f, 0.268f, 1.63f, 1.06f},
-    {96, 64, 5.79f, 2.26f, 0.684f, 0.427f, 1.67f, 1.16f},
-    {128, 32, 4.37f, 1.72f, 0.799f, 0.299f, 1.80f, 1.15f},
+    {32, 32, 2.08f, 0.94f, 2.32f, 0.62f, {{0.475f, 0.058f, 6.8f}, {0.629f, 0.014f, 4.5f}}},
+    {32, 64, 2.53f, 1.25f, 2.18f, 0.76f, {{0.559f, 0.076f, 7.3f}, {0.752f, 0.026f, 5.2f}}},
+    {32, 128, 3.49f, 1.76f, 2.46f, 0.78f, {{0.817f, 0.100f, 8.7f}, {0.931f, 0.212f, 5.9f}}},
+    {64, 32, 2.51f, 1.35f, 2.15f, 0.90f, {{0.587f, 0.087f, 6.9f}, {0.736f, 0.059f, 4.7f}}},
+    {64, 64, 3.47f, 1.45f, 2.24f, 1.06f, {{0.668f, 0.106f, 8.5f}, {0.848f, 0.117f, 5.7f}}},
+    {96, 64, 4.74f, 1.96f, 2.28f, 1.16f, {{0.816f, 0.125f, 9.6f}, {0.938f, 0.210f, 6.0f}}},
+    {128, 32, 3.32f, 1.49f, 2.41f, 1.15f, {{0.877f, 0.079f, 6.5f}, {0.950f, 0.111f, 3.6f}}},
 };
 static const WaveKFamily kFamiliesWaveK8[] = {
-    {32, 32, 3.41f, 1.19f, 0.319f, 0.082f, 1.87f, 0.47f},
-    {32, 64, 3.94f, 1.74f, 0.439f, 0.117f, 1.86f, 0.64f},
-    {64, 32, 4.03f, 1.67f, 0.401f, 0.134f, 1.95f, 0.62f},
-    {64, 48, 4.51f, 2.02f, 0.475f, 0.121f, 1.86f, 0.75f},
-    {64, 64, 5.03f, 2.45f, 0.539f, 0.187f, 1.76f, 0.88f},
-    {64, 80, 5.57f, 3.01f, 0.685f, 0.115f, 1.53f, 1.02f},
-    {64, 96, 5.96f, 3.45f, 0.747f, 0.198f, 1.73f, 1.01f},
-    {64, 112, 6.84f, 4.31f, 0.940f, 0.200f, 1.74f, 1.14f},
-    {64, 128, 7.32f, 4.24f, 0.983f, 0.344f, 1.78f, 1.15f},
-    {96, 32, 4.60f, 1.90f, 0.478f, 0.189f, 1.82f, 0.77f},
-    {96, 64, 6.07f, 3.46f, 0.705f, 0.217f, 1.74f, 1.05f},
-    {128, 32, 5.16f, 2.34f, 0.612f, 0.227f, 1.86f, 0.88f},
-    {128, 48, 6.54f, 3.52f, 0.838f, 0.198f, 1.91f, 0.93f},
-    {128, 64, 7.43f, 4.08f, 0.968f, 0.322f, 1.94f, 1.17f},
+    {32, 32, 2.43f, 1.00f, 2.29f, 0.47f, {{0.342f, 0.061f, 8.6f}, {0.409f, 0.047f, 5.2f}}},
+    {32, 64, 2.96f, 1.47f, 2.28f, 0.64f, {{0.430f, 0.141f, 9.0f}, {0.532f, 0.135f, 5.5f}}},
+    {64, 32, 3.05f, 1.41f, 2.37f, 0.62f, {{0.427f, 0.108f, 10.5f}, {0.495f, 0.086f, 5.0f}}},
+    {64, 48, 3.53f, 1.71f, 2.28f, 0.75f, {{0.496f, 0.121f, 10.0f}, {0.591f, 0.103f, 5.4f}}},
+    {64, 64, 4.05f, 2.07f, 2.18f, 0.88f, {{0.531f, 0.138f, 10.1f}, {0.595f, 0.204f, 6.0f}}},
+    {64, 80, 4.59f, 2.54f, 1.95f, 1.02f, {{0.657f, 0.137f, 9.7f}, {0.741f, 0.193f, 6.0f}}},
+    {64, 96, 4.98f, 2.91f, 2.15f, 1.01f, {{0.700f, 0.150f, 9.8f}, {0.946f, 0.097f, 6.6f}}},
+    {64, 112, 5.86f, 3.64f, 2.16f, 1.14f, {{0.849f, 0.176f, 9.9f}, {1.233f, 0.004f, 7.0f}}},
+    {64, 128, 6.34f, 3.58f, 2.20f, 1.15f, {{0.792f, 0.325f, 11.9f}, {1.238f, 0.101f, 7.2f}}},
+    {96, 32, 3.62f, 1.60f, 2.24f, 0.77f, {{0.501f, 0.164f, 13.4f}, {0.571f, 0.159f, 5.2f}}},
+    {96, 64, 5.09f, 2.92f, 2.16f, 1.05f, {{0.666f, 0.161f, 11.0f}, {0.878f, 0.079f, 6.3f}}},
+    {128, 32, 4.18f, 1.98f, 2.28f, 0.88f, {{0.647f, 0.161f, 12.6f}, {0.725f, 0.153f, 5.3f}}},
+    {128, 48, 5.56f, 2.97f, 2.33f, 0.93f, {{0.942f, 0.039f, 10.0f}, {0.981f, 0.152f, 6.7f}}},
+    {128, 64, 6.45f, 3.44f, 2.36f, 1.17f, {{0.869f, 0.220f, 11.7f}, {1.099f, 0.144f, 6.9f}}},
 };
 static const WaveKFamily kFamiliesWaveKQ4[] = {
-    {32, 32, 3.84f, 1.43f, 0.629f, 0.086f, 1.93f, 0.63f},
-    {32, 64, 4.46f, 1.88f, 0.973f, 0.115f, 1.85f, 0.79f},
-    {64, 32, 4.48f, 1.77f, 0.830f, 0.118f, 2.06f, 0.71f},
-    {64, 64, 5.32f, 2.28f, 1.222f, 0.237f, 2.05f, 0.93f},
-    {64, 96, 5.99f, 3.12f, 1.837f, 0.164f, 2.32f, 1.06f},
-    {128, 32, 5.41f, 1.72f, 1.224f, 0.307f, 2.15f, 0.83f},
+    {32, 32, 3.02f, 1.42f, 2.28f, 0.63f, {{0.662f, 0.061f, 11.7f}, {0.684f, 0.065f, 5.0f}}},
+    {32, 64, 3.64f, 1.86f, 2.20f, 0.79f, {{0.947f, 0.109f, 9.6f}, {0.990f, 0.124f, 4.6f}}},
+    {64, 32, 3.66f, 1.76f, 2.41f, 0.71f, {{0.825f, 0.093f, 9.5f}, {0.846f, 0.127f, 4.3f}}},
+    {64, 64, 4.50f, 2.26f, 2.40f, 0.93f, {{1.269f, 0.084f, 6.7f}, {1.322f, 0.076f, 3.9f}}},
+    {64, 96, 5.17f, 3.09f, 2.67f, 1.06f, {{1.680f, 0.186f, 6.7f}, {1.767f, 0.205f, 4.2f}}},
+    {128, 32, 4.59f, 1.71f, 2.50f, 0.83f, {{1.291f, 0.223f, 9.5f}, {1.323f, 0.226f, 3.0f}}},
 };
+static const WaveKRows kRowsWaveK16[2] = {{0.41f, 0.097f, 0.49f}, {0.35f, 0.136f, 0.48f}};
+static const WaveKRows kRowsWaveKNN[2] = {{0.00f, 0.200f, 0.39f}, {0.06f, 0.094f, 0.19f}};
+static const WaveKRows kRowsWaveK8[2] = {{0.36f, 0.093f, 0.36f}, {0.40f, 0.139f, 0.37f}};
+static const WaveKRows kRowsWaveKQ4[2] = {{0.00f, 0.000f, 0.18f}, {0.00f, 0.000f, 0.19f}};   // (rows of whole scale groups: aligned)
+// whether some sets of the weights stay in the Infinity Cache between calls (else the times from HBM alone count)
+static bool from_cache(int64_t N, int64_t K, int dtype) {
+  const bool q4 = dtype == SK_Q4 || dtype == SK_Q4_ZP, b16 = dtype == SK_F16 || dtype == SK_BF16;
+  return (q4 ? 0.52 : (b16 ? 2.0 : 1.0)) * N * K < 85e6;
+}
+static double unaligned_rows(const WaveKRows &m, int64_t pitch) {
+  if (pitch % 128 == 0) return 1;
+  return 1 + m.line + m.off * (pitch % 64 == 0 ? 0.5 : 1.0) * (pitch < 16384 ? pitch / 16384.0 : 1.0);
+}
 static const KernelInfo *model_pick_wavek(int64_t M, int64_t N, int64_t K, int dtype, int layout, int num_cus, sk_config *out,
-                                          double *time_us) {
+                                          Times *times) {
   const bool q4 = dtype == SK_Q4 || dtype == SK_Q4_ZP, one_byte = dtype == SK_F8E4M3 || dtype == SK_F8E5M2 || dtype == SK_I8;
   const WaveKFamily *fams = kFamiliesWaveK16;
   int nfams = (int)(sizeof(kFamiliesWaveK16) / sizeof(kFamiliesWaveK16[0]));
+  const WaveKRows *mem = kRowsWaveK16;
   if (layout == SK_LAYOUT_NN) {
     fams = kFamiliesWaveKNN;
     nfams = (int)(sizeof(kFamiliesWaveKNN) / sizeof(kFamiliesWaveKNN[0]));
+    mem = kRowsWaveKNN;
   } else if (q4) {
     fams = kFamiliesWaveKQ4;
     nfams = (int)(sizeof(kFamiliesWaveKQ4) / sizeof(kFamiliesWaveKQ4[0]));
+    mem = kRowsWaveKQ4;
   } else if (one_byte) {
     fams = kFamiliesWaveK8;
     nfams = (int)(sizeof(kFamiliesWaveK8) / sizeof(kFamiliesWaveK8[0]));
+    mem = kRowsWaveK8;
   }
   const double weight_bytes = q4 ? 0.52 : (one_byte ? 1 : 2), a_bytes = one_byte ? 1 : 2, c_bytes = dtype == SK_I8 ? 4 : 2;
-  const double memory_us = (weight_bytes * N * K + a_bytes * M * K + c_bytes * M * N) / 5.9e6;
+  const double bytes = weight_bytes * N * K + a_bytes * M * K + c_bytes * M * N;
+  const int64_t pitch = layout == SK_LAYOUT_NN ? 2 * N : (one_byte ? K : 2 * K);
+  const bool cached = from_cache(N, K, dtype);
   const KernelInfo *best = nullptr;
   double best_time = 0;
   int count;
@@ -617,14 +657,21 @@ static const KernelInfo *model_pick_wavek(int64_t M, int64_t N, int64_t K, int d
       if (s > 1 && (ipt % s != 0 || tiles * s > num_cus)) continue;
       const double busy = tiles * s < num_cus ? (double)(tiles * s) / num_cus : 1.0;
       const double rounds = (double)cdiv(tiles * s, num_cus);
-      const double core = rounds * ((double)ipt / s) * (f.iter + f.busy * busy), memory = memory_us / (1.6 * busy < 1 ? 1.6 * busy : 1.0);
-      const double c2 = core * core, m2 = memory * memory;
-      const double time = f.start + f.round * (rounds - 1) + sqrt(sqrt(c2 * c2 + m2 * m2)) +
-                          (s == 1 ? 0.0 : f.split + f.log2 * (s == 2 ? 1 : (s == 4 ? 2 : 3)));
-      // (within 2 % the larger tile: fewer bytes of the operands through the caches)
-      if (best && time >= best_time * (f.bm * f.bn > best->bm * best->bn ? 1.02 : (f.bm * f.bn < best->bm * best->bn ? 0.98 : 1.0))) continue;
+      const double past_m = (1 - (double)M / (cdiv(M, f.bm) * f.bm)) * f.bm / (f.bm + (q4 ? 0.5 : 1.0) * f.bn);
+      Times time;
+      for (int from = FROM_CACHE; from <= FROM_HBM; ++from) {
+        const double core = rounds * ((double)ipt / s) * (f.k[from].iter + f.k[from].busy * busy) * unaligned_rows(mem[from], pitch) *
+                            (1 - mem[from].empty * past_m);
+        const double memory = bytes / (f.k[from].rate * 1e6);
+        time.us[from] = f.start + f.round * (rounds - 1) + pow(pow(core, 1.6) + pow(memory, 1.6), 1 / 1.6) +
+                        (s == 1 ? 0.0 : f.split + f.log2 * (s == 2 ? 1 : (s == 4 ? 2 : 3)));
+      }
+      // (both count alike; within 2 % the larger tile: fewer bytes of the operands through the caches)
+      const double both = cached ? sqrt(time.us[FROM_CACHE] * time.us[FROM_HBM]) : time.us[FROM_HBM];
+      if (best && both >= best_time * (f.bm * f.bn > best->bm * best->bn ? 1.02 : (f.bm * f.bn < best->bm * best->bn ? 0.98 : 1.0))) continue;
       best = k;
-      best_time = time;
+      best_time = both;
+      *times = time;
       out->schedule = s == 1 ? SK_SCHED_DP : SK_SCHED_SPLIT_K;
       out->reserved[1] = s > 1 ? s : 0;
     }
@@ -634,78 +681,106 @@ static const KernelInfo *model_pick_wavek(int64_t M, int64_t N, int64_t K, int d
     out->bn = best->bn;
     out->bk = best->bk;
     out->reserved[0] = best->variant + 1;
-    *time_us = best_time;
   }
   return best;
 }
-// Whether a problem whose tile, variant, schedule and grid are open goes to them; `other_us`: the time the other tile kernels'
-// model gives (0: none of them runs it).
-static bool wavek_pays(int64_t M, int64_t N, int64_t K, int dtype, int layout, int num_cus, double wavek_us, double other_us) {
-  if (dtype == SK_Q4 || dtype == SK_Q4_ZP) {
-    // up to 64 rows the general small-M kernels: behind everywhere but with up to 32 rows on more than one round of 64-row tiles
-    // (20 x 28672 x 1280 10.4 us against 13.1, 20 x 20480 x 3072 15.8 / 19.1; 20 x 8192 x 8192 18.4 / 14.9, 64 x 4096 x 4096
-    // 16.0 / 9.4, 64 x 28672 x 1280 25.0 / 17.2)
-    if (M <= 64) return M > 32 || cdiv(N, 64) <= num_cus;
-    if (dtype == SK_Q4_ZP) return true;   // (nothing else runs them in one launch)
-    // the tile kernels that decode into LDS: fitted like the others, 128 x 128 tiles up to 128 rows, 256 x 128 beyond (mean
-    // |log error| 6 and 4 %; by this choice 35 % faster on average over 197 shapes, none slower: 512 x 4096 x 4096 33.4 us / 30.1,
-    // 128 x 8192 x 8192 41.9 / 27.5, 512 x 8192 x 8192 76.0 on the tile kernels, 103 here)
-    const int bm = M > 128 ? 256 : 128, occ = bm == 256 ? 1 : 2;
-    const int64_t tiles = cdiv(M, bm) * cdiv(N, 128), ipt = K / 64;
-    int split = 1;
-    for (int s = 2; tiles < num_cus && s <= 4; s *= 2)
-      if (tiles * s <= (int64_t)num_cus * occ && ipt % s == 0 && ipt / s >= 8) split = s;
-    int skt;
-    const bool even = tiles > num_cus && auto_tile_schedule(tiles, num_cus * occ, (int)ipt, &skt) != SK_SCHED_DP;
-    const double rounds = even ? (double)tiles / num_cus : (double)cdiv(tiles * split, num_cus);
-    const double busy = tiles * split < num_cus ? (double)(tiles * split) / num_cus : 1.0;
-    const double per = bm == 256 ? 0.667 + 0.316 * busy : 0.664 + 0.105 * busy;
-    const double tile_us = (bm == 256 ? 5.24 : 2.45) + rounds * ((double)ipt / split) * per +
-                           (split == 1 ? 0.0 : (bm == 256 ? 4.8 : 5.0) * (split == 2 ? 1 : 2));
-    return wavek_us < 0.95 * tile_us;
+
+// The kernels that such calls of up to 64 rows (96 on 96 x 32 tiles) take otherwise, fitted to 2 300 of the same timings (mean |log
+// error| 2 to 8 %):
+//     time = start + sqrt(core^2 + memory^2) + (where tiles are split) fixup + share x CTAs per tile
+//   core    iterations of the busiest CTA x (iter + busy x CTAs / CUs)
+//   memory  the operands once at `rate` TB/s, at 15 times the share of the CUs that has a CTA where that is less
+enum RowsOperands { ROWS_16, ROWS_8, ROWS_Q4, ROWS_Q4_ZP, ROWS_NN };
+struct RowsFamily {
+  int operands, bm, bn;
+  struct {
+    float start, iter, busy, rate, fixup, share;
+  } t[2];
+};
+static const RowsFamily kFamiliesRows[] = {
+    {ROWS_8, 32, 32, {{3.09f, 0.471f, 0.329f, 8.00f, 3.89f, 0.32f}, {2.87f, 0.556f, 0.948f, 8.00f, 4.10f, 0.34f}}},
+    {ROWS_8, 32, 64, {{2.79f, 0.044f, 0.948f, 8.00f, 4.00f, 0.00f}, {3.31f, 0.403f, 0.706f, 8.00f, 4.26f, 0.55f}}},
+    {ROWS_8, 64, 32, {{2.84f, 0.587f, 0.106f, 7.56f, 4.81f, 0.17f}, {2.89f, 0.591f, 0.148f, 5.56f, 5.23f, 0.16f}}},
+    {ROWS_8, 64, 64, {{3.55f, 0.000f, 1.217f, 8.00f, 4.00f, 0.00f}, {4.64f, 0.441f, 0.812f, 8.00f, 4.17f, 0.28f}}},
+    {ROWS_16, 32, 32, {{2.61f, 0.248f, 0.113f, 8.00f, 2.87f, 0.35f}, {2.30f, 0.381f, 0.320f, 8.00f, 3.30f, 0.34f}}},
+    {ROWS_16, 32, 64, {{2.79f, 0.000f, 0.889f, 8.00f, 4.00f, 0.00f}, {3.66f, 0.556f, 0.440f, 8.00f, 4.00f, 0.00f}}},
+    {ROWS_16, 64, 32, {{3.22f, 0.411f, 0.024f, 6.27f, 3.92f, 0.33f}, {3.35f, 0.397f, 0.000f, 4.63f, 4.28f, 0.31f}}},
+    {ROWS_16, 64, 64, {{3.47f, 0.000f, 1.020f, 8.00f, 4.00f, 0.00f}, {5.24f, 0.372f, 0.779f, 8.00f, 4.00f, 0.00f}}},
+    {ROWS_16, 96, 32, {{3.85f, 0.819f, 0.000f, 6.33f, 4.00f, 0.00f}, {4.09f, 0.926f, 0.000f, 5.68f, 4.00f, 0.00f}}},
+    {ROWS_NN, 128, 128, {{2.38f, 0.458f, 0.430f, 6.66f, 0.69f, 1.45f}, {2.36f, 0.635f, 0.430f, 8.00f, 0.93f, 1.52f}}},
+    {ROWS_Q4, 32, 64, {{4.52f, 0.368f, 0.217f, 4.53f, 3.53f, 0.47f}, {4.41f, 0.469f, 0.341f, 5.83f, 3.54f, 0.48f}}},
+    {ROWS_Q4, 64, 64, {{4.99f, 0.849f, 0.256f, 5.09f, 4.49f, 1.11f}, {5.37f, 0.816f, 0.353f, 5.05f, 4.62f, 1.12f}}},
+    {ROWS_Q4_ZP, 32, 64, {{5.15f, 0.448f, 0.000f, 3.24f, 3.23f, 0.54f}, {5.28f, 0.504f, 0.352f, 5.44f, 3.37f, 0.52f}}},
+    {ROWS_Q4_ZP, 64, 64, {{5.42f, 0.756f, 0.420f, 4.84f, 5.17f, 1.17f}, {5.90f, 0.747f, 0.512f, 4.96f, 5.38f, 1.16f}}},
+};
+static bool rows_times(const KernelInfo &k, const sk_plan &p, int num_cus, Times *times) {
+  const bool zp = p.dtype == SK_Q4_ZP, q4 = zp || p.dtype == SK_Q4, b16 = p.dtype == SK_F16 || p.dtype == SK_BF16;
+  const bool nn = p.layout == SK_LAYOUT_NN;
+  const int operands = q4 ? (zp ? ROWS_Q4_ZP : ROWS_Q4) : (b16 ? (nn ? ROWS_NN : ROWS_16) : ROWS_8);
+  if (!nn && k.variant != (q4 ? 0 : (b16 ? 4 : 8))) return false;
+  const double per_cta = p.streamk_tiles > 0 ? (double)p.total_tiles * p.iters_per_tile / p.grid : (double)cdiv(p.total_tiles, p.grid) * p.iters_per_tile;
+  const double bytes = (q4 ? (zp ? 0.54 : 0.52) : (b16 ? 2 : 1)) * p.N * p.K + (q4 || b16 ? 2.0 : 1.0) * p.M * p.K;
+  const double cus = p.grid < num_cus ? (double)p.grid / num_cus : 1.0;
+  for (const RowsFamily &f : kFamiliesRows) {
+    if (f.operands != operands || f.bm != k.bm || f.bn != k.bn) continue;
+    for (int from = FROM_CACHE; from <= FROM_HBM; ++from) {
+      const auto &t = f.t[from];
+      const double core = per_cta * (t.iter + t.busy * p.grid / num_cus), memory = bytes / ((t.rate < 15 * cus ? t.rate : 15 * cus) * 1e6);
+      times->us[from] = t.start + sqrt(core * core + memory * memory) + (p.streamk_tiles > 0 ? t.fixup + t.share * p.grid / p.total_tiles : 0);
+    }
+    return true;
   }
-  const bool one_byte = dtype == SK_F8E4M3 || dtype == SK_F8E5M2 || dtype == SK_I8;
-  // (16-bit weights that the Infinity Cache does not keep between calls come in slower than the fit's average of both says: 80 to
-  // 128 x 4096 x 11008 of fp16 29.5 to 31.0 us on the ring kernels, 32 to 36 here against a predicted 28)
-  if (M > 64) {
-    const bool from_hbm = !one_byte && 2 * N * K > ((int64_t)(layout == SK_LAYOUT_NN ? 48 : 64) << 20);
-    // ([K, N] weights and 97 to 128 rows, which fill the others' tiles: 128 x 5120 x 5120 29.8 us on those, 35.2 here against a
-    // predicted 24; 72 rows 29.2 / 28.2, 160 rows 34.8 / 31.9)
-    const bool full_rows = layout == SK_LAYOUT_NN && M > 96 && M <= 128;
-    // (More rows than one 128-row tile has: 320 x 4096 x 11008 of fp16 66 us on the kernels before, 50 here, 160 rows 43.4 / 40.6.)
-    const bool one_row = M <= 128 || layout == SK_LAYOUT_NN;
-    if (from_hbm && one_row) return other_us <= 0 || wavek_us < (full_rows ? 0.7 : 0.85) * other_us;
-    // The fit is of a form of these kernels that took 0.5 to 1.8 us longer to add up and store, so a tie is theirs: over 201 sizes
-    // each 22.5 % off fp8's times by this choice, 21.2 % with a margin of 5 %, no size slower (600 x 1500 x 3008 15.6 us / 9.9,
-    // 128 x 8192 x 16384 56.3 / 37.8, 128 x 6144 x 2048 9.7 / 7.0; 1024 x 1024 x 8192 of fp16 34.5 / 26.6); at 1.04 int8
-    // 320 x 11008 x 4096 would go from 25.3 to 29.6.
-    return other_us <= 0 || wavek_us < (one_byte ? 1.0 : (layout == SK_LAYOUT_NN ? 0.92 : 0.97)) * other_us;
+  return false;
+}
+// the Q4 tile kernels that decode into LDS: fitted like the others, 128 x 128 tiles up to 128 rows, 256 x 128 beyond (mean
+// |log error| 6 and 4 %)
+static double q4_tile_us(int64_t M, int64_t N, int64_t K, int num_cus) {
+  const int bm = M > 128 ? 256 : 128, occ = bm == 256 ? 1 : 2;
+  const int64_t tiles = cdiv(M, bm) * cdiv(N, 128), ipt = K / 64;
+  int split = 1;
+  for (int s = 2; tiles < num_cus && s <= 4; s *= 2)
+    if (tiles * s <= (int64_t)num_cus * occ && ipt % s == 0 && ipt / s >= 8) split = s;
+  int skt;
+  const bool even = tiles > num_cus && auto_tile_schedule(tiles, num_cus * occ, (int)ipt, &skt) != SK_SCHED_DP;
+  const double rounds = even ? (double)tiles / num_cus : (double)cdiv(tiles * split, num_cus);
+  const double busy = tiles * split < num_cus ? (double)(tiles * split) / num_cus : 1.0;
+  const double per = bm == 256 ? 0.667 + 0.316 * busy : 0.664 + 0.105 * busy;
+  return (bm == 256 ? 5.24 : 2.45) + rounds * ((double)ipt / split) * per +
+         (split == 1 ? 0.0 : (bm == 256 ? 4.8 : 5.0) * (split == 2 ? 1 : 2));
+}
+// Whether a problem whose tile, variant, schedule and grid are open goes to them: wavek's times against those of the kernel that it
+// takes otherwise (`other`, its plan), with the weights from the cache and from HBM; a call must win by both, because its caller's
+// other weights decide which it is.  The margins cover the models' errors.  On 5 900 measured sizes 43 are behind by more than 3 % in
+// either, by 16 % at most; on 1 050 others 14, by 15 % at most but for one (277 x 1792 x 15616 of bf16, 39.6 us there and 53.0 here
+// from the cache).
+static bool wavek_pays(const sk_plan &other, int num_cus, const Times &wavek) {
+  const KernelInfo *k = kernel_by_id(other.kernel_id);
+  if (!k) return false;
+  const int64_t M = other.M, N = other.N, K = other.K;
+  const int dtype = other.dtype, layout = other.layout;
+  const bool q4 = dtype == SK_Q4 || dtype == SK_Q4_ZP, b16 = dtype == SK_F16 || dtype == SK_BF16, nn = layout == SK_LAYOUT_NN;
+  Times times;
+  double margin;
+  if (k->family == FAMILY_SKINNY || (nn && M <= 64)) {
+    if (!rows_times(*k, other, num_cus, &times)) return false;
+    margin = q4 ? 1.0 : (nn ? 0.97 : 0.95);
+  } else if (dtype == SK_Q4) {
+    times.us[FROM_CACHE] = times.us[FROM_HBM] = q4_tile_us(M, N, K, num_cus);
+    margin = 0.97;
+  } else {
+    // (the tile kernels' rows suffer from their alignment as the wave-K tiles' do, the ring kernels' hardly)
+    sk_config c;
+    int split, sched;
+    const bool ring = k->variant == 9;
+    if (!(ring ? model_pick_ring(N, K, dtype, num_cus, &c, &times) : model_pick(M, N, K, dtype, layout, num_cus, &split, &sched, &times))) return true;
+    const WaveKRows *rows = nn ? kRowsWaveKNN : (b16 ? kRowsWaveK16 : kRowsWaveK8);
+    for (int from = FROM_CACHE; from <= FROM_HBM && !ring; ++from)
+      times.us[from] *= unaligned_rows(rows[from], nn ? 2 * N : (b16 ? 2 * K : K));
+    // ([K, N] weights and up to 128 rows, which fill the others' tiles: 128 x 5120 x 5120 from HBM 30.1 us on those, 35.3 here against a
+    // predicted 29, from the cache 25.2 / 23.1)
+    margin = ring ? 0.97 : (nn ? (M <= 128 ? 0.85 : 0.93) : 0.95);
   }
-  // [K, N] weights and up to 64 rows, against tiles of 128 rows and more (in us, those / these: 16 rows 4096 x 4096 21.5 / 12.0,
-  // 11008 x 4096 32.3 / 19.8, 8192 x 8192 43 / 36, 64 rows 4096 x 11008 44 / 35, 2048 x 2048 15.2 / 6.6): behind only where more than 32
-  // rows take two rounds of 64-wide tiles (33 x 20480 x 3072 40.0 / 46.8, 64 x 28672 x 8192 107 / 125, but 64 x 28672 x 1280 24 / 20)
-  if (layout == SK_LAYOUT_NN) return M <= 32 || cdiv(N, 64) <= num_cus || K < 2048;
-  // 17 to 64 rows against the kernels that stream the weights through LDS.  Times over theirs with the weights from HBM / three sets
-  // in turn, 29 shapes at 17 to 64 rows each:
-  //   more than a round of 64-wide tiles where wider ones need one   20480 x 3072 .86 / .86 (17 to 32 rows, of fp8 .86 / .82; 33 to 64 rows
-  //     of fp16 37.6 us / 27.9, of fp8 .76 / .74), 28672 x 1280 .91 / .94 and .87 / .88 from 33 rows on, 1.01 / .99 before
-  //   33 to 64 rows, few columns   fp16 768 x 1024 .80 / .79, 2048 x 1280 .52 / .49, 4096 x 1024 .85 / .79, 4096 x 8192 .95 / .81; fp8
-  //     1024 x 1024 .81 / .81, 2048 x 5120 .67 / .67, 4096 x 3584 .75 / .75; but fp16 5120 x 5120 1.05 / .83, 4096 x 11008 .97 / .96,
-  //     8192 x 3072 1.10 / .95; fp8 5120 x 5120 1.12 / .90, 14336 x 3072 1.03 / 1.02
-  //   17 to 32 rows   fp16 1504 x 3072 .86 / .84, 2048 x 1280 .65 / .62, 2048 x 8192 .93 / .92; but 1024 x 1024 1.0 / 1.0, 4096 x 1024
-  //     1.06 / .99, 1280 x 16384 1.04 / .86, 5632 x 3072 1.06 / 1.03; fp8 1024 x 1024 .89 / .91, 4096 x 2048 .96 / .90, 8192 x 1280 .87 / .82, 8192 x 3072 .93 / .93; but
-  //     11008 x 2048 1.02 / 1.03, 4096 x 8192 1.08 / .89
-  // One-byte operands of 4096 K-values and a little more stay with the streaming kernels: those are the kernels that operator calls
-  // of that length are known by (4096 x 4096 8.8 us / 7.0).
-  if (one_byte && K >= 4096 && K < 4608) return false;
-  const bool rounds = cdiv(N, 64) > num_cus;
-  if (M <= 32) {
-    if (rounds) return K >= 2048 && cdiv(N, 80) <= num_cus;
-    return one_byte ? K >= 1024 && K < 4096 && N <= 8192 : K >= 1280 && N >= 1280 && N <= 2560 && N * K <= (int64_t)16 << 20;
-  }
-  if (rounds && cdiv(N, 112) <= num_cus) return K >= 1024;
-  if (N <= 4096) return K >= 1024 && N * K <= (int64_t)(one_byte ? 48 : 36) << 20;
-  return !one_byte && N <= 6144 && K >= 1536 && N * K <= (int64_t)24 << 20;
+  return (!from_cache(N, K, dtype) || wavek.us[FROM_CACHE] < margin * times.us[FROM_CACHE]) && wavek.us[FROM_HBM] < margin * times.us[FROM_HBM];
 }
 
 // ---- fp32: tile, schedule and grid, when the caller leaves all three open ----
@@ -826,26 +901,21 @@ extern "C" int sk_make_plan(int64_t M, int64_t N, int64_t K, int dtype, int layo
   const int want_fixup = cfg ? cfg->fixup : SK_FIXUP_AUTO;
   const bool fp32_partials = want_fixup == SK_FIXUP_AUTO || want_fixup == SK_FIXUP_REDUCE || want_fixup == SK_FIXUP_ATOMIC;
   if (open && fp32_partials && by_operator && (layout == SK_LAYOUT_NT ? M > 16 : b16) && (N >= 768 || (dtype == SK_Q4_ZP && !few)) && (b16 || q4_rows || one_byte)) {
-    double wavek_us = 0, other_us = 0;
-    if (cfg) wavek = *cfg; else memset(&wavek, 0, sizeof(wavek));
-    const KernelInfo *k = model_pick_wavek(M, N, K, dtype, layout, num_cus, &wavek, &wavek_us);
-    if (k && !few && !q4_rows) {
-      sk_config ring;
-      int split, sched;
-      if (!(b16 && layout == SK_LAYOUT_NT && M <= 128 && ring_pays(N, K) && model_pick_ring(N, K, dtype, num_cus, &ring, &other_us)))
-        model_pick(M, N, K, dtype, layout, num_cus, &split, &sched, &other_us);
-    }
-    if (k && wavek_pays(M, N, K, dtype, layout, num_cus, wavek_us, other_us)) cfg = &wavek;
+    Times times;
+    wavek = *cfg;
+    sk_plan other;   // what a call takes otherwise, if any kernel runs it in one launch
+    if (model_pick_wavek(M, N, K, dtype, layout, num_cus, &wavek, &times) &&
+        (sk_make_plan(M, N, K, dtype, layout, cfg, num_cus, &other) != SK_OK || wavek_pays(other, num_cus, times)))
+      cfg = &wavek;
   }
   if (open && cfg != &wavek && (b16 || one_byte) && !few && !rows_65_to_96_stream(M, N, dtype, layout, num_cus)) {
-    double model_us = 0;
     if (cfg) modelled = *cfg; else memset(&modelled, 0, sizeof(modelled));
     if (b16 && layout == SK_LAYOUT_NT && M <= 128 && ring_pays(N, K) && fp32_partials &&
-        model_pick_ring(N, K, dtype, num_cus, &modelled, &model_us)) {
+        model_pick_ring(N, K, dtype, num_cus, &modelled)) {
       cfg = &modelled;
     } else {
       int split = 1, model_sched = SK_SCHED_AUTO;
-      if (const KernelInfo *mk = model_pick(M, N, K, dtype, layout, num_cus, &split, &model_sched, &model_us)) {
+      if (const KernelInfo *mk = model_pick(M, N, K, dtype, layout, num_cus, &split, &model_sched)) {
         modelled.bm = mk->bm; modelled.bn = mk->bn; modelled.bk = mk->bk;
         modelled.reserved[0] = mk->variant + 1;
         modelled.schedule = model_sched;

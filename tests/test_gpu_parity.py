@@ -2605,9 +2605,9 @@ def test_one_byte_weights_streamed_through_lds(sk, dtype):
             with pytest.raises(sk.StreamKError):
                 sk.make_plan(1, 256, 4096, dtype, "nt", dict(bm=bm, bn=bn, bk=bk), cus=256)
     assert len(ran) == 7
-    # what an operator call takes without a tuned configuration
+    # what a caller who names their variant alone takes
     for M, N in ((1, 4096), (16, 8192), (16, 8224), (17, 8192), (32, 8224), (33, 4096), (64, 28672)):
-        assert sk.kernel_name(sk.make_plan(M, N, 4096, dtype, "nt", sk.plan.operator_config(M, N, 4096, dtype, "nt"), cus=256).kernel_id).startswith("stream_"), (M, N)
+        assert sk.kernel_name(sk.make_plan(M, N, 4096, dtype, "nt", {"variant": 9}, cus=256).kernel_id).startswith("stream_"), (M, N)
     sk.workspace_status()
 
 

@@ -212,12 +212,19 @@ def test_the_operators_rule(sk):
         assert not wavek(16, 4096, 4096, dtype, "nt", variant=12)
         assert wavek(100, 760, 4096, dtype, "nt", variant=12) == (dtype == "q4_zp")
         assert wavek(4096, 8192, 8192, dtype, "nt", variant=12) == (dtype == "q4_zp")
-    # 17 to 64 rows: few columns, or more than one round of 64-wide tiles where wider ones need one
+    # 17 to 64 rows: few columns, or more than one round of 64-wide tiles where wider ones need one; no depth of K between others is
+    # an exception
     for dtype in ("float8_e4m3", "int8", "float16"):
         assert wavek(48, 2048, 5120, dtype, "nt", variant=12) and wavek(24, 20480, 3072, dtype, "nt", variant=12)
         assert wavek(24, 2048, 2048, dtype, "nt", variant=12) and not wavek(24, 11008, 2048, dtype, "nt", variant=12)
-        assert wavek(24, 1024, 1024, dtype, "nt", variant=12) == wavek(24, 4096, 2048, dtype, "nt", variant=12) == (dtype != "float16")
-        assert wavek(48, 4096, 4096, dtype, "nt", variant=12) == (dtype == "float16")
+        assert wavek(24, 1024, 1024, dtype, "nt", variant=12) == (dtype != "float16")
+        assert all(wavek(48, 4096, K, dtype, "nt", variant=12) for K in (4080, 4096, 4352, 4592, 4608))
+    # K unsplit on few CUs and rows that are no multiple of 128 bytes: 1.3 to 2.3 times as long as on the streaming kernels
+    for dtype in ("float16", "bfloat16"):
+        for shape in ((63, 1408, 15096), (44, 1248, 15056), (50, 1152, 6816), (26, 2056, 3752), (19, 1280, 8448), (45, 2128, 8904), (93, 6448, 4600)):
+            assert not wavek(*shape, dtype, "nt", variant=12), (dtype, shape)
+        # 65 to 96 rows over the width of the 96 x 32 streaming kernel: 80 x 8192 x 8192 38 us on it, 37 on 96 x 32 wave-K tiles, 33 on these
+        assert sk.make_plan(80, 8192, 8192, dtype, "nt", cus=256, use_tuned=False, variant=12).bn == 64
     for dtype in ("float16", "bfloat16"):
         for layout in ("nt", "nn"):
             assert not wavek(100, 4096, 4096, dtype, layout, variant=12, fixup="atomic_c")

@@ -331,7 +331,7 @@ def test_a_configuration_without_a_plan_is_asked_for_once(sk, monkeypatch):
 # (two shapes per operator whose plans split tiles: one that the smallest workspace serves, one that it does not)
 _SPLIT_SHAPES = {"gemm_f16": ("float16", (64, 256, 4096), (100, 4096, 8192)), "gemm_bf16": ("bfloat16", (64, 256, 4096), (100, 4096, 8192)),
                  "gemm_f32": ("float32", (16, 256, 2048), (512, 1024, 4096)), "gemm_f8": ("float8_e4m3", (100, 512, 8192), (300, 1024, 16384)),
-                 "gemm_i8": ("int8", (80, 256, 4096), (300, 1024, 8192)), "gemm_q4": ("q4", (64, 256, 4096), (300, 1024, 8192))}
+                 "gemm_i8": ("int8", (80, 256, 4096), (300, 1024, 16384)), "gemm_q4": ("q4", (64, 256, 4096), (300, 1024, 8192))}
 
 
 def test_split_shapes_need_the_workspaces_they_stand_for(sk):
