@@ -750,8 +750,8 @@ static double q4_tile_us(int64_t M, int64_t N, int64_t K, int num_cus) {
 }
 // Whether a problem whose tile, variant, schedule and grid are open goes to them: wavek's times against those of the kernel that it
 // takes otherwise (`other`, its plan), with the weights from the cache and from HBM; a call must win by both, because its caller's
-// other weights decide which it is.  The margins cover the models' errors.  On 5 900 measured sizes 43 are behind by more than 3 % in
-// either, by 16 % at most; on 1 050 others 14, by 15 % at most but for one (277 x 1792 x 15616 of bf16, 39.6 us there and 53.0 here
+// other weights decide which it is.  The margins cover the models' errors.  On 6 400 measured sizes the choice takes 1.1 % longer than the
+// faster of the two on average, and 46 are behind by more than 3 % in either, by 16 % at most; on 1 050 others 14, by 15 % at most but for one (277 x 1792 x 15616 of bf16, 39.6 us there and 53.0 here
 // from the cache).
 static bool wavek_pays(const sk_plan &other, int num_cus, const Times &wavek) {
   const KernelInfo *k = kernel_by_id(other.kernel_id);
@@ -884,8 +884,7 @@ extern "C" int sk_make_plan(int64_t M, int64_t N, int64_t K, int dtype, int layo
   // weight-streaming kernels take: the cost models choose kernel and split.  The kernels whose waves stream K on their own and
   // the ring kernels add up fp32 partial tiles: a fix-up that adds packed 16-bit partials into C, or exchanges them in 16 bits,
   // is a matter of the other tile kernels.  The former are for a caller who asks for SK_VARIANT_OPERATOR: a plan without it
-  // takes the kernels that plans have taken so far.  (So do products of fewer than 768 columns, for the workspaces their callers
-  // have sized -- 100 x 512 x 8192 of fp8 would take 9 us instead of 17 -- except where nothing else runs them in one launch.)
+  // takes the kernels that plans have taken so far.
   sk_config modelled, wavek;
   const bool q4_rows = dtype == SK_Q4 || dtype == SK_Q4_ZP, b16 = dtype == SK_F16 || dtype == SK_BF16;
   const bool one_byte = dtype == SK_F8E4M3 || dtype == SK_F8E5M2 || dtype == SK_I8;
@@ -900,7 +899,7 @@ extern "C" int sk_make_plan(int64_t M, int64_t N, int64_t K, int dtype, int layo
   }
   const int want_fixup = cfg ? cfg->fixup : SK_FIXUP_AUTO;
   const bool fp32_partials = want_fixup == SK_FIXUP_AUTO || want_fixup == SK_FIXUP_REDUCE || want_fixup == SK_FIXUP_ATOMIC;
-  if (open && fp32_partials && by_operator && (layout == SK_LAYOUT_NT ? M > 16 : b16) && (N >= 768 || (dtype == SK_Q4_ZP && !few)) && (b16 || q4_rows || one_byte)) {
+  if (open && fp32_partials && by_operator && (layout == SK_LAYOUT_NT ? M > 16 : b16) && (b16 || q4_rows || one_byte)) {
     Times times;
     wavek = *cfg;
     sk_plan other;   // what a call takes otherwise, if any kernel runs it in one launch

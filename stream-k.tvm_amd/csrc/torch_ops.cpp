@@ -192,8 +192,7 @@ at::Tensor gemm_q4(const c10::IValue *operands, const at::Tensor *out, const c10
     if (!is_matrix(z, at::kHalf) || !z.is_contiguous() || z.sizes() != scales.sizes()) return {};
     zeros = z.data_ptr();
   }
-  // (per-group zero points and few columns: the general implementation, as before there were kernels for these rows)
-  if (M > 1024 || (zp && M > 64 && N < 768)) return {};
+  if (M > 1024) return {};
   sk_epilogue epi;
   bool used;
   if (!epilogue(a[4], a[5], A, N, at::kHalf, &epi, &used)) return {};

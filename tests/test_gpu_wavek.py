@@ -198,8 +198,8 @@ def test_short_k_over_rows_far_apart(sk, bm, bn):
 
 
 def test_the_operators_rule(sk):
-    """Plans keep the kernels they had; an operator call takes these where the model says so, never for few columns or fix-ups
-    that they do not have."""
+    """Plans keep the kernels they had; an operator call takes these where the models say so, never for fix-ups that they do not
+    have."""
     wavek = lambda *a, **k: sk.kernel_name(sk.make_plan(*a, cus=256, use_tuned=False, **k).kernel_id).startswith("wavek_")   # noqa: E731
     for dtype in ("float16", "bfloat16", "float8_e4m3", "float8_e5m2", "int8", "q4", "q4_zp"):
         for M, N, K in ((100, 4096, 4096), (256, 4096, 4096), (128, 2048, 2048)):
@@ -210,7 +210,7 @@ def test_the_operators_rule(sk):
             else:
                 assert not wavek(M, N, K, dtype, "nt"), (dtype, M, N, K)
         assert not wavek(16, 4096, 4096, dtype, "nt", variant=12)
-        assert wavek(100, 760, 4096, dtype, "nt", variant=12) == (dtype == "q4_zp")
+        assert wavek(100, 760, 4096, dtype, "nt", variant=12) and wavek(100, 256, 4096, dtype, "nt", variant=12)   # few columns too
         assert wavek(4096, 8192, 8192, dtype, "nt", variant=12) == (dtype == "q4_zp")
     # 17 to 64 rows: few columns, or more than one round of 64-wide tiles where wider ones need one; no depth of K between others is
     # an exception

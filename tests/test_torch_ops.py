@@ -217,10 +217,11 @@ def test_native_operators_answer_like_the_general_ones(name):
         ordinary += [(A, *weights, 0.25, "e4m3")]
         other += [(A, *weights, 0.25, "e5m2"), (A.view(torch.uint8), weights[0].view(torch.uint8), 1.0, "e4m3"), (A, *weights, float("nan"), "")]
     if q4:
-        ordinary += [(A, Wq, sc, zp), (A, Wq, sc, None, 3), (torch.randn(80, K, device="cuda").half(), Wq, sc, None)]
+        ordinary += [(A, Wq, sc, zp), (A, Wq, sc, None, 3), (torch.randn(80, K, device="cuda").half(), Wq, sc, None),
+                     (torch.randn(80, K, device="cuda").half(), Wq, sc, zp)]
         other += [(A, Wq, sc, zp.to(torch.uint8)), (A, Wq, sc, zp[:, :2]), (A, Wq, sc, None, 16), (A, Wq, sc, None, 8, 64),
                   (A, Wq.t().contiguous().t(), sc, None), (A, streamk.tile_q4(Wq), sc, None, 8, 128, True),
-                  (torch.randn(80, K, device="cuda").half(), Wq, sc, zp), (torch.randn(1100, K, device="cuda").half(), Wq, sc, None)]
+                  (torch.randn(1100, K, device="cuda").half(), Wq, sc, None)]
 
     def same(a, b):
         return a is b if isinstance(a, type) or isinstance(b, type) else (a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b))
@@ -330,8 +331,8 @@ def test_a_configuration_without_a_plan_is_asked_for_once(sk, monkeypatch):
 
 # (two shapes per operator whose plans split tiles: one that the smallest workspace serves, one that it does not)
 _SPLIT_SHAPES = {"gemm_f16": ("float16", (64, 256, 4096), (100, 4096, 8192)), "gemm_bf16": ("bfloat16", (64, 256, 4096), (100, 4096, 8192)),
-                 "gemm_f32": ("float32", (16, 256, 2048), (512, 1024, 4096)), "gemm_f8": ("float8_e4m3", (100, 512, 8192), (300, 1024, 16384)),
-                 "gemm_i8": ("int8", (80, 256, 4096), (300, 1024, 16384)), "gemm_q4": ("q4", (64, 256, 4096), (300, 1024, 8192))}
+                 "gemm_f32": ("float32", (16, 256, 2048), (512, 1024, 4096)), "gemm_f8": ("float8_e4m3", (64, 256, 8192), (300, 1024, 16384)),
+                 "gemm_i8": ("int8", (64, 256, 8192), (300, 1024, 16384)), "gemm_q4": ("q4", (64, 256, 4096), (300, 1024, 8192))}
 
 
 def test_split_shapes_need_the_workspaces_they_stand_for(sk):
