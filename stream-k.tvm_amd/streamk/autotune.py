@@ -67,13 +67,12 @@ def save_cache(cache, path=None):
         json.dump(cache, f, indent=1, sort_keys=True)
 
 
-def untuned_config(M, N, K, dtype, layout="nt", cus=None):
-    """The configuration that names the plan an operator call runs where nothing has been tuned, or None if no
-    configuration does."""
+def untuned_config(M, N, K, dtype, layout="nt", cus=None, operator=True):
+    """The configuration that names the plan an operator call runs where nothing has been tuned (operator=False: the plan that
+    make_plan gives there), or None if no configuration does."""
     cus = cus or _plan.num_cus()
     try:
-        untuned = {"variant": _plan.OPERATOR_VARIANT} if M <= 64 and dtype in ("float8_e4m3", "float8_e5m2", "int8") else None
-        p = _plan.make_plan(M, N, K, dtype, layout, untuned, cus=cus, use_tuned=False)
+        p = _plan.make_plan(M, N, K, dtype, layout, _plan.untuned_operator_config(M, dtype, layout) if operator else None, cus=cus, use_tuned=False)
     except StreamKError:
         return None
     schedule = {v: k for k, v in SCHEDULES.items()}[p.schedule]
@@ -103,7 +102,8 @@ def candidate_configs(M, N, K, dtype="float16", cus=None, reduce16=True, layout=
     (autotune/streamk_fp16_autotune.py:38-53); here the axes are tile shape, kernel variant,
     schedule, grid and fix-up.  reduce16=False leaves out the candidates that exchange partial sums rounded to 16
     bits (fixup 'reduce16': within the 1e-2 every candidate is held to, but not the fp32 sums of the other fix-ups).  The
-    last candidate is the plan of an untuned call, so that a search never ends behind it."""
+    last candidates are the plan that make_plan gives and the one that an operator call runs where nothing is tuned, so that a
+    search never ends behind them."""
     cus = cus or _plan.num_cus()
     out = []
     f8 = dtype in ("float8_e4m3", "float8_e5m2", "int8")  # one-byte operands
@@ -148,7 +148,7 @@ def candidate_configs(M, N, K, dtype="float16", cus=None, reduce16=True, layout=
     if dtype != "float32" and (M > 16 or layout == "nn"):
         # tiles whose waves stream K on their own (variant 11)
         for (bm, bn) in _WAVEK_NN if layout == "nn" else (_WAVEK_Q4 if dtype in ("q4", "q4_zp") else _WAVEK):
-            if (bm >= 2 * M and bm > 32) or -(-M // bm) * -(-N // bn) > 3 * cus:
+            if (bm >= 2 * M and bm > 64) or -(-M // bm) * -(-N // bn) > 3 * cus:
                 continue
             base = dict(bm=bm, bn=bn, variant=11, raster=8 if M > bm else 0)
             out.append(dict(base, schedule="dp"))
@@ -211,9 +211,10 @@ def candidate_configs(M, N, K, dtype="float16", cus=None, reduce16=True, layout=
             if -(-M // bm) * -(-N // bn) < cus:
                 out.extend(dict(base, schedule="splitk", fixup=fixup) for fixup in ("reduce", "atomic"))
                 out.append(dict(base, schedule="splitk", split=2, fixup="reduce"))
-    untuned = untuned_config(M, N, K, dtype, layout, cus)
-    if untuned is not None and untuned not in out:
-        out.append(untuned)
+    for operator in (False, True):
+        untuned = untuned_config(M, N, K, dtype, layout, cus, operator)
+        if untuned is not None and untuned not in out:
+            out.append(untuned)
     return out
 
 

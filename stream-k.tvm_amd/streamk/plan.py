@@ -106,22 +106,31 @@ _WAVEK_DTYPES = ("float16", "bfloat16", "float8_e4m3", "float8_e5m2", "int8", "q
 SEARCH_WITH_BYTE_STREAMS = 2
 
 
+def untuned_operator_config(M, dtype, layout, long_rows=False):
+    """Configuration of an operator call that names none and whose shape is not tuned: what OPERATOR_VARIANT says, for the types and
+    layouts that have those kernels, else None (the library's heuristic).  long_rows: without the kernels whose waves stream K on
+    their own, whose tiles may have more rows than the others'."""
+    if not long_rows and (dtype in _WAVEK_DTYPES if layout == "nt" and M > 16 else layout == "nn" and dtype in ("float16", "bfloat16")):
+        return {"variant": OPERATOR_VARIANT}
+    if M <= 64 and dtype in ("float8_e4m3", "float8_e5m2", "int8"):
+        return {"variant": OPERATOR_VARIANT if not long_rows else 9}
+    return None
+
+
 def operator_config(M, N, K, dtype, layout, long_rows=False):
-    """Configuration of an operator call that names none: the tuned one (None: make_plan finds it), else what
-    OPERATOR_VARIANT says, for the types and layouts that have those kernels.  Up to 64 rows of one-byte operands a tuned
-    entry from a search that did not have the kernels which stream the weights through LDS does not speak for them: it
-    configures the plans that make_plan gives, and an operator call takes the kernels the library chooses (16 x 8192 x 8192 of
-    fp8 14.3 us, by the entry 16.7).  long_rows: without the kernels whose waves stream K on their own, whose tiles may have more
-    rows than the others'."""
-    few_bytes = M <= 64 and dtype in ("float8_e4m3", "float8_e5m2", "int8")
-    wavek = not long_rows and (dtype in _WAVEK_DTYPES if layout == "nt" and M > 16 else layout == "nn" and dtype in ("float16", "bfloat16"))
-    if not (few_bytes or wavek):
+    """Configuration of an operator call that names none: the tuned one (None: make_plan finds it), else
+    untuned_operator_config's.  Up to 64 rows of one-byte operands a tuned entry from a search that did not have the kernels
+    which stream the weights through LDS does not speak for them: it configures the plans that make_plan gives, and an operator
+    call takes the kernels the library chooses (16 x 8192 x 8192 of fp8 14.3 us, by the entry 16.7)."""
+    config = untuned_operator_config(M, dtype, layout, long_rows)
+    if config is None:
         return None
+    few_bytes = M <= 64 and dtype in ("float8_e4m3", "float8_e5m2", "int8")
     for d in dict.fromkeys((dtype, _TWIN_OF.get(dtype, dtype))):
         hit = _tuned_entry(M, N, K, d, layout)
         if hit and hit.get("search", 1) >= (SEARCH_WITH_BYTE_STREAMS if few_bytes else 0):
             return None
-    return {"variant": OPERATOR_VARIANT if wavek else 9}
+    return config
 
 
 def make_plan(M, N, K, dtype="float16", layout="nt", config=None, cus=None, use_tuned=True, **kw):

@@ -492,8 +492,8 @@ def test_one_byte_plans_keep_their_tuned_entries(monkeypatch):
 
 
 def test_autotune_offers_what_an_untuned_call_runs():
-    """The search space holds the kernels that operator calls take by themselves -- the byte-streaming, the Q4 rows and the
-    ring ones -- and, as its last resort, the very plan of an untuned call."""
+    """The search space holds the kernels that operator calls take by themselves -- the byte-streaming, the Q4 rows, the
+    ring and the wave-K ones -- and, as its last resort, the very plans of an untuned call and of make_plan."""
     import streamk
     at = sys.modules["streamk.autotune"]
 
@@ -503,22 +503,30 @@ def test_autotune_offers_what_an_untuned_call_runs():
     for dtype, kinds, shapes in (("float8_e4m3", ("stream_f8",), ((1, 4096, 4096), (24, 520, 16384), (64, 28672, 8192))), ("int8", ("stream_i8",), ((16, 8192, 8192),)),
                                  ("q4_zp", ("rows_q4zp",), ((4, 11008, 4096), (16, 1024, 16384))), ("q4", ("rows_q4", "stream_q4"), ((4, 11008, 4096), (8, 8192, 8192))),
                                  ("float16", ("_ring_",), ((100, 11008, 4096), (128, 28672, 8192), (100, 777, 3000))), ("bfloat16", ("_ring_",), ((100, 4096, 11008),)),
-                                 ("float16", ("_nt_",), ((1024, 1024, 8192), (3000, 5120, 12288), (8192, 8192, 8192))), ("float32", ("_f32_",), ((16, 4096, 4096),))):
+                                 ("float16", ("_nt_",), ((1024, 1024, 8192), (3000, 5120, 12288), (8192, 8192, 8192))), ("float32", ("_f32_",), ((16, 4096, 4096),)),
+                                 ("bfloat16", ("wavek_",), ((28, 20480, 4096), (300, 4096, 11008), (48, 2048, 5120))), ("q4", ("wavek_",), ((300, 21848, 9600), (24, 4096, 4096))),
+                                 ("q4_zp", ("wavek_",), ((160, 20480, 4096), (100, 512, 4096), (600, 2048, 4096))), ("float16 nn", ("wavek_",), ((16, 4096, 4096), (100, 4096, 4096)))):
+        dtype, layout = dtype.split()[0], "nn" if dtype.endswith(" nn") else "nt"
         for M, N, K in shapes:
             plans = []
-            for c in at.candidate_configs(M, N, K, dtype, cus=256):
+            for c in at.candidate_configs(M, N, K, dtype, cus=256, layout=layout):
                 try:
-                    plans.append(streamk.make_plan(M, N, K, dtype, "nt", c, cus=256))
+                    plans.append(streamk.make_plan(M, N, K, dtype, layout, c, cus=256))
                 except streamk.StreamKError:
                     pass
-            want = streamk.make_plan(M, N, K, dtype, "nt", streamk.plan.operator_config(M, N, K, dtype, "nt") if "8" in dtype else None, cus=256, use_tuned=False)
-            assert named(want) in [named(p) for p in plans], (dtype, M, N, K, named(want))
+            for config in (streamk.plan.untuned_operator_config(M, dtype, layout), None):
+                if config is None and dtype == "q4_zp" and M > 64:
+                    continue   # (a plain plan of them has 64 rows at most)
+                want = streamk.make_plan(M, N, K, dtype, layout, config, cus=256, use_tuned=False)
+                assert named(want) in [named(p) for p in plans], (dtype, M, N, K, named(want))
             for kind in kinds:
                 assert any(kind in streamk.kernel_name(p.kernel_id) for p in plans), (dtype, M, N, K, kind)
     for layout in ("nt", "nn"):   # ([K,N] weights: the last candidate is of that layout)
-        c = at.untuned_config(1000, 1000, 1000, "float16", layout, 256)
-        p, want = (streamk.make_plan(1000, 1000, 1000, "float16", layout, x, cus=256, use_tuned=False) for x in (c, None))
-        assert named(p) == named(want)
+        for operator in (False, True):
+            c = at.untuned_config(1000, 1000, 1000, "float16", layout, 256, operator)
+            p, want = (streamk.make_plan(1000, 1000, 1000, "float16", layout, x, cus=256, use_tuned=False)
+                       for x in (c, streamk.plan.untuned_operator_config(1000, "float16", layout) if operator else None))
+            assert named(p) == named(want)
 
 
 def test_tuned_cache_leaves_the_faster_untuned_plans_alone(monkeypatch):
