@@ -529,6 +529,16 @@ def test_autotune_offers_what_an_untuned_call_runs():
             assert named(p) == named(want)
 
 
+def test_tuned_entries_of_the_wave_k_kernels_are_a_searchs_own(sk):
+    """Entries that name them carry one search's figures: the time, the comparator's and the box's, of one run, and are ahead of
+    the comparator as that run measured it."""
+    at = sys.modules["streamk.autotune"]
+    entries = {k: v for k, v in at.load_cache(at.DEFAULT_CACHE).items() if v["config"].get("variant") == 11}
+    assert len(entries) == 7 and len({v["box_reference_tflops"] for v in entries.values()}) == 1
+    for k, v in entries.items():
+        assert v["search"] >= 3 and v["latency_ms"] < v["ref_latency_ms"], k
+
+
 def test_tuned_cache_leaves_the_faster_untuned_plans_alone(monkeypatch):
     """128 rows of fp16 / bfloat16 and four rows of Q4 at the sizes that had tuned entries for older kernels: the ring and
     the rows kernels."""
