@@ -67,7 +67,7 @@ class StreamKLinear(torch.nn.Module):
         """The plan a call with M rows runs (what forward's operator call resolves to); where that dequantises Q4 weights first,
         a plan of one launch on the packed ones."""
         N, K, dtype = self.out_features, self.in_features, self.weight_format
-        if dtype in ("q4", "q4_zp") and ops._dequantises(M, N, dtype == "q4_zp"):
+        if dtype in ("q4", "q4_zp") and ops._dequantises(M, N, K, dtype == "q4_zp"):
             return make_plan(M, N, K, dtype, "nt", operator_config(M, N, K, dtype, "nt") if dtype == "q4_zp" else None)
         return ops._plan_for("", M, N, K, dtype, "nt")
 

@@ -338,13 +338,17 @@ def _has_plan(config, M, N, K, dtype, pitch_a, pitch_b):
     return _takes_rows(plan, pitch_a, pitch_b)
 
 
-def _dequantises(M, N, zero_points):
+def _dequantises(M, N, K, zero_points):
     """Whether a call on row-major Q4 weights without a configuration dequantises them first (prefill-sized calls): beyond 1024
     rows, and with per-group zero points, whose kernels for many rows have 64 x 64 tiles, beyond 256 rows from three rounds of them
-    on, beyond 512 from two; 512 x 8192 x 8192 97 us against 103, 768 x 4096 x 11008 93 / 117, but 512 x 4096 x 4096 41 / 30,
-    320 x 8192 x 8192 99 / 76."""
-    return M > Q4_FUSED_MAX_M or (zero_points and M > 4 * Q4_MAX_M and
-                                  -(-M // 64) * -(-N // 64) > (3 if M <= 8 * Q4_MAX_M else 2) * _plan_mod.num_cus())
+    on, beyond 512 from two (512 x 8192 x 8192 97 us against 103, 768 x 4096 x 11008 93 / 117, but 512 x 4096 x 4096 41 / 30,
+    320 x 8192 x 8192 99 / 76) or, where the fp16 kernels have a long K, one and a half (517 x 3072 x 9472 62.0 / 66.9,
+    700 x 2560 x 14336 86.4 / 93.8, 849 x 1832 x 8320 51.3 / 56.5, but 656 x 2560 x 2304 .77 of the time; up to 512 rows it may be
+    either, 400 x 5120 x 8192 71.6 / 75.6, 500 x 4096 x 11008 80.3 / 76.0)."""
+    if M > Q4_FUSED_MAX_M or not zero_points or M <= 4 * Q4_MAX_M:
+        return M > Q4_FUSED_MAX_M
+    rounds = 3 if M <= 8 * Q4_MAX_M else (1.5 if K >= 8192 else 2)
+    return -(-M // 64) * -(-N // 64) > rounds * _plan_mod.num_cus()
 
 
 def _run_q4(A, Wq, scales, zeros, C, zero, group, tiled, config, bias, activation):
@@ -361,7 +365,7 @@ def _run_q4(A, Wq, scales, zeros, C, zero, group, tiled, config, bias, activatio
     if tuple(scales.shape) != (N, K // group) or not scales.is_contiguous():
         raise ValueError(f"scales must be contiguous [N, K/group]; got {tuple(scales.shape)}")
     _check_out(C, M, N, torch.float16)
-    dequantise = config == "" and not tiled and _dequantises(M, N, zeros is not None)
+    dequantise = config == "" and not tiled and _dequantises(M, N, K, zeros is not None)
     if M > Q4_MAX_M and not dequantise and not config.startswith("#") and \
             (tiled or (zeros is not None and not _has_plan(config, M, N, K, "q4_zp", 2 * A.stride(0), K // 2))):
         # The kernels for the tiled layout take at most 64 rows of A: up to 256 rows one launch per block of 64, and so do

@@ -312,6 +312,19 @@ def test_a_layers_plan_is_what_its_call_runs(sk, fmt, monkeypatch):
         assert "gemm_q4_general" in names and torch.equal(first, again)
 
 
+def test_where_zero_points_are_dequantised_first(sk, monkeypatch):
+    """Sizes on either side of each limit, as they measured."""
+    import sys
+    ops = sys.modules["streamk.ops"]
+    monkeypatch.setattr(sk.plan, "num_cus", lambda: 256)
+    first = lambda *size: ops._dequantises(*size, True)   # noqa: E731
+    for size in ((512, 8192, 8192), (768, 4096, 11008), (517, 3072, 9472), (700, 2560, 14336), (849, 1832, 8320), (1025, 256, 128)):
+        assert first(*size), size
+    for size in ((512, 4096, 4096), (320, 8192, 8192), (500, 4096, 11008), (510, 6048, 7040), (656, 2560, 2304), (256, 28672, 8192)):
+        assert not first(*size), size
+    assert not ops._dequantises(1024, 28672, 8192, False) and ops._dequantises(1025, 256, 128, False)
+
+
 def test_a_configuration_without_a_plan_is_asked_for_once(sk, monkeypatch):
     """Per-group zero points with more than 64 rows ask on every call whether one launch runs the configuration."""
     import sys
