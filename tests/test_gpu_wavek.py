@@ -21,7 +21,7 @@ def _small(rng, shape, most=2):
 
 
 def _operands(torch, dtype, rng, M, N, K, pad=0, layout="nt"):
-    """A call on A (rows `pad` elements further apart) and weights, and the exact product."""
+    """A call on A (rows `pad` elements further apart, which hold what would show) and weights, and the exact product."""
     if dtype.startswith("q4"):
         A = _small(rng, (M, K))
         q = rng.integers(0, 16, (N, K))
@@ -35,7 +35,7 @@ def _operands(torch, dtype, rng, M, N, K, pad=0, layout="nt"):
         A, W = _small(rng, (M, K)), _small(rng, (N, K))
         kind = {"float8_e4m3": torch.float8_e4m3fn, "float8_e5m2": torch.float8_e5m2}.get(dtype) or getattr(torch, dtype)
         rest = (torch.from_numpy(W if layout == "nt" else W.T.copy()).float().cuda().to(kind),)
-    dA = torch.zeros(M, K + pad, device="cuda").to(kind) if kind != torch.int8 else torch.zeros(M, K + pad, device="cuda", dtype=kind)
+    dA = torch.full((M, K + pad), float("nan"), device="cuda").to(kind) if kind != torch.int8 else torch.full((M, K + pad), 77, device="cuda", dtype=kind)
     dA[:, :K].copy_(torch.from_numpy(A).float().cuda().to(kind))
     import streamk
     f = {"float16": streamk.streamk_fp16, "bfloat16": streamk.streamk_bf16, "int8": streamk.streamk_int8}.get(dtype)
@@ -173,6 +173,55 @@ def test_equal_rows_give_equal_bits(sk, dtype, layout):
             C = C.view(rows, bm, N)
             assert (C == C[:1]).all(), (dtype, layout, bm, bn, rows, N, K, split, [(C[r] != C[0]).any(0).sum().item() for r in range(rows)])
     sk.workspace_status()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,layout", [("float16", "nt"), ("bfloat16", "nt"), ("float8_e4m3", "nt"), ("float8_e5m2", "nt"), ("q4", "nt"), ("q4_zp", "nt"),
+                                          ("float16", "nn"), ("bfloat16", "nn")])
+def test_infinities_and_nan_reach_their_own_sums(sk, dtype, layout):
+    """Infinities and NaN in A, the weights (Q4: the scales) and between A's rows, on tiles that M, N and K do not fill: the result has
+    them where the product has, through whole tiles, fixed splits and both fix-ups."""
+    import torch
+    rng = np.random.default_rng(47)
+    q4 = dtype.startswith("q4")
+    kind = {"float8_e4m3": torch.float8_e4m3fn, "float8_e5m2": torch.float8_e5m2}.get(dtype) or getattr(torch, dtype, torch.float16)
+    odd = (np.nan,) if dtype == "float8_e4m3" else (np.inf, -np.inf, np.nan)   # (e4m3 has no infinities)
+    plain = lambda t: t.float().nan_to_num(1e9, 2e9, 3e9)   # noqa: E731
+    for bm, bn in _TILES_Q4 if q4 else (_TILES if layout == "nt" else _TILES_NN):
+        M, N, K = bm + 3, 2 * bn + (5 if layout == "nt" else 8), 2176 if q4 else (1088 if kind.itemsize == 2 else 2192)
+        A = _small(rng, (M, K))
+        for i, (m, k) in enumerate(((0, 0), (M - 1, K - 1), (bm - 1, K // 2))):
+            A[m, k] = odd[i % len(odd)]
+        dA = torch.full((M, K + 16), float("nan"), device="cuda").to(kind)
+        dA[:, :K].copy_(torch.from_numpy(A).float().cuda().to(kind))
+        if q4:
+            q = rng.integers(0, 16, (N, K))
+            zeros = rng.integers(0, 16, (N, K // 128)) if dtype == "q4_zp" else np.full((N, K // 128), 8)
+            scales = 2.0 ** rng.integers(-4, -1, (N, K // 128))
+            scales[1, 0], scales[N - 1, K // 128 - 1], scales[bn, 2] = odd
+            with np.errstate(invalid="ignore"):
+                W = (q - np.repeat(zeros, 128, 1)) * np.repeat(scales, 128, 1)
+            Wq = torch.from_numpy((q[:, 0::2] | q[:, 1::2] << 4).astype(np.uint8)).cuda()
+            kw = dict(zeros=torch.from_numpy(zeros).half().cuda()) if dtype == "q4_zp" else {}
+            call = lambda **c: sk.streamk_q4(dA[:, :K], Wq, torch.from_numpy(scales).half().cuda(), **kw, **c)   # noqa: E731
+        else:
+            W = _small(rng, (N, K))
+            for i, (n, k) in enumerate(((1, 0), (N - 1, K - 1), (bn, K // 3))):
+                W[n, k] = odd[(i + 1) % len(odd)]
+            dB = torch.from_numpy(W if layout == "nt" else W.T.copy()).float().cuda().to(kind)
+            f = {torch.float16: sk.streamk_fp16, torch.bfloat16: sk.streamk_bf16}.get(kind)
+            call = (lambda **c: f(dA[:, :K], dB, layout=layout, **c)) if f else (lambda **c: sk.streamk_fp8(dA[:, :K], dB, **c))   # noqa: E731
+        with np.errstate(invalid="ignore"):
+            want = _rounded(torch, A @ W.T, dtype)
+        assert want.isnan().any() and want.isfinite().any()
+        for sched in (dict(schedule="dp"), dict(schedule="basic", grid=5, fixup="reduce"), dict(schedule="basic", grid=7, fixup="atomic")):
+            got = call(plan=sk.make_plan(M, N, K, dtype, layout, dict(sched, bm=bm, bn=bn, variant=11))).cpu()
+            assert torch.equal(plain(got), plain(want)), (dtype, layout, bm, bn, sched)
+            sk.workspace_status()
+            # (the accumulating fix-up leaves its buffers at zero: the next call must not see what this one had)
+    call, exact = _operands(torch, dtype, rng, 40, 200, 2048, layout=layout)
+    plan = sk.make_plan(40, 200, 2048, dtype, layout, dict(schedule="basic", grid=7, fixup="atomic", bm=32, bn=32, variant=11))
+    assert torch.equal(call(plan=plan).cpu(), _rounded(torch, exact, dtype))
 
 
 @pytest.mark.gpu
