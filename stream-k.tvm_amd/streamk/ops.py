@@ -146,7 +146,9 @@ def _takes_rows(plan, pitch_a, pitch_b):
     return plan.bm * pitch_a < 1 << 31 and plan.bn * pitch_b < 1 << 31
 
 
-_LONG_ROWS = "long rows"   # configuration of a call that names none and whose rows are too far apart for the plan of "": see operator_config
+# configuration of a call that names none and whose rows are too far apart for the plan of "": see operator_config (no string, so that
+# no caller's is taken for it)
+_LONG_ROWS = ("long rows",)
 
 
 def _plan_of(config, M, N, K, dtype, layout):

@@ -54,6 +54,15 @@ def test_configuration_strings_round_trip(sk):
     assert ops._config_string(None, None, {}) == ""
 
 
+def test_text_that_is_no_configuration_is_refused(sk):
+    import sys
+    ops = sys.modules["streamk.ops"]
+    for text in ("long rows", "splitk", "bm"):
+        for M in (1, 24, 200):
+            with pytest.raises(ValueError):
+                ops._plan_for(text, M, 2048, 2048, "float16", "nt")
+
+
 @pytest.mark.gpu
 def test_operator_equals_direct_c_abi_call(sk):
     """torch.ops.streamk.gemm_f16(A, B) against sk_gemm_f16 called by hand with the same plan, workspace
