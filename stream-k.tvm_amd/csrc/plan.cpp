@@ -899,7 +899,10 @@ extern "C" int sk_make_plan(int64_t M, int64_t N, int64_t K, int dtype, int layo
   }
   const int want_fixup = cfg ? cfg->fixup : SK_FIXUP_AUTO;
   const bool fp32_partials = want_fixup == SK_FIXUP_AUTO || want_fixup == SK_FIXUP_REDUCE || want_fixup == SK_FIXUP_ATOMIC;
-  if (open && fp32_partials && by_operator && (layout == SK_LAYOUT_NT ? M > 16 : b16) && (b16 || q4_rows || one_byte)) {
+  // (per-group zero points, few rows and few columns: the small-M kernels, whose sums a call on the tiled layout of these weights
+  // returns too, bit for bit)
+  const bool as_tiled = dtype == SK_Q4_ZP && few && N < 768;
+  if (open && fp32_partials && by_operator && !as_tiled && (layout == SK_LAYOUT_NT ? M > 16 : b16) && (b16 || q4_rows || one_byte)) {
     Times times;
     wavek = *cfg;
     sk_plan other;   // what a call takes otherwise, if any kernel runs it in one launch

@@ -260,6 +260,8 @@ def test_the_operators_rule(sk):
                 assert not wavek(M, N, K, dtype, "nt"), (dtype, M, N, K)
         assert not wavek(16, 4096, 4096, dtype, "nt", variant=12)
         assert wavek(100, 760, 4096, dtype, "nt", variant=12) and wavek(100, 256, 4096, dtype, "nt", variant=12)   # few columns too
+        if dtype.startswith("q4"):   # (with zero points and few rows the bits of the tiled layout's kernels)
+            assert all(wavek(M, 200, 640, dtype, "nt", variant=12) == (dtype == "q4") for M in (33, 64))
         assert wavek(4096, 8192, 8192, dtype, "nt", variant=12) == (dtype == "q4_zp")
     # 17 to 64 rows: few columns, or more than one round of 64-wide tiles where wider ones need one; no depth of K between others is
     # an exception
