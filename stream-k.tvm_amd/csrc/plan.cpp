@@ -1093,7 +1093,14 @@ extern "C" int sk_make_plan(int64_t M, int64_t N, int64_t K, int dtype, int layo
   // default tile order of the LDS-tiled 16-bit and fp8 kernels: groups of 8 tile rows.  Concurrent CTAs
   // then share B tiles as well as A tiles in the L2s: 0-20 % faster than row-major order on every shape
   // measured (no effect on the fp32 kernels, which keep the reference's order).
-  if (out->raster == 0 && k->family == FAMILY_TILE && dtype != SK_F32 && out->num_block_m > 1) out->raster = 8;
+  if (out->raster == 0 && k->family == FAMILY_TILE && dtype != SK_F32 && out->num_block_m > 1) {
+    out->raster = 8;
+    // (wave-K tiles, more than eight rows of them: groups alike.  The tiles of a short last group share little with each other and
+    // read the weights once more than they need: bf16 277 x 1792 x 15616 on nine rows of 32 x 64 tiles, 8 + 1 rows 52.2 us from the
+    // cache and 52.8 from HBM, 5 + 4 37.5 and 48.1; 530 x 1792 x 4096, nine of 64 x 64, 18.4 / 18.2 and 15.5 / 17.6; 600 x 1536 x 8192,
+    // ten of them, 26.2 / 29.0 and 25.2 / 28.5)
+    if (k->variant == 10 && out->num_block_m > 8) out->raster = (int)cdiv(out->num_block_m, cdiv(out->num_block_m, 8));
+  }
 
   // workspace: status block, fixed-size flag area, fp32 partial tiles
   int64_t ws = 0;

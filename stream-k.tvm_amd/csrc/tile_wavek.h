@@ -36,7 +36,7 @@ namespace sk {
 enum WaveKType { WK_F16 = 0, WK_BF16 = 1, WK_F8E4M3 = 2, WK_F8E5M2 = 3, WK_I8 = 4, WK_Q4 = 5, WK_Q4ZP = 6 };
 
 struct WaveKArgs : GemmArgs {
-  uint32_t start_scale;   // 2^32 / tiles of a round of the launch, rounded up (start_of)
+  uint32_t start_scale;   // 2^32 x tiles of a column in a raster group / tiles of a round of the launch, rounded up (start_of)
 };
 // Q4 weights: with the array of zero points where every group has its own
 struct WaveKQ4Args : WaveKArgs {
@@ -72,11 +72,10 @@ struct WaveKTile {
 
   // The iteration of a segment of n that a tile of column pn starts with: the XCDs' starts are spread over the segment, and a tile takes
   // that of the XCD which holds the first tile of its column -- its own XCD's but where a column straddles two, or goes on in another
-  // group of eight rows.  So all tiles of a column add up K in one order: equal rows of A give equal bits, wherever they stand in it.
-  // (first * start_scale: how far the first tile is into its round of the launch, as a fraction of 2^32)
+  // group of rows.  So all tiles of a column add up K in one order: equal rows of A give equal bits, wherever they stand in it.
+  // (pn * start_scale: how far the first tile is into its round of the launch, as a fraction of 2^32)
   static __device__ __forceinline__ int start_of(const Args &a, int pn, int n) {
-    const uint32_t first = (uint32_t)(pn * min((a.M + BM - 1) / BM, 8));
-    return (int)(((first * a.start_scale) >> 29) * (uint32_t)n >> 3);
+    return (int)((((uint32_t)pn * a.start_scale) >> 29) * (uint32_t)n >> 3);
   }
 
   // c: the wave's sums of all blocks, lane l of block v holding C[16 (v / FN) + l % 16][16 (v % FN) + 4 (l / 16) + e].  Every wave

@@ -55,7 +55,8 @@ static inline bool flat_plan(const GemmArgs &a, const DevPlan &p, int bk) {
 
 static inline uint32_t start_scale(const DevPlan &p) {
   const uint64_t round = (uint64_t)(p.grid < p.total_tiles ? p.grid : p.total_tiles);
-  return (uint32_t)((((uint64_t)1 << 32) + round - 1) / round);
+  const uint64_t group = (uint64_t)(p.raster <= 0 ? 1 : (p.raster < p.tiles_m ? p.raster : p.tiles_m));
+  return (uint32_t)(((group << 32) + round - 1) / round);
 }
 
 // ids of a type

@@ -150,7 +150,8 @@ def candidate_configs(M, N, K, dtype="float16", cus=None, reduce16=True, layout=
         for (bm, bn) in _WAVEK_NN if layout == "nn" else (_WAVEK_Q4 if dtype in ("q4", "q4_zp") else _WAVEK):
             if (bm >= 2 * M and bm > 64) or -(-M // bm) * -(-N // bn) > 3 * cus:
                 continue
-            base = dict(bm=bm, bn=bn, variant=11, raster=8 if M > bm else 0)
+            rows = -(-M // bm)   # (groups alike, as sk_make_plan makes them)
+            base = dict(bm=bm, bn=bn, variant=11, raster=0 if rows == 1 else (8 if rows <= 8 else -(-rows // -(-rows // 8))))
             out.append(dict(base, schedule="dp"))
             out.extend(dict(base, schedule="splitk", split=split, fixup="reduce") for split in (2, 4, 8)
                        if -(-M // bm) * -(-N // bn) * split <= cus)

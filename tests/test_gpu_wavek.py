@@ -288,6 +288,25 @@ def test_the_operators_rule(sk):
     assert sk.make_plan(40, 4096, 4096, "q4_zp", "nt", cus=256, use_tuned=False).kernel_id < 400
 
 
+def test_groups_of_rows_are_alike(sk):
+    """More than eight rows of tiles stand in groups of eight at most that differ by less than one row a group; other kernels and
+    rasters of the caller's as they were."""
+    for bm in (32, 64, 128):
+        for rows in range(1, 60):
+            plan = sk.make_plan(rows * bm, 512, 2048, "float16", "nt", dict(bm=bm, bn=32, variant=11, schedule="dp"), cus=256)
+            groups = -(-rows // 8)
+            if rows <= 8:
+                assert plan.raster == (8 if rows > 1 else 0)
+            else:
+                tail = rows - (groups - 1) * plan.raster
+                assert plan.raster <= 8 and plan.raster - groups < tail <= plan.raster, (bm, rows, plan.raster)
+            assert sk.make_plan(rows * bm, 512, 2048, "float16", "nt", dict(bm=bm, bn=32, variant=11, schedule="dp", raster=3), cus=256).raster == 3
+            if rows * bm > 64:
+                assert sk.make_plan(rows * bm, 512, 2048, "float16", "nt", dict(bm=64, bn=128, schedule="dp"), cus=256).raster in (0, 8)
+    # a call whose rows were eight and one
+    assert sk.make_plan(277, 1792, 15616, "bfloat16", "nt", cus=256, use_tuned=False, variant=12).raster == 5
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["float16", "float8_e4m3", "int8"])
 def test_rows_far_apart(sk, dtype):
