@@ -328,7 +328,8 @@ int sk_gemm_f32(const void *A, const void *B, void *C, int64_t M, int64_t N, int
  * that moves the nibbles through LDS and dequantises them, bit for bit as above, on their way into the fp16
  * stage of the 16x16x32 MFMA loop (256x256, 256x128 or 128x128 tiles; every schedule and fix-up).
  * A plan made with dtype SK_Q4_TILED takes Wq in the tiled layout instead (see sk_q4_tile_host): same
- * results bit for bit, the weights stream faster; at most 64 rows of A per call.
+ * results bit for bit by plans alike, the weights stream faster; at most 64 rows of A per call, any number with a plan of
+ * reserved[0] = 11 or 12 (sk_config).
  */
 int sk_gemm_q4(const void *A, const void *Wq, const void *scales, void *C, int64_t M, int64_t N,
                int64_t K, int64_t lda, int64_t ldc, int group, int zero, const sk_plan *plan,

@@ -333,7 +333,7 @@ struct KernelInfo {
   X(T, BASE + 5, 6, 4) \
   X(T, BASE + 6, 8, 2)
 
-// the same for Q4 weights (tile_wavek_q4.h; dtypes SK_Q4 id, SK_Q4_ZP id + 20):  X(id, blocks of 16 rows of A, of 16 weight rows)
+// the same for Q4 weights (tile_wavek_q4.h; dtypes SK_Q4 id, SK_Q4_ZP id + 20, SK_Q4_TILED id + 40, SK_Q4_ZP_TILED id + 60):  X(id, blocks of 16 rows of A, of 16 weight rows)
 #define SK_TILE_WAVEK_Q4_KERNELS(X) \
   X(520, 2, 2) \
   X(521, 2, 4) \

@@ -38,7 +38,7 @@ int occupancy_tile_wavek(int id) {
     FOR_WAVEK_UNITS(X)
 #undef X
   }
-  if (id >= 520 && id < 560) return occupancy_wavek_q4(id);
+  if (id >= 520 && id < 600) return occupancy_wavek_q4(id);
   return occupancy_tile_q4(id);
 }
 

@@ -33,15 +33,17 @@ __global__ __launch_bounds__(P::NT, P::WAVES_PER_EU) void sk_tile_wavek_q4_flat_
 
 int wavek_q4_kernel_infos(KernelInfo *out, int max) {
   int n = 0;
-#define INFO(id, DT, TYPE, NAME, FM, FN)                                                                                          \
+#define INFO(id, DT, TYPE, TILED, NAME, FM, FN)                                                                                   \
   if (n < max) {                                                                                                                  \
-    typedef TileWaveKQ4<TYPE, FM, FN> P;                                                                                          \
+    typedef TileWaveKQ4<TYPE, FM, FN, TILED> P;                                                                                   \
     out[n++] = KernelInfo{id, FAMILY_TILE, DT, 0, 10, P::BM, P::BN, P::BK, P::NT, P::LDS_TOTAL, P::CTAS_PER_CU, P::TILE_ELEMS, 0, \
                           0, 128, NAME "_" #FM "x" #FN};                                                                          \
   }
-#define X(id, FM, FN)                        \
-  INFO(id, 2, WK_Q4, "wavek_q4", FM, FN)     \
-  INFO(id + 20, 7, WK_Q4ZP, "wavek_q4zp", FM, FN)
+#define X(id, FM, FN)                                    \
+  INFO(id, 2, WK_Q4, false, "wavek_q4", FM, FN)          \
+  INFO(id + 20, 7, WK_Q4ZP, false, "wavek_q4zp", FM, FN) \
+  INFO(id + 40, 4, WK_Q4, true, "wavek_q4t", FM, FN)     \
+  INFO(id + 60, 9, WK_Q4ZP, true, "wavek_q4zpt", FM, FN)
   SK_TILE_WAVEK_Q4_KERNELS(X)
 #undef X
 #undef INFO
@@ -68,7 +70,9 @@ int launch_wavek_q4(int id, const GemmArgs &g, const void *zeros, const DevPlan 
   switch (id) {
 #define X(id_, FM, FN)                                                               \
   case id_: return launch<TileWaveKQ4<WK_Q4, FM, FN>>(a, p, ws, s, bias);            \
-  case id_ + 20: return launch<TileWaveKQ4<WK_Q4ZP, FM, FN>>(a, p, ws, s, bias);
+  case id_ + 20: return launch<TileWaveKQ4<WK_Q4ZP, FM, FN>>(a, p, ws, s, bias);     \
+  case id_ + 40: return launch<TileWaveKQ4<WK_Q4, FM, FN, true>>(a, p, ws, s, bias); \
+  case id_ + 60: return launch<TileWaveKQ4<WK_Q4ZP, FM, FN, true>>(a, p, ws, s, bias);
     SK_TILE_WAVEK_Q4_KERNELS(X)
 #undef X
   }
@@ -78,14 +82,16 @@ int launch_wavek_q4(int id, const GemmArgs &g, const void *zeros, const DevPlan 
 int occupancy_wavek_q4(int id) {
   int occ = 0;
   switch (id) {
-#define OCC(id_, TYPE, FM, FN)                                                                                                     \
+#define OCC(id_, TYPE, TILED, FM, FN)                                                                                              \
   case id_: {                                                                                                                      \
-    typedef TileWaveKQ4<TYPE, FM, FN> P;                                                                                           \
+    typedef TileWaveKQ4<TYPE, FM, FN, TILED> P;                                                                                    \
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, sk_tile_wavek_q4_kernel<P, true>, P::NT, 0) == hipSuccess ? occ : -1; \
   }
-#define X(id_, FM, FN)          \
-  OCC(id_, WK_Q4, FM, FN)       \
-  OCC(id_ + 20, WK_Q4ZP, FM, FN)
+#define X(id_, FM, FN)                   \
+  OCC(id_, WK_Q4, false, FM, FN)         \
+  OCC(id_ + 20, WK_Q4ZP, false, FM, FN)  \
+  OCC(id_ + 40, WK_Q4, true, FM, FN)     \
+  OCC(id_ + 60, WK_Q4ZP, true, FM, FN)
     SK_TILE_WAVEK_Q4_KERNELS(X)
 #undef X
 #undef OCC

@@ -886,7 +886,9 @@ extern "C" int sk_make_plan(int64_t M, int64_t N, int64_t K, int dtype, int layo
   // is a matter of the other tile kernels.  The former are for a caller who asks for SK_VARIANT_OPERATOR: a plan without it
   // takes the kernels that plans have taken so far.
   sk_config modelled, wavek;
-  const bool q4_rows = dtype == SK_Q4 || dtype == SK_Q4_ZP, b16 = dtype == SK_F16 || dtype == SK_BF16;
+  // (the tiled layout of Q4 weights takes what the row-major one does, so that both give the same bits)
+  const int as_rows = dtype == SK_Q4_TILED ? (int)SK_Q4 : (dtype == SK_Q4_ZP_TILED ? (int)SK_Q4_ZP : dtype);
+  const bool q4_rows = as_rows == SK_Q4 || as_rows == SK_Q4_ZP, b16 = dtype == SK_F16 || dtype == SK_BF16;
   const bool one_byte = dtype == SK_F8E4M3 || dtype == SK_F8E5M2 || dtype == SK_I8;
   const bool by_operator = cfg && cfg->reserved[0] == SK_VARIANT_OPERATOR && cfg->bm == 0 && cfg->bn == 0;
   const bool open = !cfg || (cfg->bm == 0 && cfg->bn == 0 && cfg->bk == 0 && (cfg->reserved[0] == 0 || by_operator) &&
@@ -899,15 +901,12 @@ extern "C" int sk_make_plan(int64_t M, int64_t N, int64_t K, int dtype, int layo
   }
   const int want_fixup = cfg ? cfg->fixup : SK_FIXUP_AUTO;
   const bool fp32_partials = want_fixup == SK_FIXUP_AUTO || want_fixup == SK_FIXUP_REDUCE || want_fixup == SK_FIXUP_ATOMIC;
-  // (per-group zero points, few rows and few columns: the small-M kernels, whose sums a call on the tiled layout of these weights
-  // returns too, bit for bit)
-  const bool as_tiled = dtype == SK_Q4_ZP && few && N < 768;
-  if (open && fp32_partials && by_operator && !as_tiled && (layout == SK_LAYOUT_NT ? M > 16 : b16) && (b16 || q4_rows || one_byte)) {
+  if (open && fp32_partials && by_operator && (layout == SK_LAYOUT_NT ? M > 16 : b16) && (b16 || q4_rows || one_byte)) {
     Times times;
     wavek = *cfg;
     sk_plan other;   // what a call takes otherwise, if any kernel runs it in one launch
-    if (model_pick_wavek(M, N, K, dtype, layout, num_cus, &wavek, &times) &&
-        (sk_make_plan(M, N, K, dtype, layout, cfg, num_cus, &other) != SK_OK || wavek_pays(other, num_cus, times)))
+    if (model_pick_wavek(M, N, K, as_rows, layout, num_cus, &wavek, &times) &&
+        (sk_make_plan(M, N, K, as_rows, layout, cfg, num_cus, &other) != SK_OK || wavek_pays(other, num_cus, times)))
       cfg = &wavek;
   }
   if (open && cfg != &wavek && (b16 || one_byte) && !few && !rows_65_to_96_stream(M, N, dtype, layout, num_cus)) {

@@ -21,7 +21,9 @@
 
 namespace sk {
 
-template <int TYPE_, int FM_, int FN_>
+// TILED_: the nibbles in tiles of 16 rows x one scale group, the tiles of 16 rows behind each other.  A load reads one of them, and
+// every lane gets the bytes that it gets from the row-major array: equal plans give equal bits.
+template <int TYPE_, int FM_, int FN_, bool TILED_ = false>
 struct TileWaveKQ4 : WaveKTile<TYPE_, FM_, FN_> {
   typedef WaveKTile<TYPE_, FM_, FN_> Base;
   typedef typename Base::Args Args;
@@ -82,7 +84,9 @@ struct TileWaveKQ4 : WaveKTile<TYPE_, FM_, FN_> {
     const uint32_t lda_bytes = (uint32_t)a.lda * 2, ldb_bytes = (uint32_t)a.ldb, groups_bytes = (uint32_t)a.groups * 2;
     const int rows_w = min(BN, a.N - pn * BN);
     const uint4v rsrc_a = uniform_rsrc(make_rsrc_words(a.A + (int64_t)pm * BM * a.lda, (uint32_t)min(BM, a.M - pm * BM) * lda_bytes));
-    const uint4v rsrc_w = uniform_rsrc(make_rsrc_words(reinterpret_cast<const char *>(a.B) + (int64_t)pn * BN * a.ldb, (uint32_t)rows_w * ldb_bytes));
+    // (tiled weights have whole blocks of 16 rows)
+    const uint4v rsrc_w = uniform_rsrc(make_rsrc_words(reinterpret_cast<const char *>(a.B) + (int64_t)pn * BN * a.ldb,
+                                                       (uint32_t)(TILED_ ? (rows_w + 15) & ~15 : rows_w) * ldb_bytes));
     const uint4v rsrc_s = uniform_rsrc(make_rsrc_words(a.scales + (int64_t)pn * BN * a.groups, (uint32_t)rows_w * groups_bytes));
     uint4v rsrc_z = rsrc_s;
     if constexpr (ZP) rsrc_z = uniform_rsrc(make_rsrc_words(a.zeros + (int64_t)pn * BN * a.groups, (uint32_t)rows_w * groups_bytes));
@@ -91,7 +95,9 @@ struct TileWaveKQ4 : WaveKTile<TYPE_, FM_, FN_> {
     const int row8 = lane >> 3;
     uint32_t off_a[LA], off_w[LW], off_s[LS];
     static_for<0, LA>([&](auto l) { off_a[l] = (uint32_t)(8 * l + row8) * lda_bytes + (uint32_t)((lane & 7) ^ (4 * (l & 1) + (row8 >> 1))) * 16; });
-    static_for<0, LW>([&](auto l) { off_w[l] = (uint32_t)(16 * l + (lane >> 2)) * ldb_bytes + (uint32_t)((lane & 3) ^ (lane >> 4)) * 16; });
+    static_for<0, LW>([&](auto l) {
+      off_w[l] = (uint32_t)(16 * l) * ldb_bytes + (uint32_t)(lane >> 2) * (TILED_ ? 64u : ldb_bytes) + (uint32_t)((lane & 3) ^ (lane >> 4)) * 16;
+    });
     static_for<0, LS>([&](auto l) { off_s[l] = 64 * l + lane < BN ? (uint32_t)(64 * l + lane) * groups_bytes : OOB_OFFSET; });
     const uint32_t ring = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_address(smem) + wave * RING);
     const int rot = a.M <= BM ? rotation_of(pn, n) : Base::start_of(a, pn, n);
@@ -117,7 +123,7 @@ struct TileWaveKQ4 : WaveKTile<TYPE_, FM_, FN_> {
     };
     auto issue_w = [&](auto li, const Where &q) {
       constexpr int l = decltype(li)::value;
-      if constexpr (l < LW) wavek_dma_16<l * 1024>(rsrc_w, q.slot, q.live ? off_w[l] : OOB_OFFSET, q.bytes * 64);
+      if constexpr (l < LW) wavek_dma_16<l * 1024>(rsrc_w, q.slot, q.live ? off_w[l] : OOB_OFFSET, q.bytes * (TILED_ ? 1024 : 64));
       else if constexpr (l < LW + LS) wavek_dma_2<LW * 1024 + (l - LW) * 256>(rsrc_s, q.slot, q.live ? off_s[l - LW] : OOB_OFFSET, q.bytes * 2);
       else wavek_dma_2<LW * 1024 + (l - LW) * 256>(rsrc_z, q.slot, q.live ? off_s[l - LW - LS] : OOB_OFFSET, q.bytes * 2);
     };

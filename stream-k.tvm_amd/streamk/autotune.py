@@ -147,7 +147,7 @@ def candidate_configs(M, N, K, dtype="float16", cus=None, reduce16=True, layout=
             out.extend(dict(base, schedule="basic", grid=cus, fixup=fixup) for fixup in ("reduce", "atomic"))
     if dtype != "float32" and (M > 16 or layout == "nn"):
         # tiles whose waves stream K on their own (variant 11)
-        for (bm, bn) in _WAVEK_NN if layout == "nn" else (_WAVEK_Q4 if dtype in ("q4", "q4_zp") else _WAVEK):
+        for (bm, bn) in _WAVEK_NN if layout == "nn" else (_WAVEK_Q4 if dtype.startswith("q4") else _WAVEK):
             if (bm >= 2 * M and bm > 64) or -(-M // bm) * -(-N // bn) > 3 * cus:
                 continue
             rows = -(-M // bm)   # (groups alike, as sk_make_plan makes them)

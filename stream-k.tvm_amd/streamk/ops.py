@@ -367,12 +367,13 @@ def _run_q4(A, Wq, scales, zeros, C, zero, group, tiled, config, bias, activatio
     if tuple(scales.shape) != (N, K // group) or not scales.is_contiguous():
         raise ValueError(f"scales must be contiguous [N, K/group]; got {tuple(scales.shape)}")
     _check_out(C, M, N, torch.float16)
+    name = ("q4_zp_tiled" if tiled else "q4_zp") if zeros is not None else ("q4_tiled" if tiled else "q4")
     dequantise = config == "" and not tiled and _dequantises(M, N, K, zeros is not None)
-    if M > Q4_MAX_M and not dequantise and not config.startswith("#") and \
-            (tiled or (zeros is not None and not _has_plan(config, M, N, K, "q4_zp", 2 * A.stride(0), K // 2))):
-        # The kernels for the tiled layout take at most 64 rows of A: up to 256 rows one launch per block of 64, and so do
-        # configurations that name kernels for few rows.  (Blocks of two rows and more multiply the rounded weights alike; a
-        # last block of one row takes the matrix-vector kernels and the unrounded ones.)
+    if M > Q4_MAX_M and not dequantise and not config.startswith("#") and name != "q4" and \
+            (tiled and M > 4 * Q4_MAX_M or not _has_plan(config, M, N, K, name, 2 * A.stride(0), K // 2)):
+        # Configurations that name kernels for few rows, and tiled weights where the operators' rule takes no kernel for many: up to
+        # 256 rows one launch per block of 64.  (Blocks of two rows and more multiply the rounded weights alike; a last block of
+        # one row takes the matrix-vector kernels and the unrounded ones.)
         if M <= 4 * Q4_MAX_M:
             for m0 in range(0, M, Q4_MAX_M):
                 _run_q4(A[m0:m0 + Q4_MAX_M], Wq, scales, zeros, C[m0:m0 + Q4_MAX_M], zero, group, tiled, config,
@@ -382,15 +383,15 @@ def _run_q4(A, Wq, scales, zeros, C, zero, group, tiled, config, bias, activatio
             raise ValueError("more than 256 rows of A need the row-major weights (they are dequantised once)")
         config, dequantise = "", True
     if dequantise:
-        # One pass that dequantises the weights (bit-exact device function), then the fp16 tile kernels on them.  The pass costs 26 us for 8192 x 8192 weights, under 7 % of the product from 4096 rows on, where the
-        # fused Q4 tile kernels are behind the four-wave fp16 kernel.  The buffer is kept per stream, allocated on first use;
-        # with per-group zero points it is the call's own.
+        # One pass that dequantises the weights (bit-exact device function), then the fp16 tile kernels on them.  The pass costs
+        # 26 us for 8192 x 8192 weights, under 7 % of the product from 4096 rows on, where the fused Q4 tile kernels are behind
+        # the four-wave fp16 kernel.  The buffer is kept per stream, allocated on first use; with per-group zero points it is
+        # the call's own.
         W = (_staging(N * K * 2, A.device).view(torch.float16)[:N * K].view(N, K) if zeros is None
              else torch.empty((N, K), dtype=torch.float16, device=Wq.device))
         _run_dequant_q4(Wq, scales, zeros, W, zero, group)
         _run_16bit(A, W, C, "nt", "", bias, activation, torch.float16, "float16")
         return
-    name = ("q4_zp_tiled" if tiled else "q4_zp") if zeros is not None else ("q4_tiled" if tiled else "q4")
     plan = _plan_for(config, M, N, K, name, "nt", 2 * A.stride(0), K // 2)
     if (plan.dtype in (_lib.SK_Q4_TILED, _lib.SK_Q4_ZP_TILED)) != bool(tiled):
         raise ValueError("the plan was made for the other weight layout")

@@ -101,7 +101,7 @@ _TWIN_OF = {"bfloat16": "float16", "float8_e5m2": "float8_e4m3"}
 # (variant 9) and the ones whose waves stream K on their own (variant 11) among them.  Without it a plan takes one of the
 # kernels that plans have always taken.
 OPERATOR_VARIANT = 12
-_WAVEK_DTYPES = ("float16", "bfloat16", "float8_e4m3", "float8_e5m2", "int8", "q4", "q4_zp")
+_WAVEK_DTYPES = ("float16", "bfloat16", "float8_e4m3", "float8_e5m2", "int8", "q4", "q4_zp", "q4_tiled", "q4_zp_tiled")
 # search space of the autotuner that has the former; entries carry theirs
 SEARCH_WITH_BYTE_STREAMS = 2
 

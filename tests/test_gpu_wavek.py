@@ -260,8 +260,6 @@ def test_the_operators_rule(sk):
                 assert not wavek(M, N, K, dtype, "nt"), (dtype, M, N, K)
         assert not wavek(16, 4096, 4096, dtype, "nt", variant=12)
         assert wavek(100, 760, 4096, dtype, "nt", variant=12) and wavek(100, 256, 4096, dtype, "nt", variant=12)   # few columns too
-        if dtype.startswith("q4"):   # (with zero points and few rows the bits of the tiled layout's kernels)
-            assert all(wavek(M, 200, 640, dtype, "nt", variant=12) == (dtype == "q4") for M in (33, 64))
         assert wavek(4096, 8192, 8192, dtype, "nt", variant=12) == (dtype == "q4_zp")
     # 17 to 64 rows: few columns, or more than one round of 64-wide tiles where wider ones need one; no depth of K between others is
     # an exception
@@ -286,6 +284,58 @@ def test_the_operators_rule(sk):
         assert wavek(320, 4096, 11008, dtype, "nt", variant=12) and not wavek(100, 4096, 11008, dtype, "nt", variant=12)
         assert wavek(80, 5120, 5120, dtype, "nn", variant=12) and not wavek(128, 5120, 5120, dtype, "nn", variant=12)
     assert sk.make_plan(40, 4096, 4096, "q4_zp", "nt", cus=256, use_tuned=False).kernel_id < 400
+
+
+def test_tiled_weights_take_the_plan_of_row_major_ones(sk):
+    """An operator's plan for the tiled layout of Q4 weights, wherever one for the row-major layout is of these tiles: the same tile,
+    schedule and grid."""
+    rng, seen = np.random.default_rng(48), 0
+    for dtype in ("q4", "q4_zp"):
+        for _ in range(200):
+            M, N, K = int(rng.integers(17, 257)), int(rng.integers(1, 12000)), 128 * int(rng.integers(1, 90))
+            rows = sk.make_plan(M, N, K, dtype, "nt", cus=256, use_tuned=False, variant=12)
+            if sk.kernel_name(rows.kernel_id).startswith("wavek_"):
+                tiled = sk.make_plan(M, N, K, dtype + "_tiled", "nt", cus=256, use_tuned=False, variant=12)
+                fields = ("bm", "bn", "bk", "schedule", "grid", "fixup", "raster", "streamk_tiles", "iters_per_tile", "workspace_bytes")
+                assert tiled.kernel_id == rows.kernel_id + 40 and all(getattr(tiled, f) == getattr(rows, f) for f in fields), (dtype, M, N, K)
+                seen += 1
+    assert seen > 200
+    with pytest.raises(sk.StreamKError):   # (what names no kernel for many rows has 64 of them at most)
+        sk.make_plan(65, 1024, 1024, "q4_tiled", "nt", cus=256, use_tuned=False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["q4", "q4_zp"])
+def test_tiled_weights_give_the_bits_of_row_major_ones(sk, dtype):
+    """The same call on both layouts, on values whose sums round and rows that 16 does not divide: operator calls of 17 to 256 rows
+    and every tile through whole tiles, fixed splits and both fix-ups (the accumulating one on exact sums)."""
+    import torch
+    gen = torch.Generator(device="cuda").manual_seed(49)
+    zp = dtype == "q4_zp"
+
+    def operands(M, N, K, exact=False):
+        A = torch.randint(-2, 3, (M, K), generator=gen, device="cuda").half() if exact else torch.randn(M, K, generator=gen, device="cuda").half()
+        Wq = torch.randint(0, 256, (N, K // 2), generator=gen, device="cuda", dtype=torch.uint8)
+        scales = torch.full((N, K // 128), 0.125, device="cuda").half() if exact else torch.rand(N, K // 128, generator=gen, device="cuda").half()
+        zeros = dict(zeros=torch.randint(0, 16, (N, K // 128), generator=gen, device="cuda").half()) if zp else {}
+        return (lambda **kw: sk.streamk_q4(A, Wq, scales, **zeros, **kw)), (lambda **kw: sk.streamk_q4(A, sk.tile_q4(Wq), scales, **zeros, tiled=True, **kw))
+    for M, N, K in ((17, 200, 640), (33, 3001, 1152), (64, 768, 4096), (64, 11008, 1024), (65, 775, 512), (130, 1000, 2048), (200, 260, 4096), (256, 4097, 1280)):
+        rows, tiled = operands(M, N, K)
+        name = sk.kernel_name(sk.make_plan(M, N, K, dtype, "nt", sk.plan.operator_config(M, N, K, dtype, "nt")).kernel_id)
+        if name.startswith("wavek_"):
+            assert torch.equal(rows(), tiled()), (dtype, M, N, K)
+        else:   # (the plans they take otherwise are of other kernels)
+            assert ((rows() - tiled()).float().norm() / rows().float().norm()).item() < 2e-3, (dtype, M, N, K)
+    for bm, bn in _TILES_Q4:
+        M, N, K = bm + 3, 2 * bn + 5, 2176
+        for exact, sched in ((False, dict(schedule="dp")), (False, dict(schedule="basic", grid=5, fixup="reduce")), (True, dict(schedule="basic", grid=7, fixup="atomic")), (False, dict(schedule="dp", grid=3))):
+            rows, tiled = operands(M, N, K, exact)
+            pr, pt = (sk.make_plan(M, N, K, dtype + layout, "nt", dict(sched, bm=bm, bn=bn, variant=11)) for layout in ("", "_tiled"))
+            assert torch.equal(rows(plan=pr), tiled(plan=pt)), (dtype, bm, bn, sched)
+    rows, tiled = operands(300, 256, 256)
+    with pytest.raises(ValueError):
+        tiled()
+    sk.workspace_status()
 
 
 def test_groups_of_rows_are_alike(sk):
