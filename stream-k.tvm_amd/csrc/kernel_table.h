@@ -305,7 +305,9 @@ struct KernelInfo {
   X(382, 128, 128, 64, 2, 2, 2, 6, 4, false)    \
   X(383, 128, 128, 64, 2, 2, 2, 6, 4, true)
 
-// Tiles whose waves stream K on their own (tile_wavek.h; variant 10), every one for each type; ids from 400 + 20 type on
+// Tiles whose waves stream K on their own (tile_wavek.h; variant 10), every one for each type; ids from 400 + 20 type on.
+// (128 x 32 and 128 x 48, and 128 x 32 of [K, N] weights: the operators' rule takes them for one in 6000 random sizes at most, 64-row
+// tiles being ahead; they stand for plans that name them, a search's among them)
 // (types: WaveKType):  X(type, id, blocks of 16 rows of A, of 16 weight rows)
 #define SK_TILE_WAVEK_KERNELS(X, T, BASE) \
   X(T, BASE + 0, 2, 2) \

@@ -751,8 +751,7 @@ static double q4_tile_us(int64_t M, int64_t N, int64_t K, int num_cus) {
 // Whether a problem whose tile, variant, schedule and grid are open goes to them: wavek's times against those of the kernel that it
 // takes otherwise (`other`, its plan), with the weights from the cache and from HBM; a call must win by both, because its caller's
 // other weights decide which it is.  The margins cover the models' errors.  On 6 400 measured sizes the choice takes 1.1 % longer than the
-// faster of the two on average, and 46 are behind by more than 3 % in either, by 16 % at most; on 1 050 others 14, by 15 % at most but for one (277 x 1792 x 15616 of bf16, 39.6 us there and 53.0 here
-// from the cache).
+// faster of the two on average, and 46 are behind by more than 3 % in either, by 16 % at most; on 1 050 others 14, by 15 % at most.
 static bool wavek_pays(const sk_plan &other, int num_cus, const Times &wavek) {
   const KernelInfo *k = kernel_by_id(other.kernel_id);
   if (!k) return false;

@@ -12,19 +12,16 @@
 //  * When the segment ends every wave puts its sums into its own ring and every thread adds the four waves' values of its share
 //    of the tile: pieces of 16 bytes along the rows of C, whose stores fill whole lines.
 //
-// What bounds it: a CU takes 75 to 85 GB/s of operands (its direct loads alone 107, profiles/lds_direct_load_rate.md), whether
-// they come through LDS or registers (a variant that loads to registers and writes the chunk to LDS: 77 to 80 GB/s), and what
-// passes before and behind the loop.  So it serves what fits one or two rounds of tiles.  Without the
-// interleaving of reads and refills 64 x 64 tiles took 18.3 us at 256 x 4096 x 4096, with it 16.9; every XCD walks K from a start of
-// its own (start_of), because all CTAs of one share A as well as the weights (a start per column of tiles: 2048 x 1024 x 4096 45 us,
-// so 28).
-// Weights from HBM and the Infinity Cache in turn (three sets of operands), the kernels before / these, in us: fp16
-// 128 x 4096 x 4096 17.7 / 12.9, 256 x 4096 x 4096 22.0 / 17.0, 64 x 4096 x 4096 14.0 / 9.9, 128 x 2048 x 2048 13.0 / 6.6,
-// 1024 x 1024 x 8192 32.6 / 26.0 (eager), bf16 100 x 11008 x 4096 with bias and GELU 34.6 / 28.1 (eager); int8 100 x 4096 x 4096
-// 13.1 / 8.9, 128 x 8192 x 8192 21.6 / 17.0; fp8 256 x 1024 x 8192 24.9 / 10.2, 64 x 28672 x 8192 with bias and SiLU 57.0 / 51.3 (eager).
-// Those figures are of a first form: with preloaded arguments (wavek_launch.h), one barrier in the sums over the waves in place of
-// five, stores of 16 bytes in place of 8 and the bias fetched ahead the three eager ones take 24.1, 26.0 and 48.0, and 300
-// sizes of 33 to 512 rows 3.5 % less on average, the smallest 0.5 to 1 us.
+// What bounds it: a CU takes in 60 to 100 GB/s of operands (bf16 100 x 11008 x 4096 60, fp16 256 x 4096 x 4096 88, 1024 x 1024 x 8192
+// 100; its direct loads alone 107, profiles/lds_direct_load_rate.md), through LDS or through registers alike, and 3 to 4 us pass
+// before and behind the loop.  So it serves what fits one or two rounds of tiles.  Every XCD walks K from a start of its own
+// (start_of), because all CTAs of one share A as well as the weights (a start per column of tiles: 2048 x 1024 x 4096 45 us, so 28).
+// Graphs of launches, the kernels that such calls took before / these, in us, with three sets of operands in turn and with 600 MB of
+// weights in rotation, which come from HBM: fp16 64 x 4096 x 4096 13.5 / 8.5 and 14.9 / 11.7, 128 x 2048 x 2048 13.0 / 5.6 and
+// 13.8 / 6.9, 128 x 4096 x 4096 19.0 / 11.8 and 19.4 / 15.2, 256 x 4096 x 4096 21.4 / 15.9 and 28.4 / 19.3, 1024 x 1024 x 8192
+// 32.9 / 26.8 and 38.8 / 30.5, 80 x 8192 x 8192 41.2 / 32.8 and 39.4 / 32.7; bf16 100 x 11008 x 4096 with bias and GELU 35.1 / 26.5
+// and 36.1 / 27.8; int8 100 x 4096 x 4096 12.6 / 7.3 and 16.9 / 8.7, 128 x 8192 x 8192 21.5 / 16.0 and 30.0 / 21.3; fp8
+// 100 x 512 x 8192 17.4 / 7.9 and 25.0 / 8.8, 256 x 1024 x 8192 24.7 / 8.6 and 40.2 / 10.7.
 #pragma once
 #include <type_traits>
 

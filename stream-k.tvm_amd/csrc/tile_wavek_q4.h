@@ -8,13 +8,13 @@
 //  * The fragments of a half are read beside the MFMAs of the first step of the half before, their place is refilled beside those of
 //    the second; beside a block's MFMAs stands the decode of the next block.
 //
-// What bounds it: with few rows the 75 to 85 GB/s of A and nibbles that a CU takes (tile_wavek.h), with 64 rows and more the
-// decode -- 17 vector instructions per fragment of 16 x 32 weights, whose FM MFMAs are four issue slots each.  128 x 64 and 64 x 128 tiles
+// What bounds it: with few rows what a CU takes in of A and nibbles (tile_wavek.h), with 64 rows and more the decode -- 17 vector
+// instructions per fragment of 16 x 32 weights, whose FM MFMAs are four issue slots each.  128 x 64 and 64 x 128 tiles
 // are not built: two fragment buffers beside 128 accumulators make the compiler move registers in the loop (512 x 4096 x 4096 42 and
-// 57 us, 30 on 64 x 64 tiles).  Three sets of operands in turn, the kernels before (up to 64 rows tile_skinny.h, beyond the decode
-// into LDS of tile_f16_dma.h, with per-group zero points launches of 64 rows) / these, in us: 64 x 4096 x 4096 16.2 / 10.0,
-// 64 x 8192 x 8192 25.7 / 19.4, 128 x 4096 x 4096 24.1 / 13.0, 128 x 8192 x 8192 42 / 27.5, 256 x 4096 x 4096 28.3 / 17.0; with zero
-// points 128 x 4096 x 4096 32.6 / 13.3, 256 x 4096 x 4096 63 / 17.5.
+// 57 us, 30 on 64 x 64 tiles).  The kernels before (up to 64 rows tile_skinny.h, beyond the decode into LDS of tile_f16_dma.h) /
+// these, in us, three sets of operands in turn and from HBM: 64 x 4096 x 4096 15.7 / 8.5 and 15.9 / 9.6, 64 x 8192 x 8192 26.2 / 18.7
+// and 26.6 / 22.8, 128 x 4096 x 4096 25.5 / 11.3 and 25.9 / 12.6, 128 x 8192 x 8192 42.1 / 27.1 and 41.8 / 29.5, 256 x 4096 x 4096
+// 27.3 / 15.6 and 28.5 / 16.4.
 #pragma once
 #include "q4_dequant.h"
 #include "tile_wavek.h"
