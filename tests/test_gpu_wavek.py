@@ -338,6 +338,19 @@ def test_tiled_weights_give_the_bits_of_row_major_ones(sk, dtype):
     sk.workspace_status()
 
 
+def test_whole_tiles_get_a_cta_each(sk):
+    """Fewer tiles than CUs and nothing split: as many CTAs as tiles, for few tiles too."""
+    for dtype, step in (("float16", 8), ("float8_e4m3", 16), ("int8", 16), ("q4", 128)):
+        for M, bm, bn in ((18, 32, 32), (40, 32, 32), (40, 64, 32), (100, 64, 64), (100, 128, 32)):
+            for tiles in range(1, 65):
+                for K in (step * (512 // step), 2304, 2560, 3072, 4096, 16384):
+                    plan = sk.make_plan(M, tiles * bn - 5, K, dtype, "nt", dict(bm=bm, bn=bn, variant=11, schedule="dp"), cus=256)
+                    assert plan.grid == min(plan.total_tiles, 256), (dtype, M, bm, bn, tiles, K, plan.grid)
+    for shape in ((18, 264, 3072), (21, 312, 2560), (35, 272, 2304)):
+        plan = sk.make_plan(*shape, "float8_e4m3", "nt", cus=256, use_tuned=False, variant=12)
+        assert plan.grid >= plan.total_tiles, shape
+
+
 def test_groups_of_rows_are_alike(sk):
     """More than eight rows of tiles stand in groups of eight at most that differ by less than one row a group; other kernels and
     rasters of the caller's as they were."""
