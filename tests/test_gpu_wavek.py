@@ -284,6 +284,10 @@ def test_the_operators_rule(sk):
         assert wavek(320, 4096, 11008, dtype, "nt", variant=12) and not wavek(100, 4096, 11008, dtype, "nt", variant=12)
         assert wavek(80, 5120, 5120, dtype, "nn", variant=12) and not wavek(128, 5120, 5120, dtype, "nn", variant=12)
     assert sk.make_plan(40, 4096, 4096, "q4_zp", "nt", cus=256, use_tuned=False).kernel_id < 400
+    # zero points with a long K, and large products that the two models put close to each other: 1.13 to 1.4 times as long
+    for shape, dtype in (((23, 10144, 14720), "q4_zp"), ((22, 9360, 12288), "q4_zp"), ((534, 24608, 9056), "int8"), ((307, 10656, 11072), "int8"), ((906, 2912, 8432), "float16")):
+        assert not wavek(*shape, dtype, "nt", variant=12), (dtype, shape)
+    assert wavek(48, 4096, 11008, "q4_zp", "nt", variant=12) and wavek(209, 5696, 15376, "float8_e4m3", "nt", variant=12)
 
 
 def test_tiled_weights_take_the_plan_of_row_major_ones(sk):
